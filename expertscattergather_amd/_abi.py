@@ -115,6 +115,24 @@ def pycall():
     return _pycall
 
 
+_torch_ext = False       # False: not looked for yet; None: not available
+
+
+def torch_ext():
+    """The CPython module that runs the launchers and autograd Functions on torch tensors in C++ (csrc/egs_torch.cpp), or
+    None when it has not been built or the integer calls are switched off: callers then take the Python route."""
+    global _torch_ext
+    if _torch_ext is False:
+        with _lock:
+            if _torch_ext is False:
+                try:
+                    from . import _egs_torch as mod
+                    _torch_ext = mod if mod.abi_version() == ABI_VERSION else None
+                except ImportError:
+                    _torch_ext = None
+    return None if _pycall is None else _torch_ext
+
+
 class launch_log:
     """``with launch_log() as log: ...`` - afterwards ``log.kernels`` lists the kernels the calls of this thread
     launched inside the block (include/egs_hip_testing.h)."""

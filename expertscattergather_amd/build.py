@@ -59,6 +59,7 @@ def build(verbose: bool = False, extra_flags=()) -> str:
         list(pool.map(lambda c: _run(c, verbose), cmds))
     _run([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", LIB_PATH], verbose)
     build_pycall(verbose)
+    build_torch_ext(verbose)
     return LIB_PATH
 
 
@@ -73,6 +74,25 @@ def build_pycall(verbose: bool = False) -> str:
            "-L", HERE, "-legs_hip", "-Wl,-rpath,$ORIGIN", "-o", PYCALL_PATH]
     _run(cmd, verbose)
     return PYCALL_PATH
+
+
+TORCH_EXT_PATH = os.path.join(HERE, "_egs_torch" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
+
+
+def build_torch_ext(verbose: bool = False) -> str:
+    """Compile the CPython module that runs the launchers and autograd Functions on torch tensors (host code only)."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    cxx = os.environ.get("CXX", "g++")
+    lib_dir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    inc = [arg for path in (*include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"],
+                            os.path.join(os.path.dirname(HERE), "include")) for arg in ("-isystem" if "site" in path or "dist" in path else "-I", path)]
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc, os.path.join(CSRC, "egs_torch.cpp"),
+           "-L", HERE, "-legs_hip", "-L", lib_dir, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN",
+           "-o", TORCH_EXT_PATH]
+    _run(cmd, verbose)
+    return TORCH_EXT_PATH
 
 
 if __name__ == "__main__":

@@ -490,11 +490,19 @@ def _scatter_backward_impl(Y, W, Ind, grad_X, dtype):
     return (grad_Y if y_dtype is ct else grad_Y.to(y_dtype)), (grad_W if w_dtype is ct else grad_W.to(w_dtype))
 
 
-# module globals, bound by create_kernels() (reference egs/triton_kernels.py:26-29)
-expert_gather_forward_call = None
-expert_gather_backward_call = None
-expert_scatter_forward_call = None
-expert_scatter_backward_call = None
+# The module globals expert_{gather,scatter}_{forward,backward}_call are bound by create_kernels() (reference
+# egs/triton_kernels.py:26-29), at the latest when one of them is first asked for.
+_CALLABLES = ("expert_gather_forward_call", "expert_gather_backward_call", "expert_scatter_forward_call", "expert_scatter_backward_call")
+
+
+def __getattr__(name):
+    if name in _CALLABLES:
+        create_kernels()
+        return globals()[name]
+    raise AttributeError(f"module {__name__!r} has no attribute {name!r}")
+
+
+_created = False
 _create_lock = threading.Lock()
 
 
@@ -580,10 +588,11 @@ def create_kernels() -> None:
     threads."""
     global expert_gather_forward_call, expert_gather_backward_call
     global expert_scatter_forward_call, expert_scatter_backward_call
-    if expert_scatter_backward_call is not None:
+    global _created
+    if _created:
         return
     with _create_lock:
-        if expert_scatter_backward_call is not None:
+        if _created:
             return
         _register_ops(OP_NAMESPACE)
         ops = getattr(torch.ops, OP_NAMESPACE)
@@ -592,33 +601,42 @@ def create_kernels() -> None:
 
         # The callables the Functions use.  Like the reference's (plain Python functions, egs/triton_kernels.py:569-578)
         # they run the launcher directly for tensors on the GPU in eager mode, which saves the dispatcher's
-        # round trip per call (several microseconds, more than some of the kernels take); while torch.compile is
-        # tracing, and for meta / fake tensors, they go through the registered ops, whose fake implementations
-        # describe the outputs.
+        # round trip per call (several microseconds, more than some of the kernels take): in C++ for the operands that
+        # csrc/egs_torch.cpp takes, else in Python.  While torch.compile is tracing, and for meta / fake tensors, they go
+        # through the registered ops, whose fake implementations describe the outputs.
         def gather_forward_call(X, W, Ind, out_dtype):
             if type(X) in plain and X.is_cuda and not compiling():
-                return _gather_forward_impl(X, W, Ind, out_dtype)
+                ext = _abi.torch_ext()
+                Y = None if ext is None else ext.gather_forward(X, W, Ind, out_dtype, 0, _table_cache, False)
+                return _gather_forward_impl(X, W, Ind, out_dtype) if Y is None else Y
             return ops.expert_gather_forward_call_fn(X, W, Ind, out_dtype)
 
         def gather_backward_call(X, W, Ind, grad_output, out_dtype):
             if type(X) in plain and X.is_cuda and not compiling():
-                return _gather_backward_impl(X, W, Ind, grad_output, out_dtype)
+                ext = _abi.torch_ext()
+                g = None if ext is None else ext.gather_backward(X, W, Ind, grad_output, out_dtype, _MODES[get_scatter_mode()], _table_cache)
+                return _gather_backward_impl(X, W, Ind, grad_output, out_dtype) if g is None else g
             return ops.expert_gather_backward_call_fn(X, W, Ind, grad_output, out_dtype)
 
         def scatter_forward_call(Y, W, Ind, T, out_dtype):
             if type(Y) in plain and Y.is_cuda and not compiling():
-                return _scatter_forward_impl(Y, W, Ind, T, out_dtype)
+                ext = _abi.torch_ext()
+                out = None if ext is None else ext.scatter_forward(Y, W, Ind, T, out_dtype, _MODES[get_scatter_mode()], _table_cache, False)
+                return _scatter_forward_impl(Y, W, Ind, T, out_dtype) if out is None else out
             return ops.expert_scatter_forward_call_fn(Y, W, Ind, T, out_dtype)
 
         def scatter_backward_call(Y, W, Ind, grad_X, out_dtype):
             if type(Y) in plain and Y.is_cuda and not compiling():
-                return _scatter_backward_impl(Y, W, Ind, grad_X, out_dtype)
+                ext = _abi.torch_ext()
+                g = None if ext is None else ext.scatter_backward(Y, W, Ind, grad_X, out_dtype)
+                return _scatter_backward_impl(Y, W, Ind, grad_X, out_dtype) if g is None else g
             return ops.expert_scatter_backward_call_fn(Y, W, Ind, grad_X, out_dtype)
 
         expert_gather_forward_call = gather_forward_call
         expert_gather_backward_call = gather_backward_call
         expert_scatter_forward_call = scatter_forward_call
         expert_scatter_backward_call = scatter_backward_call
+        _created = True
 
 
 def register_reference_namespace(ns: str = "mylib") -> None:
@@ -678,6 +696,37 @@ class ExpertScatterFunction(torch.autograd.Function):
         # one gradient per forward input: (Y, W, Ind, T) or (Y, W, Ind, T, out_type).  The reference returns four
         # (egs/triton_kernels.py:639), which autograd rejects when out_type is passed explicitly.
         return (grad_Y, grad_W) + (None,) * (len(ctx.needs_input_grad) - 2)
+
+
+def expert_gather(X: torch.Tensor, W: torch.Tensor, Ind: torch.Tensor, scatter_mode=None) -> torch.Tensor:
+    """What `ExpertGather` computes: `ExpertGatherFunction.apply(X, W, Ind)` with `scatter_mode` (None: the mode in force) for
+    the backward, as one C++ autograd node (csrc/egs_torch.cpp) where the operands allow it."""
+    if not torch.compiler.is_compiling():
+        ext = _abi.torch_ext()
+        if ext is not None:
+            mode = get_scatter_mode() if scatter_mode is None else _check_mode(scatter_mode)
+            Y = ext.gather_forward(X, W, Ind, torch.float32, _MODES[mode], _table_cache, True)
+            if Y is not None:
+                return Y
+    if scatter_mode is None:
+        return ExpertGatherFunction.apply(X, W, Ind)
+    with scatter_mode_scope(scatter_mode):          # bound to the autograd node: the backward runs in it too
+        return ExpertGatherFunction.apply(X, W, Ind)
+
+
+def expert_scatter(Y: torch.Tensor, W: torch.Tensor, Ind: torch.Tensor, T: int, scatter_mode=None) -> torch.Tensor:
+    """What `ExpertScatter` computes: `ExpertScatterFunction.apply(Y, W, Ind, T)` in `scatter_mode`, see `expert_gather`."""
+    if not torch.compiler.is_compiling():
+        ext = _abi.torch_ext()
+        if ext is not None:
+            mode = get_scatter_mode() if scatter_mode is None else _check_mode(scatter_mode)
+            out = ext.scatter_forward(Y, W, Ind, T, torch.float32, _MODES[mode], _table_cache, True)
+            if out is not None:
+                return out
+    if scatter_mode is None:
+        return ExpertScatterFunction.apply(Y, W, Ind, T)
+    with scatter_mode_scope(scatter_mode):
+        return ExpertScatterFunction.apply(Y, W, Ind, T)
 
 
 # ------------------------------------------------------------------------------ extras (not in the reference)

@@ -8,7 +8,7 @@ import math
 import torch
 from torch import nn
 
-from .hip_kernels import ExpertGatherFunction, ExpertScatterFunction, create_kernels, scatter_mode_scope
+from .hip_kernels import create_kernels, expert_gather, expert_scatter
 
 
 class ExpertGather(nn.Module):
@@ -41,11 +41,7 @@ class ExpertGather(nn.Module):
 
     def forward(self, x: torch.Tensor, Ind: torch.Tensor):
         """x: [B,T,I];  Ind: integers in [0,T) of shape [B,E,K]  ->  [B,E,K,J]."""
-        if self.scatter_mode is None:
-            y = ExpertGatherFunction.apply(x, self.W, Ind)
-        else:
-            with scatter_mode_scope(self.scatter_mode):     # bound to the autograd node: the backward runs in it too
-                y = ExpertGatherFunction.apply(x, self.W, Ind)
+        y = expert_gather(x, self.W, Ind, self.scatter_mode)
         if self.bias is not None:
             y = y + self.bias
         return y
@@ -84,11 +80,7 @@ class ExpertScatter(nn.Module):
 
     def forward(self, Y: torch.Tensor, Ind: torch.Tensor, T: int):
         """Y: [B,E,K,J];  Ind: [B,E,K] in [0,T);  T: output sequence length  ->  [B,T,I]."""
-        if self.scatter_mode is None:
-            y = ExpertScatterFunction.apply(Y, self.W, Ind, T)
-        else:
-            with scatter_mode_scope(self.scatter_mode):
-                y = ExpertScatterFunction.apply(Y, self.W, Ind, T)
+        y = expert_scatter(Y, self.W, Ind, T, self.scatter_mode)
         if self.bias is not None and T > 0 and Ind.numel() > 0:
             # picks[b,t,e] = how many times expert e selected token t; each adds bias[e]
             # (a pick outside [0,T) contributes nothing, as in the kernels: it is routed to slot 0 with weight 0)

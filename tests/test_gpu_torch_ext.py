@@ -1,0 +1,93 @@
+"""The C++ route of the launchers and autograd Functions (csrc/egs_torch.cpp) against the Python route: same bits for what it
+takes, and what it does not take goes to the Python route."""
+import pytest
+import torch
+
+from tests._util import make_case
+
+pytestmark = pytest.mark.gpu
+
+import expertscattergather_amd as egs
+from expertscattergather_amd import _abi
+from expertscattergather_amd import hip_kernels as hk
+
+DEV = "cuda"
+SHAPES = [(4, 64, 8, 16, 128, 64),       # one-kernel scatter with a routing table
+          (1, 1, 1, 1, 1, 1),
+          (3, 37, 5, 11, 29, 13),        # product rows through the workspace, odd sizes
+          (2, 300, 4, 200, 256, 192)]
+
+
+def step(case, dtype, ind, grad_of, mode):
+    B, T, E, K, I, J = case["shape"]
+    g, s = egs.ExpertGather(E, I, J).to(DEV, dtype), egs.ExpertScatter(E, J, I).to(DEV, dtype)
+    with torch.no_grad():
+        g.W.copy_(case["Wg"]); s.W.copy_(case["Ws"])
+    g.scatter_mode = s.scatter_mode = mode
+    x = case["X"].to(DEV).requires_grad_(True)
+    out = s(g(x, ind), ind, T)
+    out.backward(grad_of(out))
+    torch.cuda.synchronize()
+    return out.detach(), x.grad, g.W.grad, s.W.grad
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("grad", ["dense", "expanded", "sliced"])
+def test_the_two_routes_agree(shape, dtype, grad, monkeypatch):
+    B, T, E, K, I, J = shape
+    case = dict(make_case(5 + sum(shape), *shape, dtype), shape=shape)
+    wide = torch.randn(B, T, I + 24, device=DEV).to(dtype)
+    grad_of = {"dense": lambda out: case["dOut"].to(DEV), "expanded": lambda out: torch.ones((), device=DEV, dtype=dtype).expand(out.shape),
+               "sliced": lambda out: wide[..., 8:8 + I]}[grad]
+    ind_dtype = torch.int16 if dtype is torch.float16 else torch.int64
+    mode = "compact" if grad == "sliced" else None
+    Ind = case["Ind"].to(ind_dtype)
+    assert _abi.torch_ext() is not None
+    fast = step(case, dtype, Ind.to(DEV), grad_of, mode)
+    monkeypatch.setattr(_abi, "_pycall", None)
+    assert _abi.torch_ext() is None
+    slow = step(case, dtype, Ind.to(DEV), grad_of, mode)
+    for name, a, b in zip(("out", "dX", "dWg", "dWs"), fast, slow):
+        assert torch.equal(a, b), name
+
+
+def test_autograd_contract_of_the_native_nodes():
+    shape = B, T, E, K, I, J = 4, 64, 8, 16, 128, 64
+    case = make_case(9, *shape, torch.bfloat16)
+    x, W, Ind = case["X"].to(DEV).requires_grad_(True), case["Wg"].to(DEV), case["Ind"].to(DEV)
+    y = hk.expert_gather(x, W, Ind)
+    assert "Native" in y.grad_fn.name() and not hk.expert_gather(x.detach(), W, Ind).requires_grad
+    with torch.no_grad():
+        assert not hk.expert_gather(x, W, Ind).requires_grad
+    y.sum().backward()                                  # W needs no gradient: only x gets one
+    assert x.grad is not None and W.grad is None
+    with pytest.raises(RuntimeError, match="second time"):
+        y.sum().backward()
+    y = hk.expert_gather(x, W, Ind)
+    Ind[0, 0, 0] = (Ind[0, 0, 0] + 1) % T               # a saved tensor written in place is noticed
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.sum().backward()
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t, lambda t: t):
+        y = hk.expert_gather(x, W, Ind)
+    assert len(packed) >= 3
+    y.sum().backward()
+
+
+def test_what_the_native_route_declines_goes_the_python_way():
+    shape = B, T, E, K, I, J = 2, 40, 4, 8, 64, 32
+    case = make_case(11, *shape, torch.float32)
+    X, W, Ind = case["X"].to(DEV), case["Wg"].to(DEV), case["Ind"].to(DEV)
+    ext = _abi.torch_ext()
+    call = lambda x, w, i, t=torch.float32: ext.gather_forward(x, w, i, t, 0, False, False)
+    assert call(X, W, Ind) is not None
+    off = torch.empty(X.numel() + 1, device=DEV)[1:].view_as(X).copy_(X)
+    for args in [(X.transpose(0, 1).contiguous().transpose(0, 1), W, Ind), (off, W, Ind), (X.bfloat16(), W, Ind), (X.cpu(), W, Ind),
+                 (X, W, Ind.float()), (X, W, Ind, torch.bfloat16), (X[:0], W, Ind[:0]), (X, W[:3], Ind)]:
+        assert call(*args) is None
+    assert torch.equal(hk.expert_gather(off, W, Ind), hk.expert_gather(X, W, Ind))
+    with pytest.raises(ValueError):
+        hk.expert_gather(X, W[:3], Ind)
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(Exception):      # no forward-mode derivative, on either route
+        hk.expert_gather(torch.autograd.forward_ad.make_dual(X, torch.ones_like(X)), W, Ind)
