@@ -15,13 +15,13 @@
 // (rejected picks, the ragged end of a split) get an offset outside the buffer descriptor and
 // arrive as zeros.
 //
-// Preconditions (checked by the host, which otherwise uses dw_kernel): 16-bit elements,
+// Preconditions (checked by the host, which otherwise uses tiled_dw_kernel): 16-bit elements,
 // I % 8 == 0, J % 8 == 0, 16-byte aligned rows, operands below 2 GiB.
 //
 // Replaces the reference's expert_gather_scatter_dW_kernel (egs/triton_kernels.py:261-356) on
 // these shapes.
 #pragma once
-#include "egs_dw.h"
+#include "egs_device.h"
 #include "egs_rows_gemm_dl.h"
 #include "egs_small.h"
 
@@ -30,8 +30,21 @@ namespace egs {
 constexpr int kDlThreads = 512;      // 8 wavefronts
 constexpr int kDwChunkRows = 1024;   // three-stage form: reduction rows whose offsets are staged in LDS at a time
 
+struct DwParams {
+    const char *Xs;         // [B,T,I] strided source (gathered through Ind)
+    const char *Ys;         // [B,E,K,J] dense
+    const void *Ind;
+    float *part;            // S > 1: [S] fp32 partial sums in the output's layout
+    char *dW;               // final output when S == 1
+    int32_t B, T, E, K, I, J;
+    int64_t ldx_b, ldx_t;
+    int32_t ind_dtype;
+    int32_t i_tiles, j_tiles;      // 256-row and BQ-column tiles
+    int32_t S, rows_per_split;     // rows_per_split is a multiple of the slab depth
+    int32_t out_dtype, dw_layout;  // used when S == 1
+};
 struct DwDlParams {
-    DwParams d;               // i_tiles / j_tiles count 256-row and BQ-column tiles here
+    DwParams d;
     uint32_t x_bytes, y_bytes;
 };
 

@@ -1,4 +1,4 @@
-// Launch side of the tiled weight gradient: dw_kernel, or dw_dl_kernel for large well-formed 16-bit
+// Launch side of the tiled weight gradient: tiled_dw_kernel, or dw_dl_kernel for large well-formed 16-bit
 // shapes, followed by the fixed-order sum over splits.
 #include "egs_host.h"
 #include "egs_dw_dl.h"
@@ -19,10 +19,6 @@ int dw_general(const void *Xs, const void *Ys, const void *Ind, void *dW, void *
     p.B = d->B; p.T = d->T; p.E = d->E; p.K = d->K; p.I = d->I; p.J = d->J;
     p.ldx_b = ldx_b; p.ldx_t = ldx_t;
     p.ind_dtype = ind_dtype;
-    p.x_vec = aligned_to(Xs, 16) && (ldx_b * ES) % 16 == 0 && (ldx_t * ES) % 16 == 0;
-    p.y_vec = aligned_to(Ys, 16) && ((int64_t)d->J * ES) % 16 == 0;
-    p.o_vec = aligned_to(dW, 16) && d->J % 4 == 0;
-    p.i_tiles = pl.i_tiles; p.j_tiles = pl.j_tiles; p.S = pl.S; p.rows_per_split = pl.rows_per_split;
     p.out_dtype = out_dtype; p.dw_layout = dw_layout;
     const uint64_t x_span = d->B > 0 && d->T > 0
         ? ((uint64_t)(d->B - 1) * (uint64_t)ldx_b + (uint64_t)(d->T - 1) * (uint64_t)ldx_t + (uint64_t)d->I) * ES : 0;
@@ -51,19 +47,20 @@ int dw_general(const void *Xs, const void *Ys, const void *Ind, void *dW, void *
         }
         return EGS_OK;
     }
-    const int64_t grid = (int64_t)8 * ceil_div(d->E, 8) * pl.i_tiles * pl.j_tiles * pl.S;
-    if (grid > INT32_MAX) return EGS_ERR_BAD_SHAPE;
-    switch (act_dtype) {
-    case EGS_F32: hipLaunchKernelGGL((dw_kernel<ElemF32, 128, 64, 32>), dim3((unsigned)grid), dim3(kThreads), 0, s, p); break;
-    case EGS_F16: hipLaunchKernelGGL((dw_kernel<ElemF16, 128, 64, 64>), dim3((unsigned)grid), dim3(kThreads), 0, s, p); break;
-    default: hipLaunchKernelGGL((dw_kernel<ElemBF16, 128, 64, 64>), dim3((unsigned)grid), dim3(kThreads), 0, s, p); break;
-    }
-    EGS_CHECK_LAUNCH("dw_kernel");
-    if (pl.S > 1) {
-        hipLaunchKernelGGL(dw_reduce_kernel, dim3(grid_1d(w_elems, 4096)), dim3(kThreads), 0, s, (const float *)workspace,
-                           (char *)dW, pl.S, d->E, d->I, d->J, out_dtype, dw_layout);
-        EGS_CHECK_LAUNCH("dw_reduce_kernel");
-    }
+    TiledDwParams q;
+    memset(&q, 0, sizeof(q));
+    q.Xs = p.Xs; q.Ys = p.Ys; q.Ind = Ind; q.dW = pl.S > 1 ? (char *)workspace : (char *)dW;
+    q.x_bytes = (int64_t)x_span; q.y_bytes = (int64_t)y_span;
+    q.ldx_b = ldx_b; q.ldx_t = ldx_t;
+    q.B = d->B; q.T = d->T; q.E = d->E; q.K = d->K; q.I = d->I; q.J = d->J;
+    q.ind_dtype = ind_dtype; q.out_dtype = out_dtype; q.eji = dw_layout != 0;
+    q.i_tiles = pl.i_tiles; q.j_tiles = pl.j_tiles; q.S = pl.S; q.picks_per_split = pl.picks_per_split;
+    q.edges = (d->I * ES) % 16 != 0 || (d->J * ES) % 16 != 0;
+    const int rc = act_dtype == EGS_F32 ? tiled_dw_f32(q, s) : act_dtype == EGS_F16 ? tiled_dw_f16(q, s) : tiled_dw_bf16(q, s);
+    if (rc != EGS_OK || pl.S <= 1) return rc;
+    hipLaunchKernelGGL(tiled_dw_sum_kernel, dim3(grid_1d((w_elems + 3) / 4, 4096)), dim3(kThreads), 0, s, (const float *)workspace,
+                       (char *)dW, pl.S, (int64_t)w_elems, out_dtype);
+    EGS_CHECK_LAUNCH("tiled_dw_sum_kernel");
     return EGS_OK;
 }
 

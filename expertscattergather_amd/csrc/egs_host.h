@@ -11,7 +11,8 @@
 #include "../../include/egs_hip.h"
 #include "egs_device.h"
 #include "egs_rows_gemm.h"
-#include "egs_dw.h"
+#include "egs_tiled.h"
+#include "egs_token_sum.h"
 
 namespace egs {
 namespace host {
@@ -70,11 +71,14 @@ inline int grid_1d(size_t items, int cap = 8192)
     return (int)(g > (size_t)cap ? (size_t)cap : g);
 }
 
+// row stride (elements) of product rows in the workspace: whole 16-byte (fp32) or 8-byte pieces for token_sum / segment_sum
+inline int product_ld(int I) { return (I + 3) & ~3; }
+
 // LDS the counting-sort routing table needs with `nw` wavefronts per batch element
 inline size_t csr_count_lds(int T, int nw) { return ((size_t)(nw + 1) * T + 1) * 4; }
 
 struct DwPlan {
-    int BI, BJ, BK, i_tiles, j_tiles, S, rows_per_split;   // general tiled kernel
+    int i_tiles, j_tiles, S, picks_per_split;              // general tiled kernel
     bool small_ok;                                          // shape admits the small-expert kernel
     int s_i_tiles, s_j_tiles, s_S, s_rows_per_split;        // its plan
     bool big_ok;                                            // shape admits the direct-to-LDS kernel (256 x BQ tiles)
@@ -101,6 +105,15 @@ inline bool dw_big_takes(const DwPlan &pl, const void *Xs, const void *Ys, const
 int rows_gemm_gather(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans, hipStream_t s);
 // scatter products: epi = EPI_STORE / EPI_STORE_F32 (rows in pick order) or EPI_ATOMIC_F32 (fp32 atomics on the output)
 int rows_gemm_scatter(RowsGemmParams &p, int act_dtype, bool w_trans, int epi, hipStream_t s);
+
+// ---- egs_tiled_<type>.hip: tiled products and weight gradients for operands of any size and alignment
+int tiled_rows_f32(TiledRowsParams &p, bool w_trans, hipStream_t s);
+int tiled_rows_f16(TiledRowsParams &p, bool w_trans, hipStream_t s);
+int tiled_rows_bf16(TiledRowsParams &p, bool w_trans, hipStream_t s);
+int tiled_rows_fp8w(TiledRowsParams &p, bool w_trans, hipStream_t s);
+int tiled_dw_f32(TiledDwParams &p, hipStream_t s);
+int tiled_dw_f16(TiledDwParams &p, hipStream_t s);
+int tiled_dw_bf16(TiledDwParams &p, hipStream_t s);
 
 // ---- egs_pass_launch.hip: the one-kernel GEMM-scatter in passes (thousands of picks per batch element, 16-bit types)
 struct PassPlan { bool ok; int units_per_pass; size_t lds; };

@@ -139,7 +139,7 @@ ScatterPlan plan_scatter(const egs_dims *d, int mode, int act_dtype, ScatterPath
     // long segments (tokens picked more than kLongSegment times): records and fp32 partial rows
     pl.long_tab_at = at;  at += align_up((size_t)d->B * long_tab_stride((int)N) * 4, 256);
     pl.long_part_at = at; at += align_up((size_t)d->B * long_max_slots((int)N) * d->I * 4, 256);
-    pl.rows_at = at;    at += align_up((size_t)d->B * N * d->I * row_es, 256);
+    pl.rows_at = at;    at += align_up((size_t)d->B * N * product_ld(d->I) * row_es, 256);
     pl.bytes = at;
     return pl;
 }
@@ -148,23 +148,20 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
 {
     DwPlan pl;
     memset(&pl, 0, sizeof(pl));
-    pl.BI = 128; pl.BJ = 64;
-    pl.BK = act_dtype == EGS_F32 ? 32 : 64;
-    pl.i_tiles = ceil_div(d->I, pl.BI);
-    pl.j_tiles = ceil_div(d->J, pl.BJ);
+    // any shape: 32 x 64 tiles (fp32: 32 x 32), the picks split only where there are more than a workgroup's four wavefronts
+    // reduce in about the time the second pass would cost (1024) and too few tiles to fill the device
     const int64_t Me = (int64_t)d->B * d->K;
+    pl.i_tiles = ceil_div(d->I, 32);
+    pl.j_tiles = ceil_div(d->J, act_dtype == EGS_F32 ? 32 : 64);
     const int64_t base = (int64_t)d->E * pl.i_tiles * pl.j_tiles;
-    int64_t S = base > 0 ? (512 + base - 1) / base : 1;
-    const int64_t max_s = Me > 0 ? (Me + pl.BK - 1) / pl.BK : 1;
-    if (S > max_s) S = max_s;
-    if (S > 64) S = 64;
+    int64_t S = base > 0 ? 512 / base : 1;
+    if (S > (Me + 1023) / 1024) S = (Me + 1023) / 1024;
     if (S < 1) S = 1;
-    int64_t rows = Me > 0 ? (Me + S - 1) / S : pl.BK;
-    rows = (rows + pl.BK - 1) / pl.BK * pl.BK;
+    int64_t rows = Me > 0 ? ((Me + S - 1) / S + 127) / 128 * 128 : 128;
     S = Me > 0 ? (Me + rows - 1) / rows : 1;
     pl.S = (int)S;
-    pl.rows_per_split = (int)rows;
-    pl.bytes_general = S > 1 ? align_up((size_t)S * d->E * d->I * d->J * 4, 256) : 0;
+    pl.picks_per_split = (int)(rows < INT32_MAX ? rows : INT32_MAX);
+    pl.bytes_general = S > 1 ? align_up((size_t)S * d->E * d->I * d->J * 4, 256) : 256;     // never none: this path always has a workspace
 
     // large 16-bit shapes: 256 x 256 (or 256 x 128) tiles, 64-row slabs, splits only to give every CU a workgroup
     // (C4: 2 splits 42 us, 4 splits 49 us, none 50 us)
@@ -651,7 +648,7 @@ int launch_segment_sum(const void *rows, bool rows_f32, const int32_t *seg_off, 
     SegSumParams sp;
     memset(&sp, 0, sizeof(sp));
     sp.P = rows; sp.seg_off = seg_off; sp.perm = perm; sp.out = (char *)Out;
-    sp.B = d->B; sp.T = d->T; sp.N = N; sp.I = d->I;
+    sp.B = d->B; sp.T = d->T; sp.N = N; sp.I = d->I; sp.ldp = product_ld(d->I);
     while ((1 << sp.tpr_log2) < iv && sp.tpr_log2 < 8) ++sp.tpr_log2;      // threads sharing an output row (<= 256)
     sp.gx = ceil_div(d->T, kThreads >> sp.tpr_log2);
     sp.gy = d->B;
@@ -677,6 +674,36 @@ int launch_segment_sum(const void *rows, bool rows_f32, const int32_t *seg_off, 
 #undef EGS_SEGSUM
     EGS_CHECK_LAUNCH(fuse ? "segsum_dwreduce_kernel" : "segment_sum_kernel");
     if (fuse) reduce->q.S = 1;              // second pass done
+    return EGS_OK;
+}
+
+// the same without a routing table, for up to kTokenSumPicks picks per batch element
+int launch_token_sum(const void *rows, bool rows_f32, const void *Ind, int ind_dtype, void *Out, const egs_dims *d, int act_dtype, hipStream_t s)
+{
+    TokenSumParams p;
+    memset(&p, 0, sizeof(p));
+    p.P = rows; p.Ind = Ind; p.out = (char *)Out;
+    p.B = d->B; p.T = d->T; p.N = d->E * d->K; p.I = d->I; p.ldp = product_ld(d->I);
+    p.ind_dtype = ind_dtype;
+    // at most 64 threads (256 columns) per row, so that a hot token's segment has at least four groups of threads to share it
+    p.tpr_log2 = 3;
+    while ((4 << p.tpr_log2) < d->I && p.tpr_log2 < 6) ++p.tpr_log2;
+    p.c_blocks = ceil_div(d->I, 4 << p.tpr_log2);
+    // tokens per workgroup: one per group of threads, more (each workgroup reads all indices of its batch element) once that
+    // alone makes a thousand workgroups
+    const int groups = kThreads >> p.tpr_log2;
+    p.tb = groups;
+    while (p.tb < kTokenSumTokens && (int64_t)d->B * ceil_div(d->T, p.tb) * p.c_blocks > 1024) p.tb *= 2;
+    p.t_blocks = ceil_div(d->T, p.tb);
+    const int64_t grid = (int64_t)d->B * p.t_blocks * p.c_blocks;
+    if (grid > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
+    const size_t lds = token_sum_lds(p.N);
+    if (act_dtype == EGS_F32) hipLaunchKernelGGL((token_sum_kernel<ElemF32, float>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
+    else if (act_dtype == EGS_F16 && rows_f32) hipLaunchKernelGGL((token_sum_kernel<ElemF16, float>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
+    else if (act_dtype == EGS_F16) hipLaunchKernelGGL((token_sum_kernel<ElemF16, uint16_t>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
+    else if (rows_f32) hipLaunchKernelGGL((token_sum_kernel<ElemBF16, float>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
+    else hipLaunchKernelGGL((token_sum_kernel<ElemBF16, uint16_t>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
+    EGS_CHECK_LAUNCH("token_sum_kernel");
     return EGS_OK;
 }
 
@@ -1072,8 +1099,15 @@ int gemm_scatter_impl(const void *Y, const void *W, const void *Ind, void *Out, 
             p.a_bytes = span < (1ull << 31) ? (uint32_t)span : 0;
             // the routing table may ride along with the (first) product launch (large shapes); otherwise it is a
             // launch of its own
-            p.csr_blocks = (b0 == 0 && N > 0) ? d->B : 0; p.csr_done = 0;
+            const bool no_table = N >= 1 && N <= kTokenSumPicks && !(dw != nullptr && dw->done && dw->q.S > 1);
+            p.csr_blocks = (b0 == 0 && N > 0 && !no_table) ? d->B : 0; p.csr_done = 0;
             rc = rows_gemm_scatter(p, act_dtype, w_trans, rows_f32 ? EPI_STORE_F32 : EPI_STORE, s);
+            if (rc == EGS_OK && no_table) {
+                rc = launch_token_sum(rows, rows_f32, (const char *)Ind + (size_t)b0 * N * ind_size(ind_dtype), ind_dtype,
+                                      (char *)Out + (size_t)b0 * d->T * d->I * ES, &sub, act_dtype, s);
+                if (rc != EGS_OK) return rc;
+                continue;
+            }
             if (rc == EGS_OK && b0 == 0 && !p.csr_done)
                 rc = launch_routing_table(Ind, ind_dtype, d, seg_off, perm, rank_tmp, cnt, long_tab, s);
             if (rc != EGS_OK) return rc;

@@ -532,10 +532,10 @@ static __global__ __launch_bounds__(1024) void csr_sort_kernel(const void *Ind, 
 // exactly once (tokens nobody picked become zero).  P rows hold PT (float, or 16-bit values
 // of the element type TT); VW elements per thread.
 struct SegSumParams {
-    const void *P;              // product rows [B, N, I], fp32 or 16-bit
+    const void *P;              // product rows [B, N, ldp], fp32 or 16-bit
     const int32_t *seg_off, *perm;
     char *out;                  // [B, T, I]
-    int32_t B, T, N, I;
+    int32_t B, T, N, I, ldp;
     int32_t tpr_log2;           // 2^tpr_log2 threads share an output row
     int32_t gx, gy;             // logical grid: gx row groups x gy batch slots
     int32_t *long_tab;          // long-segment records (see emit_long_tokens), or nullptr
@@ -590,7 +590,7 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
             }
         };
         const int32_t *pb = perm + (size_t)b * N;
-        const PT *Pb = P + (size_t)b * N * I + (size_t)iv * VW;
+        const PT *Pb = P + (size_t)b * N * sp.ldp + (size_t)iv * VW;
         int s = s0;
         if constexpr (VW >= 4) {
             struct alignas(16) F32x8 { f32x4 lo, hi; };
@@ -619,7 +619,7 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
 #pragma unroll
                 for (int u = 0; u < LB; ++u) q[u] = pb[s + u];
 #pragma unroll
-                for (int u = 0; u < LB; ++u) v[u] = *reinterpret_cast<const vec_t *>(Pb + (size_t)q[u] * I);
+                for (int u = 0; u < LB; ++u) v[u] = *reinterpret_cast<const vec_t *>(Pb + (size_t)q[u] * sp.ldp);
 #pragma unroll
                 for (int u = 0; u < LB; ++u) add_vec(v[u]);
             }
@@ -632,13 +632,13 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
 #pragma unroll
                 for (int u = 0; u < RB; ++u) q[u] = pb[min(s + u, s1 - 1)];
 #pragma unroll
-                for (int u = 0; u < RB; ++u) v[u] = *reinterpret_cast<const vec_t *>(Pb + (size_t)q[u] * I);
+                for (int u = 0; u < RB; ++u) v[u] = *reinterpret_cast<const vec_t *>(Pb + (size_t)q[u] * sp.ldp);
 #pragma unroll
                 for (int u = 0; u < RB; ++u)
                     if (u < nb) add_vec(v[u]);
             }
         } else {
-            for (; s < s1; ++s) add_row(Pb + (size_t)pb[s] * I);
+            for (; s < s1; ++s) add_row(Pb + (size_t)pb[s] * sp.ldp);
         }
         size_t at = row * I + (size_t)iv * VW;
         if constexpr (TT::ES == 4) {
@@ -698,7 +698,7 @@ __device__ __forceinline__ void segment_sum_long_body(const SegSumParams &sp, co
     float *part = sp.long_part + ((size_t)b * slots + slot) * I;
 
     for (int iv = tid; iv < IV; iv += kThreads) {
-        const PT *Pb = P + (size_t)b * N * I + (size_t)iv * VW;
+        const PT *Pb = P + (size_t)b * N * sp.ldp + (size_t)iv * VW;
         float acc[VW];
 #pragma unroll
         for (int x = 0; x < VW; ++x) acc[x] = 0.f;
@@ -717,7 +717,7 @@ __device__ __forceinline__ void segment_sum_long_body(const SegSumParams &sp, co
             for (int u = 0; u < 8; ++u) q[u] = pb[s + u];
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const PT *src = Pb + (size_t)q[u] * I;
+                const PT *src = Pb + (size_t)q[u] * sp.ldp;
                 if constexpr (VW == 4) {
                     typedef typename std::conditional<sizeof(PT) == 4, f32x4, u32x2>::type vec_t;
                     *reinterpret_cast<vec_t *>(v[u]) = *reinterpret_cast<const vec_t *>(src);
@@ -729,7 +729,7 @@ __device__ __forceinline__ void segment_sum_long_body(const SegSumParams &sp, co
             for (int u = 0; u < 8; ++u) add_elems(v[u]);
         }
         for (; s < s1; ++s) {
-            const PT *src = Pb + (size_t)pb[s] * I;
+            const PT *src = Pb + (size_t)pb[s] * sp.ldp;
             PT v[VW];
 #pragma unroll
             for (int x = 0; x < VW; ++x) v[x] = src[x];

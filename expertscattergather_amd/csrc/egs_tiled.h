@@ -1,0 +1,690 @@
+// Tiled rows x weight products and weight gradients for operands of ANY size and alignment: odd row lengths, views that
+// start anywhere, few picks, few experts.  The specialised kernels (egs_small*.h, egs_rows_gemm_dl.h, egs_dw_tile.h,
+// egs_dw_dl.h) take the shapes they are made for; everything else runs here.
+//
+// What such calls are bound by is not arithmetic but the chain  index -> row -> LDS -> matrix instruction  and the number of
+// workgroups: a 95 x 65 expert with 74 picks is one 128 x 128 tile, and the kernel this replaces walked its three 32-deep
+// slabs one memory round trip after the other, reading rows that do not start on 16 bytes element by element.  Hence:
+//   * every operand is read 16 bytes at a time wherever a row starts (global memory takes any alignment); the one chunk per
+//     tensor that would reach past its end is read a little earlier and shifted, row tails are masked in the last slab;
+//   * up to four slabs are requested before the first is used, and the LDS tile is double-buffered: one barrier per slab;
+//   * tiles come in 64 or 128 rows x 32 .. 128 columns, so that a ragged width wastes little and a small problem still has
+//     many workgroups; workgroups are dealt to the XCDs evenly for any number of experts.
+#pragma once
+#include "egs_device.h"
+
+namespace egs {
+
+typedef u32x4 u32x4_any __attribute__((aligned(1)));        // 16 bytes at any address (global memory)
+typedef u32x2 u32x2_any __attribute__((aligned(1)));
+typedef f32x4 f32x4_any __attribute__((aligned(1)));
+
+// 128-bit logical right shift by 8 * bytes, 0 <= bytes < 16
+__device__ __forceinline__ u32x4 shift_right_bytes(const u32x4 &v, int bytes)
+{
+    uint64_t lo = (uint64_t)v[0] | ((uint64_t)v[1] << 32), hi = (uint64_t)v[2] | ((uint64_t)v[3] << 32);
+    if (bytes >= 8) { lo = hi; hi = 0; }
+    const int s = 8 * (bytes & 7);
+    if (s != 0) { lo = (lo >> s) | (hi << (64 - s)); hi >>= s; }
+    return u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+
+// Workgroup -> linear tile number: XCD x (workgroups are dealt to the eight XCDs in turn) takes the x-th eighth of `total`
+// consecutive tiles, so neighbours in the numbering share an L2 and no XCD gets more than one tile more than another.
+__device__ __forceinline__ int balanced_tile(int bid, int total)
+{
+    const int per = (total + 7) >> 3;
+    const int t = (bid & 7) * per + (bid >> 3);
+    return (bid >> 3) < per && t < total ? t : -1;
+}
+
+struct TiledRowsParams {
+    const char *A;              // gather: [B,T,R] source; else dense [B,E,K,R] rows
+    const char *W;              // [E,R,N] (W_TRANS) or [E,N,R]
+    const void *Ind;            // gather only
+    char *C;                    // [B,E,K,ldc] rows, element type or fp32
+    const float *w_scale;       // [E,N] or nullptr
+    int64_t a_bytes, w_bytes;   // extents of A and W, at least 16
+    int64_t lda_b, lda_t;       // element strides of the source (gather)
+    int32_t B, T, E, K, R, N, ldc;
+    int32_t ind_dtype, gather, out_f32;
+    int32_t m_tiles, n_tiles;
+    int32_t rows_major;         // numbering of the tiles: 1 = row tiles outermost (their source rows share an L2), 0 = experts outermost
+};
+
+// bytes of LDS: two stages of A and W tiles
+template <class TT, bool W_TRANS, int TM, int TN>
+struct TiledLds {
+    static constexpr int CH = 8, BKE = CH * TT::VEC;            // 128-byte row pieces per slab
+    static constexpr int A = 64 * TM * CH * 16;
+    // [reduction][column] weight tiles.  16-bit: an odd number of 32-byte units per row and 128 more bytes every eight rows, so
+    // that the 16 row pieces of a transpose read fall two deep on every bank; fp32: rows 4 banks apart modulo 16
+    static constexpr int WROW = TT::ES == 2 ? 32 * (TN | 1) : (16 * TN + 4) * 4;
+    static constexpr int W = W_TRANS ? (TT::ES == 2 ? BKE * WROW + (BKE / 8) * 128 : BKE * WROW) : 16 * TN * CH * 16;
+    static constexpr int STAGE = A + W;
+    static constexpr int BYTES = 2 * STAGE;
+};
+
+// 64 * TM rows x 16 * TN columns per workgroup of four wavefronts, each 16 * TM rows x all columns.
+template <class TT, int WES, bool W_TRANS, int TM, int TN>
+__global__ __launch_bounds__(kThreads) void tiled_rows_kernel(TiledRowsParams p)
+{
+    constexpr int ES = TT::ES, VEC = TT::VEC;
+    constexpr bool W_FP8 = WES == 1;
+    typedef TiledLds<TT, W_TRANS, TM, TN> L;
+    constexpr int CH = L::CH, BKE = L::BKE, KSTEPS = CH / 4;
+    constexpr int BM = 64 * TM, BN = 16 * TN;
+    constexpr int NA = BM * CH / kThreads;                              // A chunks per thread and slab
+    // W chunks (16 source bytes) per slab: W_TRANS rows of BN columns, else BN rows of CH chunks (fp8: half as many)
+    constexpr int WPR = W_TRANS ? BN * WES / 16 : CH * WES / ES;        // chunks per source row
+    constexpr int WCH = WPR * (W_TRANS ? BKE : BN);
+    constexpr int NW = (WCH + kThreads - 1) / kThreads;
+    constexpr int D = NA + NW <= 5 ? 4 : 2;                             // slabs in flight in registers
+    extern __shared__ __attribute__((aligned(16))) char smem_tiled[];
+
+    const int total = p.E * p.m_tiles * p.n_tiles;
+    const int lin = balanced_tile((int)blockIdx.x, total);
+    if (lin < 0) return;
+    int e, mt, nt;
+    if (p.rows_major) { mt = lin / (p.E * p.n_tiles); const int r = lin - mt * p.E * p.n_tiles; e = r / p.n_tiles; nt = r - e * p.n_tiles; }
+    else { e = lin / (p.m_tiles * p.n_tiles); const int r = lin - e * p.m_tiles * p.n_tiles; mt = r / p.n_tiles; nt = r - mt * p.n_tiles; }
+    const int m0 = mt * BM, n0 = nt * BN;
+    const int tid = (int)threadIdx.x;
+    const int R = p.R, N = p.N, Me = p.B * p.K;
+    const int nk = (R + BKE - 1) / BKE;
+
+    // ---------------- this thread's rows of A (chunk tid % CH of rows tid / CH + i * (256 / CH)); the index words travel first
+    const int ac = tid % CH;
+    int64_t apick[NA];
+    uint64_t iw[NA];
+    int ab[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        const int m = min(m0 + tid / CH + i * (kThreads / CH), Me - 1);
+        ab[i] = m / p.K;
+        apick[i] = ((int64_t)ab[i] * p.E + e) * p.K + (m - ab[i] * p.K);
+        iw[i] = 0;
+    }
+    if (p.gather) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) iw[i] = load_index_word(p.Ind, p.ind_dtype, apick[i]);
+    }
+
+    // ---------------- weight side
+    const char *We = p.W + (int64_t)e * R * N * WES;
+    const char *w_last = p.W + p.w_bytes - 16;
+    u32x4 wreg[D][NW];
+    auto w_at = [&](int kt, int i) -> const char * {                    // address of chunk i of slab kt, before the clamp
+        const int v = min(tid + i * kThreads, WCH - 1);
+        if constexpr (W_TRANS) {
+            const int r = min(kt * BKE + v / WPR, R - 1);
+            int n = n0 + (v % WPR) * (16 / WES);
+            if (n >= N) n = n0;
+            return We + ((int64_t)r * N + n) * WES;
+        } else {
+            const int n = min(n0 + v / WPR, N - 1);
+            int k = kt * BKE + (v % WPR) * (16 / WES);
+            if (k >= R) k = 0;
+            return We + ((int64_t)n * R + k) * WES;
+        }
+    };
+    auto issue_w = [&](int kt, u32x4 (&set)[NW]) {
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            const char *at = w_at(kt, i);
+            set[i] = *reinterpret_cast<const u32x4_any *>(at < w_last ? at : w_last);
+        }
+    };
+    // the same chunks in A
+    const char *arow[NA];
+    int alive = 0;
+    const char *a_last = p.A + p.a_bytes - 16;
+    u32x4 areg[D][NA];
+    auto a_at = [&](int kt, int i) -> const char * {
+        int k = kt * BKE + ac * VEC;
+        if (k >= R) k = 0;
+        return arow[i] + (int64_t)k * ES;
+    };
+    auto issue_a = [&](int kt, u32x4 (&set)[NA]) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const char *at = a_at(kt, i);
+            set[i] = *reinterpret_cast<const u32x4_any *>(at < a_last ? at : a_last);
+        }
+    };
+
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (d < nk) issue_w(d, wreg[d]);
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        const int m = m0 + tid / CH + i * (kThreads / CH);
+        if (p.gather) {
+            const int64_t t = decode_index_word(iw[i], p.Ind, p.ind_dtype, apick[i]);
+            const bool ok = m < Me && t >= 0 && t < (int64_t)p.T;
+            arow[i] = p.A + (ok ? ((int64_t)ab[i] * p.lda_b + t * p.lda_t) * ES : 0);
+            alive |= (int)ok << i;
+        } else {
+            arow[i] = p.A + apick[i] * R * ES;
+            alive |= (int)(m < Me) << i;
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (d < nk) issue_a(d, areg[d]);
+
+    // ---------------- registers -> LDS.  `edge` (the last slab, and every slab of a matrix whose rows are shorter than a chunk):
+    // chunks that were read early are shifted into place and what lies past the reduction length is cleared on both sides
+    const bool short_rows = (int64_t)N * WES < 16;
+    auto commit_a = [&](const u32x4 (&set)[NA], int kt, char *stage) {
+        u32x4 *tile = reinterpret_cast<u32x4 *>(stage);
+        const bool edge = kt >= nk - 1;
+        const int left = (R - kt * BKE - ac * VEC) * ES;                // valid bytes of this thread's chunk
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            u32x4 v = set[i];
+            if (edge) {
+                const char *at = a_at(kt, i);
+                if (at > a_last) v = shift_right_bytes(v, (int)(at - a_last));
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const int nb = left - 4 * x;
+                    v[x] &= nb >= 4 ? 0xffffffffu : nb == 2 ? 0xffffu : 0u;
+                }
+            }
+            if (!((alive >> i) & 1)) v = u32x4{0u, 0u, 0u, 0u};
+            tile[tile_chunk_index<CH>(tid / CH + i * (kThreads / CH), ac)] = v;
+        }
+    };
+    auto w_off = [&](int r, int col_bytes) -> int {                     // byte offset in a [reduction][column] tile
+        return ES == 2 ? r * L::WROW + (r >> 3) * 128 + col_bytes : r * L::WROW + col_bytes;
+    };
+    auto commit_w = [&](const u32x4 (&set)[NW], int kt, char *stage) {
+        char *tile = stage + L::A;
+        const bool edge = kt >= nk - 1 || (W_TRANS && short_rows);
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            const int v = tid + i * kThreads;
+            if (WCH % kThreads != 0 && v >= WCH) continue;
+            u32x4 w = set[i];
+            if (edge) {
+                const char *at = w_at(kt, i);
+                if (at > w_last) w = shift_right_bytes(w, (int)(at - w_last));
+                if constexpr (W_TRANS) {
+                    if (kt * BKE + v / WPR >= R) w = u32x4{0u, 0u, 0u, 0u};
+                } else {
+                    const int left = (R - kt * BKE - (v % WPR) * (16 / WES)) * WES;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) {
+                        const int nb = left - 4 * x;
+                        w[x] &= nb >= 4 ? 0xffffffffu : nb <= 0 ? 0u : 0xffffffffu >> (32 - 8 * nb);
+                    }
+                }
+            }
+            if constexpr (W_TRANS) {
+                const int r = v / WPR, cb = (v % WPR) * (W_FP8 ? 32 : 16);
+                if constexpr (W_FP8) {
+                    *reinterpret_cast<u32x4 *>(tile + w_off(r, cb)) = fp8x8_to_bf16_chunk(w[0], w[1]);
+                    *reinterpret_cast<u32x4 *>(tile + w_off(r, cb) + 16) = fp8x8_to_bf16_chunk(w[2], w[3]);
+                } else {
+                    *reinterpret_cast<u32x4 *>(tile + w_off(r, cb)) = w;
+                }
+            } else {
+                u32x4 *t4 = reinterpret_cast<u32x4 *>(tile);
+                const int n = v / WPR, c = v % WPR;
+                if constexpr (W_FP8) {
+                    t4[tile_chunk_index<CH>(n, 2 * c)] = fp8x8_to_bf16_chunk(w[0], w[1]);
+                    t4[tile_chunk_index<CH>(n, 2 * c + 1)] = fp8x8_to_bf16_chunk(w[2], w[3]);
+                } else {
+                    t4[tile_chunk_index<CH>(n, c)] = w;
+                }
+            }
+        }
+    };
+
+    // ---------------- LDS -> matrix instructions
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int a = lane & 15, g = lane >> 4;
+    const int wave_m0 = wave * 16 * TM;
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](const char *stage) {
+        const u32x4 *ta = reinterpret_cast<const u32x4 *>(stage);
+        const char *tw = stage + L::A;
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+            u32x4 mf[TM], nf[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) mf[i] = ta[tile_chunk_index<CH>(wave_m0 + i * 16 + a, ks * 4 + g)];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                if constexpr (!W_TRANS) {
+                    nf[j] = reinterpret_cast<const u32x4 *>(tw)[tile_chunk_index<CH>(j * 16 + a, ks * 4 + g)];
+                } else if constexpr (ES == 2) {
+                    // transpose reads: lane (a, g) points at reduction row 32 ks + 8 g + 4 h + a / 4, columns 4 (a % 4) .. + 3
+                    const char *at = tw + w_off(ks * 32 + g * 8 + (a >> 2), j * 32 + (a & 3) * 8);
+                    const u32x2 lo = lds_read_tr16(at), hi = lds_read_tr16(at + 4 * L::WROW);
+                    nf[j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        nf[j][c] = *reinterpret_cast<const uint32_t *>(tw + w_off(ks * 16 + g * 4 + c, (j * 16 + a) * 4));
+                }
+            }
+            if constexpr (ES == 2) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) mma_chunk<TT>(acc[i][j], nf[j], mf[i]);
+            } else {            // accumulators in turn: an fp32 matrix instruction then never waits for the one before it
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int j = 0; j < TN; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bits_f32(nf[j][c]), bits_f32(mf[i][c]), acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+    // One barrier per slab: a wavefront that writes slab kt + 1 has passed slab kt's barrier, before which every wavefront had
+    // finished with slab kt - 1, the stage's previous content.  The steady state issues unconditionally, so that the compiler can
+    // count the outstanding loads and waits for one slab's only.
+    static_assert(D % 2 == 0, "stage parity is static");
+    int kt = 0;
+    for (; kt + 2 * D <= nk; kt += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            char *stage = smem_tiled + (d & 1) * L::STAGE;
+            commit_a(areg[d], kt + d, stage);
+            commit_w(wreg[d], kt + d, stage);
+            issue_a(kt + d + D, areg[d]);
+            issue_w(kt + d + D, wreg[d]);
+            __syncthreads();
+            compute(stage);
+        }
+    }
+    for (; kt < nk; kt += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            if (kt + d < nk) {
+                char *stage = smem_tiled + (d & 1) * L::STAGE;
+                commit_a(areg[d], kt + d, stage);
+                commit_w(wreg[d], kt + d, stage);
+                if (kt + d + D < nk) { issue_a(kt + d + D, areg[d]); issue_w(kt + d + D, wreg[d]); }
+                __syncthreads();
+                compute(stage);
+            }
+        }
+    }
+
+    // ---------------- results: lane (a, g) holds columns 16 j + 4 g .. + 3 of row 16 i + a; regrouped so that adjacent lanes
+    // store adjacent pieces of a row
+    const int srow = lane >> 2, sg = lane & 3;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int m = m0 + wave_m0 + i * 16 + srow, mm = min(m, Me - 1);
+        const int b = mm / p.K;
+        const int64_t pick = ((int64_t)b * p.E + e) * p.K + (mm - b * p.K);
+        char *crow = p.C + pick * p.ldc * (p.out_f32 ? 4 : ES);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            f32x4 v = acc[i][j];
+            if (p.w_scale != nullptr) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] *= p.w_scale[(int64_t)e * N + min(n0 + j * 16 + g * 4 + r, N - 1)];
+            }
+            v = __builtin_bit_cast(f32x4, lanes_16g_a_to_4a_g(__builtin_bit_cast(u32x4, v), lane));
+            const int n = n0 + j * 16 + sg * 4;
+            if (m >= Me || n >= N) continue;
+            if (n + 4 <= N) {
+                if (ES == 4 || p.out_f32) *reinterpret_cast<f32x4_any *>(crow + (int64_t)n * 4) = v;
+                else *reinterpret_cast<u32x2_any *>(crow + (int64_t)n * 2) = u32x2{pack2<TT>(v[0], v[1]), pack2<TT>(v[2], v[3])};
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (n + r >= N) continue;
+                    if (ES == 4 || p.out_f32) reinterpret_cast<float *>(crow)[n + r] = v[r];
+                    else reinterpret_cast<uint16_t *>(crow)[n + r] = (uint16_t)f32_to_elem_bits<TT>(v[r]);
+                }
+            }
+        }
+    }
+}
+
+// Operands of less than 16 bytes: one thread per product, element by element.
+template <class TT, int WES, bool W_TRANS>
+__global__ __launch_bounds__(kThreads) void tiny_rows_kernel(TiledRowsParams p)
+{
+    const int64_t total = (int64_t)p.B * p.E * p.K * p.N;
+    auto elem = [](const char *at) -> float {
+        if constexpr (TT::ES == 4) return *reinterpret_cast<const float *>(at);
+        else return TT::ID == 2 ? bf16_bits_to_f32(*reinterpret_cast<const uint16_t *>(at)) : f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(at));
+    };
+    for (int64_t at = (int64_t)blockIdx.x * kThreads + threadIdx.x; at < total; at += (int64_t)gridDim.x * kThreads) {
+        const int64_t pick = at / p.N;
+        const int n = (int)(at - pick * p.N), e = (int)(pick / p.K % p.E);
+        const char *row = p.A + pick * p.R * TT::ES;
+        if (p.gather) {
+            const int32_t t = load_token(p.Ind, p.ind_dtype, pick, p.T);
+            row = t < 0 ? nullptr : p.A + (pick / p.K / p.E * p.lda_b + (int64_t)t * p.lda_t) * TT::ES;
+        }
+        float v = 0.f;
+        for (int r = 0; row != nullptr && r < p.R; ++r) {
+            const int64_t w = (int64_t)e * p.R * p.N + (W_TRANS ? (int64_t)r * p.N + n : (int64_t)n * p.R + r);
+            float wv;
+            if constexpr (WES == 1) wv = __builtin_amdgcn_cvt_f32_fp8((int)(uint32_t)(uint8_t)p.W[w], 0);
+            else wv = elem(p.W + w * TT::ES);
+            v += elem(row + (int64_t)r * TT::ES) * wv;
+        }
+        if (p.w_scale != nullptr) v *= p.w_scale[(int64_t)e * p.N + n];
+        if (TT::ES == 4 || p.out_f32) reinterpret_cast<float *>(p.C)[pick * p.ldc + n] = v;
+        else reinterpret_cast<uint16_t *>(p.C)[pick * p.ldc + n] = (uint16_t)f32_to_elem_bits<TT>(v);
+    }
+}
+
+// ------------------------------------------------------------------------------ weight gradient
+struct TiledDwParams {
+    const char *Xs;             // [B,T,I] rows, element strides (ldx_b, ldx_t, 1)
+    const char *Ys;             // [B,E,K,J] dense
+    const void *Ind;
+    char *dW;                   // [E,I,J] or [E,J,I] in out_dtype; S > 1: fp32 [S] of them, in the same layout
+    int64_t x_bytes, y_bytes;   // extents, at least 16
+    int64_t ldx_b, ldx_t;
+    int32_t B, T, E, K, I, J;
+    int32_t ind_dtype, out_dtype, eji;
+    int32_t i_tiles, j_tiles, S, picks_per_split;
+    int32_t edges;              // some row is not a whole number of chunks: chunks may have to be read early and shifted
+};
+// what a pick that does not exist reads instead of a row
+static __device__ const u32x4 kZeroChunk = {0u, 0u, 0u, 0u};
+
+template <class TT>
+struct TiledDw {
+    static constexpr int ES = TT::ES, TI = 32, TJ = ES == 2 ? 64 : 32;
+    static constexpr int XB = TI * ES, YB = TJ * ES;                    // bytes of a pick's piece
+    static constexpr int XS = ES == 2 ? XB : 192, YS = ES == 2 ? YB : 192;      // strides in the staging tile (fp32: padded)
+    static constexpr int STAGE = 32 * (XS + YS);                        // one step of 32 picks
+    static constexpr int TAB = 2 * 64 * 16;                             // byte offsets of both rows of two chunks of 64 picks
+    static constexpr int RS = TJ + 4;                                   // floats per row of the exchange tile
+    static constexpr int EXCHANGE = TI * RS * 4;
+    static constexpr int PER_WAVE = (TAB + STAGE > EXCHANGE ? TAB + STAGE : EXCHANGE);
+    static constexpr int BYTES = 4 * PER_WAVE;
+};
+
+// A workgroup owns a 32 x TJ tile of dW(e) for one split of the expert's picks; its four wavefronts take consecutive parts of
+// them, two 32-pick steps of rows in flight each, and are summed through LDS in wavefront order (as in egs_dw_tile.h, whose
+// swizzles the 16-bit staging tiles use; there the operands are aligned and read through buffer descriptors).
+template <class TT>
+__global__ __launch_bounds__(kThreads) void tiled_dw_kernel(TiledDwParams p)
+{
+    typedef TiledDw<TT> L;
+    constexpr int ES = TT::ES, VEC = TT::VEC, TJ = L::TJ, NWV = kThreads / 64;
+    constexpr int XL = L::XB / 16, XN = 32 * XL / 64, YL = L::YB / 16, YN = 32 * YL / 64;
+    constexpr int NY = TJ / 16;
+    extern __shared__ __attribute__((aligned(16))) char smem_tiled_dw[];
+
+    const int per_e = p.i_tiles * p.j_tiles * p.S;
+    const int lin = balanced_tile((int)blockIdx.x, p.E * per_e);
+    if (lin < 0) return;
+    const int e = lin / per_e;
+    int rest = lin - e * per_e;
+    const int split = rest / (p.i_tiles * p.j_tiles);
+    rest -= split * (p.i_tiles * p.j_tiles);
+    const int i0 = (rest / p.j_tiles) * L::TI, j0 = (rest % p.j_tiles) * TJ;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int a = lane & 15, g = lane >> 4;
+    const int Me = p.B * p.K;
+    const int lo = split * p.picks_per_split, hi = min(Me, lo + p.picks_per_split);
+    const int per_wave = ((hi - lo + NWV - 1) / NWV + 31) & ~31;
+    const int w_begin = min(hi, lo + wave * per_wave), w_end = min(hi, w_begin + per_wave);
+    const int nsteps = (w_end - w_begin + 31) >> 5;
+
+    char *mine = smem_tiled_dw + wave * L::PER_WAVE;
+    int64_t *tab = reinterpret_cast<int64_t *>(mine);                   // [2][x: 64 | y: 64], -1: no such pick
+    char *stage = mine + L::TAB;
+
+    const int xp = lane / XL, xcn = lane % XL, yp = lane / YL, ycn = lane % YL;
+    const int xc = i0 + xcn * VEC, yc = j0 + ycn * VEC;
+    const bool x_in = xc < p.I, y_in = yc < p.J;
+    const int64_t x_last = p.x_bytes - 16, y_last = p.y_bytes - 16;
+
+    uint64_t iw = 0;
+    auto pick_of = [&](int c, int &m, int &b) -> int64_t {
+        m = w_begin + c * 64 + lane;
+        const int mm = min(m, Me - 1);
+        b = mm / p.K;
+        return ((int64_t)b * p.E + e) * p.K + (mm - b * p.K);
+    };
+    auto load_idx = [&](int c) { int m, b; iw = load_index_word(p.Ind, p.ind_dtype, pick_of(c, m, b)); };
+    auto store_tab = [&](int c) {
+        int m, b;
+        const int64_t pick = pick_of(c, m, b);
+        const int64_t t = decode_index_word(iw, p.Ind, p.ind_dtype, pick);
+        const bool live = m < w_end && t >= 0 && t < (int64_t)p.T;
+        int64_t *at = tab + (c & 1) * 128;
+        at[lane] = live ? ((int64_t)b * p.ldx_b + t * p.ldx_t) * ES : -1;
+        at[64 + lane] = live ? pick * p.J * ES : -1;
+    };
+    u32x4 rx[2][XN], ry[2][YN];
+    int sx[2][XN], sy[2][YN];                                           // bytes by which a chunk was read early
+    auto fetch = [&](const char *base, int64_t off, int col, bool in, int64_t last, int &early) -> u32x4 {
+        // an offset from `base` in every case (also to the zeros): the compiler then knows the load is a global one
+        int64_t at = off + (int64_t)col * ES;
+        early = 0;
+        if (p.edges && off >= 0 && at > last) { early = (int)(at - last); at = last; }
+        if (off < 0 || !in) { at = reinterpret_cast<const char *>(&kZeroChunk) - base; early = 0; }
+        return *reinterpret_cast<const u32x4_any *>(base + at);
+    };
+    auto issue = [&](int s, u32x4 (&x)[XN], u32x4 (&y)[YN], int (&ex)[XN], int (&ey)[YN]) {
+        const int64_t *at = tab + ((s >> 1) & 1) * 128 + (s & 1) * 32;
+#pragma unroll
+        for (int h = 0; h < XN; ++h) x[h] = fetch(p.Xs, at[h * (64 / XL) + xp], xc, x_in, x_last, ex[h]);
+#pragma unroll
+        for (int h = 0; h < YN; ++h) y[h] = fetch(p.Ys, at[64 + h * (64 / YL) + yp], yc, y_in, y_last, ey[h]);
+    };
+    // see dw_tile_body for the 16-bit swizzles
+    const int fr = a >> 2;
+    const int xkey = ((fr >> 1) & 1) ^ (g & 1), ykey = (fr & 3) ^ g;
+    const int at0 = ES == 2 ? (g * 8 + fr) * 64 + (a & 3) * 8 : g * L::XS + a * 4, at1 = at0 + 4 * 64;
+    const int yat0 = ES == 2 ? (g * 8 + fr) * 128 + (a & 3) * 8 : g * L::YS + a * 4, yat1 = yat0 + 4 * 128;
+    const int wr = ES == 2 ? xp * 64 + (((xcn >> 1) ^ ((xp >> 1) & 1) ^ ((xp >> 3) & 1)) << 5) + (xcn & 1) * 16 : xp * L::XS + xcn * 16;
+    const int ywr = ES == 2 ? yp * 128 + (((ycn >> 1) ^ (yp & 3)) << 5) + (ycn & 1) * 16 : yp * L::YS + ycn * 16;
+    constexpr int XT = 32 * L::XS;
+    auto put = [&](u32x4 (&x)[XN], u32x4 (&y)[YN], const int (&ex)[XN], const int (&ey)[YN]) {
+        if (p.edges) {
+            int any = 0;
+#pragma unroll
+            for (int h = 0; h < XN; ++h) any |= ex[h];
+#pragma unroll
+            for (int h = 0; h < YN; ++h) any |= ey[h];
+            if (__any(any)) {
+#pragma unroll
+                for (int h = 0; h < XN; ++h) x[h] = shift_right_bytes(x[h], ex[h]);
+#pragma unroll
+                for (int h = 0; h < YN; ++h) y[h] = shift_right_bytes(y[h], ey[h]);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < XN; ++h) *reinterpret_cast<u32x4 *>(stage + h * (64 / XL) * L::XS + wr) = x[h];
+#pragma unroll
+        for (int h = 0; h < YN; ++h)
+            *reinterpret_cast<u32x4 *>(stage + XT + h * (64 / YL) * L::YS + (ES == 2 ? ywr ^ ((h & 3) << 5) : ywr)) = y[h];
+    };
+    struct Frag16 { u32x4 v; };
+    struct Frag32 { float v[8]; };
+    typedef typename std::conditional<ES == 2, Frag16, Frag32>::type Frag;
+    f32x4 acc[2][NY];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < NY; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto get = [&](Frag (&pf)[2], Frag (&qf)[NY]) {
+        if constexpr (ES == 2) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                const u32x2 l = lds_read_tr16(stage + at0 + ((x ^ xkey) << 5)), h = lds_read_tr16(stage + at1 + ((x ^ xkey) << 5));
+                pf[x].v = u32x4{l[0], l[1], h[0], h[1]};
+            }
+#pragma unroll
+            for (int y = 0; y < NY; ++y) {
+                const u32x2 l = lds_read_tr16(stage + XT + yat0 + ((y ^ ykey) << 5)), h = lds_read_tr16(stage + XT + yat1 + ((y ^ ykey) << 5));
+                qf[y].v = u32x4{l[0], l[1], h[0], h[1]};
+            }
+        } else {
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) pf[x].v[k] = *reinterpret_cast<const float *>(stage + at0 + k * 4 * L::XS + x * 64);
+#pragma unroll
+            for (int y = 0; y < NY; ++y)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) qf[y].v[k] = *reinterpret_cast<const float *>(stage + XT + yat0 + k * 4 * L::YS + y * 64);
+        }
+    };
+    auto multiply = [&](const Frag (&pf)[2], const Frag (&qf)[NY]) {
+        if constexpr (ES == 2) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < NY; ++y) mma_chunk<TT>(acc[x][y], qf[y].v, pf[x].v);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+#pragma unroll
+                    for (int y = 0; y < NY; ++y)
+                        acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[y].v[k], pf[x].v[k], acc[x][y], 0, 0, 0);
+        }
+    };
+    // Steps beyond the last read kZeroChunk; nothing in the loop is conditional on them, so the loads in flight stay countable.
+    // Step s: its fragments out of the staging tile, step s + 1's rows into it (a wavefront's LDS accesses happen in order, so one
+    // tile is enough), step s + 3's rows requested, then the matrix instructions of step s.
+    if (nsteps > 0) {
+        load_idx(0); store_tab(0);
+        load_idx(1);
+        issue(0, rx[0], ry[0], sx[0], sy[0]);
+        issue(1, rx[1], ry[1], sx[1], sy[1]);
+        store_tab(1);
+        load_idx(2);
+        put(rx[0], ry[0], sx[0], sy[0]);
+        issue(2, rx[0], ry[0], sx[0], sy[0]);
+        for (int s = 0; s < nsteps; s += 2) {
+            Frag pf[2], qf[NY];
+            get(pf, qf);
+            __builtin_amdgcn_sched_barrier(0);
+            put(rx[1], ry[1], sx[1], sy[1]);
+            issue(s + 3, rx[1], ry[1], sx[1], sy[1]);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(pf, qf);
+            get(pf, qf);
+            __builtin_amdgcn_sched_barrier(0);
+            put(rx[0], ry[0], sx[0], sy[0]);
+            store_tab((s >> 1) + 2);
+            load_idx((s >> 1) + 3);
+            issue(s + 4, rx[0], ry[0], sx[0], sy[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(pf, qf);
+        }
+    }
+    __syncthreads();
+
+    // lane (a, g) holds rows i0 + 16 x + a, columns j0 + 16 y + 4 g .. + 3 of its wavefront's share
+    float *red = reinterpret_cast<float *>(smem_tiled_dw);
+    constexpr int RS = L::RS, PW = L::PER_WAVE / 4;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < NY; ++y)
+            *reinterpret_cast<f32x4 *>(red + wave * PW + (x * 16 + a) * RS + y * 16 + g * 4) = acc[x][y];
+    __syncthreads();
+    const bool eji = p.eji != 0;
+    const int out_dtype = p.S > 1 ? 0 : p.out_dtype;
+    const int64_t base = p.S > 1 ? (int64_t)split * p.E * p.I * p.J : 0;
+    for (int item = tid; item < 8 * TJ; item += kThreads) {
+        const int gi_l = eji ? item & 31 : item / (TJ / 4), gj_l = (eji ? item >> 5 : item % (TJ / 4)) * 4;
+        f32x4 v = *reinterpret_cast<const f32x4 *>(red + gi_l * RS + gj_l);
+#pragma unroll
+        for (int w = 1; w < NWV; ++w) {
+            const f32x4 u = *reinterpret_cast<const f32x4 *>(red + w * PW + gi_l * RS + gj_l);
+            v[0] += u[0]; v[1] += u[1]; v[2] += u[2]; v[3] += u[3];
+        }
+        const int gi = i0 + gi_l, gj = j0 + gj_l;
+        if (gi >= p.I || gj >= p.J) continue;
+        if (!eji && gj + 4 <= p.J) {
+            const int64_t at = base + ((int64_t)e * p.I + gi) * p.J + gj;
+            if (out_dtype == 0) *reinterpret_cast<f32x4_any *>(p.dW + at * 4) = v;
+            else if (out_dtype == 1) *reinterpret_cast<u32x2_any *>(p.dW + at * 2) = u32x2{pack2<ElemF16>(v[0], v[1]), pack2<ElemF16>(v[2], v[3])};
+            else *reinterpret_cast<u32x2_any *>(p.dW + at * 2) = u32x2{pack2<ElemBF16>(v[0], v[1]), pack2<ElemBF16>(v[2], v[3])};
+        } else {
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                if (gj + x >= p.J) continue;
+                const int64_t at = base + (eji ? ((int64_t)e * p.J + gj + x) * p.I + gi : ((int64_t)e * p.I + gi) * p.J + gj + x);
+                if (out_dtype == 0) reinterpret_cast<float *>(p.dW)[at] = v[x];
+                else reinterpret_cast<uint16_t *>(p.dW)[at] =
+                         (uint16_t)((out_dtype == 1 ? pack2<ElemF16>(v[x], 0.f) : pack2<ElemBF16>(v[x], 0.f)) & 0xffffu);
+            }
+        }
+    }
+}
+
+// sums of S fp32 parts of n elements in increasing order, rounded once
+static __global__ __launch_bounds__(kThreads) void tiled_dw_sum_kernel(const float *part, char *dW, int S, int64_t n, int out_dtype)
+{
+    const int64_t n4 = (n + 3) / 4;
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n4; i += (int64_t)gridDim.x * kThreads) {
+        const int64_t at = i * 4 + 4 <= n ? i * 4 : n >= 4 ? n - 4 : 0;      // the last thread redoes a few sums rather than go element by element
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        const int live = n >= 4 ? 4 : (int)n;
+        for (int s = 0; s < S; ++s) {
+            const float *src = part + (int64_t)s * n + at;
+            if (live == 4) { const f32x4 u = *reinterpret_cast<const f32x4_any *>(src); v[0] += u[0]; v[1] += u[1]; v[2] += u[2]; v[3] += u[3]; }
+            else for (int x = 0; x < live; ++x) v[x] += src[x];
+        }
+        if (live == 4) {
+            if (out_dtype == 0) *reinterpret_cast<f32x4_any *>(dW + at * 4) = v;
+            else if (out_dtype == 1) *reinterpret_cast<u32x2_any *>(dW + at * 2) = u32x2{pack2<ElemF16>(v[0], v[1]), pack2<ElemF16>(v[2], v[3])};
+            else *reinterpret_cast<u32x2_any *>(dW + at * 2) = u32x2{pack2<ElemBF16>(v[0], v[1]), pack2<ElemBF16>(v[2], v[3])};
+        } else {
+            for (int x = 0; x < live; ++x) {
+                if (out_dtype == 0) reinterpret_cast<float *>(dW)[at + x] = v[x];
+                else reinterpret_cast<uint16_t *>(dW)[at + x] =
+                         (uint16_t)((out_dtype == 1 ? pack2<ElemF16>(v[x], 0.f) : pack2<ElemBF16>(v[x], 0.f)) & 0xffffu);
+            }
+        }
+    }
+}
+
+// Operands of less than 16 bytes: one thread per element of dW, pick by pick.
+template <class TT>
+__global__ __launch_bounds__(kThreads) void tiny_dw_kernel(TiledDwParams p)
+{
+    auto elem = [](const char *at) -> float {
+        if constexpr (TT::ES == 4) return *reinterpret_cast<const float *>(at);
+        else return TT::ID == 2 ? bf16_bits_to_f32(*reinterpret_cast<const uint16_t *>(at)) : f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(at));
+    };
+    const int64_t total = (int64_t)p.E * p.I * p.J;
+    for (int64_t w = (int64_t)blockIdx.x * kThreads + threadIdx.x; w < total; w += (int64_t)gridDim.x * kThreads) {
+        const int e = (int)(w / ((int64_t)p.I * p.J));
+        const int64_t ij = w - (int64_t)e * p.I * p.J;
+        const int i = (int)(p.eji ? ij % p.I : ij / p.J), j = (int)(p.eji ? ij / p.I : ij % p.J);
+        float v = 0.f;
+        for (int m = 0; m < p.B * p.K; ++m) {
+            const int b = m / p.K;
+            const int64_t pick = ((int64_t)b * p.E + e) * p.K + (m - b * p.K);
+            const int32_t t = load_token(p.Ind, p.ind_dtype, pick, p.T);
+            if (t < 0) continue;
+            v += elem(p.Xs + ((int64_t)b * p.ldx_b + (int64_t)t * p.ldx_t + i) * TT::ES) * elem(p.Ys + (pick * p.J + j) * TT::ES);
+        }
+        if (p.out_dtype == 0) reinterpret_cast<float *>(p.dW)[w] = v;
+        else reinterpret_cast<uint16_t *>(p.dW)[w] =
+                 (uint16_t)((p.out_dtype == 1 ? pack2<ElemF16>(v, 0.f) : pack2<ElemBF16>(v, 0.f)) & 0xffffu);
+    }
+}
+
+}  // namespace egs

@@ -1,0 +1,211 @@
+// Second half of the GEMM-scatter with product rows in memory, without a routing table: every workgroup finds the picks of its
+// own few tokens in Ind, puts them in order and adds their product rows up.
+//
+//   out[b,t,:] = sum of P[b,q,:] over the picks q of batch element b with Ind[b,q] = t, in increasing q
+//
+// With the table built by a launch of its own (csr_count_kernel, 5 .. 15 us for a few hundred picks: one workgroup per batch
+// element, a chain of phases) the table took as long as the sums.  Up to kTokenSumPicks picks per batch element it is cheaper
+// that each workgroup reads all of the batch element's indices - a few KB out of the L2, all in flight at once - keeps those
+// of its tokens, and sorts what is left, of which there is little.  The order of the additions is the order of the picks
+// (tokens with more than kTokenSumHot of them: in contiguous shares, added in order), a function of Ind alone:
+// bitwise reproducible.
+#pragma once
+#include "egs_device.h"
+
+namespace egs {
+
+constexpr int kTokenSumPicks = 4096;        // most picks per batch element
+constexpr int kTokenSumTokens = 32;         // most tokens per workgroup
+constexpr int kTokenSumHot = 64;            // longer segments are shared by the whole workgroup
+
+struct TokenSumParams {
+    const void *P;              // product rows [B, N, ldp], fp32 or the 16-bit element type
+    const void *Ind;            // [B, N]
+    char *out;                  // [B, T, I]
+    int32_t B, T, N, I, ldp;
+    int32_t ind_dtype;
+    int32_t tb;                 // tokens per workgroup
+    int32_t tpr_log2;           // 2^tpr_log2 threads share a row (4 columns each)
+    int32_t t_blocks, c_blocks; // workgroups per batch element: token blocks x column blocks of 4 << tpr_log2 columns
+};
+
+// bytes of LDS: picks of the workgroup's tokens as found, and in order; counters of four wavefronts
+__host__ __device__ inline size_t token_sum_lds(int N)
+{
+    const size_t list = (size_t)4 * (((N + 3) / 4 + 63) / 64 * 64);     // four wavefronts' shares
+    return list * 8 + (4 * kTokenSumTokens + kTokenSumTokens + 4) * 4 + kThreads * 16;
+}
+
+template <class TT, class PT>
+__global__ __launch_bounds__(kThreads) void token_sum_kernel(TokenSumParams p)
+{
+    extern __shared__ __attribute__((aligned(16))) char smem_token_sum[];
+    const int N = p.N, T = p.T;
+    const int share = ((N + 3) / 4 + 63) / 64 * 64;                     // picks a wavefront looks at
+    f32x4 *part = reinterpret_cast<f32x4 *>(smem_token_sum);            // [256] partial sums of hot tokens
+    int32_t *found = reinterpret_cast<int32_t *>(smem_token_sum + kThreads * 16);       // [4][share] pick | local token << 16, rank in the next
+    int32_t *order = found + 4 * share;                                 // picks of the tokens, in order
+    int32_t *hist = order + 4 * share;                                  // [4][kTokenSumTokens]
+    int32_t *first = hist + 4 * kTokenSumTokens;                        // [kTokenSumTokens + 1]
+
+    int blk = (int)blockIdx.x;
+    const int cb = blk % p.c_blocks;
+    blk /= p.c_blocks;
+    const int b = blk / p.t_blocks, t0 = (blk - b * p.t_blocks) * p.tb;
+    const int tb = min(p.tb, T - t0);
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint64_t before = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+
+    // ---- the picks of this workgroup's tokens, in increasing order, wavefront by wavefront
+    const int64_t base = (int64_t)b * N;
+    const int q0 = wave * share;
+    int have = 0;                                                       // found so far (uniform)
+    if (lane < kTokenSumTokens) hist[wave * kTokenSumTokens + lane] = 0;
+    constexpr int U = 8;
+    for (int c0 = 0; c0 < share; c0 += U * 64) {
+        uint64_t w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) w[u] = load_index_word(p.Ind, p.ind_dtype, base + min(q0 + c0 + u * 64 + lane, N - 1));
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int q = q0 + c0 + u * 64 + lane;
+            const int64_t t = decode_index_word(w[u], p.Ind, p.ind_dtype, base + min(q, N - 1));
+            const bool mine = c0 + u * 64 < share && q < N && t >= t0 && t < t0 + tb;
+            const uint64_t who = __ballot(mine);
+            if (mine) found[q0 + have + __popcll(who & before)] = q | ((int32_t)(t - t0) << 16);
+            have += __popcll(who);
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    // ---- rank of each among the wavefront's picks of the same token (a wavefront's LDS accesses happen in order)
+    for (int c0 = 0; c0 < have; c0 += 64) {
+        const int i = c0 + lane;
+        const int ent = i < have ? found[q0 + i] : 0;
+        const int tl = ent >> 16;
+        uint64_t same = __ballot(i < have);
+        if (i >= have) same = 0;
+#pragma unroll
+        for (int bit = 0; bit < 5; ++bit) {
+            const uint64_t ones = __ballot((tl >> bit) & 1);
+            same &= ((tl >> bit) & 1) ? ones : ~ones;
+        }
+        if (i < have) {
+            const int rank = __popcll(same & before), start = hist[wave * kTokenSumTokens + tl];
+            order[q0 + i] = start + rank;                               // parked; replaced below
+            if ((same >> lane) == 1ull) hist[wave * kTokenSumTokens + tl] = start + __popcll(same);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    // ranks into registers before `order` gets its real contents
+    constexpr int MAXR = kTokenSumPicks / 4 / 64;
+    int rk[MAXR];
+#pragma unroll
+    for (int c = 0; c < MAXR; ++c) rk[c] = c * 64 + lane < have ? order[q0 + c * 64 + lane] : 0;
+    __syncthreads();
+    if (wave == 0) {                                                    // counts -> starts: over wavefronts, then over tokens
+        int n[4], sum = 0;
+        if (lane < kTokenSumTokens) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) { n[w] = hist[w * kTokenSumTokens + lane]; sum += n[w]; }
+        }
+        int incl = sum;
+#pragma unroll
+        for (int d = 1; d < kTokenSumTokens; d <<= 1) {
+            const int o = __shfl_up(incl, d);
+            if (lane >= d) incl += o;
+        }
+        if (lane < kTokenSumTokens) {
+            int at = incl - sum;
+            first[lane] = at;
+            if (lane == kTokenSumTokens - 1) first[kTokenSumTokens] = incl;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) { hist[w * kTokenSumTokens + lane] = at; at += n[w]; }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < MAXR; ++c)
+        if (c * 64 + lane < have) {
+            const int ent = found[q0 + c * 64 + lane];
+            order[hist[wave * kTokenSumTokens + (ent >> 16)] + rk[c]] = ent & 0xffff;
+        }
+    __syncthreads();
+
+    // ---- sums: 2^tpr_log2 threads per token, four columns each
+    const int tpr = 1 << p.tpr_log2, groups = kThreads >> p.tpr_log2;
+    const int grp = tid >> p.tpr_log2, ct = tid & (tpr - 1);
+    const int col = (cb * tpr + ct) * 4;
+    const bool live = col < p.I;
+    const PT *Pb = reinterpret_cast<const PT *>(p.P) + base * p.ldp + (live ? col : 0);
+    typedef typename std::conditional<sizeof(PT) == 4, f32x4, u32x2>::type vec_t;
+    auto add = [&](f32x4 &acc, const vec_t &v) {
+        if constexpr (sizeof(PT) == 4) {
+#pragma unroll
+            for (int x = 0; x < 4; ++x) acc[x] += v[x];
+        } else {
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                const uint32_t h = (v[x >> 1] >> (16 * (x & 1))) & 0xffffu;
+                acc[x] += TT::ID == 2 ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
+            }
+        }
+    };
+    auto sum_of = [&](int s0, int s1) -> f32x4 {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        constexpr int LB = 16, RB = 4;
+        int s = s0;
+        for (; s + LB <= s1; s += LB) {
+            vec_t v[LB];
+#pragma unroll
+            for (int u = 0; u < LB; ++u) v[u] = *reinterpret_cast<const vec_t *>(Pb + (int64_t)order[s + u] * p.ldp);
+#pragma unroll
+            for (int u = 0; u < LB; ++u) add(acc, v[u]);
+        }
+        for (; s < s1; s += RB) {
+            vec_t v[RB];
+#pragma unroll
+            for (int u = 0; u < RB; ++u) v[u] = *reinterpret_cast<const vec_t *>(Pb + (int64_t)order[min(s + u, s1 - 1)] * p.ldp);
+#pragma unroll
+            for (int u = 0; u < RB; ++u)
+                if (s + u < s1) add(acc, v[u]);
+        }
+        return acc;
+    };
+    auto store = [&](int tl, const f32x4 &acc) {
+        if (!live) return;
+        char *dst = p.out + (((int64_t)b * T + t0 + tl) * p.I + col) * TT::ES;
+        if (col + 4 <= p.I) {
+            if constexpr (TT::ES == 4) *reinterpret_cast<f32x4 __attribute__((aligned(4))) *>(dst) = acc;
+            else *reinterpret_cast<u32x2 __attribute__((aligned(2))) *>(dst) = u32x2{pack2<TT>(acc[0], acc[1]), pack2<TT>(acc[2], acc[3])};
+        } else {
+            for (int x = 0; col + x < p.I; ++x) {
+                if constexpr (TT::ES == 4) reinterpret_cast<float *>(dst)[x] = acc[x];
+                else reinterpret_cast<uint16_t *>(dst)[x] = (uint16_t)f32_to_elem_bits<TT>(acc[x]);
+            }
+        }
+    };
+    for (int tl = grp; tl < tb; tl += groups) {
+        const int s0 = first[tl], s1 = first[tl + 1];
+        if (groups > 1 && s1 - s0 > kTokenSumHot) continue;
+        store(tl, sum_of(s0, s1));
+    }
+    if (groups == 1) return;
+    for (int tl = 0; tl < tb; ++tl) {                                   // hot tokens: a share of the segment per group
+        const int s0 = first[tl], len = first[tl + 1] - s0;
+        if (len <= kTokenSumHot) continue;                              // uniform
+        const int each = (len + groups - 1) / groups;
+        __syncthreads();
+        part[tid] = sum_of(s0 + min(len, grp * each), s0 + min(len, (grp + 1) * each));
+        __syncthreads();
+        if (grp == 0) {
+            f32x4 acc = part[ct];
+            for (int gi = 1; gi < groups; ++gi) {
+                const f32x4 v = part[gi * tpr + ct];
+                acc[0] += v[0]; acc[1] += v[1]; acc[2] += v[2]; acc[3] += v[3];
+            }
+            store(tl, acc);
+        }
+    }
+}
+
+}  // namespace egs

@@ -1,0 +1,73 @@
+"""The kernels for operands of any size and alignment (csrc/egs_tiled.h, csrc/egs_token_sum.h) where they can go wrong: edges of
+tiles and slabs, rows shorter than a chunk, operands of a few bytes, picks that do not exist, hot tokens; against the oracle."""
+import pytest
+import torch
+
+from oracle import egs_oracle as O
+from tests._util import assert_close, make_case, np64
+from tests.test_gpu_parity import dev, run_all
+
+pytestmark = pytest.mark.gpu
+
+from expertscattergather_amd import _abi
+from expertscattergather_amd import hip_kernels as hk
+
+SHAPES = [
+    (1, 2, 1, 1, 3, 1), (1, 1, 2, 2, 1, 5), (2, 3, 2, 2, 7, 2),     # operands below 16 bytes, and just above
+    (3, 9, 2, 5, 5, 3),                 # rows shorter than a chunk on both sides
+    (2, 40, 9, 33, 63, 65), (2, 40, 3, 32, 65, 63),                 # one element off a slab and a tile
+    (4, 50, 5, 16, 520, 17),            # nine slabs, a column tile with one column in its second 16
+    (2, 70, 7, 65, 129, 81),            # 130 picks per expert: one row tile and two rows; widths of 80 and 144
+    (6, 30, 11, 29, 97, 131),           # tokens picked tens of times
+    (40, 33, 13, 64, 72, 100),          # 2560 picks per expert: 128-row tiles, splits of the weight gradient
+]
+
+
+@pytest.mark.parametrize("mode", ["deterministic", "atomic"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_any_size_matches_the_oracle(shape, dtype, mode):
+    B, T, E, K, I, J = shape
+    case = make_case(300 + sum(shape), *shape, dtype, ind_dtype=torch.int16 if dtype is torch.float16 else torch.int64)
+    Ind = case["Ind"].clone()
+    if E * K > 40:
+        g = torch.Generator().manual_seed(1)
+        Ind[torch.rand(Ind.shape, generator=g) < 0.3] = T // 2      # a token with a third of the picks: shared by the workgroup
+        Ind[0, 0, 0], Ind[-1, -1, -1], Ind[-1, 0, 0] = T, -1, 30000
+    bad = (Ind < 0) | (Ind >= T)
+    safe = Ind.clone(); safe[bad] = 0
+    keep = (~bad).numpy()[..., None]
+    got = run_all(dict(case, Ind=Ind), T, mode)
+    X, Wg, Ws, Y, dOut = (np64(case[k]) for k in ("X", "Wg", "Ws", "Y", "dOut"))
+    Yk, In = Y * keep, safe.to(torch.int64).numpy()
+    dX, dWg = O.gather_backward(X, Wg, In, Yk)
+    dY, dWs = O.scatter_backward(Yk, Ws, In, dOut)
+    for name, ref in (("Y", O.gather_forward(X, Wg, In) * keep), ("out", O.scatter_forward(Yk, Ws, In, T)), ("dX", dX), ("dWg", dWg),
+                      ("dY", dY * keep), ("dWs", dWs)):
+        if mode == "atomic" and dtype is not torch.float32 and name in ("out", "dX"):     # one more rounding per pick
+            assert abs(np64(got[name]) - ref).max() <= 2 ** (-6 if dtype is torch.bfloat16 else -9) * abs(ref).max() + 1e-30
+        else:
+            assert_close(got[name], ref, dtype, f"{name} {shape} {dtype} {mode}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_odd_views_and_values_that_are_not_finite_stay_where_they_are(dtype):
+    """X as a view with odd strides that ends at its storage's last element, W and Y off the 16-byte grid (through the C ABI's
+    Python route they would be copied); a NaN row reaches only its own picks although row tails are read 16 bytes at a time."""
+    B, T, E, K, I, J = 3, 21, 4, 9, 37, 29
+    case = make_case(77, B, T, E, K, I, J, dtype)
+    X = case["X"].clone()
+    X[1, 5] = float("nan")
+    wide = torch.full((B * T * 41,), float("nan"), dtype=dtype, device="cuda")
+    Xv = wide[wide.numel() - ((B - 1) * T * 41 + (T - 1) * 41 + I):].as_strided((B, T, I), (T * 41, 41, 1))
+    Xv.copy_(X)
+    W, Ind = dev(case["Wg"]), dev(case["Ind"])
+    Wo = torch.empty(W.numel() + 1, dtype=dtype, device="cuda")[1:].view(W.shape).copy_(W)
+    Yo = torch.empty(B * E * K * J + 1, dtype=dtype, device="cuda")[1:].view(B, E, K, J)
+    rc = _abi.lib().egs_expert_gather_forward(Xv.data_ptr(), Wo.data_ptr(), Ind.data_ptr(), Yo.data_ptr(), _abi.Dims(B, T, E, K, I, J),
+                                              T * 41, 41, hk.dtype_to_type_id(dtype), _abi.IND_I64, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    hit = ((case["Ind"] == 5) & (torch.arange(B) == 1)[:, None, None])[..., None]
+    assert torch.isnan(Yo.cpu().float()).eq(hit.expand(B, E, K, J)).all()
+    want = O.gather_forward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy())
+    assert_close(torch.where(hit, torch.from_numpy(want).to(dtype), Yo.cpu()), want, dtype, "Y")
