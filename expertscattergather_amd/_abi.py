@@ -24,7 +24,7 @@ IND_I16, IND_I32, IND_I64, IND_U8 = 0, 1, 2, 3
 W_EIJ, W_EJI = 0, 1
 SCATTER_DETERMINISTIC, SCATTER_ATOMIC, SCATTER_COMPACT = 0, 1, 2
 OP_GATHER_GEMM, OP_GEMM_SCATTER, OP_DW, OP_GATHER_BACKWARD, OP_SCATTER_BACKWARD = 0, 1, 2, 3, 4
-ACT_NONE, ACT_RELU, ACT_GELU, ACT_SILU, ACT_GELU_TANH = 0, 1, 2, 3, 4
+ACT_NONE, ACT_RELU, ACT_GELU, ACT_SILU, ACT_GELU_TANH, ACT_ROUND_FIRST = 0, 1, 2, 3, 4, 16
 EGS_ERR_UNSUPPORTED = -9
 ABI_VERSION = 1
 
@@ -55,10 +55,12 @@ SIGNATURES = {
     "egs_expert_gather_backward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _dp, _i64, _i64, _i, _i, _i, _vp]),
     "egs_expert_scatter_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _dp, _i, _i, _i, _vp]),
     "egs_expert_scatter_backward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _dp, _i64, _i64, _i, _i, _vp]),
+    "egs_expert_choice_router": (_i, [_vp, _vp, _vp, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _i, _i, _vp]),
     "egs_validate_indices": (_i, [_vp, _i, _i64, ctypes.c_int32, _vp, _vp]),
     "egs_routing_table_bytes": (_sz, [_dp, _i]),
     "egs_stream_capture_id": (_i, [_vp, ctypes.POINTER(ctypes.c_ulonglong)]),
     "egs_expert_gather_forward_table": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _dp, _i64, _i64, _i, _i, _vp]),
+    "egs_expert_gather_act_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _dp, _i64, _i64, _i, _i, _i, _vp]),
     "egs_expert_scatter_forward_table": (_i, [_vp, _vp, _vp, _vp, _sz, _vp, _vp, _sz, _dp, _i, _i, _i, _vp]),
     "egs_expert_gather_backward_table": (_i, [_vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _sz, _dp, _i64, _i64, _i, _i, _i, _vp]),
     "egs_expert_mlp_supported": (_i, [_dp, _i]),

@@ -103,6 +103,49 @@ template <> __device__ __forceinline__ void mma_chunk<ElemF32>(f32x4 &acc, const
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(bits_f32(p[c]), bits_f32(q[c]), acc, 0, 0, 0);
 }
 
+// ---------------------------------------------------------------------------- activations (values of egs_activation)
+// Applied to fp32 products before they are rounded.  The transcendental ones are for 16-bit results and written with the hardware
+// exponential and reciprocal (a few instructions per value instead of the ~100 of the library erff / tanhf):
+// gelu_tanh(v) = v * sigmoid(2u); erf by the rational approximation of Abramowitz & Stegun 7.1.26 (absolute error < 1.5e-7, far
+// below the rounding to a 16-bit type that follows).
+enum Activation { ACT_NONE = 0, ACT_RELU = 1, ACT_GELU = 2, ACT_SILU = 3, ACT_GELU_TANH = 4, ACT_ROUND_FIRST = 16 };
+
+// `each(fn)` applies fn to every value; `act` is uniform
+template <class Each> __device__ __forceinline__ void apply_activation(int act, Each each)
+{
+    switch (act & 15) {
+    case ACT_RELU: each([](float v) { return v < 0.f ? 0.f : v; }); break;
+    case ACT_GELU:
+        each([](float v) {
+            const float x = fabsf(v) * 0.70710678118654752f;
+            const float t = __frcp_rn(1.f + 0.3275911f * x);
+            const float poly = ((((1.061405429f * t - 1.453152027f) * t + 1.421413741f) * t - 0.284496736f) * t + 0.254829592f) * t;
+            const float erf_abs = 1.f - poly * __expf(-x * x);
+            return 0.5f * v * (1.f + copysignf(erf_abs, v));
+        });
+        break;
+    case ACT_SILU: each([](float v) { return v * __frcp_rn(1.f + __expf(-v)); }); break;
+    case ACT_GELU_TANH:
+        each([](float v) {
+            const float u = 0.7978845608028654f * (v + 0.044715f * v * v * v);
+            return v * __frcp_rn(1.f + __expf(-2.f * u));
+        });
+        break;
+    default: break;
+    }
+}
+
+// the same on products that ACT_ROUND_FIRST asks to be rounded to the element type before (as if they had been stored)
+template <class TT, class Each> __device__ __forceinline__ void apply_activation_of(int act, Each each)
+{
+    if (act & ACT_ROUND_FIRST)
+        each([](float v) {
+            if constexpr (TT::ID == 2) return bits_f32(pack2<TT>(v, 0.f) << 16);
+            else return f16_bits_to_f32(pack2<TT>(v, 0.f) & 0xffffu);
+        });
+    apply_activation(act, each);
+}
+
 // ---------------------------------------------------------------------------- index decode
 // Ind is read in its own integer width and never narrowed.  Branch-free for every width (so that
 // several index loads can be in flight): one 8-byte load of the aligned window that contains the

@@ -270,7 +270,7 @@ int rows_xcd_blocks(int map, int tiles_per_e, int E)
 
 bool make_gather_small(const void *X, const void *W, const void *Ind, void *Y, const egs_dims *d, int64_t ldx_b,
                        int64_t ldx_t, int act_dtype, int w_dtype, int ind_dtype, int w_layout, SmallRowsJob &j,
-                       const RoutingTable *build = nullptr)
+                       const RoutingTable *build = nullptr, int act = ACT_NONE)
 {
     const int R = d->I, N = d->J;
     if (g_force_generic || w_dtype != act_dtype || !small_shape_ok(act_dtype, R, N)) return false;
@@ -288,6 +288,7 @@ bool make_gather_small(const void *X, const void *W, const void *Ind, void *Y, c
     p.tiles_per_e = (int)((Me + 255) / 256);
     if ((int64_t)8 * (ceil_div(d->E, 8) + 1) * (p.tiles_per_e + 8) > INT32_MAX / 2) return false;
     p.rows_share_xcd = rows_xcd_map(d, R, N, 2, p.tiles_per_e);
+    p.act = act;
     j.R = R; j.act_dtype = act_dtype; j.gather = true; j.out_f32 = false; j.lds = 0;
     j.nmajor = (w_layout == EGS_W_EIJ);                 // [E,I,J] = [E,R,N]
     if (build != nullptr) {             // the routing table of a later scatter rides along: B more workgroups, first in line
@@ -962,12 +963,12 @@ int check_table_arg(void *table, size_t table_bytes, const egs_dims *d, int act_
 // ------------------------------------------------------------------------------ implementations
 int gather_gemm_impl(const void *X, const void *W, const void *Ind, void *Y, const float *w_scale,
                      const egs_dims *d, int64_t ldx_b, int64_t ldx_t, int act_dtype, int w_dtype, int ind_dtype,
-                     int w_layout, hipStream_t s, const RoutingTable *build = nullptr)
+                     int w_layout, hipStream_t s, const RoutingTable *build = nullptr, int act = ACT_NONE)
 {
     const int ES = elem_size(act_dtype), WES = elem_size(w_dtype);
     if (w_scale == nullptr) {
         SmallRowsJob j;
-        if (make_gather_small(X, W, Ind, Y, d, ldx_b, ldx_t, act_dtype, w_dtype, ind_dtype, w_layout, j, build))
+        if (make_gather_small(X, W, Ind, Y, d, ldx_b, ldx_t, act_dtype, w_dtype, ind_dtype, w_layout, j, build, act))
             return launch_rows_small_job(j, nullptr, nullptr, s);
     }
     if (w_scale == nullptr && act_dtype == EGS_F32 && w_dtype == EGS_F32) {
@@ -983,6 +984,7 @@ int gather_gemm_impl(const void *X, const void *W, const void *Ind, void *Y, con
     memset(&p, 0, sizeof(p));
     p.A = (const char *)X; p.W = (const char *)W; p.Ind = Ind; p.C = (char *)Y; p.w_scale = w_scale;
     p.B = d->B; p.T = d->T; p.E = d->E; p.K = d->K;
+    p.act = act;
     p.R = d->I; p.N = d->J;
     p.lda_b = ldx_b; p.lda_t = ldx_t;
     p.ind_dtype = ind_dtype;
@@ -1443,19 +1445,30 @@ size_t egs_routing_table_bytes(const egs_dims *d, int dtype)
     return l.ok ? l.bytes : 0;
 }
 
-int egs_expert_gather_forward_table(const void *X, const void *W, const void *Ind, void *Y, void *table, size_t table_bytes,
-                                    const egs_dims *d, int64_t ldx_b, int64_t ldx_t,
-                                    int dtype, int ind_dtype, void *stream)
+int egs_expert_gather_act_forward(const void *X, const void *W, const void *Ind, void *Y, void *table, size_t table_bytes,
+                                  const egs_dims *d, int64_t ldx_b, int64_t ldx_t,
+                                  int dtype, int ind_dtype, int activation, void *stream)
 {
     int rc = validate_gather(X, W, Ind, Y, nullptr, d, ldx_b, ldx_t, dtype, dtype, ind_dtype, EGS_W_EIJ);
     if (rc != EGS_OK) return rc;
+    const int act = activation & ~EGS_ACT_ROUND_FIRST;
+    if (act < EGS_ACT_NONE || act > EGS_ACT_GELU_TANH) return EGS_ERR_BAD_MODE;
+    if (act <= EGS_ACT_RELU) activation = act;      // the same values either way
+    if (dtype == EGS_F32 && act != EGS_ACT_NONE) return EGS_ERR_UNSUPPORTED;      // the approximations are for 16-bit results
     RoutingTable tab;
     bool have_tab = false;
     rc = check_table_arg(table, table_bytes, d, dtype, tab, have_tab);
     if (rc != EGS_OK) return rc;
     if ((size_t)d->B * d->E * d->K * d->J == 0) return EGS_OK;
     return gather_gemm_impl(X, W, Ind, Y, nullptr, d, ldx_b, ldx_t, dtype, dtype, ind_dtype, EGS_W_EIJ, (hipStream_t)stream,
-                            have_tab ? &tab : nullptr);
+                            have_tab ? &tab : nullptr, activation);
+}
+
+int egs_expert_gather_forward_table(const void *X, const void *W, const void *Ind, void *Y, void *table, size_t table_bytes,
+                                    const egs_dims *d, int64_t ldx_b, int64_t ldx_t,
+                                    int dtype, int ind_dtype, void *stream)
+{
+    return egs_expert_gather_act_forward(X, W, Ind, Y, table, table_bytes, d, ldx_b, ldx_t, dtype, ind_dtype, EGS_ACT_NONE, stream);
 }
 
 int egs_expert_scatter_backward(const void *Y, const void *W, const void *Ind, const void *grad_Out,

@@ -32,8 +32,6 @@
 
 namespace egs {
 
-enum MlpAct { MLP_ACT_NONE = 0, MLP_ACT_RELU = 1, MLP_ACT_GELU = 2, MLP_ACT_SILU = 3, MLP_ACT_GELU_TANH = 4 };
-
 struct MlpFusedParams {
     const char *X;          // [B,T,I] rows, strides (ldx_b, ldx_t, 1) in elements
     const char *Wg;         // [E,I,J]
@@ -45,7 +43,7 @@ struct MlpFusedParams {
     int32_t ind_dtype;
     int32_t slices;         // I / kFusedCols
     int32_t perm_at, cnt_at, zero_at;   // as in ScatterFusedParams
-    int32_t act;            // MlpAct
+    int32_t act;            // Activation
 };
 
 // KS1 = I / 32 (matrix-instruction steps of the gather product; I is also the output width), JT = J / 16
@@ -184,30 +182,7 @@ __device__ __forceinline__ void mlp_fused_body(const MlpFusedParams &p, const in
 #pragma unroll
                     for (int r = 0; r < 4; ++r) acc1[h][t][r] = fn(acc1[h][t][r]);
         };
-        // The transcendental ones are written with the hardware exponential and reciprocal (a few instructions per value
-        // instead of the ~100 of the library erff / tanhf: every slice workgroup repeats them).  gelu_tanh(v) = v * sigmoid(2u);
-        // erf by the rational approximation of Abramowitz & Stegun 7.1.26 (absolute error < 1.5e-7, far below the rounding
-        // to a 16-bit type that follows).
-        switch (p.act) {
-        case MLP_ACT_RELU: activate([](float v) { return fmaxf(v, 0.f); }); break;
-        case MLP_ACT_GELU:
-            activate([](float v) {
-                const float x = fabsf(v) * 0.70710678118654752f;
-                const float t = __frcp_rn(1.f + 0.3275911f * x);
-                const float poly = ((((1.061405429f * t - 1.453152027f) * t + 1.421413741f) * t - 0.284496736f) * t + 0.254829592f) * t;
-                const float erf_abs = 1.f - poly * __expf(-x * x);
-                return 0.5f * v * (1.f + copysignf(erf_abs, v));
-            });
-            break;
-        case MLP_ACT_SILU: activate([](float v) { return v * __frcp_rn(1.f + __expf(-v)); }); break;
-        case MLP_ACT_GELU_TANH:
-            activate([](float v) {
-                const float u = 0.7978845608028654f * (v + 0.044715f * v * v * v);
-                return v * __frcp_rn(1.f + __expf(-2.f * u));
-            });
-            break;
-        default: break;
-        }
+        apply_activation(p.act, activate);
         f32x4 acc2[2][2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) { acc2[h][0] = f32x4{0.f, 0.f, 0.f, 0.f}; acc2[h][1] = f32x4{0.f, 0.f, 0.f, 0.f}; }

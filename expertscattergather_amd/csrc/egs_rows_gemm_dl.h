@@ -364,7 +364,24 @@ __global__ __launch_bounds__(dl_threads(BM, BN), (BK == 32 && dl_threads(BM, BN)
             for (int r0 = wave * ROWS_PER_INSTR; r0 < ROWS_PER_PASS; r0 += NW * ROWS_PER_INSTR) {
                 const int row = r0 + lrow;
                 const int64_t co = c_off[half * ROWS_PER_PASS + row];
-                const u32x4 v = *reinterpret_cast<const u32x4 *>(smem + row * ROW_BYTES + ((lchunk ^ (row & 15)) << 4));
+                u32x4 v = *reinterpret_cast<const u32x4 *>(smem + row * ROW_BYTES + ((lchunk ^ (row & 15)) << 4));
+                if constexpr (GATHER && OES == 2 && WES == 2) {
+                    // on the rounded values, as a pass of its own over them would: here they are out of the accumulators, eight to a lane
+                    if (p.act != ACT_NONE) {
+                        float f[8];
+#pragma unroll
+                        for (int x = 0; x < 8; ++x) {
+                            const uint32_t h = (v[x >> 1] >> (16 * (x & 1))) & 0xffffu;
+                            f[x] = TT::ID == 2 ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
+                        }
+                        apply_activation(p.act, [&](auto fn) {
+#pragma unroll
+                            for (int x = 0; x < 8; ++x) f[x] = fn(f[x]);
+                        });
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) v[x] = pack2<TT>(f[2 * x], f[2 * x + 1]);
+                    }
+                }
                 if (co >= 0 && n_here < N) *reinterpret_cast<u32x4 *>(p.C + co * OES + (size_t)n_here * OES) = v;
             }
         }

@@ -42,6 +42,7 @@ struct SmallRowsParams {
     // routing-table build riding along (csr_blocks = B, or 0): see csr_count_body; csr_split: two workgroups per batch
     // element (csr_blocks = 2 B), see csr_count_half_body
     int32_t csr_blocks, csr_split;
+    int32_t act;            // Activation of the results (GATHER only)
     int32_t *seg_off, *perm, *rank_tmp, *long_tab;
 };
 
@@ -198,6 +199,14 @@ __device__ __forceinline__ void rows_small_body(const SmallRowsParams &p, const 
         if (st == 2) {
 #pragma unroll
             for (int tn = 0; tn < TN; ++tn) acc[tn] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        if constexpr (GATHER) {
+            apply_activation_of<TT>(p.act, [&](auto fn) {
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[tn][r] = fn(acc[tn][r]);
+            });
         }
         if (st != 0) {
             if constexpr (OES == 4) {

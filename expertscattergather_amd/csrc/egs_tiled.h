@@ -49,6 +49,7 @@ struct TiledRowsParams {
     int32_t B, T, E, K, R, N, ldc;
     int32_t ind_dtype, gather, out_f32;
     int32_t m_tiles, n_tiles;
+    int32_t act;                // Activation of the results (16-bit types)
     int32_t rows_major;         // numbering of the tiles: 1 = row tiles outermost (their source rows share an L2), 0 = experts outermost
 };
 
@@ -323,6 +324,15 @@ __global__ __launch_bounds__(kThreads) void tiled_rows_kernel(TiledRowsParams p)
 
     // ---------------- results: lane (a, g) holds columns 16 j + 4 g .. + 3 of row 16 i + a; regrouped so that adjacent lanes
     // store adjacent pieces of a row
+    auto each = [&](auto fn) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[i][j][r] = fn(acc[i][j][r]);
+    };
+    if constexpr (WES == 2) apply_activation_of<TT>(p.act, each);
     const int srow = lane >> 2, sg = lane & 3;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -381,6 +391,7 @@ __global__ __launch_bounds__(kThreads) void tiny_rows_kernel(TiledRowsParams p)
             v += elem(row + (int64_t)r * TT::ES) * wv;
         }
         if (p.w_scale != nullptr) v *= p.w_scale[(int64_t)e * p.N + n];
+        if constexpr (TT::ES == 2) apply_activation_of<TT>(p.act, [&](auto fn) { v = fn(v); });
         if (TT::ES == 4 || p.out_f32) reinterpret_cast<float *>(p.C)[pick * p.ldc + n] = v;
         else reinterpret_cast<uint16_t *>(p.C)[pick * p.ldc + n] = (uint16_t)f32_to_elem_bits<TT>(v);
     }

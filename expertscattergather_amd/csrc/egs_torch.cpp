@@ -123,13 +123,13 @@ struct Scratch {                // per call, from the caching allocator: stream-
 };
 
 // ------------------------------------------------------------------------------ the four launchers
-Tensor gather_forward(const Problem &p, const Tensor &X, const Tensor &W, const Tensor &Ind, const Tensor &build)
+Tensor gather_forward(const Problem &p, const Tensor &X, const Tensor &W, const Tensor &Ind, const Tensor &build, int act = EGS_ACT_NONE)
 {
     Tensor Y = empty_gpu({p.d.B, p.d.E, p.d.K, p.d.J}, X.scalar_type(), p);
-    const int rc = egs_expert_gather_forward_table(X.const_data_ptr(), W.const_data_ptr(), Ind.const_data_ptr(), Y.data_ptr(),
-                                                   build.defined() ? build.data_ptr() : nullptr,
-                                                   build.defined() ? (size_t)build.numel() : 0, &p.d, (int64_t)p.d.T * p.d.I, p.d.I, p.dt,
-                                                   p.ind, stream_of(X));
+    const int rc = egs_expert_gather_act_forward(X.const_data_ptr(), W.const_data_ptr(), Ind.const_data_ptr(), Y.data_ptr(),
+                                                 build.defined() ? build.data_ptr() : nullptr,
+                                                 build.defined() ? (size_t)build.numel() : 0, &p.d, (int64_t)p.d.T * p.d.I, p.d.I, p.dt,
+                                                 p.ind, act, stream_of(X));
     raise_status(rc, "expert_gather_forward_call");
     return Y;
 }
@@ -449,6 +449,76 @@ PyObject *py_scatter_backward(PyObject *, PyObject *const *a, Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
+// router(logits, K, ind_dtype) -> (Ind, scores) or None
+PyObject *py_router(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    if (!want(n, 3, "router")) return nullptr;
+    if (!plain_object(a[0]) || !PyLong_CheckExact(a[1]) || !THPDtype_Check(a[2])) Py_RETURN_NONE;
+    const Tensor &logits = THPVariable_Unpack(a[0]);
+    const at::ScalarType it = ((THPDtype *)a[2])->scalar_type;
+    const long long K = PyLong_AsLongLong(a[1]);
+    const int dt = plain(logits) ? type_id(logits.scalar_type()) : -1, ind = ind_type_id(it);
+    if (dt < 0 || ind < 0 || logits.dim() != 3 || !logits.is_contiguous() || !no_modes() || has_tangent(logits) ||
+        logits.device().index() != c10::hip::current_device() || (at::GradMode::is_enabled() && logits.requires_grad()))
+        Py_RETURN_NONE;
+    const int64_t B = logits.size(0), T = logits.size(1), E = logits.size(2);
+    if (B < 1 || T < 1 || E < 1 || K < 1 || K > T || B > INT32_MAX || T > INT32_MAX || E > INT32_MAX) Py_RETURN_NONE;
+    Tensor Ind, scores;
+    int rc;
+    {
+        NoGil nogil;
+        Problem p{};
+        p.dev = logits.device().index();
+        Ind = empty_gpu({B, E, K}, it, p);
+        scores = empty_gpu({B, E, K}, at::kFloat, p);
+        rc = egs_expert_choice_router(logits.const_data_ptr(), Ind.data_ptr(), (float *)scores.data_ptr(), (int32_t)B, (int32_t)T, (int32_t)E,
+                                      (int32_t)K, dt, ind, stream_of(logits));
+    }
+    if (rc == EGS_ERR_UNSUPPORTED) Py_RETURN_NONE;
+    raise_status(rc, "expert_choice_router");
+    return pair({Ind, scores});
+    END_HANDLE_TH_ERRORS
+}
+
+// mlp_forward(X, W_gather, W_scatter, Ind, activation, mode, keep_table, block) -> out, or None.  block: by the one-kernel block
+// where it takes the operands; else the gather with the activation in its launch, and the scatter
+PyObject *py_mlp_forward(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    if (!want(n, 8, "mlp_forward")) return nullptr;
+    for (int i = 0; i < 4; ++i)
+        if (!plain_object(a[i])) Py_RETURN_NONE;
+    const Tensor &X = THPVariable_Unpack(a[0]), &Wg = THPVariable_Unpack(a[1]), &Ws = THPVariable_Unpack(a[2]), &Ind = THPVariable_Unpack(a[3]);
+    const Problem p = problem_of(X, Wg, Ind, true, true, 0);
+    if (!p.ok || !no_modes() || !plain(Ws) || Ws.dim() != 3 || Ws.scalar_type() != X.scalar_type() || Ws.device() != X.device() ||
+        !dense16(Ws) || Ws.size(0) != p.d.E || Ws.size(1) != p.d.J || Ws.size(2) != p.d.I)
+        Py_RETURN_NONE;
+    const int act = (int)PyLong_AsLong(a[4]) & ~EGS_ACT_ROUND_FIRST, round = (int)PyLong_AsLong(a[4]) & EGS_ACT_ROUND_FIRST, mode = (int)PyLong_AsLong(a[5]);
+    Tensor out;
+    if (flag(a[7]) && egs_expert_mlp_supported(&p.d, p.dt)) {
+        NoGil nogil;
+        out = empty_gpu({p.d.B, p.d.T, p.d.I}, X.scalar_type(), p);
+        const int rc = egs_expert_mlp_forward(X.const_data_ptr(), Wg.const_data_ptr(), Ws.const_data_ptr(), Ind.const_data_ptr(), out.data_ptr(),
+                                              &p.d, (int64_t)p.d.T * p.d.I, p.d.I, p.dt, p.ind, act, stream_of(X));
+        raise_status(rc, "expert_mlp_forward");
+    } else {
+        if (p.dt == EGS_F32 && act != EGS_ACT_NONE) Py_RETURN_NONE;
+        TableState ts = table_state(a[3], Ind, p, flag(a[6]));
+        Tensor table = ts.table;
+        const bool build = ts.applies && !table.defined();
+        {
+            NoGil nogil;
+            if (build) table = empty_gpu({(int64_t)ts.bytes}, at::kByte, p);
+            const Tensor Y = gather_forward(p, X, Wg, Ind, build ? table : Tensor(), act | round);
+            out = scatter_forward(p, Y, Ws, Ind, table, mode);
+        }
+        if (build) keep_table(a[3], ts.key, table);
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
 PyObject *py_abi_version(PyObject *, PyObject *) { return PyLong_FromLong(egs_abi_version()); }
 
 PyMethodDef methods[] = {
@@ -456,6 +526,8 @@ PyMethodDef methods[] = {
     {"scatter_forward", (PyCFunction)(void (*)(void))py_scatter_forward, METH_FASTCALL, "out, or None: not for this way"},
     {"gather_backward", (PyCFunction)(void (*)(void))py_gather_backward, METH_FASTCALL, "(grad_X, grad_W), or None: not for this way"},
     {"scatter_backward", (PyCFunction)(void (*)(void))py_scatter_backward, METH_FASTCALL, "(grad_Y, grad_W), or None: not for this way"},
+    {"router", (PyCFunction)(void (*)(void))py_router, METH_FASTCALL, "(Ind, scores), or None: not for this way"},
+    {"mlp_forward", (PyCFunction)(void (*)(void))py_mlp_forward, METH_FASTCALL, "out, or None: not for this way"},
     {"abi_version", py_abi_version, METH_NOARGS, "ABI version of the library this module is linked to"},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -855,8 +855,19 @@ def _mlp_forward_impl(X: torch.Tensor, W_gather: torch.Tensor, W_scatter: torch.
     T = X.shape[1]
     d = _abi.Dims(B, T, E, K, I, J)
     lib = _abi.lib()
-    if ct is not torch.float32 and (force_block or _mlp_block_pays(B, E, K, I, J, act)) \
-            and lib.egs_expert_mlp_supported(d, dtype_to_type_id(ct)):
+    ext = _abi.torch_ext()
+    if ext is not None:
+        # The activation rides in the gather's launch here, so the block has only one launch of its own to save: it wins where
+        # its workgroups walk at most eight 32-pick units (bf16, relu, block / two launches in us: B64 T256 E8 K32 I128 J64
+        # 9.7 / 10.7, E16 13.3 / 11.5, E32 22.4 / 15.2; B16 T128 E8 K16 I64 J64 7.5 / 10.6)
+        few = E * ((K + 31) // 32) <= 8 and 8 * ((B + 7) // 8) * (I // 32) <= 256
+        # products rounded before the activation where the block is not what these sizes are (by its own rule) specified by
+        pays = _mlp_block_pays(B, E, K, I, J, act) and I in (32, 64, 128) and J in (32, 64) and E * K <= 1024
+        out = ext.mlp_forward(X, W_gather, W_scatter, Ind, act if pays else act | _abi.ACT_ROUND_FIRST, _MODES[get_scatter_mode()], _table_cache, force_block or few)
+        if out is not None:
+            return out
+    block = ct is not torch.float32 and (force_block or _mlp_block_pays(B, E, K, I, J, act))
+    if block and lib.egs_expert_mlp_supported(d, dtype_to_type_id(ct)):
         res_dtype = X.dtype
         Xs, ld_b, ld_t = _rows_source(X, ct)
         Wg = _dense16(W_gather, ct); Ws = _dense16(W_scatter, ct); Indc = Ind.contiguous()
@@ -869,6 +880,10 @@ def _mlp_forward_impl(X: torch.Tensor, W_gather: torch.Tensor, W_scatter: torch.
         if rc != _abi.EGS_ERR_UNSUPPORTED:
             _abi.check(rc, "expert_mlp_forward")
     with torch.no_grad():
+        if ext is not None:
+            create_kernels()
+            Y = _TORCH_ACT[act](expert_gather_forward_call(X, W_gather, Ind, torch.float32))
+            return expert_scatter_forward_call(Y, W_scatter, Ind, T, torch.float32)
         Y = _TORCH_ACT[act](_gather_forward_impl(X, W_gather, Ind, torch.float32))
         return _scatter_forward_impl(Y, W_scatter, Ind, T, torch.float32)
 

@@ -4,12 +4,15 @@ The reference draws ``Ind`` at random in its tests and benchmark (test_all.py:16
 and ships no router; in a model ``Ind[b, e, :]`` is what expert ``e`` picks from batch element ``b``.
 This is the usual expert-choice rule: every expert takes the K tokens with the highest affinity, so
 tokens are distinct within one ``(b, e)`` and may repeat across experts — the ``configs[0..2]`` input
-distribution of the benchmark.  Plain torch (``topk`` runs on the GPU); the scores come back with the
-indices so that a caller can weight the gathered rows.
+distribution of the benchmark.  On the GPU, and where no gradient is asked of the scores, this is one HIP kernel
+(csrc/egs_router.hip); else plain torch.  The scores come back with the indices so that a caller can weight the
+gathered rows.
 """
 from __future__ import annotations
 
 import torch
+
+from . import _abi
 
 
 def expert_choice_router(logits: torch.Tensor, K: int, ind_dtype: torch.dtype = torch.int64):
@@ -26,6 +29,11 @@ def expert_choice_router(logits: torch.Tensor, K: int, ind_dtype: torch.dtype = 
         raise ValueError("Unknown dtype")
     if T - 1 > torch.iinfo(ind_dtype).max:
         raise ValueError(f"{ind_dtype} cannot hold token ids up to {T - 1}")
+    if type(logits) is torch.Tensor and logits.is_cuda and not torch.compiler.is_compiling():
+        ext = _abi.torch_ext()
+        routed = None if ext is None else ext.router(logits, K, ind_dtype)
+        if routed is not None:
+            return routed
     affinity = torch.softmax(logits.float(), dim=-1).transpose(1, 2)      # [B, E, T]
     scores, ind = torch.topk(affinity, K, dim=-1)
     return ind.to(ind_dtype), scores

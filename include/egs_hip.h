@@ -241,7 +241,8 @@ typedef enum egs_activation {
     EGS_ACT_RELU = 1,
     EGS_ACT_GELU = 2,           /* erf form (torch.nn.functional.gelu default) */
     EGS_ACT_SILU = 3,
-    EGS_ACT_GELU_TANH = 4       /* tanh approximation */
+    EGS_ACT_GELU_TANH = 4,      /* tanh approximation */
+    EGS_ACT_ROUND_FIRST = 16    /* flag of egs_expert_gather_act_forward: the products are rounded to the element type first */
 } egs_activation;
 
 /* 1 if egs_expert_mlp_forward takes these sizes (with dense operands that start on a 16-byte boundary), else 0 */
@@ -254,6 +255,13 @@ int egs_expert_mlp_forward(const void *X, const void *Wg, const void *Ws, const 
 /* ---------------------------------------------------------------------------------------
  * Launcher-level entry points (one per reference callable)
  * ------------------------------------------------------------------------------------- */
+
+/* egs_expert_gather_forward_table with an activation applied to the products before they are stored (table may be null).
+ * Large products round to the element type before it in any case.  16-bit types; fp32 with an
+ * activation returns EGS_ERR_UNSUPPORTED. */
+int egs_expert_gather_act_forward(const void *X, const void *W, const void *Ind, void *Y, void *table, size_t table_bytes,
+                                  const egs_dims *d, int64_t ldx_b, int64_t ldx_t,
+                                  int dtype, int ind_dtype, int activation, void *stream);
 
 /* expert_gather_forward_call(X, W[E,I,J], Ind) -> Y          reference egs/triton_kernels.py:367-392 */
 int egs_expert_gather_forward(const void *X, const void *W, const void *Ind, void *Y,
@@ -278,6 +286,16 @@ int egs_expert_scatter_backward(const void *Y, const void *W, const void *Ind, c
                                 void *workspace, size_t workspace_bytes, const egs_dims *d,
                                 int64_t ldg_b, int64_t ldg_t,
                                 int dtype, int ind_dtype, void *stream);
+
+/* ---------------------------------------------------------------------------------------
+ * Expert-choice router (no counterpart in the reference, which draws Ind at random)
+ * ------------------------------------------------------------------------------------- */
+
+/* scores[b,e,:] = the K largest of softmax over experts of logits[b,:,e], descending, Ind[b,e,:] their tokens.
+ * logits [B,T,E] dense in fp32 / fp16 / bf16, scores fp32.  EGS_ERR_UNSUPPORTED where a column does not fit a
+ * compute unit's LDS (T above about 9000) or K > 512. */
+int egs_expert_choice_router(const void *logits, void *Ind, float *scores, int32_t B, int32_t T, int32_t E, int32_t K,
+                             int logits_dtype, int ind_dtype, void *stream);
 
 /* ---------------------------------------------------------------------------------------
  * Debug helper (no counterpart in the reference, which never checks Ind)

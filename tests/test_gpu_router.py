@@ -1,0 +1,49 @@
+"""The one-kernel expert-choice router (csrc/egs_router.hip) against torch on the CPU: the same tokens in the same order, at sizes
+where a wavefront's column, the row loads or the selection have remainders; ties, and what stays with torch."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from expertscattergather_amd import _abi
+from expertscattergather_amd.router import expert_choice_router
+
+SHAPES = [(1, 1, 1, 1), (3, 17, 5, 4), (2, 64, 9, 64), (2, 65, 64, 33), (64, 256, 32, 32), (1, 1024, 70, 100), (2, 1025, 3, 257), (1, 4096, 20, 512)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("B,T,E,K", SHAPES, ids=lambda v: str(v))
+def test_router_matches_topk(B, T, E, K, dtype):
+    gen = torch.Generator().manual_seed(B + T + E + K)
+    logits = torch.randn(B, T, E, generator=gen).to(dtype)
+    ind_dtype = torch.int16 if dtype is torch.float16 else torch.int64
+    with _abi.launch_log() as log:
+        Ind, scores = expert_choice_router(logits.cuda(), K, ind_dtype)
+    assert log.kernels == ["router_kernel"] and Ind.dtype is ind_dtype and scores.dtype is torch.float32
+    aff = torch.softmax(logits.double(), -1).transpose(1, 2)
+    want = aff.topk(K, -1)[0]
+    Ind, scores = Ind.cpu().long(), scores.cpu()
+    assert ((Ind >= 0) & (Ind < T)).all() and (Ind.sort(-1)[0].diff(dim=-1) > 0).all()
+    assert torch.allclose(scores.double(), want, rtol=1e-5, atol=0)
+    assert torch.allclose(scores.double(), aff.gather(-1, Ind), rtol=1e-5, atol=0)
+    assert (scores.diff(dim=-1) <= 0).all()
+
+
+def test_ties_take_the_lowest_tokens_and_a_nan_comes_first():
+    logits = torch.zeros(2, 100, 3)
+    logits[1, 40] = float("nan")
+    Ind, scores = expert_choice_router(logits.cuda(), 7)
+    assert Ind[0].tolist() == [[0, 1, 2, 3, 4, 5, 6]] * 3
+    assert Ind[1].tolist() == [[40, 0, 1, 2, 3, 4, 5]] * 3 and torch.isnan(scores[1, :, 0]).all()
+
+
+def test_gradients_and_strided_logits_stay_with_torch():
+    logits = torch.randn(2, 33, 4, device="cuda", requires_grad=True)
+    with _abi.launch_log() as log:
+        Ind, scores = expert_choice_router(logits, 5)
+        expert_choice_router(logits.detach().transpose(0, 1), 2)
+    assert log.kernels == []
+    scores.sum().backward()
+    assert logits.grad is not None
+    fast, _ = expert_choice_router(logits.detach(), 5)
+    assert torch.equal(fast, Ind)
