@@ -60,7 +60,10 @@ SIGNATURES = {
     "egs_routing_table_bytes": (_sz, [_dp, _i]),
     "egs_stream_capture_id": (_i, [_vp, ctypes.POINTER(ctypes.c_ulonglong)]),
     "egs_expert_gather_forward_table": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _dp, _i64, _i64, _i, _i, _vp]),
-    "egs_expert_gather_act_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _dp, _i64, _i64, _i, _i, _i, _vp]),
+    "egs_expert_gather_act_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _sz, _dp, _i64, _i64, _i, _i, _i, _vp]),
+    "egs_expert_scatter_bias_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _vp, _vp, _sz, _dp, _i, _i, _i, _vp]),
+    "egs_gather_bias_grad": (_i, [_vp, _vp, _dp, _i, _vp]),
+    "egs_scatter_bias_grad": (_i, [_vp, _vp, _vp, _dp, _i64, _i64, _i, _i, _vp]),
     "egs_expert_scatter_forward_table": (_i, [_vp, _vp, _vp, _vp, _sz, _vp, _vp, _sz, _dp, _i, _i, _i, _vp]),
     "egs_expert_gather_backward_table": (_i, [_vp, _vp, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _sz, _dp, _i64, _i64, _i, _i, _i, _vp]),
     "egs_expert_mlp_supported": (_i, [_dp, _i]),

@@ -115,6 +115,10 @@ int tiled_dw_f32(TiledDwParams &p, hipStream_t s);
 int tiled_dw_f16(TiledDwParams &p, hipStream_t s);
 int tiled_dw_bf16(TiledDwParams &p, hipStream_t s);
 
+// ---- egs_bias.hip: biases added in place, for launches that did not take them along
+int bias_rows(void *Y, const void *bias, const egs_dims *d, int act_dtype, hipStream_t s);
+int bias_scatter(void *Out, const void *bias, const void *Ind, const egs_dims *d, int act_dtype, int ind_dtype, hipStream_t s);
+
 // ---- egs_pass_launch.hip: the one-kernel GEMM-scatter in passes (thousands of picks per batch element, 16-bit types)
 struct PassPlan { bool ok; int units_per_pass; size_t lds; };
 PassPlan scatter_pass_plan(const void *Y, const void *W, const void *Out, const egs_dims *d, int act_dtype);

@@ -963,18 +963,20 @@ int check_table_arg(void *table, size_t table_bytes, const egs_dims *d, int act_
 // ------------------------------------------------------------------------------ implementations
 int gather_gemm_impl(const void *X, const void *W, const void *Ind, void *Y, const float *w_scale,
                      const egs_dims *d, int64_t ldx_b, int64_t ldx_t, int act_dtype, int w_dtype, int ind_dtype,
-                     int w_layout, hipStream_t s, const RoutingTable *build = nullptr, int act = ACT_NONE)
+                     int w_layout, hipStream_t s, const RoutingTable *build = nullptr, int act = ACT_NONE, const void *bias = nullptr)
 {
     const int ES = elem_size(act_dtype), WES = elem_size(w_dtype);
     if (w_scale == nullptr) {
         SmallRowsJob j;
-        if (make_gather_small(X, W, Ind, Y, d, ldx_b, ldx_t, act_dtype, w_dtype, ind_dtype, w_layout, j, build, act))
-            return launch_rows_small_job(j, nullptr, nullptr, s);
+        if (make_gather_small(X, W, Ind, Y, d, ldx_b, ldx_t, act_dtype, w_dtype, ind_dtype, w_layout, j, build, act)) {
+            const int rc = launch_rows_small_job(j, nullptr, nullptr, s);
+            return rc == EGS_OK && bias != nullptr ? bias_rows(Y, bias, d, act_dtype, s) : rc;
+        }
     }
     if (w_scale == nullptr && act_dtype == EGS_F32 && w_dtype == EGS_F32) {
         bool used = false;
         const int rc = gather_small_f32(X, W, Ind, Y, d, ldx_b, ldx_t, ind_dtype, w_layout, s, used, build);
-        if (used) return rc;
+        if (used) return rc == EGS_OK && bias != nullptr ? bias_rows(Y, bias, d, act_dtype, s) : rc;
     }
     if (build != nullptr) {             // no launch for the table to ride in: a launch of its own
         const int rc = launch_routing_table(Ind, ind_dtype, d, build->seg, build->perm, nullptr, nullptr, nullptr, s);
@@ -984,7 +986,7 @@ int gather_gemm_impl(const void *X, const void *W, const void *Ind, void *Y, con
     memset(&p, 0, sizeof(p));
     p.A = (const char *)X; p.W = (const char *)W; p.Ind = Ind; p.C = (char *)Y; p.w_scale = w_scale;
     p.B = d->B; p.T = d->T; p.E = d->E; p.K = d->K;
-    p.act = act;
+    p.act = act; p.bias = bias;
     p.R = d->I; p.N = d->J;
     p.lda_b = ldx_b; p.lda_t = ldx_t;
     p.ind_dtype = ind_dtype;
@@ -998,15 +1000,34 @@ int gather_gemm_impl(const void *X, const void *W, const void *Ind, void *Y, con
             ? ((uint64_t)(d->B - 1) * (uint64_t)ldx_b + (uint64_t)(d->T - 1) * (uint64_t)ldx_t + (uint64_t)d->I) * ES : 0;
         p.a_bytes = span < (1ull << 31) ? (uint32_t)span : 0;
     }
-    return rows_gemm_gather(p, act_dtype, w_dtype == EGS_FP8_E4M3, w_trans, s);
+    const int rc = rows_gemm_gather(p, act_dtype, w_dtype == EGS_FP8_E4M3, w_trans, s);
+    return rc == EGS_OK && bias != nullptr && !p.bias_done ? bias_rows(Y, bias, d, act_dtype, s) : rc;
 }
+
+int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, void *workspace,
+                      const egs_dims *d, int act_dtype, int ind_dtype, int w_layout, int mode, SmallDwJob *dw,
+                      DwTileJob *dwt, hipStream_t s, const RoutingTable *use, const void *bias, bool &with_rows);
 
 // `dw` (optional): a weight gradient of the same call whose first pass may share the product
 // launch and whose second pass may share the reduction launch
 int gemm_scatter_impl(const void *Y, const void *W, const void *Ind, void *Out, void *workspace,
                       const egs_dims *d, int act_dtype, int ind_dtype, int w_layout, int mode, SmallDwJob *dw,
-                      DwTileJob *dwt, hipStream_t s, const RoutingTable *use = nullptr)
+                      DwTileJob *dwt, hipStream_t s, const RoutingTable *use = nullptr, const void *bias = nullptr)
 {
+    if (bias != nullptr) {              // rows of the tiled products come with it; everything else gets it afterwards
+        bool with_rows = false;
+        const int rc = gemm_scatter_rows(Y, W, Ind, Out, workspace, d, act_dtype, ind_dtype, w_layout, mode, dw, dwt, s, use, bias, with_rows);
+        return rc == EGS_OK && !with_rows ? bias_scatter(Out, bias, Ind, d, act_dtype, ind_dtype, s) : rc;
+    }
+    bool none;
+    return gemm_scatter_rows(Y, W, Ind, Out, workspace, d, act_dtype, ind_dtype, w_layout, mode, dw, dwt, s, use, nullptr, none);
+}
+
+int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, void *workspace,
+                      const egs_dims *d, int act_dtype, int ind_dtype, int w_layout, int mode, SmallDwJob *dw,
+                      DwTileJob *dwt, hipStream_t s, const RoutingTable *use, const void *bias, bool &with_rows)
+{
+    with_rows = false;
     const int ES = elem_size(act_dtype);
     const size_t out_elems = (size_t)d->B * d->T * d->I;
     if (out_elems == 0) return EGS_OK;
@@ -1103,7 +1124,9 @@ int gemm_scatter_impl(const void *Y, const void *W, const void *Ind, void *Out, 
             // launch of its own
             const bool no_table = N >= 1 && N <= kTokenSumPicks && !(dw != nullptr && dw->done && dw->q.S > 1);
             p.csr_blocks = (b0 == 0 && N > 0 && !no_table) ? d->B : 0; p.csr_done = 0;
+            p.bias = bias;
             rc = rows_gemm_scatter(p, act_dtype, w_trans, rows_f32 ? EPI_STORE_F32 : EPI_STORE, s);
+            with_rows = p.bias_done != 0;
             if (rc == EGS_OK && no_table) {
                 rc = launch_token_sum(rows, rows_f32, (const char *)Ind + (size_t)b0 * N * ind_size(ind_dtype), ind_dtype,
                                       (char *)Out + (size_t)b0 * d->T * d->I * ES, &sub, act_dtype, s);
@@ -1424,18 +1447,26 @@ int egs_expert_scatter_forward(const void *Y, const void *W, const void *Ind, vo
     return egs_gemm_scatter(Y, W, Ind, Out, workspace, workspace_bytes, d, dtype, ind_dtype, EGS_W_EJI, mode, stream);
 }
 
-int egs_expert_scatter_forward_table(const void *Y, const void *W, const void *Ind, const void *table, size_t table_bytes,
-                                     void *Out, void *workspace, size_t workspace_bytes, const egs_dims *d,
-                                     int dtype, int ind_dtype, int mode, void *stream)
+int egs_expert_scatter_bias_forward(const void *Y, const void *W, const void *bias, const void *Ind, const void *table, size_t table_bytes,
+                                    void *Out, void *workspace, size_t workspace_bytes, const egs_dims *d,
+                                    int dtype, int ind_dtype, int mode, void *stream)
 {
     int rc = validate_scatter(Y, W, Ind, Out, workspace, workspace_bytes, d, dtype, ind_dtype, EGS_W_EJI, mode);
     if (rc != EGS_OK) return rc;
+    if (bias != nullptr && !aligned_to(bias, elem_size(dtype))) return EGS_ERR_ALIGNMENT;
     RoutingTable tab;
     bool have_tab = false;
     rc = check_table_arg(const_cast<void *>(table), table_bytes, d, dtype, tab, have_tab);
     if (rc != EGS_OK) return rc;
     return gemm_scatter_impl(Y, W, Ind, Out, workspace, d, dtype, ind_dtype, EGS_W_EJI, mode, nullptr, nullptr,
-                             (hipStream_t)stream, have_tab ? &tab : nullptr);
+                             (hipStream_t)stream, have_tab ? &tab : nullptr, bias);
+}
+
+int egs_expert_scatter_forward_table(const void *Y, const void *W, const void *Ind, const void *table, size_t table_bytes,
+                                     void *Out, void *workspace, size_t workspace_bytes, const egs_dims *d,
+                                     int dtype, int ind_dtype, int mode, void *stream)
+{
+    return egs_expert_scatter_bias_forward(Y, W, nullptr, Ind, table, table_bytes, Out, workspace, workspace_bytes, d, dtype, ind_dtype, mode, stream);
 }
 
 size_t egs_routing_table_bytes(const egs_dims *d, int dtype)
@@ -1445,7 +1476,7 @@ size_t egs_routing_table_bytes(const egs_dims *d, int dtype)
     return l.ok ? l.bytes : 0;
 }
 
-int egs_expert_gather_act_forward(const void *X, const void *W, const void *Ind, void *Y, void *table, size_t table_bytes,
+int egs_expert_gather_act_forward(const void *X, const void *W, const void *bias, const void *Ind, void *Y, void *table, size_t table_bytes,
                                   const egs_dims *d, int64_t ldx_b, int64_t ldx_t,
                                   int dtype, int ind_dtype, int activation, void *stream)
 {
@@ -1455,20 +1486,21 @@ int egs_expert_gather_act_forward(const void *X, const void *W, const void *Ind,
     if (act < EGS_ACT_NONE || act > EGS_ACT_GELU_TANH) return EGS_ERR_BAD_MODE;
     if (act <= EGS_ACT_RELU) activation = act;      // the same values either way
     if (dtype == EGS_F32 && act != EGS_ACT_NONE) return EGS_ERR_UNSUPPORTED;      // the approximations are for 16-bit results
+    if (bias != nullptr && (act != EGS_ACT_NONE || !aligned_to(bias, elem_size(dtype)))) return act != EGS_ACT_NONE ? EGS_ERR_UNSUPPORTED : EGS_ERR_ALIGNMENT;
     RoutingTable tab;
     bool have_tab = false;
     rc = check_table_arg(table, table_bytes, d, dtype, tab, have_tab);
     if (rc != EGS_OK) return rc;
     if ((size_t)d->B * d->E * d->K * d->J == 0) return EGS_OK;
     return gather_gemm_impl(X, W, Ind, Y, nullptr, d, ldx_b, ldx_t, dtype, dtype, ind_dtype, EGS_W_EIJ, (hipStream_t)stream,
-                            have_tab ? &tab : nullptr, activation);
+                            have_tab ? &tab : nullptr, activation, bias);
 }
 
 int egs_expert_gather_forward_table(const void *X, const void *W, const void *Ind, void *Y, void *table, size_t table_bytes,
                                     const egs_dims *d, int64_t ldx_b, int64_t ldx_t,
                                     int dtype, int ind_dtype, void *stream)
 {
-    return egs_expert_gather_act_forward(X, W, Ind, Y, table, table_bytes, d, ldx_b, ldx_t, dtype, ind_dtype, EGS_ACT_NONE, stream);
+    return egs_expert_gather_act_forward(X, W, nullptr, Ind, Y, table, table_bytes, d, ldx_b, ldx_t, dtype, ind_dtype, EGS_ACT_NONE, stream);
 }
 
 int egs_expert_scatter_backward(const void *Y, const void *W, const void *Ind, const void *grad_Out,

@@ -31,6 +31,8 @@ struct RowsGemmParams {
     int64_t lda_b, lda_t;   // element strides of the [B,T,R] source (gather)
     int32_t ind_dtype;
     int32_t a_vec, w_vec, c_vec;   // 1 when 16-byte accesses are safe on that tensor
+    const void *bias;       // [E,N] in the element type, added to every row of its expert; bias_done: the launch took it along
+    int32_t bias_done;
     int32_t act;            // Activation of a gather's results (not rows_gemm_kernel)
     int32_t m_tiles, n_tiles;
     uint32_t a_bytes;       // extent of A in bytes when it is below 2 GiB, else 0 (direct-load kernel only)

@@ -25,7 +25,7 @@ int launch_rows_atomic(RowsGemmParams &p, hipStream_t s)
 }
 
 // anything the direct-to-LDS kernels do not take
-int launch_rows_tiled(const RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans, bool gather, int epi, hipStream_t s)
+int launch_rows_tiled(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans, bool gather, int epi, hipStream_t s)
 {
     TiledRowsParams q;
     memset(&q, 0, sizeof(q));
@@ -36,7 +36,8 @@ int launch_rows_tiled(const RowsGemmParams &p, int act_dtype, bool fp8_w, bool w
     q.lda_b = p.lda_b; q.lda_t = p.lda_t;
     q.B = p.B; q.T = p.T; q.E = p.E; q.K = p.K; q.R = p.R; q.N = p.N;
     q.ldc = gather ? p.N : product_ld(p.N);
-    q.ind_dtype = p.ind_dtype; q.gather = gather; q.out_f32 = epi == EPI_STORE_F32; q.act = p.act;
+    q.ind_dtype = p.ind_dtype; q.gather = gather; q.out_f32 = epi == EPI_STORE_F32; q.act = p.act; q.bias = (const char *)p.bias;
+    p.bias_done = p.bias != nullptr;
     // which operand to keep in one XCD's L2: source rows that several experts pick, or the experts' weights
     q.rows_major = gather && (double)p.B * p.T * p.R * ES > (double)p.E * p.R * p.N * WES;
     if (fp8_w) return tiled_rows_fp8w(q, w_trans, s);

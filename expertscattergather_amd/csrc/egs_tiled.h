@@ -44,6 +44,7 @@ struct TiledRowsParams {
     const void *Ind;            // gather only
     char *C;                    // [B,E,K,ldc] rows, element type or fp32
     const float *w_scale;       // [E,N] or nullptr
+    const char *bias;           // [E,N] in the element type, or nullptr
     int64_t a_bytes, w_bytes;   // extents of A and W, at least 16
     int64_t lda_b, lda_t;       // element strides of the source (gather)
     int32_t B, T, E, K, R, N, ldc;
@@ -324,6 +325,20 @@ __global__ __launch_bounds__(kThreads) void tiled_rows_kernel(TiledRowsParams p)
 
     // ---------------- results: lane (a, g) holds columns 16 j + 4 g .. + 3 of row 16 i + a; regrouped so that adjacent lanes
     // store adjacent pieces of a row
+    auto as_float = [](const char *at) -> float {
+        if constexpr (ES == 4) return *reinterpret_cast<const float *>(at);
+        else return TT::ID == 2 ? bf16_bits_to_f32(*reinterpret_cast<const uint16_t *>(at)) : f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(at));
+    };
+    if (p.bias != nullptr) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float v = as_float(p.bias + ((int64_t)e * N + min(n0 + j * 16 + g * 4 + r, N - 1)) * ES);
+#pragma unroll
+                for (int i = 0; i < TM; ++i) acc[i][j][r] += v;
+            }
+    }
     auto each = [&](auto fn) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -391,6 +406,7 @@ __global__ __launch_bounds__(kThreads) void tiny_rows_kernel(TiledRowsParams p)
             v += elem(row + (int64_t)r * TT::ES) * wv;
         }
         if (p.w_scale != nullptr) v *= p.w_scale[(int64_t)e * p.N + n];
+        if (p.bias != nullptr) v += elem(p.bias + ((int64_t)e * p.N + n) * TT::ES);
         if constexpr (TT::ES == 2) apply_activation_of<TT>(p.act, [&](auto fn) { v = fn(v); });
         if (TT::ES == 4 || p.out_f32) reinterpret_cast<float *>(p.C)[pick * p.ldc + n] = v;
         else reinterpret_cast<uint16_t *>(p.C)[pick * p.ldc + n] = (uint16_t)f32_to_elem_bits<TT>(v);

@@ -123,10 +123,12 @@ struct Scratch {                // per call, from the caching allocator: stream-
 };
 
 // ------------------------------------------------------------------------------ the four launchers
-Tensor gather_forward(const Problem &p, const Tensor &X, const Tensor &W, const Tensor &Ind, const Tensor &build, int act = EGS_ACT_NONE)
+Tensor gather_forward(const Problem &p, const Tensor &X, const Tensor &W, const Tensor &Ind, const Tensor &build, int act = EGS_ACT_NONE,
+                      const Tensor &bias = Tensor())
 {
     Tensor Y = empty_gpu({p.d.B, p.d.E, p.d.K, p.d.J}, X.scalar_type(), p);
-    const int rc = egs_expert_gather_act_forward(X.const_data_ptr(), W.const_data_ptr(), Ind.const_data_ptr(), Y.data_ptr(),
+    const int rc = egs_expert_gather_act_forward(X.const_data_ptr(), W.const_data_ptr(), bias.defined() ? bias.const_data_ptr() : nullptr,
+                                                 Ind.const_data_ptr(), Y.data_ptr(),
                                                  build.defined() ? build.data_ptr() : nullptr,
                                                  build.defined() ? (size_t)build.numel() : 0, &p.d, (int64_t)p.d.T * p.d.I, p.d.I, p.dt,
                                                  p.ind, act, stream_of(X));
@@ -134,11 +136,13 @@ Tensor gather_forward(const Problem &p, const Tensor &X, const Tensor &W, const 
     return Y;
 }
 
-Tensor scatter_forward(const Problem &p, const Tensor &Y, const Tensor &W, const Tensor &Ind, const Tensor &table, int mode)
+Tensor scatter_forward(const Problem &p, const Tensor &Y, const Tensor &W, const Tensor &Ind, const Tensor &table, int mode,
+                       const Tensor &bias = Tensor())
 {
     Tensor out = empty_gpu({p.d.B, p.d.T, p.d.I}, Y.scalar_type(), p);
     Scratch ws(EGS_OP_GEMM_SCATTER, mode, p);
-    const int rc = egs_expert_scatter_forward_table(Y.const_data_ptr(), W.const_data_ptr(), Ind.const_data_ptr(),
+    const int rc = egs_expert_scatter_bias_forward(Y.const_data_ptr(), W.const_data_ptr(), bias.defined() ? bias.const_data_ptr() : nullptr,
+                                                    Ind.const_data_ptr(),
                                                     table.defined() ? table.const_data_ptr() : nullptr,
                                                     table.defined() ? (size_t)table.numel() : 0, out.data_ptr(), ws.ptr, ws.bytes, &p.d,
                                                     p.dt, p.ind, mode, stream_of(Y));
@@ -146,8 +150,10 @@ Tensor scatter_forward(const Problem &p, const Tensor &Y, const Tensor &W, const
     return out;
 }
 
-std::pair<Tensor, Tensor> gather_backward(const Problem &p, const Tensor &X, const Tensor &W, const Tensor &Ind, const Tensor &table,
-                                          const Tensor &grad_in, int mode)
+struct Grads { Tensor in, W, bias; };
+
+Grads gather_backward(const Problem &p, const Tensor &X, const Tensor &W, const Tensor &Ind, const Tensor &table,
+                                          const Tensor &grad_in, int mode, bool with_bias = false)
 {
     const Tensor grad = dense16(grad_in) ? grad_in : grad_in.clone(at::MemoryFormat::Contiguous);
     Tensor gX = empty_gpu({p.d.B, p.d.T, p.d.I}, X.scalar_type(), p);
@@ -159,10 +165,15 @@ std::pair<Tensor, Tensor> gather_backward(const Problem &p, const Tensor &X, con
                                                     gW.data_ptr(), ws.ptr, ws.bytes, &p.d, (int64_t)p.d.T * p.d.I, p.d.I, p.dt, p.ind, mode,
                                                     stream_of(X));
     raise_status(rc, "expert_gather_backward_call");
-    return {gX, gW};
+    Tensor gb;
+    if (with_bias) {
+        gb = empty_gpu({p.d.E, 1, p.d.J}, X.scalar_type(), p);
+        raise_status(egs_gather_bias_grad(grad.const_data_ptr(), gb.data_ptr(), &p.d, p.dt, stream_of(X)), "egs_gather_bias_grad");
+    }
+    return {gX, gW, gb};
 }
 
-std::pair<Tensor, Tensor> scatter_backward(const Problem &p, const Tensor &Y, const Tensor &W, const Tensor &Ind, const Tensor &grad_in)
+Grads scatter_backward(const Problem &p, const Tensor &Y, const Tensor &W, const Tensor &Ind, const Tensor &grad_in, bool with_bias = false)
 {
     // rows of the incoming gradient may be strided (unit stride inside a row, everything on the 16-byte grid); what else
     // comes - an expanded scalar, a transposed view - is copied
@@ -188,7 +199,14 @@ std::pair<Tensor, Tensor> scatter_backward(const Problem &p, const Tensor &Y, co
                                          gW.data_ptr(), ws.ptr, ws.bytes, &p.d, (int64_t)p.d.T * p.d.I, p.d.I, p.dt, p.ind, stream_of(Y));
     }
     raise_status(rc, "expert_scatter_backward_call");
-    return {gY, gW};
+    Tensor gb;
+    if (with_bias) {
+        gb = empty_gpu({p.d.E, 1, p.d.I}, Y.scalar_type(), p);
+        if (grad.is_contiguous()) { ld_t = p.d.I; ld_b = (int64_t)p.d.T * p.d.I; }
+        raise_status(egs_scatter_bias_grad(grad.const_data_ptr(), Ind.const_data_ptr(), gb.data_ptr(), &p.d, ld_b, ld_t, p.dt, p.ind, stream_of(Y)),
+                     "egs_scatter_bias_grad");
+    }
+    return {gY, gW, gb};
 }
 
 // ------------------------------------------------------------------------------ routing table kept with Ind
@@ -275,12 +293,13 @@ void keep_table(PyObject *ind_obj, const TableKey &k, const Tensor &table)
 // Same contract as the Python Functions of hip_kernels.py: what is saved is the inputs (and the routing table that was
 // valid in the forward); the scatter mode is the forward's; both gradients are always computed.
 struct ExpertGatherFunctionNative : public torch::autograd::Function<ExpertGatherFunctionNative> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &X, const Tensor &W, const Tensor &Ind, const std::optional<Tensor> &table, bool build,
-                          int64_t mode)
+    static Tensor forward(AutogradContext *ctx, const Tensor &X, const Tensor &W, const Tensor &Ind, const std::optional<Tensor> &bias,
+                          const std::optional<Tensor> &table, bool build, int64_t mode)
     {
         ctx->save_for_backward({X, W, Ind, table.value_or(Tensor())});
         ctx->saved_data["mode"] = mode;
-        return gather_forward(problem_of(X, W, Ind, true, true, 0), X, W, Ind, build ? *table : Tensor());
+        ctx->saved_data["bias"] = bias.has_value();
+        return gather_forward(problem_of(X, W, Ind, true, true, 0), X, W, Ind, build ? *table : Tensor(), EGS_ACT_NONE, bias.value_or(Tensor()));
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
@@ -289,18 +308,19 @@ struct ExpertGatherFunctionNative : public torch::autograd::Function<ExpertGathe
         const Problem p = problem_of(X, W, Ind, true, true, 0);
         TORCH_CHECK(p.ok && plain(grads[0]) && grads[0].scalar_type() == X.scalar_type(), "expert_gather_backward: unexpected operands");
         at::AutoDispatchBelowADInplaceOrView below;
-        auto g = gather_backward(p, X, W, Ind, saved[3], grads[0], (int)ctx->saved_data["mode"].toInt());
-        return {g.first, g.second, Tensor(), Tensor(), Tensor(), Tensor()};
+        Grads g = gather_backward(p, X, W, Ind, saved[3], grads[0], (int)ctx->saved_data["mode"].toInt(), ctx->saved_data["bias"].toBool());
+        return {g.in, g.W, Tensor(), g.bias, Tensor(), Tensor(), Tensor()};
     }
 };
 
 struct ExpertScatterFunctionNative : public torch::autograd::Function<ExpertScatterFunctionNative> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &Y, const Tensor &W, const Tensor &Ind, const std::optional<Tensor> &table, int64_t T,
-                          int64_t mode)
+    static Tensor forward(AutogradContext *ctx, const Tensor &Y, const Tensor &W, const Tensor &Ind, const std::optional<Tensor> &bias,
+                          const std::optional<Tensor> &table, int64_t T, int64_t mode)
     {
         ctx->save_for_backward({Y, W, Ind});
         ctx->saved_data["T"] = T;
-        return scatter_forward(problem_of(Y, W, Ind, false, false, T), Y, W, Ind, table.value_or(Tensor()), (int)mode);
+        ctx->saved_data["bias"] = bias.has_value();
+        return scatter_forward(problem_of(Y, W, Ind, false, false, T), Y, W, Ind, table.value_or(Tensor()), (int)mode, bias.value_or(Tensor()));
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
@@ -309,14 +329,20 @@ struct ExpertScatterFunctionNative : public torch::autograd::Function<ExpertScat
         const Problem p = problem_of(Y, W, Ind, false, false, ctx->saved_data["T"].toInt());
         TORCH_CHECK(p.ok && plain(grads[0]) && grads[0].scalar_type() == Y.scalar_type(), "expert_scatter_backward: unexpected operands");
         at::AutoDispatchBelowADInplaceOrView below;
-        auto g = scatter_backward(p, Y, W, Ind, grads[0]);
-        return {g.first, g.second, Tensor(), Tensor(), Tensor(), Tensor()};
+        Grads g = scatter_backward(p, Y, W, Ind, grads[0], ctx->saved_data["bias"].toBool());
+        return {g.in, g.W, Tensor(), g.bias, Tensor(), Tensor(), Tensor()};
     }
 };
 
-bool records(const Tensor &a, const Tensor &b)
+bool records(const Tensor &a, const Tensor &b, const Tensor &c)
 {
-    return at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad());
+    return at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad() || (c.defined() && c.requires_grad()));
+}
+// [E,1,N] in the operands' type, dense
+bool bias_fits(const Tensor &b, const Tensor &W, int64_t E, int64_t N)
+{
+    return plain(b) && b.dim() == 3 && b.size(0) == E && b.size(1) == 1 && b.size(2) == N && b.scalar_type() == W.scalar_type() &&
+           b.device() == W.device() && b.is_contiguous();
 }
 std::optional<Tensor> some(const Tensor &t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
 bool has_tangent(const Tensor &t) { return t._fw_grad(0).defined(); }
@@ -352,17 +378,23 @@ PyObject *pair(std::pair<Tensor, Tensor> &&t)
     return Py_BuildValue("(NN)", a, b);
 }
 
-// gather_forward(X, W, Ind, out_dtype, mode, keep_table, record) -> Y or None; record: with an autograd node where one is due
+// gather_forward(X, W, Ind, out_dtype, mode, keep_table, record, bias or None) -> Y or None; record: with an autograd node where
+// one is due
 PyObject *py_gather_forward(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
-    if (!want(n, 7, "gather_forward")) return nullptr;
-    if (!plain_object(a[0]) || !plain_object(a[1]) || !plain_object(a[2])) Py_RETURN_NONE;
+    if (!want(n, 8, "gather_forward")) return nullptr;
+    if (!plain_object(a[0]) || !plain_object(a[1]) || !plain_object(a[2]) || (a[7] != Py_None && !plain_object(a[7]))) Py_RETURN_NONE;
     const Tensor &X = THPVariable_Unpack(a[0]), &W = THPVariable_Unpack(a[1]), &Ind = THPVariable_Unpack(a[2]);
     const Problem p = problem_of(X, W, Ind, true, true, 0);
     if (!p.ok || !type_fits(a[3], X) || !no_modes()) Py_RETURN_NONE;
     const bool record = flag(a[6]);
-    if (record && (has_tangent(X) || has_tangent(W))) Py_RETURN_NONE;
+    Tensor bias;
+    if (a[7] != Py_None) {
+        bias = THPVariable_Unpack(a[7]);
+        if (!bias_fits(bias, W, p.d.E, p.d.J)) Py_RETURN_NONE;
+    }
+    if (record && (has_tangent(X) || has_tangent(W) || (bias.defined() && has_tangent(bias)))) Py_RETURN_NONE;
     TableState ts = table_state(a[2], Ind, p, flag(a[5]));
     Tensor table = ts.table, Y;
     const int64_t mode = PyLong_AsLong(a[4]);
@@ -370,20 +402,21 @@ PyObject *py_gather_forward(PyObject *, PyObject *const *a, Py_ssize_t n)
     {
         NoGil nogil;
         if (build) table = empty_gpu({(int64_t)ts.bytes}, at::kByte, p);
-        if (record && records(X, W)) Y = ExpertGatherFunctionNative::apply(X, W, Ind, some(table), build, mode);
-        else Y = gather_forward(p, X, W, Ind, build ? table : Tensor());
+        if (record && records(X, W, bias)) Y = ExpertGatherFunctionNative::apply(X, W, Ind, some(bias), some(table), build, mode);
+        else Y = gather_forward(p, X, W, Ind, build ? table : Tensor(), EGS_ACT_NONE, bias);
     }
     if (build) keep_table(a[2], ts.key, table);
     return THPVariable_Wrap(std::move(Y));
     END_HANDLE_TH_ERRORS
 }
 
-// scatter_forward(Y, W, Ind, T, out_dtype, mode, keep_table, record) -> out or None
+// scatter_forward(Y, W, Ind, T, out_dtype, mode, keep_table, record, bias or None) -> out or None
 PyObject *py_scatter_forward(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
-    if (!want(n, 8, "scatter_forward")) return nullptr;
-    if (!plain_object(a[0]) || !plain_object(a[1]) || !plain_object(a[2]) || !PyLong_CheckExact(a[3])) Py_RETURN_NONE;
+    if (!want(n, 9, "scatter_forward")) return nullptr;
+    if (!plain_object(a[0]) || !plain_object(a[1]) || !plain_object(a[2]) || !PyLong_CheckExact(a[3]) || (a[8] != Py_None && !plain_object(a[8])))
+        Py_RETURN_NONE;
     const Tensor &Y = THPVariable_Unpack(a[0]), &W = THPVariable_Unpack(a[1]), &Ind = THPVariable_Unpack(a[2]);
     int overflow = 0;
     const int64_t T = PyLong_AsLongLongAndOverflow(a[3], &overflow);
@@ -391,14 +424,19 @@ PyObject *py_scatter_forward(PyObject *, PyObject *const *a, Py_ssize_t n)
     const Problem p = problem_of(Y, W, Ind, false, false, T);
     if (!p.ok || !type_fits(a[4], Y) || !no_modes()) Py_RETURN_NONE;
     const bool record = flag(a[7]);
-    if (record && (has_tangent(Y) || has_tangent(W))) Py_RETURN_NONE;
+    Tensor bias;
+    if (a[8] != Py_None) {
+        bias = THPVariable_Unpack(a[8]);
+        if (!bias_fits(bias, W, p.d.E, p.d.I)) Py_RETURN_NONE;
+    }
+    if (record && (has_tangent(Y) || has_tangent(W) || (bias.defined() && has_tangent(bias)))) Py_RETURN_NONE;
     const int mode = (int)PyLong_AsLong(a[5]);
     const TableState ts = table_state(a[2], Ind, p, flag(a[6]));
     Tensor out;
     {
         NoGil nogil;
-        if (record && records(Y, W)) out = ExpertScatterFunctionNative::apply(Y, W, Ind, some(ts.table), T, (int64_t)mode);
-        else out = scatter_forward(p, Y, W, Ind, ts.table, mode);
+        if (record && records(Y, W, bias)) out = ExpertScatterFunctionNative::apply(Y, W, Ind, some(bias), some(ts.table), T, (int64_t)mode);
+        else out = scatter_forward(p, Y, W, Ind, ts.table, mode, bias);
     }
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
@@ -418,12 +456,12 @@ PyObject *py_gather_backward(PyObject *, PyObject *const *a, Py_ssize_t n)
         Py_RETURN_NONE;
     const int mode = (int)PyLong_AsLong(a[5]);
     const TableState ts = table_state(a[2], Ind, p, flag(a[6]));
-    std::pair<Tensor, Tensor> g;
+    Grads g;
     {
         NoGil nogil;
         g = gather_backward(p, X, W, Ind, ts.table, G, mode);
     }
-    return pair(std::move(g));
+    return pair({g.in, g.W});
     END_HANDLE_TH_ERRORS
 }
 
@@ -440,12 +478,12 @@ PyObject *py_scatter_backward(PyObject *, PyObject *const *a, Py_ssize_t n)
     if (!p.ok || !type_fits(a[4], Y) || !no_modes() || !plain(G) || G.scalar_type() != Y.scalar_type() || G.device() != Y.device() ||
         G.size(0) != p.d.B || G.size(2) != p.d.I || !dense16(G))
         Py_RETURN_NONE;
-    std::pair<Tensor, Tensor> g;
+    Grads g;
     {
         NoGil nogil;
         g = scatter_backward(p, Y, W, Ind, G);
     }
-    return pair(std::move(g));
+    return pair({g.in, g.W});
     END_HANDLE_TH_ERRORS
 }
 

@@ -607,7 +607,7 @@ def create_kernels() -> None:
         def gather_forward_call(X, W, Ind, out_dtype):
             if type(X) in plain and X.is_cuda and not compiling():
                 ext = _abi.torch_ext()
-                Y = None if ext is None else ext.gather_forward(X, W, Ind, out_dtype, 0, _table_cache, False)
+                Y = None if ext is None else ext.gather_forward(X, W, Ind, out_dtype, 0, _table_cache, False, None)
                 return _gather_forward_impl(X, W, Ind, out_dtype) if Y is None else Y
             return ops.expert_gather_forward_call_fn(X, W, Ind, out_dtype)
 
@@ -621,7 +621,7 @@ def create_kernels() -> None:
         def scatter_forward_call(Y, W, Ind, T, out_dtype):
             if type(Y) in plain and Y.is_cuda and not compiling():
                 ext = _abi.torch_ext()
-                out = None if ext is None else ext.scatter_forward(Y, W, Ind, T, out_dtype, _MODES[get_scatter_mode()], _table_cache, False)
+                out = None if ext is None else ext.scatter_forward(Y, W, Ind, T, out_dtype, _MODES[get_scatter_mode()], _table_cache, False, None)
                 return _scatter_forward_impl(Y, W, Ind, T, out_dtype) if out is None else out
             return ops.expert_scatter_forward_call_fn(Y, W, Ind, T, out_dtype)
 
@@ -698,35 +698,51 @@ class ExpertScatterFunction(torch.autograd.Function):
         return (grad_Y, grad_W) + (None,) * (len(ctx.needs_input_grad) - 2)
 
 
-def expert_gather(X: torch.Tensor, W: torch.Tensor, Ind: torch.Tensor, scatter_mode=None) -> torch.Tensor:
+def expert_gather(X: torch.Tensor, W: torch.Tensor, Ind: torch.Tensor, scatter_mode=None, bias=None) -> torch.Tensor:
     """What `ExpertGather` computes: `ExpertGatherFunction.apply(X, W, Ind)` with `scatter_mode` (None: the mode in force) for
-    the backward, as one C++ autograd node (csrc/egs_torch.cpp) where the operands allow it."""
+    the backward, plus `bias` [E,1,J]; as one C++ autograd node (csrc/egs_torch.cpp) where the operands allow it."""
     if not torch.compiler.is_compiling():
         ext = _abi.torch_ext()
         if ext is not None:
             mode = get_scatter_mode() if scatter_mode is None else _check_mode(scatter_mode)
-            Y = ext.gather_forward(X, W, Ind, torch.float32, _MODES[mode], _table_cache, True)
+            Y = ext.gather_forward(X, W, Ind, torch.float32, _MODES[mode], _table_cache, True, bias)
             if Y is not None:
                 return Y
     if scatter_mode is None:
-        return ExpertGatherFunction.apply(X, W, Ind)
-    with scatter_mode_scope(scatter_mode):          # bound to the autograd node: the backward runs in it too
-        return ExpertGatherFunction.apply(X, W, Ind)
+        Y = ExpertGatherFunction.apply(X, W, Ind)
+    else:
+        with scatter_mode_scope(scatter_mode):          # bound to the autograd node: the backward runs in it too
+            Y = ExpertGatherFunction.apply(X, W, Ind)
+    return Y if bias is None else Y + bias
 
 
-def expert_scatter(Y: torch.Tensor, W: torch.Tensor, Ind: torch.Tensor, T: int, scatter_mode=None) -> torch.Tensor:
-    """What `ExpertScatter` computes: `ExpertScatterFunction.apply(Y, W, Ind, T)` in `scatter_mode`, see `expert_gather`."""
+def expert_scatter(Y: torch.Tensor, W: torch.Tensor, Ind: torch.Tensor, T: int, scatter_mode=None, bias=None) -> torch.Tensor:
+    """What `ExpertScatter` computes: `ExpertScatterFunction.apply(Y, W, Ind, T)` in `scatter_mode`, plus bias[e] of `bias`
+    [E,1,I] for every pick of expert e on the token it lands on; see `expert_gather`."""
     if not torch.compiler.is_compiling():
         ext = _abi.torch_ext()
         if ext is not None:
             mode = get_scatter_mode() if scatter_mode is None else _check_mode(scatter_mode)
-            out = ext.scatter_forward(Y, W, Ind, T, torch.float32, _MODES[mode], _table_cache, True)
+            out = ext.scatter_forward(Y, W, Ind, T, torch.float32, _MODES[mode], _table_cache, True, bias)
             if out is not None:
                 return out
     if scatter_mode is None:
-        return ExpertScatterFunction.apply(Y, W, Ind, T)
-    with scatter_mode_scope(scatter_mode):
-        return ExpertScatterFunction.apply(Y, W, Ind, T)
+        out = ExpertScatterFunction.apply(Y, W, Ind, T)
+    else:
+        with scatter_mode_scope(scatter_mode):
+            out = ExpertScatterFunction.apply(Y, W, Ind, T)
+    if bias is not None and T > 0 and Ind.numel() > 0:
+        # picks[b,t,e] = how many times expert e selected token t; each adds bias[e]
+        # (a pick outside [0,T) contributes nothing, as in the kernels: it is routed to slot 0 with weight 0)
+        B, E, K = Ind.shape
+        picks = torch.zeros(B, T, E, device=out.device, dtype=torch.float32)
+        e_ids = torch.arange(E, device=out.device).view(1, E, 1).expand(B, E, K).reshape(B, E * K)
+        ind = Ind.to(torch.int64).reshape(B, E * K)
+        valid = (ind >= 0) & (ind < T)
+        flat = torch.where(valid, ind * E + e_ids, torch.zeros_like(ind))
+        picks.view(B, T * E).scatter_add_(1, flat, valid.to(torch.float32))
+        out = out + (picks @ bias[:, 0, :].float()).to(out.dtype)
+    return out
 
 
 # ------------------------------------------------------------------------------ extras (not in the reference)

@@ -256,12 +256,22 @@ int egs_expert_mlp_forward(const void *X, const void *Wg, const void *Ws, const 
  * Launcher-level entry points (one per reference callable)
  * ------------------------------------------------------------------------------------- */
 
-/* egs_expert_gather_forward_table with an activation applied to the products before they are stored (table may be null).
- * Large products round to the element type before it in any case.  16-bit types; fp32 with an
- * activation returns EGS_ERR_UNSUPPORTED. */
-int egs_expert_gather_act_forward(const void *X, const void *W, const void *Ind, void *Y, void *table, size_t table_bytes,
+/* egs_expert_gather_forward_table with a bias [E,J] added to, or an activation applied to, the products before they are stored
+ * (table and bias may be null).  Large products round to the element type before it in any case.  Activations: 16-bit types;
+ * fp32 with an activation, or both at once, returns EGS_ERR_UNSUPPORTED. */
+int egs_expert_gather_act_forward(const void *X, const void *W, const void *bias, const void *Ind, void *Y, void *table, size_t table_bytes,
                                   const egs_dims *d, int64_t ldx_b, int64_t ldx_t,
                                   int dtype, int ind_dtype, int activation, void *stream);
+
+/* egs_expert_scatter_forward_table with a bias [E,I]: every pick of expert e inside [0,T) adds bias[e] to its token */
+int egs_expert_scatter_bias_forward(const void *Y, const void *W, const void *bias, const void *Ind, const void *table, size_t table_bytes,
+                                    void *Out, void *workspace, size_t workspace_bytes, const egs_dims *d,
+                                    int dtype, int ind_dtype, int mode, void *stream);
+
+/* gradients of the biases: grad_bias[e,:] = sum over the expert's picks of grad_Y[b,e,k,:], or of grad_Out[b,Ind[b,e,k],:] */
+int egs_gather_bias_grad(const void *grad_Y, void *grad_bias, const egs_dims *d, int dtype, void *stream);
+int egs_scatter_bias_grad(const void *grad_Out, const void *Ind, void *grad_bias, const egs_dims *d, int64_t ldg_b, int64_t ldg_t,
+                          int dtype, int ind_dtype, void *stream);
 
 /* expert_gather_forward_call(X, W[E,I,J], Ind) -> Y          reference egs/triton_kernels.py:367-392 */
 int egs_expert_gather_forward(const void *X, const void *W, const void *Ind, void *Y,

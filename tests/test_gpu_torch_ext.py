@@ -18,17 +18,19 @@ SHAPES = [(4, 64, 8, 16, 128, 64),       # one-kernel scatter with a routing tab
           (2, 300, 4, 200, 256, 192)]
 
 
-def step(case, dtype, ind, grad_of, mode):
+def step(case, dtype, ind, grad_of, mode, bias=False):
     B, T, E, K, I, J = case["shape"]
-    g, s = egs.ExpertGather(E, I, J).to(DEV, dtype), egs.ExpertScatter(E, J, I).to(DEV, dtype)
+    g, s = egs.ExpertGather(E, I, J, bias=bias).to(DEV, dtype), egs.ExpertScatter(E, J, I, bias=bias).to(DEV, dtype)
     with torch.no_grad():
         g.W.copy_(case["Wg"]); s.W.copy_(case["Ws"])
+        if bias:
+            g.bias.copy_(case["X"][0, 0, :1].expand(E, 1, J) + torch.arange(E)[:, None, None]); s.bias.copy_(case["dOut"][0, 0].expand(E, 1, I))
     g.scatter_mode = s.scatter_mode = mode
     x = case["X"].to(DEV).requires_grad_(True)
     out = s(g(x, ind), ind, T)
     out.backward(grad_of(out))
     torch.cuda.synchronize()
-    return out.detach(), x.grad, g.W.grad, s.W.grad
+    return (out.detach(), x.grad, g.W.grad, s.W.grad) + ((g.bias.grad, s.bias.grad) if bias else ())
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
@@ -50,6 +52,27 @@ def test_the_two_routes_agree(shape, dtype, grad, monkeypatch):
     slow = step(case, dtype, Ind.to(DEV), grad_of, mode)
     for name, a, b in zip(("out", "dX", "dWg", "dWs"), fast, slow):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("shape", SHAPES + [(40, 30, 3, 30, 70, 33)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("mode", ["deterministic", "atomic"])
+def test_biases_and_their_gradients(shape, dtype, mode, monkeypatch):
+    """Added by the launch itself or by one of its own (csrc/egs_bias.hip), against the composition from torch operations; picks
+    outside [0, T) bring no bias in the scatter, and one in the gather."""
+    B, T, E, K, I, J = shape
+    case = dict(make_case(19 + sum(shape), *shape, dtype), shape=shape)
+    Ind = case["Ind"].clone()
+    if E * K > 1:
+        Ind[0, 0, 0], Ind[-1, -1, -1] = T, -1
+    grad_of = lambda out: case["dOut"].to(DEV)
+    fast = step(case, dtype, Ind.to(DEV), grad_of, mode, True)
+    monkeypatch.setattr(_abi, "_pycall", None)
+    slow = step(case, dtype, Ind.to(DEV), grad_of, mode, True)
+    tol = {torch.float32: 2e-5, torch.float16: 4e-3, torch.bfloat16: 3e-2}[dtype]
+    for name, a, b in zip(("out", "dX", "dWg", "dWs", "db_gather", "db_scatter"), fast, slow):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        assert (a.float() - b.float()).abs().max() <= tol * b.float().abs().max(), name
 
 
 def test_autograd_contract_of_the_native_nodes():
@@ -80,7 +103,7 @@ def test_what_the_native_route_declines_goes_the_python_way():
     case = make_case(11, *shape, torch.float32)
     X, W, Ind = case["X"].to(DEV), case["Wg"].to(DEV), case["Ind"].to(DEV)
     ext = _abi.torch_ext()
-    call = lambda x, w, i, t=torch.float32: ext.gather_forward(x, w, i, t, 0, False, False)
+    call = lambda x, w, i, t=torch.float32: ext.gather_forward(x, w, i, t, 0, False, False, None)
     assert call(X, W, Ind) is not None
     off = torch.empty(X.numel() + 1, device=DEV)[1:].view_as(X).copy_(X)
     for args in [(X.transpose(0, 1).contiguous().transpose(0, 1), W, Ind), (off, W, Ind), (X.bfloat16(), W, Ind), (X.cpu(), W, Ind),
