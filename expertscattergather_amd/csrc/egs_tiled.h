@@ -67,9 +67,15 @@ struct TiledLds {
     static constexpr int BYTES = 2 * STAGE;
 };
 
+// Wavefronts per SIMD that the registers are bounded for: where there are workgroups enough, several of them to a CU hide one's
+// round trips behind the others' matrix instructions (DEEP = false: two slabs in flight each; B53 K41 E29 I111 J75 fp32 gather
+// 25.8 us with one or two workgroups to a CU, see launch_tiled for the figures now); a problem of a few workgroups keeps four
+// slabs in flight instead and takes the registers it likes.
+template <int TM, int TN, bool DEEP> constexpr int tiled_waves() { return DEEP ? 1 : TM * TN <= 2 ? 4 : TM * TN <= 6 ? 3 : 2; }
+
 // 64 * TM rows x 16 * TN columns per workgroup of four wavefronts, each 16 * TM rows x all columns.
-template <class TT, int WES, bool W_TRANS, int TM, int TN>
-__global__ __launch_bounds__(kThreads) void tiled_rows_kernel(TiledRowsParams p)
+template <class TT, int WES, bool W_TRANS, int TM, int TN, bool DEEP>
+__global__ __launch_bounds__(kThreads, (tiled_waves<TM, TN, DEEP>())) void tiled_rows_kernel(TiledRowsParams p)
 {
     constexpr int ES = TT::ES, VEC = TT::VEC;
     constexpr bool W_FP8 = WES == 1;
@@ -81,7 +87,7 @@ __global__ __launch_bounds__(kThreads) void tiled_rows_kernel(TiledRowsParams p)
     constexpr int WPR = W_TRANS ? BN * WES / 16 : CH * WES / ES;        // chunks per source row
     constexpr int WCH = WPR * (W_TRANS ? BKE : BN);
     constexpr int NW = (WCH + kThreads - 1) / kThreads;
-    constexpr int D = NA + NW <= 5 ? 4 : 2;                             // slabs in flight in registers
+    constexpr int D = DEEP ? 4 : 2;                                     // slabs in flight in registers
     extern __shared__ __attribute__((aligned(16))) char smem_tiled[];
 
     const int total = p.E * p.m_tiles * p.n_tiles;
@@ -112,134 +118,106 @@ __global__ __launch_bounds__(kThreads) void tiled_rows_kernel(TiledRowsParams p)
         for (int i = 0; i < NA; ++i) iw[i] = load_index_word(p.Ind, p.ind_dtype, apick[i]);
     }
 
-    // ---------------- weight side
+    // ---------------- weight side: byte offsets from the expert's matrix.  A chunk may lie past the reduction length, past the last
+    // column or past the matrix: those values are cleared, never stored, or read early (`w_last`: the last 16 bytes of W)
     const char *We = p.W + (int64_t)e * R * N * WES;
-    const char *w_last = p.W + p.w_bytes - 16;
-    u32x4 wreg[D][NW];
-    auto w_at = [&](int kt, int i) -> const char * {                    // address of chunk i of slab kt, before the clamp
+    const int64_t to_end = p.w_bytes - 16 - (int64_t)e * R * N * WES;
+    const uint32_t w_last = to_end > 0xffffff00ll ? 0xffffff00u : (uint32_t)to_end;
+    const uint32_t w_step = (uint32_t)BKE * (W_TRANS ? (uint32_t)N : 1u) * WES;
+    uint32_t woff[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
         const int v = min(tid + i * kThreads, WCH - 1);
-        if constexpr (W_TRANS) {
-            const int r = min(kt * BKE + v / WPR, R - 1);
-            int n = n0 + (v % WPR) * (16 / WES);
-            if (n >= N) n = n0;
-            return We + ((int64_t)r * N + n) * WES;
-        } else {
-            const int n = min(n0 + v / WPR, N - 1);
-            int k = kt * BKE + (v % WPR) * (16 / WES);
-            if (k >= R) k = 0;
-            return We + ((int64_t)n * R + k) * WES;
-        }
-    };
+        if constexpr (W_TRANS) woff[i] = ((uint32_t)(v / WPR) * (uint32_t)N + (uint32_t)n0) * WES + (uint32_t)(v % WPR) * 16u;
+        else woff[i] = (uint32_t)min(n0 + v / WPR, N - 1) * (uint32_t)R * WES + (uint32_t)(v % WPR) * 16u;
+    }
+    u32x4 wreg[D][NW];
     auto issue_w = [&](int kt, u32x4 (&set)[NW]) {
 #pragma unroll
-        for (int i = 0; i < NW; ++i) {
-            const char *at = w_at(kt, i);
-            set[i] = *reinterpret_cast<const u32x4_any *>(at < w_last ? at : w_last);
-        }
+        for (int i = 0; i < NW; ++i) set[i] = *reinterpret_cast<const u32x4_any *>(We + min(woff[i] + (uint32_t)kt * w_step, w_last));
     };
-    // the same chunks in A
-    const char *arow[NA];
+    int64_t arow[NA];           // byte offsets (always from p.A: the compiler then knows the loads are global ones)
     int alive = 0;
-    const char *a_last = p.A + p.a_bytes - 16;
+    const int64_t a_last = p.a_bytes - 16;
     u32x4 areg[D][NA];
-    auto a_at = [&](int kt, int i) -> const char * {
-        int k = kt * BKE + ac * VEC;
-        if (k >= R) k = 0;
-        return arow[i] + (int64_t)k * ES;
-    };
     auto issue_a = [&](int kt, u32x4 (&set)[NA]) {
 #pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            const char *at = a_at(kt, i);
-            set[i] = *reinterpret_cast<const u32x4_any *>(at < a_last ? at : a_last);
-        }
+        for (int i = 0; i < NA; ++i) set[i] = *reinterpret_cast<const u32x4_any *>(p.A + min(arow[i] + kt * (CH * 16), a_last));
     };
 
+    // slabs beyond the last are requested as the last one again: no load is conditional, so that the compiler can count the
+    // outstanding ones and waits for one slab's only
 #pragma unroll
-    for (int d = 0; d < D; ++d)
-        if (d < nk) issue_w(d, wreg[d]);
+    for (int d = 0; d < D; ++d) issue_w(min(d, nk - 1), wreg[d]);
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
         const int m = m0 + tid / CH + i * (kThreads / CH);
         if (p.gather) {
             const int64_t t = decode_index_word(iw[i], p.Ind, p.ind_dtype, apick[i]);
             const bool ok = m < Me && t >= 0 && t < (int64_t)p.T;
-            arow[i] = p.A + (ok ? ((int64_t)ab[i] * p.lda_b + t * p.lda_t) * ES : 0);
+            arow[i] = (ok ? ((int64_t)ab[i] * p.lda_b + t * p.lda_t) * ES : 0) + ac * 16;
             alive |= (int)ok << i;
         } else {
-            arow[i] = p.A + apick[i] * R * ES;
+            arow[i] = apick[i] * R * ES + ac * 16;
             alive |= (int)(m < Me) << i;
         }
     }
 #pragma unroll
-    for (int d = 0; d < D; ++d)
-        if (d < nk) issue_a(d, areg[d]);
+    for (int d = 0; d < D; ++d) issue_a(min(d, nk - 1), areg[d]);
 
     // ---------------- registers -> LDS.  `edge` (the last slab, and every slab of a matrix whose rows are shorter than a chunk):
     // chunks that were read early are shifted into place and what lies past the reduction length is cleared on both sides
-    const bool short_rows = (int64_t)N * WES < 16;
-    auto commit_a = [&](const u32x4 (&set)[NA], int kt, char *stage) {
-        u32x4 *tile = reinterpret_cast<u32x4 *>(stage);
-        const bool edge = kt >= nk - 1;
-        const int left = (R - kt * BKE - ac * VEC) * ES;                // valid bytes of this thread's chunk
-#pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            u32x4 v = set[i];
-            if (edge) {
-                const char *at = a_at(kt, i);
-                if (at > a_last) v = shift_right_bytes(v, (int)(at - a_last));
-#pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    const int nb = left - 4 * x;
-                    v[x] &= nb >= 4 ? 0xffffffffu : nb == 2 ? 0xffffu : 0u;
-                }
-            }
-            if (!((alive >> i) & 1)) v = u32x4{0u, 0u, 0u, 0u};
-            tile[tile_chunk_index<CH>(tid / CH + i * (kThreads / CH), ac)] = v;
-        }
-    };
+    const bool short_rows = W_TRANS && (int64_t)N * WES < 16;
     auto w_off = [&](int r, int col_bytes) -> int {                     // byte offset in a [reduction][column] tile
         return ES == 2 ? r * L::WROW + (r >> 3) * 128 + col_bytes : r * L::WROW + col_bytes;
     };
-    auto commit_w = [&](const u32x4 (&set)[NW], int kt, char *stage) {
-        char *tile = stage + L::A;
-        const bool edge = kt >= nk - 1 || (W_TRANS && short_rows);
+    auto clear_past = [](u32x4 &v, int left) {                          // keeps the first `left` bytes
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const int nb = left - 4 * x;
+            v[x] &= nb >= 4 ? 0xffffffffu : nb <= 0 ? 0u : 0xffffffffu >> (32 - 8 * nb);
+        }
+    };
+    auto fix_edge = [&](u32x4 (&av)[NA], u32x4 (&wv)[NW], int kt) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const int64_t past = arow[i] + kt * (CH * 16) - a_last;
+            if (past > 0) av[i] = shift_right_bytes(av[i], (int)min(past, (int64_t)15));
+            clear_past(av[i], R * ES - kt * (CH * 16) - ac * 16);
+        }
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            const int v = min(tid + i * kThreads, WCH - 1);
+            const uint32_t off = woff[i] + (uint32_t)kt * w_step;
+            if (off > w_last) wv[i] = shift_right_bytes(wv[i], (int)min(off - w_last, 15u));
+            if constexpr (W_TRANS) { if (kt * BKE + v / WPR >= R) wv[i] = u32x4{0u, 0u, 0u, 0u}; }
+            else clear_past(wv[i], (R - kt * BKE) * WES - (v % WPR) * 16);
+        }
+    };
+    auto commit = [&](u32x4 (&av)[NA], u32x4 (&wv)[NW], char *stage) {
+        u32x4 *ta = reinterpret_cast<u32x4 *>(stage);
+        char *tw = stage + L::A;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const uint32_t keep = (alive >> i) & 1 ? 0xffffffffu : 0u;
+            ta[tile_chunk_index<CH>(tid / CH + i * (kThreads / CH), ac)] = u32x4{av[i][0] & keep, av[i][1] & keep, av[i][2] & keep, av[i][3] & keep};
+        }
 #pragma unroll
         for (int i = 0; i < NW; ++i) {
             const int v = tid + i * kThreads;
             if (WCH % kThreads != 0 && v >= WCH) continue;
-            u32x4 w = set[i];
-            if (edge) {
-                const char *at = w_at(kt, i);
-                if (at > w_last) w = shift_right_bytes(w, (int)(at - w_last));
-                if constexpr (W_TRANS) {
-                    if (kt * BKE + v / WPR >= R) w = u32x4{0u, 0u, 0u, 0u};
-                } else {
-                    const int left = (R - kt * BKE - (v % WPR) * (16 / WES)) * WES;
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) {
-                        const int nb = left - 4 * x;
-                        w[x] &= nb >= 4 ? 0xffffffffu : nb <= 0 ? 0u : 0xffffffffu >> (32 - 8 * nb);
-                    }
-                }
-            }
-            if constexpr (W_TRANS) {
-                const int r = v / WPR, cb = (v % WPR) * (W_FP8 ? 32 : 16);
-                if constexpr (W_FP8) {
-                    *reinterpret_cast<u32x4 *>(tile + w_off(r, cb)) = fp8x8_to_bf16_chunk(w[0], w[1]);
-                    *reinterpret_cast<u32x4 *>(tile + w_off(r, cb) + 16) = fp8x8_to_bf16_chunk(w[2], w[3]);
-                } else {
-                    *reinterpret_cast<u32x4 *>(tile + w_off(r, cb)) = w;
-                }
+            const u32x4 w = wv[i];
+            const int r = v / WPR, c = v % WPR;
+            if constexpr (W_TRANS && W_FP8) {
+                *reinterpret_cast<u32x4 *>(tw + w_off(r, c * 32)) = fp8x8_to_bf16_chunk(w[0], w[1]);
+                *reinterpret_cast<u32x4 *>(tw + w_off(r, c * 32) + 16) = fp8x8_to_bf16_chunk(w[2], w[3]);
+            } else if constexpr (W_TRANS) {
+                *reinterpret_cast<u32x4 *>(tw + w_off(r, c * 16)) = w;
+            } else if constexpr (W_FP8) {
+                reinterpret_cast<u32x4 *>(tw)[tile_chunk_index<CH>(r, 2 * c)] = fp8x8_to_bf16_chunk(w[0], w[1]);
+                reinterpret_cast<u32x4 *>(tw)[tile_chunk_index<CH>(r, 2 * c + 1)] = fp8x8_to_bf16_chunk(w[2], w[3]);
             } else {
-                u32x4 *t4 = reinterpret_cast<u32x4 *>(tile);
-                const int n = v / WPR, c = v % WPR;
-                if constexpr (W_FP8) {
-                    t4[tile_chunk_index<CH>(n, 2 * c)] = fp8x8_to_bf16_chunk(w[0], w[1]);
-                    t4[tile_chunk_index<CH>(n, 2 * c + 1)] = fp8x8_to_bf16_chunk(w[2], w[3]);
-                } else {
-                    t4[tile_chunk_index<CH>(n, c)] = w;
-                }
+                reinterpret_cast<u32x4 *>(tw)[tile_chunk_index<CH>(r, c)] = w;
             }
         }
     };
@@ -253,11 +231,12 @@ __global__ __launch_bounds__(kThreads) void tiled_rows_kernel(TiledRowsParams p)
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto compute = [&](const char *stage) {
+    auto compute = [&](const char *stage, int left) {                   // `left`: reduction elements from this slab on
         const u32x4 *ta = reinterpret_cast<const u32x4 *>(stage);
         const char *tw = stage + L::A;
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ++ks) {
+            if (ks > 0 && ks * 4 * VEC >= left) break;
             u32x4 mf[TM], nf[TN];
 #pragma unroll
             for (int i = 0; i < TM; ++i) mf[i] = ta[tile_chunk_index<CH>(wave_m0 + i * 16 + a, ks * 4 + g)];
@@ -293,90 +272,101 @@ __global__ __launch_bounds__(kThreads) void tiled_rows_kernel(TiledRowsParams p)
         }
     };
     // One barrier per slab: a wavefront that writes slab kt + 1 has passed slab kt's barrier, before which every wavefront had
-    // finished with slab kt - 1, the stage's previous content.  The steady state issues unconditionally, so that the compiler can
-    // count the outstanding loads and waits for one slab's only.
+    // finished with slab kt - 1, the stage's previous content.  The rounds before the last request and consume without a condition,
+    // so that the compiler can count the outstanding loads and waits for one slab's only; the last round requests nothing more.
     static_assert(D % 2 == 0, "stage parity is static");
     int kt = 0;
-    for (; kt + 2 * D <= nk; kt += D) {
+    for (; kt + D < nk && !short_rows; kt += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             char *stage = smem_tiled + (d & 1) * L::STAGE;
-            commit_a(areg[d], kt + d, stage);
-            commit_w(wreg[d], kt + d, stage);
-            issue_a(kt + d + D, areg[d]);
-            issue_w(kt + d + D, wreg[d]);
+            commit(areg[d], wreg[d], stage);
+            issue_a(min(kt + d + D, nk - 1), areg[d]);
+            issue_w(min(kt + d + D, nk - 1), wreg[d]);
             __syncthreads();
-            compute(stage);
+            compute(stage, BKE);
         }
     }
-    for (; kt < nk; kt += D) {
+    for (;;) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            if (kt + d < nk) {
-                char *stage = smem_tiled + (d & 1) * L::STAGE;
-                commit_a(areg[d], kt + d, stage);
-                commit_w(wreg[d], kt + d, stage);
-                if (kt + d + D < nk) { issue_a(kt + d + D, areg[d]); issue_w(kt + d + D, wreg[d]); }
-                __syncthreads();
-                compute(stage);
-            }
+            if (kt + d >= nk) break;
+            char *stage = smem_tiled + (d & 1) * L::STAGE;
+            if (kt + d == nk - 1 || short_rows) fix_edge(areg[d], wreg[d], kt + d);
+            commit(areg[d], wreg[d], stage);
+            __syncthreads();
+            compute(stage, R - (kt + d) * BKE);
+        }
+        kt += D;
+        if (kt >= nk) break;                                            // `short_rows` alone goes on: every slab is an edge
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            issue_a(min(kt + d, nk - 1), areg[d]);
+            issue_w(min(kt + d, nk - 1), wreg[d]);
         }
     }
 
-    // ---------------- results: lane (a, g) holds columns 16 j + 4 g .. + 3 of row 16 i + a; regrouped so that adjacent lanes
-    // store adjacent pieces of a row
+    // ---------------- results.  Lane (a, g) holds columns 16 j + 4 g .. + 3 of row 16 i + a; sixteen rows at a time go through a
+    // piece of LDS of the wavefront's own and leave as whole row segments.  One short loop does everything else to a value: unrolled
+    // over the tile, the activations alone were tens of KB of code, fetched anew by every launch.
+    constexpr int ORS = BN + 4;                                         // floats per row
+    static_assert(4 * 16 * ORS * 4 <= L::BYTES, "the slabs' LDS holds it");
+    float *mine = reinterpret_cast<float *>(smem_tiled) + wave * 16 * ORS;
     auto as_float = [](const char *at) -> float {
         if constexpr (ES == 4) return *reinterpret_cast<const float *>(at);
         else return TT::ID == 2 ? bf16_bits_to_f32(*reinterpret_cast<const uint16_t *>(at)) : f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(at));
     };
-    if (p.bias != nullptr) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float v = as_float(p.bias + ((int64_t)e * N + min(n0 + j * 16 + g * 4 + r, N - 1)) * ES);
-#pragma unroll
-                for (int i = 0; i < TM; ++i) acc[i][j][r] += v;
-            }
-    }
-    auto each = [&](auto fn) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[i][j][r] = fn(acc[i][j][r]);
-    };
-    if constexpr (WES == 2) apply_activation_of<TT>(p.act, each);
-    const int srow = lane >> 2, sg = lane & 3;
+    const int orow = lane >> 3, ocol = (lane & 7) * 4;                  // eight lanes per row: rows orow and orow + 8, 32 columns at a time
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-        const int m = m0 + wave_m0 + i * 16 + srow, mm = min(m, Me - 1);
-        const int b = mm / p.K;
-        const int64_t pick = ((int64_t)b * p.E + e) * p.K + (mm - b * p.K);
-        char *crow = p.C + pick * p.ldc * (p.out_f32 ? 4 : ES);
+        int64_t crow[2];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            f32x4 v = acc[i][j];
-            if (p.w_scale != nullptr) {
+        for (int h = 0; h < 2; ++h) {
+            const int m = m0 + wave_m0 + i * 16 + h * 8 + orow, mm = min(m, Me - 1), b = mm / p.K;
+            crow[h] = m < Me ? (((int64_t)b * p.E + e) * p.K + (mm - b * p.K)) * p.ldc : -1;
+        }
 #pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] *= p.w_scale[(int64_t)e * N + min(n0 + j * 16 + g * 4 + r, N - 1)];
+        for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4 *>(mine + a * ORS + j * 16 + g * 4) = acc[i][j];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+        for (int c = ocol; c < BN && n0 + c < N; c += 32) {
+            const int n = n0 + c;
+            f32x4 v[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[h] = *reinterpret_cast<const f32x4 *>(mine + (h * 8 + orow) * ORS + c);
+            if (p.w_scale != nullptr || p.bias != nullptr) {
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const int64_t at = (int64_t)e * N + min(n + x, N - 1);
+                    const float f = p.w_scale != nullptr ? p.w_scale[at] : 1.f, add = p.bias != nullptr ? as_float(p.bias + at * ES) : 0.f;
+                    v[0][x] = v[0][x] * f + add;
+                    v[1][x] = v[1][x] * f + add;
+                }
             }
-            v = __builtin_bit_cast(f32x4, lanes_16g_a_to_4a_g(__builtin_bit_cast(u32x4, v), lane));
-            const int n = n0 + j * 16 + sg * 4;
-            if (m >= Me || n >= N) continue;
-            if (n + 4 <= N) {
-                if (ES == 4 || p.out_f32) *reinterpret_cast<f32x4_any *>(crow + (int64_t)n * 4) = v;
-                else *reinterpret_cast<u32x2_any *>(crow + (int64_t)n * 2) = u32x2{pack2<TT>(v[0], v[1]), pack2<TT>(v[2], v[3])};
-            } else {
+            if constexpr (WES == 2)
+                apply_activation_of<TT>(p.act, [&](auto fn) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (n + r >= N) continue;
-                    if (ES == 4 || p.out_f32) reinterpret_cast<float *>(crow)[n + r] = v[r];
-                    else reinterpret_cast<uint16_t *>(crow)[n + r] = (uint16_t)f32_to_elem_bits<TT>(v[r]);
+                    for (int h = 0; h < 2; ++h)
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) v[h][x] = fn(v[h][x]);
+                });
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (crow[h] < 0) continue;
+                char *dst = p.C + (crow[h] + n) * (ES == 4 || p.out_f32 ? 4 : 2);
+                if (n + 4 <= N) {
+                    if (ES == 4 || p.out_f32) *reinterpret_cast<f32x4_any *>(dst) = v[h];
+                    else *reinterpret_cast<u32x2_any *>(dst) = u32x2{pack2<TT>(v[h][0], v[h][1]), pack2<TT>(v[h][2], v[h][3])};
+                } else {
+                    for (int x = 0; n + x < N; ++x) {
+                        if (ES == 4 || p.out_f32) reinterpret_cast<float *>(dst)[x] = v[h][x];
+                        else reinterpret_cast<uint16_t *>(dst)[x] = (uint16_t)f32_to_elem_bits<TT>(v[h][x]);
+                    }
                 }
             }
         }
+        __builtin_amdgcn_wave_barrier();
     }
 }
 

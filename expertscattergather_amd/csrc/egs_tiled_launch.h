@@ -5,7 +5,7 @@
 namespace egs {
 namespace host {
 
-template <class TT, int WES, bool W_TRANS, int TM, int TN>
+template <class TT, int WES, bool W_TRANS, int TM, int TN, bool DEEP = false>
 int launch_tiled_one(TiledRowsParams &p, hipStream_t s)
 {
     p.m_tiles = ceil_div(p.B * p.K, 64 * TM);
@@ -14,9 +14,9 @@ int launch_tiled_one(TiledRowsParams &p, hipStream_t s)
     if (total > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
     static LdsGrant told;
     constexpr size_t lds = TiledLds<TT, W_TRANS, TM, TN>::BYTES;
-    const int rc = allow_large_lds((const void *)tiled_rows_kernel<TT, WES, W_TRANS, TM, TN>, told, lds, "hipFuncSetAttribute(tiled_rows_kernel)");
+    const int rc = allow_large_lds((const void *)tiled_rows_kernel<TT, WES, W_TRANS, TM, TN, DEEP>, told, lds, "hipFuncSetAttribute(tiled_rows_kernel)");
     if (rc != EGS_OK) return rc;
-    hipLaunchKernelGGL((tiled_rows_kernel<TT, WES, W_TRANS, TM, TN>), dim3((unsigned)(8 * ((total + 7) / 8))), dim3(kThreads), lds, s, p);
+    hipLaunchKernelGGL((tiled_rows_kernel<TT, WES, W_TRANS, TM, TN, DEEP>), dim3((unsigned)(8 * ((total + 7) / 8))), dim3(kThreads), lds, s, p);
     EGS_CHECK_LAUNCH("tiled_rows_kernel");
     return EGS_OK;
 }
@@ -24,7 +24,9 @@ int launch_tiled_one(TiledRowsParams &p, hipStream_t s)
 template <class TT, int WES, bool W_TRANS>
 int launch_tiled(TiledRowsParams &p, hipStream_t s)
 {
-    if (p.a_bytes < 16 || p.w_bytes < 16) {
+    // (offsets inside an expert's matrix are 32-bit, the slab past its end included)
+    const bool huge = (uint64_t)p.R * p.N * WES + 128ull * p.N * WES + 4096 > 0xff000000ull;
+    if (p.a_bytes < 16 || p.w_bytes < 16 || huge) {
         hipLaunchKernelGGL((tiny_rows_kernel<TT, WES, W_TRANS>), dim3(grid_1d((size_t)p.B * p.E * p.K * p.N)), dim3(kThreads), 0, s, p);
         EGS_CHECK_LAUNCH("tiny_rows_kernel");
         return EGS_OK;
@@ -38,6 +40,8 @@ int launch_tiled(TiledRowsParams &p, hipStream_t s)
     auto tiles = [&](int bm) { return (int64_t)p.E * ((Me + bm - 1) / bm) * ceil_div(p.N, 16 * tn); };
     const int tm = Me > 64 && tiles(128) >= 512 ? 2 : 1;
     while (tm == 1 && tn > 2 && tiles(64) < 256) tn = tn > 4 ? 4 : 2;
+    if (tm == 1 && tn <= 4 && tiles(64) <= 512)
+        return tn == 2 ? launch_tiled_one<TT, WES, W_TRANS, 1, 2, true>(p, s) : launch_tiled_one<TT, WES, W_TRANS, 1, 4, true>(p, s);
     switch (tm * 16 + tn) {
     case 16 + 2: return launch_tiled_one<TT, WES, W_TRANS, 1, 2>(p, s);
     case 16 + 4: return launch_tiled_one<TT, WES, W_TRANS, 1, 4>(p, s);
