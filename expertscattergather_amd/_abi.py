@@ -55,7 +55,8 @@ SIGNATURES = {
     "egs_expert_gather_backward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _dp, _i64, _i64, _i, _i, _i, _vp]),
     "egs_expert_scatter_forward": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _dp, _i, _i, _i, _vp]),
     "egs_expert_scatter_backward": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _dp, _i64, _i64, _i, _i, _vp]),
-    "egs_expert_choice_router": (_i, [_vp, _vp, _vp, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _i, _i, _vp]),
+    "egs_expert_choice_router_workspace_bytes": (_sz, [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32]),
+    "egs_expert_choice_router": (_i, [_vp, _vp, _vp, _vp, _sz, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _i, _i, _vp]),
     "egs_validate_indices": (_i, [_vp, _i, _i64, ctypes.c_int32, _vp, _vp]),
     "egs_routing_table_bytes": (_sz, [_dp, _i]),
     "egs_stream_capture_id": (_i, [_vp, ctypes.POINTER(ctypes.c_ulonglong)]),

@@ -510,8 +510,11 @@ PyObject *py_router(PyObject *, PyObject *const *a, Py_ssize_t n)
         p.dev = logits.device().index();
         Ind = empty_gpu({B, E, K}, it, p);
         scores = empty_gpu({B, E, K}, at::kFloat, p);
-        rc = egs_expert_choice_router(logits.const_data_ptr(), Ind.data_ptr(), (float *)scores.data_ptr(), (int32_t)B, (int32_t)T, (int32_t)E,
-                                      (int32_t)K, dt, ind, stream_of(logits));
+        const size_t ws_bytes = egs_expert_choice_router_workspace_bytes((int32_t)B, (int32_t)T, (int32_t)E);
+        Tensor ws;
+        if (ws_bytes > 0) ws = empty_gpu({(int64_t)ws_bytes}, at::kByte, p);
+        rc = egs_expert_choice_router(logits.const_data_ptr(), Ind.data_ptr(), (float *)scores.data_ptr(), ws_bytes > 0 ? ws.data_ptr() : nullptr,
+                                      ws_bytes, (int32_t)B, (int32_t)T, (int32_t)E, (int32_t)K, dt, ind, stream_of(logits));
     }
     if (rc == EGS_ERR_UNSUPPORTED) Py_RETURN_NONE;
     raise_status(rc, "expert_choice_router");

@@ -303,9 +303,10 @@ int egs_expert_scatter_backward(const void *Y, const void *W, const void *Ind, c
 
 /* scores[b,e,:] = the K largest of softmax over experts of logits[b,:,e], descending, Ind[b,e,:] their tokens.
  * logits [B,T,E] dense in fp32 / fp16 / bf16, scores fp32.  EGS_ERR_UNSUPPORTED where a column does not fit a
- * compute unit's LDS (T above about 9000) or K > 512. */
-int egs_expert_choice_router(const void *logits, void *Ind, float *scores, int32_t B, int32_t T, int32_t E, int32_t K,
-                             int logits_dtype, int ind_dtype, void *stream);
+ * compute unit's LDS (T above about 9000) or K > 512.  Many logits per batch element need a workspace: its size, or 0. */
+size_t egs_expert_choice_router_workspace_bytes(int32_t B, int32_t T, int32_t E);
+int egs_expert_choice_router(const void *logits, void *Ind, float *scores, void *workspace, size_t workspace_bytes, int32_t B,
+                             int32_t T, int32_t E, int32_t K, int logits_dtype, int ind_dtype, void *stream);
 
 /* ---------------------------------------------------------------------------------------
  * Debug helper (no counterpart in the reference, which never checks Ind)

@@ -8,7 +8,9 @@ pytestmark = pytest.mark.gpu
 from expertscattergather_amd import _abi
 from expertscattergather_amd.router import expert_choice_router
 
-SHAPES = [(1, 1, 1, 1), (3, 17, 5, 4), (2, 64, 9, 64), (2, 65, 64, 33), (64, 256, 32, 32), (1, 1024, 70, 100), (2, 1025, 3, 257), (1, 4096, 20, 512)]
+SHAPES = [(1, 1, 1, 1), (3, 17, 5, 4), (2, 64, 9, 64), (2, 65, 64, 33), (64, 256, 32, 32), (1, 1024, 60, 100), (2, 1025, 3, 257), (1, 4096, 20, 512),
+          (1, 257, 7, 129), (64, 300, 33, 20), (1, 4097, 17, 65), (40, 1025, 17, 65)]
+LARGE = [(1, 1024, 70, 100), (1, 700, 140, 30), (2, 3000, 40, 130), (64, 800, 129, 9)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
@@ -27,6 +29,19 @@ def test_router_matches_topk(B, T, E, K, dtype):
     assert torch.allclose(scores.double(), want, rtol=1e-5, atol=0)
     assert torch.allclose(scores.double(), aff.gather(-1, Ind), rtol=1e-5, atol=0)
     assert (scores.diff(dim=-1) <= 0).all()
+
+
+@pytest.mark.parametrize("B,T,E,K", LARGE, ids=lambda v: str(v))
+def test_large_logits_have_their_row_sums_first(B, T, E, K):
+    logits = torch.randn(B, T, E, generator=torch.Generator().manual_seed(T))
+    logits[0, 3, 1] = float("nan")
+    with _abi.launch_log() as log:
+        Ind, scores = expert_choice_router(logits.cuda(), K)
+    assert log.kernels == ["router_stats_kernel", "router_kernel"]
+    assert (Ind[0, :, 0] == 3).all() and scores[0, :, 0].isnan().all()
+    aff = torch.softmax(logits.double(), -1).transpose(1, 2).nan_to_num(9.0)
+    scores = scores.cpu().double().nan_to_num(9.0)
+    assert torch.allclose(scores, aff.topk(K, -1)[0], rtol=1e-5, atol=0) and torch.allclose(scores, aff.gather(-1, Ind.cpu()), rtol=1e-5, atol=0)
 
 
 def test_ties_take_the_lowest_tokens_and_a_nan_comes_first():
