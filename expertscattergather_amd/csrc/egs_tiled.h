@@ -55,10 +55,10 @@ struct TiledRowsParams {
 };
 
 // bytes of LDS: two stages of A and W tiles
-template <class TT, bool W_TRANS, int TM, int TN>
+template <class TT, bool W_TRANS, int TN>
 struct TiledLds {
     static constexpr int CH = 8, BKE = CH * TT::VEC;            // 128-byte row pieces per slab
-    static constexpr int A = 64 * TM * CH * 16;
+    static constexpr int A = 64 * CH * 16;
     // [reduction][column] weight tiles.  16-bit: an odd number of 32-byte units per row and 128 more bytes every eight rows, so
     // that the 16 row pieces of a transpose read fall two deep on every bank; fp32: rows 4 banks apart modulo 16
     static constexpr int WROW = TT::ES == 2 ? 32 * (TN | 1) : (16 * TN + 4) * 4;
@@ -67,27 +67,24 @@ struct TiledLds {
     static constexpr int BYTES = 2 * STAGE;
 };
 
-// Wavefronts per SIMD that the registers are bounded for: where there are workgroups enough, several of them to a CU hide one's
-// round trips behind the others' matrix instructions (DEEP = false: two slabs in flight each; B53 K41 E29 I111 J75 fp32 gather
-// 25.8 us with one or two workgroups to a CU, see launch_tiled for the figures now); a problem of a few workgroups keeps four
-// slabs in flight instead and takes the registers it likes.
-template <int TM, int TN, bool DEEP> constexpr int tiled_waves() { return DEEP ? 1 : TM * TN <= 2 ? 4 : TM * TN <= 6 ? 3 : 2; }
-
-// 64 * TM rows x 16 * TN columns per workgroup of four wavefronts, each 16 * TM rows x all columns.
-template <class TT, int WES, bool W_TRANS, int TM, int TN, bool DEEP>
-__global__ __launch_bounds__(kThreads, (tiled_waves<TM, TN, DEEP>())) void tiled_rows_kernel(TiledRowsParams p)
+// 64 rows x 16 * TN columns per workgroup of four wavefronts, each 16 rows x all columns, two slabs in flight in registers.  What
+// hides one workgroup's round trips is the others of its compute unit, so the registers are bounded for three or four.
+// (128-row tiles were level or slower at all of 42 shapes but where they left fewer columns over; four slabs in flight gave
+// 4% at R1000 and a few tiles, and cost occupancy elsewhere.)
+template <class TT, int WES, bool W_TRANS, int TN>
+__global__ __launch_bounds__(kThreads, TN <= 2 ? 4 : 3) void tiled_rows_kernel(TiledRowsParams p)
 {
     constexpr int ES = TT::ES, VEC = TT::VEC;
     constexpr bool W_FP8 = WES == 1;
-    typedef TiledLds<TT, W_TRANS, TM, TN> L;
+    typedef TiledLds<TT, W_TRANS, TN> L;
     constexpr int CH = L::CH, BKE = L::BKE, KSTEPS = CH / 4;
-    constexpr int BM = 64 * TM, BN = 16 * TN;
+    constexpr int BM = 64, BN = 16 * TN;
     constexpr int NA = BM * CH / kThreads;                              // A chunks per thread and slab
     // W chunks (16 source bytes) per slab: W_TRANS rows of BN columns, else BN rows of CH chunks (fp8: half as many)
     constexpr int WPR = W_TRANS ? BN * WES / 16 : CH * WES / ES;        // chunks per source row
     constexpr int WCH = WPR * (W_TRANS ? BKE : BN);
     constexpr int NW = (WCH + kThreads - 1) / kThreads;
-    constexpr int D = DEEP ? 4 : 2;                                     // slabs in flight in registers
+    constexpr int D = 2;                                                // slabs in flight in registers
     extern __shared__ __attribute__((aligned(16))) char smem_tiled[];
 
     const int total = p.E * p.m_tiles * p.n_tiles;
@@ -225,21 +222,18 @@ __global__ __launch_bounds__(kThreads, (tiled_waves<TM, TN, DEEP>())) void tiled
     // ---------------- LDS -> matrix instructions
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int a = lane & 15, g = lane >> 4;
-    const int wave_m0 = wave * 16 * TM;
-    f32x4 acc[TM][TN];
+    const int wave_m0 = wave * 16;
+    f32x4 acc[TN];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < TN; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto compute = [&](const char *stage, int left) {                   // `left`: reduction elements from this slab on
         const u32x4 *ta = reinterpret_cast<const u32x4 *>(stage);
         const char *tw = stage + L::A;
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ++ks) {
             if (ks > 0 && ks * 4 * VEC >= left) break;
-            u32x4 mf[TM], nf[TN];
-#pragma unroll
-            for (int i = 0; i < TM; ++i) mf[i] = ta[tile_chunk_index<CH>(wave_m0 + i * 16 + a, ks * 4 + g)];
+            const u32x4 mf = ta[tile_chunk_index<CH>(wave_m0 + a, ks * 4 + g)];
+            u32x4 nf[TN];
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 if constexpr (!W_TRANS) {
@@ -257,17 +251,13 @@ __global__ __launch_bounds__(kThreads, (tiled_waves<TM, TN, DEEP>())) void tiled
             }
             if constexpr (ES == 2) {
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) mma_chunk<TT>(acc[i][j], nf[j], mf[i]);
+                for (int j = 0; j < TN; ++j) mma_chunk<TT>(acc[j], nf[j], mf);
             } else {            // accumulators in turn: an fp32 matrix instruction then never waits for the one before it
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
 #pragma unroll
-                    for (int i = 0; i < TM; ++i)
-#pragma unroll
-                        for (int j = 0; j < TN; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bits_f32(nf[j][c]), bits_f32(mf[i][c]), acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < TN; ++j)
+                        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bits_f32(nf[j][c]), bits_f32(mf[c]), acc[j], 0, 0, 0);
             }
         }
     };
@@ -306,9 +296,9 @@ __global__ __launch_bounds__(kThreads, (tiled_waves<TM, TN, DEEP>())) void tiled
         }
     }
 
-    // ---------------- results.  Lane (a, g) holds columns 16 j + 4 g .. + 3 of row 16 i + a; sixteen rows at a time go through a
-    // piece of LDS of the wavefront's own and leave as whole row segments.  One short loop does everything else to a value: unrolled
-    // over the tile, the activations alone were tens of KB of code, fetched anew by every launch.
+    // ---------------- results.  Lane (a, g) holds columns 16 j + 4 g .. + 3 of row a of the wavefront's; they go through a piece of
+    // LDS of its own and leave as whole row segments.  One short loop does everything else to a value: unrolled over the tile, the
+    // activations alone were tens of KB of code, fetched anew by every launch.
     constexpr int ORS = BN + 4;                                         // floats per row
     static_assert(4 * 16 * ORS * 4 <= L::BYTES, "the slabs' LDS holds it");
     float *mine = reinterpret_cast<float *>(smem_tiled) + wave * 16 * ORS;
@@ -318,55 +308,51 @@ __global__ __launch_bounds__(kThreads, (tiled_waves<TM, TN, DEEP>())) void tiled
     };
     const int orow = lane >> 3, ocol = (lane & 7) * 4;                  // eight lanes per row: rows orow and orow + 8, 32 columns at a time
     __syncthreads();
+    int64_t crow[2];
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        int64_t crow[2];
+    for (int h = 0; h < 2; ++h) {
+        const int m = m0 + wave_m0 + h * 8 + orow, mm = min(m, Me - 1), b = mm / p.K;
+        crow[h] = m < Me ? (((int64_t)b * p.E + e) * p.K + (mm - b * p.K)) * p.ldc : -1;
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4 *>(mine + a * ORS + j * 16 + g * 4) = acc[j];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+    for (int c = ocol; c < BN && n0 + c < N; c += 32) {
+        const int n = n0 + c;
+        f32x4 v[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) v[h] = *reinterpret_cast<const f32x4 *>(mine + (h * 8 + orow) * ORS + c);
+        if (p.w_scale != nullptr || p.bias != nullptr) {
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                const int64_t at = (int64_t)e * N + min(n + x, N - 1);
+                const float f = p.w_scale != nullptr ? p.w_scale[at] : 1.f, add = p.bias != nullptr ? as_float(p.bias + at * ES) : 0.f;
+                v[0][x] = v[0][x] * f + add;
+                v[1][x] = v[1][x] * f + add;
+            }
+        }
+        if constexpr (WES == 2)
+            apply_activation_of<TT>(p.act, [&](auto fn) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) v[h][x] = fn(v[h][x]);
+            });
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int m = m0 + wave_m0 + i * 16 + h * 8 + orow, mm = min(m, Me - 1), b = mm / p.K;
-            crow[h] = m < Me ? (((int64_t)b * p.E + e) * p.K + (mm - b * p.K)) * p.ldc : -1;
-        }
-#pragma unroll
-        for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4 *>(mine + a * ORS + j * 16 + g * 4) = acc[i][j];
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll 1
-        for (int c = ocol; c < BN && n0 + c < N; c += 32) {
-            const int n = n0 + c;
-            f32x4 v[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) v[h] = *reinterpret_cast<const f32x4 *>(mine + (h * 8 + orow) * ORS + c);
-            if (p.w_scale != nullptr || p.bias != nullptr) {
-#pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    const int64_t at = (int64_t)e * N + min(n + x, N - 1);
-                    const float f = p.w_scale != nullptr ? p.w_scale[at] : 1.f, add = p.bias != nullptr ? as_float(p.bias + at * ES) : 0.f;
-                    v[0][x] = v[0][x] * f + add;
-                    v[1][x] = v[1][x] * f + add;
-                }
-            }
-            if constexpr (WES == 2)
-                apply_activation_of<TT>(p.act, [&](auto fn) {
-#pragma unroll
-                    for (int h = 0; h < 2; ++h)
-#pragma unroll
-                        for (int x = 0; x < 4; ++x) v[h][x] = fn(v[h][x]);
-                });
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                if (crow[h] < 0) continue;
-                char *dst = p.C + (crow[h] + n) * (ES == 4 || p.out_f32 ? 4 : 2);
-                if (n + 4 <= N) {
-                    if (ES == 4 || p.out_f32) *reinterpret_cast<f32x4_any *>(dst) = v[h];
-                    else *reinterpret_cast<u32x2_any *>(dst) = u32x2{pack2<TT>(v[h][0], v[h][1]), pack2<TT>(v[h][2], v[h][3])};
-                } else {
-                    for (int x = 0; n + x < N; ++x) {
-                        if (ES == 4 || p.out_f32) reinterpret_cast<float *>(dst)[x] = v[h][x];
-                        else reinterpret_cast<uint16_t *>(dst)[x] = (uint16_t)f32_to_elem_bits<TT>(v[h][x]);
-                    }
+            if (crow[h] < 0) continue;
+            char *dst = p.C + (crow[h] + n) * (ES == 4 || p.out_f32 ? 4 : 2);
+            if (n + 4 <= N) {
+                if (ES == 4 || p.out_f32) *reinterpret_cast<f32x4_any *>(dst) = v[h];
+                else *reinterpret_cast<u32x2_any *>(dst) = u32x2{pack2<TT>(v[h][0], v[h][1]), pack2<TT>(v[h][2], v[h][3])};
+            } else {
+                for (int x = 0; n + x < N; ++x) {
+                    if (ES == 4 || p.out_f32) reinterpret_cast<float *>(dst)[x] = v[h][x];
+                    else reinterpret_cast<uint16_t *>(dst)[x] = (uint16_t)f32_to_elem_bits<TT>(v[h][x]);
                 }
             }
         }
-        __builtin_amdgcn_wave_barrier();
     }
 }
 

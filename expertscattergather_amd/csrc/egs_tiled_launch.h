@@ -5,18 +5,18 @@
 namespace egs {
 namespace host {
 
-template <class TT, int WES, bool W_TRANS, int TM, int TN, bool DEEP = false>
+template <class TT, int WES, bool W_TRANS, int TN>
 int launch_tiled_one(TiledRowsParams &p, hipStream_t s)
 {
-    p.m_tiles = ceil_div(p.B * p.K, 64 * TM);
+    p.m_tiles = ceil_div(p.B * p.K, 64);
     p.n_tiles = ceil_div(p.N, 16 * TN);
     const int64_t total = (int64_t)p.E * p.m_tiles * p.n_tiles;
     if (total > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
     static LdsGrant told;
-    constexpr size_t lds = TiledLds<TT, W_TRANS, TM, TN>::BYTES;
-    const int rc = allow_large_lds((const void *)tiled_rows_kernel<TT, WES, W_TRANS, TM, TN, DEEP>, told, lds, "hipFuncSetAttribute(tiled_rows_kernel)");
+    constexpr size_t lds = TiledLds<TT, W_TRANS, TN>::BYTES;
+    const int rc = allow_large_lds((const void *)tiled_rows_kernel<TT, WES, W_TRANS, TN>, told, lds, "hipFuncSetAttribute(tiled_rows_kernel)");
     if (rc != EGS_OK) return rc;
-    hipLaunchKernelGGL((tiled_rows_kernel<TT, WES, W_TRANS, TM, TN, DEEP>), dim3((unsigned)(8 * ((total + 7) / 8))), dim3(kThreads), lds, s, p);
+    hipLaunchKernelGGL((tiled_rows_kernel<TT, WES, W_TRANS, TN>), dim3((unsigned)(8 * ((total + 7) / 8))), dim3(kThreads), lds, s, p);
     EGS_CHECK_LAUNCH("tiled_rows_kernel");
     return EGS_OK;
 }
@@ -31,29 +31,22 @@ int launch_tiled(TiledRowsParams &p, hipStream_t s)
         EGS_CHECK_LAUNCH("tiny_rows_kernel");
         return EGS_OK;
     }
-    // Tile shape.  Columns: what covers N with the least left over, at most 128.  Rows: 128 where that still gives every CU two
-    // workgroups, else 64.  Then narrower columns while the device (256 CUs) is not covered: these products are bound by the
-    // latency of their slabs, and rows fetched again by the next column tile come out of the L2.
-    const int64_t Me = (int64_t)p.B * p.K;
-    const int at_most_8 = ceil_div(ceil_div(p.N, ceil_div(p.N, 128)), 16);
-    int tn = at_most_8 <= 2 ? 2 : at_most_8 <= 4 ? 4 : at_most_8 <= 6 ? at_most_8 : 8;
-    auto tiles = [&](int bm) { return (int64_t)p.E * ((Me + bm - 1) / bm) * ceil_div(p.N, 16 * tn); };
-    const int tm = Me > 64 && tiles(128) >= 512 ? 2 : 1;
-    while (tm == 1 && tn > 2 && tiles(64) < 256) tn = tn > 4 ? 4 : 2;
-    if (tm == 1 && tn <= 4 && tiles(64) <= 512)
-        return tn == 2 ? launch_tiled_one<TT, WES, W_TRANS, 1, 2, true>(p, s) : launch_tiled_one<TT, WES, W_TRANS, 1, 4, true>(p, s);
-    switch (tm * 16 + tn) {
-    case 16 + 2: return launch_tiled_one<TT, WES, W_TRANS, 1, 2>(p, s);
-    case 16 + 4: return launch_tiled_one<TT, WES, W_TRANS, 1, 4>(p, s);
-    case 16 + 5: return launch_tiled_one<TT, WES, W_TRANS, 1, 5>(p, s);
-    case 16 + 6: return launch_tiled_one<TT, WES, W_TRANS, 1, 6>(p, s);
-    case 16 + 8: return launch_tiled_one<TT, WES, W_TRANS, 1, 8>(p, s);
-    case 32 + 2: return launch_tiled_one<TT, WES, W_TRANS, 2, 2>(p, s);
-    case 32 + 4: return launch_tiled_one<TT, WES, W_TRANS, 2, 4>(p, s);
-    case 32 + 5: return launch_tiled_one<TT, WES, W_TRANS, 2, 5>(p, s);
-    case 32 + 6: return launch_tiled_one<TT, WES, W_TRANS, 2, 6>(p, s);
-    default: return launch_tiled_one<TT, WES, W_TRANS, 2, 8>(p, s);
+    // Columns per tile: what takes the fewest rounds of the 256 CUs, each as long as the tile's matrix instructions and the fixed
+    // part of a tile (fetching 64 rows, and what a slab's barriers cost) let it be, measured at 42 shapes.  80 columns only where
+    // the matrix instructions are the larger part (fp32: E35 of 6000 picks, R185 N67 71 us, 78 with 96 columns; 16-bit 35 and 33).
+    const int64_t Me = (int64_t)p.B * p.K, row_tiles = p.E * ((Me + 63) / 64);
+    int tn = 0;
+    double least = 0;
+    for (const int c : {6, 5, 4, 2}) {
+        if (c == 5 && TT::ES == 2) continue;
+        const double cost = (double)((row_tiles * ceil_div(p.N, 16 * c) + 255) / 256) * (c + (TT::ES == 2 ? 1.5 : 1.0));
+        if (tn == 0 || cost < least) { least = cost; tn = c; }
     }
+    if constexpr (TT::ES == 4) {
+        if (tn == 5) return launch_tiled_one<TT, WES, W_TRANS, 5>(p, s);
+    }
+    return tn == 6 ? launch_tiled_one<TT, WES, W_TRANS, 6>(p, s)
+                   : tn == 4 ? launch_tiled_one<TT, WES, W_TRANS, 4>(p, s) : launch_tiled_one<TT, WES, W_TRANS, 2>(p, s);
 }
 
 template <class TT>
