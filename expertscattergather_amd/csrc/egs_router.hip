@@ -52,20 +52,25 @@ __global__ __launch_bounds__(256) void router_stats_kernel(RouterParams p, PT lo
     const int rl = (int)threadIdx.x & 15;
     const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4), rows = (int64_t)p.B * p.T;
     const int64_t at = (row < rows ? row : rows - 1) * p.E;
-    float m = -INFINITY, s = 0.f;
-    float v[8];
+    float v[8], m = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = logit(logits, at + min(rl + i * 16, p.E - 1));      // (the last again: no matter to a maximum)
 #pragma unroll
     for (int i = 0; i < 8; ++i) m = fmaxf(m, v[i]);
     for (int e = rl + 128; e < p.E; e += 16) m = fmaxf(m, logit(logits, at + e));
 #pragma unroll
-    for (int x = 1; x < 16; x *= 2) m = fmaxf(m, __shfl_xor(m, x));
+    for (int x = 8; x > 0; x /= 2) m = fmaxf(m, __shfl_xor(m, x));
+    // the sum in torch's order (every 64th expert in turn, then pairwise, the furthest first), and so its bits
+    float q[4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) s += rl + i * 16 < p.E ? expf(v[i] - m) : 0.f;
-    for (int e = rl + 128; e < p.E; e += 16) s += expf(logit(logits, at + e) - m);
+    for (int i = 0; i < 4; ++i) {
+        q[i] = rl + i * 16 < p.E ? expf(v[i] - m) : 0.f;
+        q[i] += rl + i * 16 + 64 < p.E ? expf(v[i + 4] - m) : 0.f;
+        for (int e = rl + i * 16 + 128; e < p.E; e += 64) q[i] += expf(logit(logits, at + e) - m);
+    }
+    float s = (q[0] + q[2]) + (q[1] + q[3]);
 #pragma unroll
-    for (int x = 1; x < 16; x *= 2) s += __shfl_xor(s, x);
+    for (int x = 8; x > 0; x /= 2) s += __shfl_xor(s, x);
     if (rl == 0 && row < rows) p.stats[row] = float2{m, s};
 }
 
@@ -99,8 +104,8 @@ __global__ __launch_bounds__(64 * WV * WPE) void router_kernel(RouterParams p, P
         constexpr int OWN = WV < L ? 1 : WV / L;        // of this workgroup's experts, those in one lane
         const int rl = tid % L, rg = tid / L;
         auto reduce4 = [](float v, auto op) {           // every lane of the four gets the result (no LDS round trip)
-            v = op(v, bits_f32(__builtin_amdgcn_update_dpp(0, (int)f32_bits(v), 0xb1, 0xf, 0xf, false)));       // quad_perm 1 0 3 2
             v = op(v, bits_f32(__builtin_amdgcn_update_dpp(0, (int)f32_bits(v), 0x4e, 0xf, 0xf, false)));       // quad_perm 2 3 0 1
+            v = op(v, bits_f32(__builtin_amdgcn_update_dpp(0, (int)f32_bits(v), 0xb1, 0xf, 0xf, false)));       // quad_perm 1 0 3 2
             return v;
         };
         for (int t0 = 0; t0 < T; t0 += U * ROWS) {
@@ -118,16 +123,20 @@ __global__ __launch_bounds__(64 * WV * WPE) void router_kernel(RouterParams p, P
 #pragma unroll
                 for (int i = 1; i < MAXI; ++i) m = fmaxf(m, v[u][i]);
                 m = reduce4(m, [](float x, float y) { return fmaxf(x, y); });
-                float s = 0.f, own[OWN];
+                float own[OWN];
 #pragma unroll
                 for (int i = 0; i < MAXI; ++i) {
                     float x = expf(v[u][i] - m);
-                    x = rl + i * L < E ? x : 0.f;
-                    s += x;
+                    v[u][i] = x = rl + i * L < E ? x : 0.f;
 #pragma unroll
                     for (int w = 0; w < OWN; ++w) own[w] = i == 0 || e0 / L + w == i ? x : own[w];
                 }
-                s = reduce4(s, [](float x, float y) { return x + y; });
+                // added pairwise, the furthest experts first: torch's order, and so its bits, and so the same picks
+#pragma unroll
+                for (int h = MAXI / 2; h > 0; h /= 2)
+#pragma unroll
+                    for (int i = 0; i < h; ++i) v[u][i] += v[u][i + h];
+                const float s = reduce4(v[u][0], [](float x, float y) { return x + y; });
                 const int t = t0 + u * ROWS + rg;
 #pragma unroll
                 for (int w = 0; w < OWN; ++w) {
