@@ -1,4 +1,4 @@
-// Launch side of the tiled weight gradient: tiled_dw_kernel, or dw_dl_kernel for large well-formed 16-bit
+// Launch side of the tiled weight gradient: tiled_dw_kernel, tiled_dw_wide_kernel for few picks, or dw_dl_kernel for large well-formed 16-bit
 // shapes, followed by the fixed-order sum over splits.
 #include "egs_host.h"
 #include "egs_dw_dl.h"
@@ -55,6 +55,7 @@ int dw_general(const void *Xs, const void *Ys, const void *Ind, void *dW, void *
     q.B = d->B; q.T = d->T; q.E = d->E; q.K = d->K; q.I = d->I; q.J = d->J;
     q.ind_dtype = ind_dtype; q.out_dtype = out_dtype; q.eji = dw_layout != 0;
     q.i_tiles = pl.i_tiles; q.j_tiles = pl.j_tiles; q.S = pl.S; q.picks_per_split = pl.picks_per_split;
+    q.wide = pl.wide;
     q.edges = (d->I * ES) % 16 != 0 || (d->J * ES) % 16 != 0;
     const int rc = act_dtype == EGS_F32 ? tiled_dw_f32(q, s) : act_dtype == EGS_F16 ? tiled_dw_f16(q, s) : tiled_dw_bf16(q, s);
     if (rc != EGS_OK || pl.S <= 1) return rc;

@@ -144,6 +144,17 @@ ScatterPlan plan_scatter(const egs_dims *d, int mode, int act_dtype, ScatterPath
     return pl;
 }
 
+// Experts of few picks: dW itself is what takes the time, and tiled_dw_wide_kernel writes it as whole rows.  Each of its workgroups
+// goes through all picks, so there have to be enough of them for the number of picks (a tile and 32 picks take about as long in
+// every kernel).  us, this kernel and the next best: bf16 B1 T256 E128 K4 I1024 J128 16 and 82, B3 T169 E86 K58 I384 J64 14.5 and
+// 17, fp32 B16 E50 K32 I300 J150 54 and 58; with fewer tiles bf16 B4 E6 K21 I64 J64 6.7 and 4.5, with more picks fp32 B32 E50 K32
+// I100 J75 49 and 32.
+int64_t dw_wide_tiles(const egs_dims *d, int act_dtype)
+{
+    return (int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, act_dtype == EGS_F32 ? 64 : 128);
+}
+bool dw_few_picks(const egs_dims *d, int act_dtype) { return (int64_t)d->B * d->K <= 256 && dw_wide_tiles(d, act_dtype) >= 256; }
+
 DwPlan plan_dw(const egs_dims *d, int act_dtype)
 {
     DwPlan pl;
@@ -161,6 +172,7 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
     S = Me > 0 ? (Me + rows - 1) / rows : 1;
     pl.S = (int)S;
     pl.picks_per_split = (int)(rows < INT32_MAX ? rows : INT32_MAX);
+    pl.wide = Me <= 128 || dw_few_picks(d, act_dtype) || (Me <= 512 && dw_wide_tiles(d, act_dtype) >= 512);
     pl.bytes_general = S > 1 ? align_up((size_t)S * d->E * d->I * d->J * 4, 256) : 256;     // never none: this path always has a workspace
 
     // large 16-bit shapes: 256 x 256 (or 256 x 128) tiles, 64-row slabs, splits only to give every CU a workgroup
@@ -185,7 +197,7 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
 
     // small experts: 64 x 64 tiles, up to 1024 picks per workgroup, enough workgroups to cover the device
     pl.small_ok = act_dtype != EGS_F32 && d->I % 8 == 0 && d->J % 8 == 0 && d->I >= 8 && d->J >= 8 && d->I <= 128 &&
-                  d->J <= 128 && Me > 0 && d->E > 0;
+                  d->J <= 128 && Me > 0 && d->E > 0 && !dw_few_picks(d, act_dtype);
     if (pl.small_ok) {
         pl.s_i_tiles = ceil_div(d->I, 64);
         pl.s_j_tiles = ceil_div(d->J, 64);
@@ -366,6 +378,7 @@ bool make_dw_tile(const void *Xs, const void *Ys, const void *Ind, void *dW, con
     if (d->I % 8 || d->J % 8 || d->I < 8 || d->J < 8 || d->I > 2048 || d->J > 128) return false;
     const int64_t Me = (int64_t)d->B * d->K;
     if (Me == 0 || d->E == 0 || d->T == 0) return false;
+    if (dw_few_picks(d, act_dtype)) return false;
     if (ES == 2 && d->I > 128 && d->J > 64 && Me >= 256) return false;      // the 256-row tiles of the direct-to-LDS kernel do better there
     const int it = ceil_div(d->I, 32), jt = ceil_div(d->J, wide ? 64 : 32);
     if ((int64_t)d->E * it * jt < (wide ? 64 : 128)) return false;

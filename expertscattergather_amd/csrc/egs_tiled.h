@@ -400,6 +400,7 @@ struct TiledDwParams {
     int32_t B, T, E, K, I, J;
     int32_t ind_dtype, out_dtype, eji;
     int32_t i_tiles, j_tiles, S, picks_per_split;
+    int32_t wide;               // tiled_dw_wide_kernel (S = 1)
     int32_t edges;              // some row is not a whole number of chunks: chunks may have to be read early and shifted
 };
 // what a pick that does not exist reads instead of a row
@@ -631,6 +632,179 @@ __global__ __launch_bounds__(kThreads) void tiled_dw_kernel(TiledDwParams p)
                 if (out_dtype == 0) reinterpret_cast<float *>(p.dW)[at] = v[x];
                 else reinterpret_cast<uint16_t *>(p.dW)[at] =
                          (uint16_t)((out_dtype == 1 ? pack2<ElemF16>(v[x], 0.f) : pack2<ElemBF16>(v[x], 0.f)) & 0xffffu);
+            }
+        }
+    }
+}
+
+// The same for experts of few picks, where dW itself is what takes the time: 64 rows x 256 bytes of columns per workgroup, a
+// wavefront 16 rows x all columns, the picks in slabs of 32 that the four wavefronts share.  (Splitting the picks over wavefronts
+// and adding four partial tiles up, as above, took 344 us for the 134 MB of fp32 dW at B1 E128 K4 I1024 J256; this way 53.)
+template <class TT>
+struct TiledDwWide {
+    static constexpr int ES = TT::ES, TI = 64, TJ = 256 / ES, NJ = TJ / 16;
+    // bytes of a pick's row in the tiles: an odd number of 32-byte units and 128 more bytes every eight rows for transpose reads
+    // (see TiledLds), fp32 rows 4 banks apart modulo 16
+    static constexpr int XROW = ES == 2 ? TI * 2 + 32 : (TI + 4) * 4, YROW = ES == 2 ? TJ * 2 + 32 : (TJ + 4) * 4;
+    static constexpr int X = 32 * XROW + 512, Y = 32 * YROW + 512;
+    static constexpr int STAGE = X + Y;
+    static constexpr int RS = TJ + 4;                                   // floats per row of a wavefront's results
+    static constexpr int TAB_AT = 2 * STAGE > 64 * RS * 4 ? 2 * STAGE : 64 * RS * 4;
+    static constexpr int BYTES = TAB_AT + 4 * 64 * 8;
+};
+
+template <class TT>
+__global__ __launch_bounds__(kThreads, 3) void tiled_dw_wide_kernel(TiledDwParams p)
+{
+    typedef TiledDwWide<TT> L;
+    constexpr int ES = TT::ES, VEC = TT::VEC, TI = L::TI, TJ = L::TJ, NJ = L::NJ;
+    constexpr int XL = TI * ES / 16, YL = 16;                           // chunks per pick: 8 (fp32 16) of X, 16 of Y
+    constexpr int XN = 32 * XL / kThreads, YN = 32 * YL / kThreads;
+    extern __shared__ __attribute__((aligned(16))) char smem_tiled_dww[];
+    const int per_e = p.i_tiles * p.j_tiles;
+    const int lin = balanced_tile((int)blockIdx.x, p.E * per_e);
+    if (lin < 0) return;
+    const int e = lin / per_e, rest = lin - e * per_e;
+    const int i0 = (rest / p.j_tiles) * TI, j0 = (rest % p.j_tiles) * TJ;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int a = lane & 15, g = lane >> 4;
+    const int Me = p.B * p.K, nslabs = (Me + 31) >> 5;
+    const int xp = tid / XL, xc = tid % XL, yp = tid / YL, yc = tid % YL;
+    const bool x_in = i0 + xc * VEC < p.I, y_in = j0 + yc * VEC < p.J;
+    const int64_t x_last = p.x_bytes - 16, y_last = p.y_bytes - 16;
+
+    // byte offsets of a slab's rows, made by the first half of wavefront 0 two slabs ahead; -1: no such pick
+    int64_t *tab = reinterpret_cast<int64_t *>(smem_tiled_dww + L::TAB_AT);       // [4][X: 32 | Y: 32]
+    uint64_t iw = 0;
+    auto pick_of = [&](int s, int &b, bool &ok) -> int64_t {
+        const int m = s * 32 + (lane & 31), mm = min(m, Me - 1);
+        ok = m < Me;
+        b = mm / p.K;
+        return ((int64_t)b * p.E + e) * p.K + (mm - b * p.K);
+    };
+    auto load_idx = [&](int s) { int b; bool ok; iw = load_index_word(p.Ind, p.ind_dtype, pick_of(s, b, ok)); };
+    auto store_tab = [&](int s) {
+        int b; bool ok;
+        const int64_t pick = pick_of(s, b, ok), t = decode_index_word(iw, p.Ind, p.ind_dtype, pick);
+        ok = ok && t >= 0 && t < (int64_t)p.T;
+        if (lane < 32) {
+            tab[(s & 3) * 64 + lane] = ok ? ((int64_t)b * p.ldx_b + t * p.ldx_t) * ES : -1;
+            tab[(s & 3) * 64 + 32 + lane] = ok ? pick * p.J * ES : -1;
+        }
+    };
+    u32x4 rx[XN], ry[YN];
+    // no load is conditional: what must not count - picks that do not exist, columns past the matrix - is read somewhere in bounds and
+    // cleared on the way into LDS; a chunk at the end of an operand is read early and shifted
+    int shift_x[XN], shift_y[YN];
+    auto issue = [&](int s) {
+        auto fetch = [&](const char *base, int64_t row, int at_in_row, bool in, int64_t last, int &shift) -> u32x4 {
+            const bool ok = row >= 0 && in;
+            const int64_t at = ok ? row + at_in_row : 0, from = min(at, last);
+            shift = ok ? (int)(at - from) : 16;
+            return *reinterpret_cast<const u32x4_any *>(base + from);
+        };
+        const int64_t *row = tab + (s & 3) * 64;
+#pragma unroll
+        for (int h = 0; h < XN; ++h) rx[h] = fetch(p.Xs, row[h * (kThreads / XL) + xp], i0 * ES + xc * 16, x_in, x_last, shift_x[h]);
+#pragma unroll
+        for (int h = 0; h < YN; ++h) ry[h] = fetch(p.Ys, row[32 + h * (kThreads / YL) + yp], j0 * ES + yc * 16, y_in, y_last, shift_y[h]);
+    };
+    auto row_at = [&](int r, int stride) { return r * stride + (ES == 2 ? (r >> 3) * 128 : 0); };
+    auto put = [&](char *stage) {
+        auto settle = [](u32x4 v, int shift) -> u32x4 {
+            if (__any(shift != 0)) {
+                const u32x4 moved = shift_right_bytes(v, min(shift, 15));
+#pragma unroll
+                for (int x = 0; x < 4; ++x) v[x] = shift >= 16 ? 0u : moved[x];
+            }
+            return v;
+        };
+#pragma unroll
+        for (int h = 0; h < XN; ++h)
+            *reinterpret_cast<u32x4 *>(stage + row_at(h * (kThreads / XL) + xp, L::XROW) + xc * 16) = settle(rx[h], shift_x[h]);
+#pragma unroll
+        for (int h = 0; h < YN; ++h)
+            *reinterpret_cast<u32x4 *>(stage + L::X + row_at(h * (kThreads / YL) + yp, L::YROW) + yc * 16) = settle(ry[h], shift_y[h]);
+    };
+    f32x4 acc[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const char *stage) {
+        const char *sy = stage + L::X;
+        if constexpr (ES == 2) {
+            // transpose reads: lane (a, g) points at pick 8 g + 4 h + a / 4, columns 4 (a % 4) .. + 3
+            auto read = [&](const char *tile, int stride, int col) -> u32x4 {
+                const char *at = tile + row_at(g * 8 + (a >> 2), stride) + col * 2 + (a & 3) * 8;
+                const u32x2 lo = lds_read_tr16(at), hi = lds_read_tr16(at + 4 * stride);
+                return u32x4{lo[0], lo[1], hi[0], hi[1]};
+            };
+            const u32x4 xf = read(stage, L::XROW, wave * 16);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) mma_chunk<TT>(acc[j], read(sy, L::YROW, j * 16), xf);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float xv = *reinterpret_cast<const float *>(stage + (k * 4 + g) * L::XROW + (wave * 16 + a) * 4);
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(*reinterpret_cast<const float *>(sy + (k * 4 + g) * L::YROW + (j * 16 + a) * 4), xv,
+                                                                  acc[j], 0, 0, 0);
+            }
+        }
+    };
+    // one barrier per slab, as in tiled_rows_kernel; slabs beyond the last are requested like any other
+    if (wave == 0) {
+        load_idx(0); store_tab(0);
+        load_idx(1); store_tab(1);
+        load_idx(2);
+    }
+    __syncthreads();
+    issue(0);
+    for (int s = 0; s < nslabs; ++s) {
+        char *stage = smem_tiled_dww + (s & 1) * L::STAGE;
+        put(stage);
+        issue(s + 1);
+        if (wave == 0) { store_tab(s + 2); load_idx(s + 3); }
+        __syncthreads();
+        multiply(stage);
+    }
+    __syncthreads();
+
+    // lane (a, g) holds row i0 + 16 wave + a, columns j0 + 16 j + 4 g .. + 3; through LDS, so that whole row (or, [E,J,I], column)
+    // segments leave
+    float *red = reinterpret_cast<float *>(smem_tiled_dww) + wave * 16 * L::RS;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) *reinterpret_cast<f32x4 *>(red + a * L::RS + j * 16 + g * 4) = acc[j];
+    auto pack = [&](float x, float y) -> uint32_t { return p.out_dtype == 1 ? pack2<ElemF16>(x, y) : pack2<ElemBF16>(x, y); };
+    const int oes = p.out_dtype == 0 ? 4 : 2;
+    const bool eji = p.eji != 0;
+    if (eji) __syncthreads();
+    else __builtin_amdgcn_wave_barrier();
+    // four values along the output's rows at a time: [E,I,J] a wavefront's own 16 rows, [E,J,I] all 64 of the workgroup's
+#pragma unroll 1
+    for (int v = lane; v < 4 * TJ; v += 64) {
+        int gi, gj;
+        f32x4 r;
+        if (eji) {
+            const int il = (v & 15) * 4, jl = wave * (TJ / 4) + (v >> 4);
+            const float *at = reinterpret_cast<const float *>(smem_tiled_dww) + il * L::RS + jl;
+            gi = i0 + il; gj = j0 + jl;
+            r = f32x4{at[0], at[L::RS], at[2 * L::RS], at[3 * L::RS]};
+        } else {
+            const int il = v / (TJ / 4), jl = v % (TJ / 4) * 4;
+            gi = i0 + wave * 16 + il; gj = j0 + jl;
+            r = *reinterpret_cast<const f32x4 *>(red + il * L::RS + jl);
+        }
+        if (gi >= p.I || gj >= p.J) continue;
+        const int live = min(4, eji ? p.I - gi : p.J - gj);
+        char *dst = p.dW + (eji ? ((int64_t)e * p.J + gj) * p.I + gi : ((int64_t)e * p.I + gi) * p.J + gj) * oes;
+        if (live == 4) {
+            if (oes == 4) *reinterpret_cast<f32x4_any *>(dst) = r;
+            else *reinterpret_cast<u32x2_any *>(dst) = u32x2{pack(r[0], r[1]), pack(r[2], r[3])};
+        } else {
+            for (int x = 0; x < live; ++x) {
+                if (oes == 4) reinterpret_cast<float *>(dst)[x] = r[x];
+                else reinterpret_cast<uint16_t *>(dst)[x] = (uint16_t)(pack(r[x], 0.f) & 0xffffu);
             }
         }
     }

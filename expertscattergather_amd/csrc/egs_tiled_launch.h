@@ -58,6 +58,18 @@ int launch_tiled_dw(TiledDwParams &p, hipStream_t s)
         EGS_CHECK_LAUNCH("tiny_dw_kernel");
         return EGS_OK;
     }
+    if (p.wide) {
+        typedef TiledDwWide<TT> L;
+        p.i_tiles = ceil_div(p.I, L::TI); p.j_tiles = ceil_div(p.J, L::TJ);
+        const int64_t wide = (int64_t)p.E * p.i_tiles * p.j_tiles;
+        if (wide > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
+        static LdsGrant told;
+        const int rc = allow_large_lds((const void *)tiled_dw_wide_kernel<TT>, told, L::BYTES, "hipFuncSetAttribute(tiled_dw_wide_kernel)");
+        if (rc != EGS_OK) return rc;
+        hipLaunchKernelGGL(tiled_dw_wide_kernel<TT>, dim3((unsigned)(8 * ((wide + 7) / 8))), dim3(kThreads), L::BYTES, s, p);
+        EGS_CHECK_LAUNCH("tiled_dw_wide_kernel");
+        return EGS_OK;
+    }
     const int64_t total = (int64_t)p.E * p.i_tiles * p.j_tiles * p.S;
     if (total > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
     static_assert(TiledDw<TT>::BYTES <= 64 * 1024, "no grant needed");

@@ -71,3 +71,25 @@ def test_odd_views_and_values_that_are_not_finite_stay_where_they_are(dtype):
     assert torch.isnan(Yo.cpu().float()).eq(hit.expand(B, E, K, J)).all()
     want = O.gather_forward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy())
     assert_close(torch.where(hit, torch.from_numpy(want).to(dtype), Yo.cpu()), want, dtype, "Y")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("shape", [(1, 20, 70, 4, 200, 150), (5, 60, 45, 43, 140, 135), (1, 30, 130, 17, 128, 128), (3, 9, 300, 11, 5, 63)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_weight_gradient_of_experts_with_few_picks(shape, dtype):
+    """tiled_dw_wide_kernel: one slab, several, a part of one; both output layouts; picks that do not exist do not count, whatever
+    their rows hold."""
+    B, T, E, K, I, J = shape
+    case = make_case(sum(shape), *shape, dtype)
+    Ind, Y = case["Ind"].clone(), case["Y"].clone()
+    Ind[0, 0, 0], Ind[-1, -1, -1] = T, -1
+    Y[0, 0, 0] = Y[-1, -1, -1] = float("nan")
+    with _abi.launch_log() as log:
+        _, dWg = hk.expert_gather_backward_call(dev(case["X"]), dev(case["Wg"]), dev(Ind), dev(Y), dtype)
+        _, dWs = hk.expert_scatter_backward_call(dev(Y), dev(case["Ws"]), dev(Ind), dev(case["dOut"]), dtype)
+    assert log.kernels.count("tiled_dw_wide_kernel") == 2, log.kernels
+    safe = Ind.clamp(0, T - 1).numpy()
+    Yk = np64(Y)
+    Yk[0, 0, 0] = Yk[-1, -1, -1] = 0
+    assert_close(dWg, O.gather_backward(np64(case["X"]), np64(case["Wg"]), safe, Yk)[1], dtype, "dWg")
+    assert_close(dWs, O.scatter_backward(Yk, np64(case["Ws"]), safe, np64(case["dOut"]))[1], dtype, "dWs")
