@@ -145,10 +145,10 @@ ScatterPlan plan_scatter(const egs_dims *d, int mode, int act_dtype, ScatterPath
 }
 
 // Experts of few picks: dW itself is what takes the time, and tiled_dw_wide_kernel writes it as whole rows.  Each of its workgroups
-// goes through all picks, so there have to be enough of them for the number of picks (a tile and 32 picks take about as long in
-// every kernel).  us, this kernel and the next best: bf16 B1 T256 E128 K4 I1024 J128 16 and 82, B3 T169 E86 K58 I384 J64 14.5 and
-// 17, fp32 B16 E50 K32 I300 J150 54 and 58; with fewer tiles bf16 B4 E6 K21 I64 J64 6.7 and 4.5, with more picks fp32 B32 E50 K32
-// I100 J75 49 and 32.
+// goes through all picks, so there have to be enough of them for the number of picks.  us, this kernel and the next best: bf16 B1
+// T256 E128 K4 I1024 J128 16 and 82, B3 T169 E86 K58 I384 J64 11 and 17; with fewer tiles bf16 B4 E6 K21 I64 J64 6.7 and 4.5.
+// Sizes that only tiled_dw_kernel takes otherwise: fp32 B16 E50 K32 I300 J150 41 and 58 (750 tiles), bf16 B20 E60 K100 I500 J250 76
+// and 138 (960), fp32 B32 E128 K64 I100 J75 110 and 102 (512), bf16 B6 E20 K80 I100 J60 15 and 7 (40).
 int64_t dw_wide_tiles(const egs_dims *d, int act_dtype)
 {
     return (int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, act_dtype == EGS_F32 ? 64 : 128);
@@ -172,7 +172,7 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
     S = Me > 0 ? (Me + rows - 1) / rows : 1;
     pl.S = (int)S;
     pl.picks_per_split = (int)(rows < INT32_MAX ? rows : INT32_MAX);
-    pl.wide = Me <= 128 || dw_few_picks(d, act_dtype) || (Me <= 512 && dw_wide_tiles(d, act_dtype) >= 512);
+    pl.wide = Me <= 128 || (Me <= 512 && dw_wide_tiles(d, act_dtype) >= 256) || dw_wide_tiles(d, act_dtype) >= 768;
     pl.bytes_general = S > 1 ? align_up((size_t)S * d->E * d->I * d->J * 4, 256) : 256;     // never none: this path always has a workspace
 
     // large 16-bit shapes: 256 x 256 (or 256 x 128) tiles, 64-row slabs, splits only to give every CU a workgroup

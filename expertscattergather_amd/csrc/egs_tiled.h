@@ -639,7 +639,7 @@ __global__ __launch_bounds__(kThreads) void tiled_dw_kernel(TiledDwParams p)
 
 // The same for experts of few picks, where dW itself is what takes the time: 64 rows x 256 bytes of columns per workgroup, a
 // wavefront 16 rows x all columns, the picks in slabs of 32 that the four wavefronts share.  (Splitting the picks over wavefronts
-// and adding four partial tiles up, as above, took 344 us for the 134 MB of fp32 dW at B1 E128 K4 I1024 J256; this way 53.)
+// and adding four partial tiles up, as above, took 344 us for the 134 MB of fp32 dW at B1 E128 K4 I1024 J256; this way 46.)
 template <class TT>
 struct TiledDwWide {
     static constexpr int ES = TT::ES, TI = 64, TJ = 256 / ES, NJ = TJ / 16;
@@ -650,7 +650,7 @@ struct TiledDwWide {
     static constexpr int STAGE = X + Y;
     static constexpr int RS = TJ + 4;                                   // floats per row of a wavefront's results
     static constexpr int TAB_AT = 2 * STAGE > 64 * RS * 4 ? 2 * STAGE : 64 * RS * 4;
-    static constexpr int BYTES = TAB_AT + 4 * 64 * 8;
+    static constexpr int TAB = 256, BYTES = TAB_AT + 2 * TAB * 8;
 };
 
 template <class TT>
@@ -673,58 +673,52 @@ __global__ __launch_bounds__(kThreads, 3) void tiled_dw_wide_kernel(TiledDwParam
     const bool x_in = i0 + xc * VEC < p.I, y_in = j0 + yc * VEC < p.J;
     const int64_t x_last = p.x_bytes - 16, y_last = p.y_bytes - 16;
 
-    // byte offsets of a slab's rows, made by the first half of wavefront 0 two slabs ahead; -1: no such pick
-    int64_t *tab = reinterpret_cast<int64_t *>(smem_tiled_dww + L::TAB_AT);       // [4][X: 32 | Y: 32]
-    uint64_t iw = 0;
-    auto pick_of = [&](int s, int &b, bool &ok) -> int64_t {
-        const int m = s * 32 + (lane & 31), mm = min(m, Me - 1);
-        ok = m < Me;
-        b = mm / p.K;
-        return ((int64_t)b * p.E + e) * p.K + (mm - b * p.K);
-    };
-    auto load_idx = [&](int s) { int b; bool ok; iw = load_index_word(p.Ind, p.ind_dtype, pick_of(s, b, ok)); };
-    auto store_tab = [&](int s) {
-        int b; bool ok;
-        const int64_t pick = pick_of(s, b, ok), t = decode_index_word(iw, p.Ind, p.ind_dtype, pick);
-        ok = ok && t >= 0 && t < (int64_t)p.T;
-        if (lane < 32) {
-            tab[(s & 3) * 64 + lane] = ok ? ((int64_t)b * p.ldx_b + t * p.ldx_t) * ES : -1;
-            tab[(s & 3) * 64 + 32 + lane] = ok ? pick * p.J * ES : -1;
+    // byte offsets of the rows of kTab picks, -1: no such pick.  (Made slab by slab, the index words kept the rows' loads waiting.)
+    constexpr int kTab = L::TAB;
+    int64_t *tab = reinterpret_cast<int64_t *>(smem_tiled_dww + L::TAB_AT);       // [X: kTab | Y: kTab]
+    auto make_tab = [&](int s) {                                        // from slab s on
+#pragma unroll
+        for (int at = tid; at < kTab; at += kThreads) {
+            if (s * 32 + at - tid >= Me + 96) break;                    // (two slabs beyond the last are looked up)
+            const int m = s * 32 + at, mm = min(m, Me - 1), b = mm / p.K;
+            const int64_t pick = ((int64_t)b * p.E + e) * p.K + (mm - b * p.K);
+            const int64_t t = decode_index_word(load_index_word(p.Ind, p.ind_dtype, pick), p.Ind, p.ind_dtype, pick);
+            const bool ok = m < Me && t >= 0 && t < (int64_t)p.T;
+            tab[at] = ok ? ((int64_t)b * p.ldx_b + t * p.ldx_t) * ES : -1;
+            tab[kTab + at] = ok ? pick * p.J * ES : -1;
         }
     };
-    u32x4 rx[XN], ry[YN];
+    u32x4 rx[2][XN], ry[2][YN];
     // no load is conditional: what must not count - picks that do not exist, columns past the matrix - is read somewhere in bounds and
     // cleared on the way into LDS; a chunk at the end of an operand is read early and shifted
-    int shift_x[XN], shift_y[YN];
-    auto issue = [&](int s) {
+    int shift_x[2][XN], shift_y[2][YN];
+    auto issue = [&](int s, int q) {
         auto fetch = [&](const char *base, int64_t row, int at_in_row, bool in, int64_t last, int &shift) -> u32x4 {
             const bool ok = row >= 0 && in;
             const int64_t at = ok ? row + at_in_row : 0, from = min(at, last);
             shift = ok ? (int)(at - from) : 16;
             return *reinterpret_cast<const u32x4_any *>(base + from);
         };
-        const int64_t *row = tab + (s & 3) * 64;
+        const int64_t *row = tab + s % (kTab / 32) * 32;
 #pragma unroll
-        for (int h = 0; h < XN; ++h) rx[h] = fetch(p.Xs, row[h * (kThreads / XL) + xp], i0 * ES + xc * 16, x_in, x_last, shift_x[h]);
+        for (int h = 0; h < XN; ++h) rx[q][h] = fetch(p.Xs, row[h * (kThreads / XL) + xp], i0 * ES + xc * 16, x_in, x_last, shift_x[q][h]);
 #pragma unroll
-        for (int h = 0; h < YN; ++h) ry[h] = fetch(p.Ys, row[32 + h * (kThreads / YL) + yp], j0 * ES + yc * 16, y_in, y_last, shift_y[h]);
+        for (int h = 0; h < YN; ++h) ry[q][h] = fetch(p.Ys, row[kTab + h * (kThreads / YL) + yp], j0 * ES + yc * 16, y_in, y_last, shift_y[q][h]);
     };
     auto row_at = [&](int r, int stride) { return r * stride + (ES == 2 ? (r >> 3) * 128 : 0); };
-    auto put = [&](char *stage) {
+    auto put = [&](char *stage, int q) {
         auto settle = [](u32x4 v, int shift) -> u32x4 {
-            if (__any(shift != 0)) {
-                const u32x4 moved = shift_right_bytes(v, min(shift, 15));
+            if (__any(shift & 15)) v = shift_right_bytes(v, shift & 15);            // (at an operand's end)
 #pragma unroll
-                for (int x = 0; x < 4; ++x) v[x] = shift >= 16 ? 0u : moved[x];
-            }
+            for (int x = 0; x < 4; ++x) v[x] = shift >= 16 ? 0u : v[x];
             return v;
         };
 #pragma unroll
         for (int h = 0; h < XN; ++h)
-            *reinterpret_cast<u32x4 *>(stage + row_at(h * (kThreads / XL) + xp, L::XROW) + xc * 16) = settle(rx[h], shift_x[h]);
+            *reinterpret_cast<u32x4 *>(stage + row_at(h * (kThreads / XL) + xp, L::XROW) + xc * 16) = settle(rx[q][h], shift_x[q][h]);
 #pragma unroll
         for (int h = 0; h < YN; ++h)
-            *reinterpret_cast<u32x4 *>(stage + L::X + row_at(h * (kThreads / YL) + yp, L::YROW) + yc * 16) = settle(ry[h], shift_y[h]);
+            *reinterpret_cast<u32x4 *>(stage + L::X + row_at(h * (kThreads / YL) + yp, L::YROW) + yc * 16) = settle(ry[q][h], shift_y[q][h]);
     };
     f32x4 acc[NJ];
 #pragma unroll
@@ -752,21 +746,23 @@ __global__ __launch_bounds__(kThreads, 3) void tiled_dw_wide_kernel(TiledDwParam
             }
         }
     };
-    // one barrier per slab, as in tiled_rows_kernel; slabs beyond the last are requested like any other
-    if (wave == 0) {
-        load_idx(0); store_tab(0);
-        load_idx(1); store_tab(1);
-        load_idx(2);
-    }
+    // one barrier per slab, as in tiled_rows_kernel, two slabs in flight; those beyond the last are requested like any other
+    make_tab(0);
     __syncthreads();
-    issue(0);
-    for (int s = 0; s < nslabs; ++s) {
-        char *stage = smem_tiled_dww + (s & 1) * L::STAGE;
-        put(stage);
-        issue(s + 1);
-        if (wave == 0) { store_tab(s + 2); load_idx(s + 3); }
-        __syncthreads();
-        multiply(stage);
+    issue(0, 0);
+    issue(1, 1);
+    for (int s0 = 0; s0 < nslabs; s0 += 2) {
+        if ((s0 + 2) % (kTab / 32) == 0) { make_tab(s0 + 2); __syncthreads(); }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int s = s0 + q;
+            if (s >= nslabs) break;
+            char *stage = smem_tiled_dww + q * L::STAGE;
+            put(stage, q);
+            issue(s + 2, q);
+            __syncthreads();
+            multiply(stage);
+        }
     }
     __syncthreads();
 
