@@ -742,6 +742,13 @@ int launch_scatter_fused_one(const ScatterFusedParams &p, size_t lds, int blocks
                                            "hipFuncSetAttribute(scatter_fused_multi_kernel)");
         if (rc_lds != EGS_OK) return rc_lds;
         hipLaunchKernelGGL((scatter_fused_multi_kernel<TT, W_NMAJOR, KS>), dim3(blocks), dim3(kFusedThreads), lds, s, p);
+    } else if (p.run > 1) {             // (a weight gradient of the same call follows alone)
+        name = "scatter_fused_runs_kernel";
+        static LdsGrant told_runs;
+        const int rc_lds = allow_large_lds((const void *)scatter_fused_runs_kernel<TT, W_NMAJOR, KS>, told_runs, lds,
+                                           "hipFuncSetAttribute(scatter_fused_runs_kernel)");
+        if (rc_lds != EGS_OK) return rc_lds;
+        hipLaunchKernelGGL((scatter_fused_runs_kernel<TT, W_NMAJOR, KS>), dim3(blocks), dim3(kFusedThreads), lds, s, p);
     } else if (p.tab_seg != nullptr && dwt != nullptr && !dwt->wide && TT::ES == 2) {
       if constexpr (TT::ES == 2) {
         name = "scatter_fused_dwtile_table_kernel";
@@ -877,13 +884,25 @@ int scatter_fused(const void *Y, const void *W, const void *Ind, void *Out, cons
     if (!fp.ok) return EGS_ERR_UNSUPPORTED;
     const size_t lds = fp.lds;
     const int slices = N / kFusedCols;
-    const int64_t blocks = (int64_t)8 * ceil_div(d->B, 8) * slices;
+    // More slices than CUs: runs of slices with one sort.  A CU does its workgroups' slices one after the other, however many fit
+    // its LDS, and a sort takes 0.6 of a slice's time; the run with the shortest rounds was the fastest at 12 of 12 sizes (B64
+    // T256 E32 K32 I768 J64: runs of 6, 61 -> 47 us; B128 T64 E8 K16 I1024 J64: 16, 73 -> 37).
+    int run = 1;
+    if (fp.experts_per_pass == d->E) {
+        double least = 0;
+        for (int r = 1; r <= slices; ++r) {
+            const double cost = (double)(((int64_t)d->B * ceil_div(slices, r) + 255) / 256) * (r + 0.6);
+            if (r == 1 || cost < least) { least = cost; run = r; }
+        }
+    }
+    const int64_t blocks = (int64_t)8 * ceil_div(d->B, 8) * ceil_div(slices, run);
     ScatterFusedParams p;
     memset(&p, 0, sizeof(p));
     p.A = (const char *)Y; p.W = (const char *)W; p.Ind = Ind; p.out = (char *)Out;
     p.B = d->B; p.T = d->T; p.E = d->E; p.K = d->K; p.N = N;
     p.ind_dtype = ind_dtype;
     p.slices = slices;
+    p.run = run;
     p.experts_per_pass = fp.experts_per_pass;
     if (use != nullptr && fused_reads_table(fp, d, act_dtype)) { p.tab_seg = use->seg; p.tab_perm = use->perm; }
     p.perm_at = (int32_t)((int64_t)fp.experts_per_pass * d->K * kFusedCols * 4);

@@ -3,8 +3,9 @@
 //   out[b, t, c0:c0+32] = sum over the picks (e, k) of token t, in routing-table order, of
 //                         A[b, e, k, :] . W(e)[:, c0:c0+32]
 //
-// A workgroup owns one batch element b and one 32-column slice of the output.  It
-//   (0) sorts the picks of b by token in LDS (the counting sort of csr_count_body; the slices of
+// A workgroup owns one batch element b and one 32-column slice of the output, or several in turn where there are more than CUs.
+// It
+//   (0) sorts the picks of b by token in LDS (the counting sort of csr_count_body; the workgroups of
 //       one batch element repeat it, which is cheaper than a launch of its own),
 //   (1) multiplies every pick's row by its expert's weight slice on the MFMAs (operands straight
 //       from global memory into registers, several (expert, 32-pick) units in flight per wavefront)
@@ -44,6 +45,7 @@ struct ScatterFusedParams {
     int32_t B, T, E, K, N;
     int32_t ind_dtype;
     int32_t slices;         // N / kFusedCols
+    int32_t run;            // RUNS: slices that a workgroup does one after the other
     int32_t perm_at, cnt_at;    // byte offsets of the table and of the sort's counters in dynamic LDS (rows start at 0)
     int32_t zero_at;            // ... and of 128 bytes of zeros (128-byte aligned), scatter_fused_zero_at()
     int32_t xcd_batch;          // consecutive batch elements per XCD: 1, 2, 4 or 8
@@ -69,7 +71,7 @@ __host__ __device__ inline size_t scatter_fused_lds(int T, int NP, int rows)
 }
 __host__ __device__ inline size_t scatter_fused_lds(int T, int NP) { return scatter_fused_lds(T, NP, NP); }
 
-template <class TT, bool W_NMAJOR, int KS, bool MULTI = false, bool TABLE = false>
+template <class TT, bool W_NMAJOR, int KS, bool MULTI = false, bool TABLE = false, bool RUNS = false>
 __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, const int block, char *smem)
 {
     // KS = reduction length in MFMA steps of four 16-byte chunks: 32 elements of a 16-bit type, 16 of fp32
@@ -90,14 +92,15 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
     // slices of one batch element sit on one XCD (ids congruent modulo 8 share an XCD), so that its
     // rows are fetched from memory once
     const int grp = block & 7, idx = block >> 3;
-    const int qb = idx / p.slices, slice = idx % p.slices;
+    const int runs = RUNS ? (p.slices + p.run - 1) / p.run : p.slices, qb = idx / runs;
+    const int slice = (idx - qb * runs) * (RUNS ? p.run : 1), slice_end = RUNS ? min(slice + p.run, p.slices) : slice + 1;
     // XCD grp takes runs of xcd_batch consecutive batch elements (a power of two up to 8: the batch elements of one 256-pick
     // row tile of the gather that wrote this scatter's rows, which ran on the XCD of the same number), i.e. the elements
     // xcd_batch * grp .. + xcd_batch - 1 of every 8 * xcd_batch; a last incomplete block: grp of every 8
     const int nb = p.xcd_batch;
     const int b = (qb | (nb - 1)) < ((p.B + 7) >> 3) ? ((qb / nb) * 8 + grp) * nb + (qb & (nb - 1)) : qb * 8 + grp;
     if (b >= p.B) return;
-    const int c0 = slice * kFusedCols;
+    int c0 = slice * kFusedCols;
     const int T = p.T, E = p.E, K = p.K, N = p.N, NP = E * K;
 
     float *rows = reinterpret_cast<float *>(smem);
@@ -254,53 +257,65 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
     };
 
     if constexpr (!MULTI) {
-        for (int u0 = wave; u0 < E * KT2; u0 += NWV * kFusedDepth) {
+        for (int sl = slice; sl < slice_end; ++sl) {
+            if (sl > slice) __syncthreads();            // everybody is done with the last slice's rows
+            for (int u0 = wave; u0 < E * KT2; u0 += NWV * kFusedDepth) {
 #pragma unroll
-            for (int d = 0; d < kFusedDepth; ++d) {
-                // the request for the unit kAhead further on goes out before this one is multiplied: a CU's wavefronts
-                // then take turns at its one address path instead of all queueing there first and multiplying afterwards
-                if constexpr (kAhead < kFusedDepth) load_unit(buf[(d + kAhead) % kFusedDepth], u0 + NWV * (d + kAhead), 0, E);
-                compute_unit(buf[d], u0 + NWV * d, E);
-                if constexpr (kAhead == kFusedDepth) load_unit(buf[d], u0 + NWV * d + NWV * kFusedDepth, 0, E);
-            }
-        }
-        __syncthreads();
-
-        // ---------------- (2) per token: add its product rows in table order; 4 threads x 8 columns per token.
-        // The table entries of a segment are read four at a time without looking at its end (what follows in LDS is the next
-        // segment or the sort's counters: inside the allocation either way); an entry past the end selects a row of zeros
-        // instead of its own, so that the additions need no condition.  Entry q stands for byte (q << 7) | ((q & 7) << 4),
-        // chunk 0 of row q in the rows' XOR order: a thread's two chunks are one XOR away each.  (The phase is bound by
-        // vector-ALU issue - two wavefronts per SIMD, all in it at once - so it is written for few instructions per pick.)
-        const uint32_t c2 = (uint32_t)(tid & 3) << 5, zero_sel = (uint32_t)p.zero_at;
-        for (int t = tid >> 2; t < T; t += kFusedThreads >> 2) {
-            const int s0 = seg[t], s1 = seg[t + 1];
-            f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
-            for (int s = s0; s < s1; s += 4) {
-                const int n = s1 - s;
-                uint32_t en[4];
-                f32x4 v[4][2];
-#pragma unroll
-                for (int x = 0; x < 4; ++x) en[x] = (uint32_t)perm[s + x];
-#pragma unroll
-                for (int x = 0; x < 4; ++x) {
-                    const uint32_t at = kEncoded ? en[x] : (en[x] << 7) | ((en[x] & 7u) << 4);
-                    const uint32_t sel = (x < n) ? at : zero_sel;
-                    v[x][0] = *reinterpret_cast<const f32x4 *>(smem + (sel ^ c2));
-                    v[x][1] = *reinterpret_cast<const f32x4 *>(smem + (sel ^ (c2 | 16u)));
+                for (int d = 0; d < kFusedDepth; ++d) {
+                    // the request for the unit kAhead further on goes out before this one is multiplied: a CU's wavefronts
+                    // then take turns at its one address path instead of all queueing there first and multiplying afterwards
+                    if constexpr (kAhead < kFusedDepth) load_unit(buf[(d + kAhead) % kFusedDepth], u0 + NWV * (d + kAhead), 0, E);
+                    compute_unit(buf[d], u0 + NWV * d, E);
+                    if constexpr (kAhead == kFusedDepth) load_unit(buf[d], u0 + NWV * d + NWV * kFusedDepth, 0, E);
                 }
-#pragma unroll
-                for (int x = 0; x < 4; ++x) { lo += v[x][0]; hi += v[x][1]; }
             }
-            char *dst = p.out + (((size_t)b * T + t) * N + c0 + (tid & 3) * 8) * ES;
-            if constexpr (ES == 4) {
-                reinterpret_cast<f32x4 *>(dst)[0] = lo;
-                reinterpret_cast<f32x4 *>(dst)[1] = hi;
-            } else {
-                u32x4 w;
-                w[0] = pack2<TT>(lo[0], lo[1]); w[1] = pack2<TT>(lo[2], lo[3]);
-                w[2] = pack2<TT>(hi[0], hi[1]); w[3] = pack2<TT>(hi[2], hi[3]);
-                *reinterpret_cast<u32x4 *>(dst) = w;
+            __syncthreads();
+            // the next slice's first operands travel while this one's rows are added
+            const int at0 = c0 + (tid & 3) * 8;
+            if constexpr (RUNS) {
+                c0 += kFusedCols;
+                if (sl + 1 < slice_end) {
+#pragma unroll
+                    for (int d = 0; d < kAhead; ++d) load_unit(buf[d], wave + NWV * d, 0, E);
+                }
+            }
+
+            // ---------------- (2) per token: add its product rows in table order; 4 threads x 8 columns per token.
+            // The table entries of a segment are read four at a time without looking at its end (what follows in LDS is the next
+            // segment or the sort's counters: inside the allocation either way); an entry past the end selects a row of zeros
+            // instead of its own, so that the additions need no condition.  Entry q stands for byte (q << 7) | ((q & 7) << 4),
+            // chunk 0 of row q in the rows' XOR order: a thread's two chunks are one XOR away each.  (The phase is bound by
+            // vector-ALU issue - two wavefronts per SIMD, all in it at once - so it is written for few instructions per pick.)
+            const uint32_t c2 = (uint32_t)(tid & 3) << 5, zero_sel = (uint32_t)p.zero_at;
+            for (int t = tid >> 2; t < T; t += kFusedThreads >> 2) {
+                const int s0 = seg[t], s1 = seg[t + 1];
+                f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
+                for (int s = s0; s < s1; s += 4) {
+                    const int n = s1 - s;
+                    uint32_t en[4];
+                    f32x4 v[4][2];
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) en[x] = (uint32_t)perm[s + x];
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) {
+                        const uint32_t at = kEncoded ? en[x] : (en[x] << 7) | ((en[x] & 7u) << 4);
+                        const uint32_t sel = (x < n) ? at : zero_sel;
+                        v[x][0] = *reinterpret_cast<const f32x4 *>(smem + (sel ^ c2));
+                        v[x][1] = *reinterpret_cast<const f32x4 *>(smem + (sel ^ (c2 | 16u)));
+                    }
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) { lo += v[x][0]; hi += v[x][1]; }
+                }
+                char *dst = p.out + (((size_t)b * T + t) * N + at0) * ES;
+                if constexpr (ES == 4) {
+                    reinterpret_cast<f32x4 *>(dst)[0] = lo;
+                    reinterpret_cast<f32x4 *>(dst)[1] = hi;
+                } else {
+                    u32x4 w;
+                    w[0] = pack2<TT>(lo[0], lo[1]); w[1] = pack2<TT>(lo[2], lo[3]);
+                    w[2] = pack2<TT>(hi[0], hi[1]); w[3] = pack2<TT>(hi[2], hi[3]);
+                    *reinterpret_cast<u32x4 *>(dst) = w;
+                }
             }
         }
     } else {
@@ -369,6 +384,14 @@ __global__ __launch_bounds__(kFusedThreads) void scatter_fused_kernel(ScatterFus
 {
     extern __shared__ __attribute__((aligned(16))) char smem_fused[];
     scatter_fused_body<TT, W_NMAJOR, KS>(p, (int)blockIdx.x, smem_fused);
+}
+
+// more slices than the device has CUs for: a run of them per workgroup, with one sort
+template <class TT, bool W_NMAJOR, int KS>
+__global__ __launch_bounds__(kFusedThreads) void scatter_fused_runs_kernel(ScatterFusedParams p)
+{
+    extern __shared__ __attribute__((aligned(16))) char smem_fused_runs[];
+    scatter_fused_body<TT, W_NMAJOR, KS, false, false, true>(p, (int)blockIdx.x, smem_fused_runs);
 }
 
 // more picks per batch element than LDS holds product rows for: groups of experts, one after the other
