@@ -40,6 +40,9 @@ struct RowsGemmParams {
     // (direct-load kernel only; csr_done reports that the launch took it along)
     // csr_parts workgroups share a batch element's table (csr_blocks = B * csr_parts; set by the launcher)
     int32_t csr_blocks, csr_done, csr_threads, csr_parts;
+    // rows_gemm_dl_kernel, fp32 product rows: tile numbers, which its workgroups go through in strides of their number; whether there
+    // are more rows than stay in the memory-side cache until they are read
+    int32_t tile_blocks, stream_rows;
     int32_t *seg_off, *perm, *rank_tmp, *long_tab;
 };
 

@@ -11,6 +11,9 @@
 //     CU) and 256 x 256 x 32 with four stages compile as well but measured slower on every benchmark
 //     configuration (the loads are bound by bandwidth beyond the L2, not by latency, and 32-deep slabs
 //     pay twice the barriers).
+//   * fp32 product rows (the scatter's) may be launched with one workgroup per CU, which does every 256th tile: its pipeline goes
+//     on from one tile to the next (the next tile's first slab is requested with the last slab of the current one, and lands while
+//     that is multiplied), so that neither its latency nor the way to its addresses stands between two tiles.
 //   * Rows that are fetched through Ind are just per-lane byte offsets into the buffer
 //     descriptor; rows that do not exist get an offset outside it and arrive as zeros.
 //   * K-major operands ([row][reduction]) are read back with 16-byte LDS reads (XOR swizzle set
@@ -94,72 +97,97 @@ __global__ __launch_bounds__(dl_threads(BM, BN), (BK == 32 && dl_threads(BM, BN)
         }
         block -= p.csr_blocks;
     }
-    int e, tile;
-    if (!decode_expert_tile(block, p.m_tiles * p.n_tiles, p.E, e, tile)) return;
-    const int mt = tile / p.n_tiles, nt = tile - mt * p.n_tiles;
-    const int m0 = mt * BM, n0 = nt * BN;
+    // PERSIST: tiles block, block + stride, ... of one XCD (the stride is a multiple of 8)
+    constexpr bool PERSIST = !GATHER && EPI == EPI_STORE_F32 && NSTAGE == 2;
+    const int stride = PERSIST ? (int)gridDim.x - p.csr_blocks : 0;
+    int e, m0, n0;
+    auto find_tile = [&]() -> bool {                    // `block`, or the next one that exists
+        int tile;
+        while (!decode_expert_tile(block, p.m_tiles * p.n_tiles, p.E, e, tile)) {
+            if (!PERSIST || (block += stride) >= p.tile_blocks) return false;
+        }
+        const int mt = tile / p.n_tiles;
+        m0 = mt * BM; n0 = (tile - mt * p.n_tiles) * BN;
+        return true;
+    };
+    if (!find_tile()) return;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int R = p.R, N = p.N;
     const int Me = p.B * p.K;
 
     // ---------------- per-row bookkeeping: byte offset each tile row reads from, element offset it writes to
-    if (tid < BM) {
-        int m = m0 + tid;
-        uint32_t ao = kVoffInvalid;
-        int64_t co = -1;
-        if (m < Me) {
-            int b = m / p.K, k = m - b * p.K;
-            int64_t pick = ((int64_t)b * p.E + e) * p.K + k;
-            if constexpr (GATHER) {
-                int32_t t = load_token(p.Ind, p.ind_dtype, pick, p.T);
-                if (t >= 0) ao = (uint32_t)(((int64_t)b * p.lda_b + (int64_t)t * p.lda_t) * 2);
-            } else {
-                ao = (uint32_t)(pick * R * 2);
+    auto row_table = [&]() {
+        if (tid < BM) {
+            int m = m0 + tid;
+            uint32_t ao = kVoffInvalid;
+            int64_t co = -1;
+            if (m < Me) {
+                int b = m / p.K, k = m - b * p.K;
+                int64_t pick = ((int64_t)b * p.E + e) * p.K + k;
+                if constexpr (GATHER) {
+                    int32_t t = load_token(p.Ind, p.ind_dtype, pick, p.T);
+                    if (t >= 0) ao = (uint32_t)(((int64_t)b * p.lda_b + (int64_t)t * p.lda_t) * 2);
+                } else {
+                    ao = (uint32_t)(pick * R * 2);
+                }
+                co = pick * N;
             }
-            co = pick * N;
+            if constexpr (!PERSIST) a_voff[tid] = ao;
+            c_off[tid] = co;
         }
-        a_voff[tid] = ao;
-        c_off[tid] = co;
+    };
+    if constexpr (!PERSIST) {
+        row_table();
+        __syncthreads();
     }
-    __syncthreads();
 
     const u32x4 rs_a = make_rsrc(p.A, p.a_bytes);
-    const u32x4 rs_w = make_rsrc(p.W + (size_t)e * R * N * WES, (uint32_t)((size_t)R * N * WES));
+    u32x4 rs_w;
 
     // ---------------- loader set-up.  One load covers 1 KB of a tile = 64 / CR rows of a K-major tile;
     // lane l lands on row (64 / CR) j + l / CR, physical chunk l % CR, and therefore fetches the logical
     // chunk (l % CR) ^ key(row).
     uint32_t pv[PL], qv[QL];
+    auto aim = [&]() {
+        rs_w = make_rsrc(p.W + (size_t)e * R * N * WES, (uint32_t)((size_t)R * N * WES));
 #pragma unroll
-    for (int jj = 0; jj < PL; ++jj) {
-        const int row = (wave * PL + jj) * (64 / CR) + lane / CR;
-        const uint32_t ao = a_voff[row];
-        pv[jj] = ao == kVoffInvalid ? kVoffInvalid : ao + (((lane % CR) ^ kmajor_key_rows<CR>(row)) << 4);
-    }
-#pragma unroll
-    for (int jj = 0; jj < QL; ++jj) {
-        if constexpr (!W_TRANS) {
-            const int row = (wave * QL + jj) * (64 / CR) + lane / CR;
-            const int n = n0 + row;
-            qv[jj] = n < N ? (uint32_t)n * (uint32_t)R * 2 + (((lane % CR) ^ kmajor_key_rows<CR>(row)) << 4) : kVoffInvalid;
-        } else if constexpr (W_FP8) {
-            // bytes, [BK reduction rows][16 chunks]: a load covers 4 rows; lane l lands on row 4j + l/16, physical
-            // chunk l%16; chunks are XORed with the low four bits of the row so that the 32 rows one transpose
-            // read touches spread over all banks
-            const int row = (wave * QL + jj) * 4 + (lane >> 4);
-            const int n = n0 + ((lane & 15) ^ (row & 15)) * 16;
-            qv[jj] = n < N ? (uint32_t)row * (uint32_t)N + n : kVoffInvalid;
-        } else {
-            // [BK reduction rows][BN/8 chunks]: a load covers 2 (4) rows of 32 (16) chunks; lane l lands on
-            // row 2j + l/32 (4j + l/16), physical chunk l%32 (l%16)
-            constexpr int LPR = WROW / 16;               // lanes (chunks) per row
-            const int row = (wave * QL + jj) * (64 / LPR) + lane / LPR;
-            const int pc = lane % LPR;
-            const int n = n0 + ((((pc >> 1) ^ tr_swizzle(row)) << 1) | (pc & 1)) * 8;
-            qv[jj] = n < N ? ((uint32_t)row * (uint32_t)N + n) * 2 : kVoffInvalid;
+        for (int jj = 0; jj < PL; ++jj) {
+            const int row = (wave * PL + jj) * (64 / CR) + lane / CR;
+            uint32_t ao;
+            if constexpr (PERSIST) {
+                const int m = m0 + row, b = m / p.K;
+                ao = m < Me ? (uint32_t)((((int64_t)b * p.E + e) * p.K + (m - b * p.K)) * R * 2) : kVoffInvalid;
+            } else {
+                ao = a_voff[row];
+            }
+            pv[jj] = ao == kVoffInvalid ? kVoffInvalid : ao + (((lane % CR) ^ kmajor_key_rows<CR>(row)) << 4);
         }
-    }
+#pragma unroll
+        for (int jj = 0; jj < QL; ++jj) {
+            if constexpr (!W_TRANS) {
+                const int row = (wave * QL + jj) * (64 / CR) + lane / CR;
+                const int n = n0 + row;
+                qv[jj] = n < N ? (uint32_t)n * (uint32_t)R * 2 + (((lane % CR) ^ kmajor_key_rows<CR>(row)) << 4) : kVoffInvalid;
+            } else if constexpr (W_FP8) {
+                // bytes, [BK reduction rows][16 chunks]: a load covers 4 rows; lane l lands on row 4j + l/16, physical
+                // chunk l%16; chunks are XORed with the low four bits of the row so that the 32 rows one transpose
+                // read touches spread over all banks
+                const int row = (wave * QL + jj) * 4 + (lane >> 4);
+                const int n = n0 + ((lane & 15) ^ (row & 15)) * 16;
+                qv[jj] = n < N ? (uint32_t)row * (uint32_t)N + n : kVoffInvalid;
+            } else {
+                // [BK reduction rows][BN/8 chunks]: a load covers 2 (4) rows of 32 (16) chunks; lane l lands on
+                // row 2j + l/32 (4j + l/16), physical chunk l%32 (l%16)
+                constexpr int LPR = WROW / 16;               // lanes (chunks) per row
+                const int row = (wave * QL + jj) * (64 / LPR) + lane / LPR;
+                const int pc = lane % LPR;
+                const int n = n0 + ((((pc >> 1) ^ tr_swizzle(row)) << 1) | (pc & 1)) * 8;
+                qv[jj] = n < N ? ((uint32_t)row * (uint32_t)N + n) * 2 : kVoffInvalid;
+            }
+        }
+    };
+    aim();
     auto issue = [&](int kt, int stage) {
         char *pbase = smem + stage * STAGE + wave * (PL * 1024);
         char *qbase = smem + stage * STAGE + P_BYTES + wave * (QL * 1024);
@@ -206,14 +234,18 @@ __global__ __launch_bounds__(dl_threads(BM, BN), (BK == 32 && dl_threads(BM, BN)
             }
         }
 
-    const int nk = R / BK;
+    const int nk = R / BK;                              // at least two
 #pragma unroll
     for (int st = 0; st < NSTAGE - 1; ++st)
         if (st < nk) issue(st, st);
     int stage = 0;
+    bool later_tile = false, another = false;
+    do {
+    const int tile_n0 = n0;
     for (int kt = 0; kt < nk; ++kt) {
-        // slab kt has landed once at most the loads of the slabs issued after it are outstanding
-        {
+        // slab kt has landed once at most the loads of the slabs issued after it are outstanding (a later tile's first slab: it
+        // had before the stores of the tile before it, which may still be under way)
+        if (!later_tile || kt > 0) {
             const int later = min(nk - 1 - kt, NSTAGE - 2);     // slabs requested after slab kt that may stay in flight
             if (NSTAGE >= 4 && later >= 2) wait_vmem<(NSTAGE >= 4 ? 2 * (PL + QL) : 0)>();
             else if (NSTAGE >= 3 && later >= 1) wait_vmem<(NSTAGE >= 3 ? PL + QL : 0)>();
@@ -224,6 +256,15 @@ __global__ __launch_bounds__(dl_threads(BM, BN), (BK == 32 && dl_threads(BM, BN)
             int fill = stage + NSTAGE - 1;
             if (fill >= NSTAGE) fill -= NSTAGE;
             issue(kt + NSTAGE - 1, fill);
+        }
+        if constexpr (PERSIST) {
+            // past the barrier everybody is done with the stores of the tile before, and the next barrier publishes the table
+            if (kt == 0) row_table();
+            if (kt + 1 == nk) {
+                block += stride;
+                another = block < p.tile_blocks && find_tile();
+                if (another) { aim(); issue(0, stage ^ 1); }
+            }
         }
         const char *tile_m = smem + stage * STAGE;
         const char *tile_n = tile_m + P_BYTES;
@@ -282,10 +323,12 @@ __global__ __launch_bounds__(dl_threads(BM, BN), (BK == 32 && dl_threads(BM, BN)
         }
         if (++stage == NSTAGE) stage = 0;
     }
+    if constexpr (PERSIST) wait_vmem<0>();              // the next tile's first slab, before the stores join the count
 
     constexpr int OES = (EPI == EPI_STORE_F32) ? 4 : 2;
-    if constexpr (OES == 4) {
-        // fp32 product rows: measured slightly faster straight from registers than through LDS
+    if (OES == 4 && !p.stream_rows) {
+        // fp32 product rows that the next launch finds in the memory-side cache: slightly faster straight from registers than
+        // through LDS
         // ---------------- epilogue.  After the MFMAs lane (a, g) holds, for row 16 i + a, the four columns
         // 16 j + 4 g .. + 3.  The values are regrouped across lanes first (lane 4 r + c takes piece c of row r),
         // so that the four pieces of a row, 64 contiguous bytes of fp32 or 32 of a 16-bit type, leave from
@@ -297,21 +340,11 @@ __global__ __launch_bounds__(dl_threads(BM, BN), (BK == 32 && dl_threads(BM, BN)
             char *crow = p.C + co * OES;
     #pragma unroll
             for (int j = 0; j < TN; ++j) {
-                f32x4 v = acc[i][j];
-                if (p.w_scale != nullptr) {
-                    const int nn = n0 + wave_n0 + j * 16 + g * 4;
-    #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] *= nn + r < N ? p.w_scale[(size_t)e * N + nn + r] : 0.f;
-                }
-                const int n = n0 + wave_n0 + j * 16 + sg * 4;      // N % 8 == 0 and n % 4 == 0: the 4 columns are all in or all out
-                if constexpr (OES == 4) {
-                    const u32x4 w = lanes_16g_a_to_4a_g(__builtin_bit_cast(u32x4, v), lane);
-                    if (co >= 0 && n < N) *reinterpret_cast<u32x4 *>(crow + (size_t)n * 4) = w;
-                } else {
-                    u32x4 w = {pack2<TT>(v[0], v[1]), pack2<TT>(v[2], v[3]), 0u, 0u};
-                    w = lanes_16g_a_to_4a_g(w, lane);
-                    if (co >= 0 && n < N) *reinterpret_cast<u32x2 *>(crow + (size_t)n * 2) = u32x2{w[0], w[1]};
-                }
+                const f32x4 v = acc[i][j];
+                const int n = tile_n0 + wave_n0 + j * 16 + sg * 4;      // N % 8 == 0 and n % 4 == 0: the 4 columns are all in or all out
+                const u32x4 w = lanes_16g_a_to_4a_g(__builtin_bit_cast(u32x4, v), lane);
+                if (co >= 0 && n < N) *reinterpret_cast<u32x4 *>(crow + (size_t)n * 4) = w;
+                acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
         }
     } else {
@@ -382,10 +415,18 @@ __global__ __launch_bounds__(dl_threads(BM, BN), (BK == 32 && dl_threads(BM, BN)
                         for (int x = 0; x < 4; ++x) v[x] = pack2<TT>(f[2 * x], f[2 * x + 1]);
                     }
                 }
-                if (co >= 0 && n_here < N) *reinterpret_cast<u32x4 *>(p.C + co * OES + (size_t)n_here * OES) = v;
+                if (co >= 0 && n_here < N) {
+                    // more product rows than that cache holds: whole lines, past the caches (bf16 B32 T2048 E256 K64 J512 I2048:
+                    // 1.82 -> 1.68 ms for the 4.3 GB, and 0.93 -> 0.88 ms to add them up; 64-byte pieces past the caches 2.03)
+                    u32x4 *dst = reinterpret_cast<u32x4 *>(p.C + co * OES + (size_t)n_here * OES);
+                    if constexpr (OES == 4) __builtin_nontemporal_store(v, dst);
+                    else *dst = v;
+                }
             }
         }
     }
+    later_tile = true;
+    } while (PERSIST && another);
 }
 
 }  // namespace egs

@@ -77,6 +77,12 @@ int launch_rows_dl(RowsGemmParams &p, bool &used, hipStream_t s)
             p.csr_parts = (int)(parts < 1 ? 1 : parts > 8 ? 8 : parts);
             p.csr_blocks *= p.csr_parts;
         }
+        p.tile_blocks = (int)grid;
+        p.stream_rows = !GATHER && EPI == EPI_STORE_F32 && (uint64_t)Me * p.E * p.N * 4 > (256ull << 20);
+        // A workgroup per CU goes through its share of the tiles without refilling its pipeline between them (C3: 41 -> 37 us per
+        // group); where table workgroups come first the shares would end at different times (C4: 36 -> 40 us), and rows that are
+        // streamed need the LDS for that.
+        if (!GATHER && EPI == EPI_STORE_F32 && p.csr_blocks == 0 && !p.stream_rows && grid > 256) grid = 256;
         grid += p.csr_blocks;
         if (grid > INT32_MAX) return EGS_ERR_BAD_SHAPE;
         p.csr_done = p.csr_blocks > 0;
