@@ -20,7 +20,7 @@
 //     up by choosing which global chunk each lane fetches); a weight stored [reduction][column]
 //     stays that way in LDS and is read with the transpose read, so no register transposes.
 //
-// Preconditions (checked by the host, which otherwise uses rows_gemm_kernel): 16-bit elements,
+// Preconditions (checked by the host, which otherwise uses tiled_rows_kernel): 16-bit elements,
 // R % 64 == 0, N % 8 == 0, 16-byte aligned rows, operands below 2 GiB.  fp8 (e4m3) weights in the
 // [reduction][column] layout are supported with bf16 activations (N % 16 == 0): the bytes go to LDS as
 // they are, the 8-bit transpose read hands each lane eight reduction-consecutive values and those are
