@@ -1038,7 +1038,7 @@ int gather_gemm_impl(const void *X, const void *W, const void *Ind, void *Y, con
 
 int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, void *workspace,
                       const egs_dims *d, int act_dtype, int ind_dtype, int w_layout, int mode, SmallDwJob *dw,
-                      DwTileJob *dwt, hipStream_t s, const RoutingTable *use, const void *bias, bool &with_rows);
+                      DwTileJob *dwt, hipStream_t s, const RoutingTable *use, const void *bias, bool &bias_done);
 
 // `dw` (optional): a weight gradient of the same call whose first pass may share the product
 // launch and whose second pass may share the reduction launch
@@ -1046,20 +1046,16 @@ int gemm_scatter_impl(const void *Y, const void *W, const void *Ind, void *Out, 
                       const egs_dims *d, int act_dtype, int ind_dtype, int w_layout, int mode, SmallDwJob *dw,
                       DwTileJob *dwt, hipStream_t s, const RoutingTable *use = nullptr, const void *bias = nullptr)
 {
-    if (bias != nullptr) {              // rows of the tiled products come with it; everything else gets it afterwards
-        bool with_rows = false;
-        const int rc = gemm_scatter_rows(Y, W, Ind, Out, workspace, d, act_dtype, ind_dtype, w_layout, mode, dw, dwt, s, use, bias, with_rows);
-        return rc == EGS_OK && !with_rows ? bias_scatter(Out, bias, Ind, d, act_dtype, ind_dtype, s) : rc;
-    }
-    bool none;
-    return gemm_scatter_rows(Y, W, Ind, Out, workspace, d, act_dtype, ind_dtype, w_layout, mode, dw, dwt, s, use, nullptr, none);
+    bool bias_done = false;
+    const int rc = gemm_scatter_rows(Y, W, Ind, Out, workspace, d, act_dtype, ind_dtype, w_layout, mode, dw, dwt, s, use, bias, bias_done);
+    return rc == EGS_OK && bias != nullptr && !bias_done ? bias_scatter(Out, bias, Ind, d, act_dtype, ind_dtype, s) : rc;
 }
 
 int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, void *workspace,
                       const egs_dims *d, int act_dtype, int ind_dtype, int w_layout, int mode, SmallDwJob *dw,
-                      DwTileJob *dwt, hipStream_t s, const RoutingTable *use, const void *bias, bool &with_rows)
+                      DwTileJob *dwt, hipStream_t s, const RoutingTable *use, const void *bias, bool &bias_done)
 {
-    with_rows = false;
+    bias_done = false;
     const int ES = elem_size(act_dtype);
     const size_t out_elems = (size_t)d->B * d->T * d->I;
     if (out_elems == 0) return EGS_OK;
@@ -1145,6 +1141,16 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
         p.C = (char *)rows;
         p.c_vec = d->I % 4 == 0;
         p.seg_off = seg_off; p.perm = perm; p.rank_tmp = rank_tmp; p.long_tab = long_tab;
+        // Whether the rows come with the bias is each group's own answer: a last group with fewer rows per expert than the large
+        // product kernel takes runs the tiled one, which adds it.  Consecutive groups without it get it in one launch.
+        int bare = 0;                   // batch elements from here up to the current group have no bias yet
+        auto add_bias_up_to = [&](int b_end) -> int {
+            if (bias == nullptr || bare >= b_end) return EGS_OK;
+            egs_dims part = *d;
+            part.B = b_end - bare;
+            return bias_scatter((char *)Out + (size_t)bare * d->T * d->I * ES, bias, (const char *)Ind + (size_t)bare * N * ind_size(ind_dtype),
+                                &part, act_dtype, ind_dtype, s);
+        };
         for (int b0 = 0; b0 < d->B; b0 += G) {
             egs_dims sub = *d;
             sub.B = d->B - b0 < G ? d->B - b0 : G;
@@ -1156,9 +1162,12 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
             // launch of its own
             const bool no_table = N >= 1 && N <= kTokenSumPicks && !(dw != nullptr && dw->done && dw->q.S > 1);
             p.csr_blocks = (b0 == 0 && N > 0 && !no_table) ? d->B : 0; p.csr_done = 0;
-            p.bias = bias;
+            p.bias = bias; p.bias_done = 0;
             rc = rows_gemm_scatter(p, act_dtype, w_trans, rows_f32 ? EPI_STORE_F32 : EPI_STORE, s);
-            with_rows = p.bias_done != 0;
+            if (rc == EGS_OK && p.bias_done) {
+                rc = add_bias_up_to(b0);
+                bare = b0 + sub.B;
+            }
             if (rc == EGS_OK && no_table) {
                 rc = launch_token_sum(rows, rows_f32, (const char *)Ind + (size_t)b0 * N * ind_size(ind_dtype), ind_dtype,
                                       (char *)Out + (size_t)b0 * d->T * d->I * ES, &sub, act_dtype, s);
@@ -1174,7 +1183,8 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
                                     b0 + G >= d->B ? dw : nullptr, s);
             if (rc != EGS_OK) return rc;
         }
-        return EGS_OK;
+        bias_done = true;
+        return add_bias_up_to(d->B);
     }
     if (rc != EGS_OK) return rc;
     return launch_segment_sum(rows, rows_f32, seg_off, perm, long_tab, long_part, Out, d, act_dtype, dw, s);

@@ -15,7 +15,7 @@ from tests._util import assert_close, np64
 
 pytestmark = pytest.mark.gpu
 
-from expertscattergather_amd import hip_kernels as hk, workloads as wl
+from expertscattergather_amd import _abi, hip_kernels as hk, workloads as wl
 
 hk.create_kernels()
 DEV = "cuda"
@@ -164,6 +164,30 @@ def test_scatter_cut_into_uneven_batch_groups():
     for b in (0, 6, 7, 13, 14, 19):
         ref = O.scatter_forward(np64(Y[b:b + 1]), np64(inp["Ws"]), Indn[b:b + 1], T, acc=np.float64)
         assert_close(out[b:b + 1], ref, cfg.dtype, f"out[{b}]")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("dims, kernels", [
+    ((10, 256, 128, 64, 1024, 128), ["rows_gemm_dl_kernel", "rows_gemm_dl_kernel", "tiled_rows_kernel"]),       # groups of 4, 4 and 2
+    ((19, 300, 37, 255, 1024, 192), ["rows_gemm_dl_kernel"] * 6 + ["tiled_rows_kernel"]),                       # six of 3 and one of 1
+    ((8, 256, 128, 64, 1024, 128), ["rows_gemm_dl_kernel"] * 2)], ids=["4+4+2", "6x3+1", "4+4"])
+def test_bias_of_a_scatter_cut_into_batch_groups(dims, kernels, dtype):
+    """A last group with fewer rows per expert than the large product kernel takes runs the tiled one, which adds the bias to its rows;
+    the other groups' bias is added afterwards.  Elements on both sides of every group boundary against the oracle."""
+    B, T, E, K, I, J = dims
+    gen = torch.Generator().manual_seed(sum(dims))
+    Y, Ws = torch.randn(B, E, K, J, generator=gen).to(dtype), (torch.randn(E, J, I, generator=gen) / J ** 0.5).to(dtype)
+    bias, Ind = torch.randn(E, 1, I, generator=gen).to(dtype), torch.randint(0, T, (B, E, K), generator=gen)
+    Yd, Wd, Id, bd = (t.to(DEV) for t in (Y, Ws, Ind, bias))
+    with _abi.launch_log() as log:
+        out = hk.expert_scatter(Yd, Wd, Id, T, "deterministic", bd)
+    assert [k for k in log.kernels if "rows" in k] == kernels, log.kernels
+    G = -(-B // len(kernels))
+    for b in sorted({x for g in range(0, B, G) for x in (g, min(g + G, B) - 1)}):
+        ref = O.scatter_forward(np64(Y[b:b + 1]), np64(Ws), Ind[b:b + 1].numpy(), T, acc=np.float64)
+        picks = torch.zeros(T, E, dtype=torch.float64).index_put_((Ind[b].reshape(-1), torch.arange(E).repeat_interleave(K)),
+                                                                  torch.ones((), dtype=torch.float64), accumulate=True)
+        assert_close(out[b:b + 1], ref + (picks.numpy() @ np64(bias[:, 0]))[None], dtype, f"out[{b}]")
 
 
 def test_c5_fp8_weights_forward():
