@@ -289,17 +289,49 @@ void keep_table(PyObject *ind_obj, const TableKey &k, const Tensor &table)
     if (rc != 0) throw python_error();
 }
 
+// hip_kernels.py, which owns the switch of set_routing_table_cache (borrowed; null: gone, or not imported under its name)
+PyObject *g_owner_name = nullptr, *g_cache_name = nullptr;      // "expertscattergather_amd.hip_kernels", "_table_cache"
+PyObject *owner()
+{
+    PyObject *modules = PyImport_GetModuleDict();
+    return modules == nullptr ? nullptr : PyDict_GetItem(modules, g_owner_name);
+}
+
+struct Gil {                    // for the autograd engine's threads, which have a thread state but not the lock
+    PyGILState_STATE state;
+    Gil() : state(PyGILState_Ensure()) {}
+    ~Gil() { PyGILState_Release(state); }
+};
+
+// The table that a backward may use: the one kept with Ind NOW, under the same conditions as in any other call.  (One remembered
+// from the forward would outlive a capture, invalidate_routing_table and set_routing_table_cache(False).)  `Ind` as the node
+// saved it is the caller's object; what saved-tensor hooks made of it has no table, and the indices are sorted.
+Tensor table_of_backward(const Tensor &Ind, const Problem &p)
+{
+    if (egs_routing_table_bytes(&p.d, p.dt) == 0) return Tensor();
+    Gil gil;
+    PyObject *module = owner(), *enabled = module == nullptr ? nullptr : PyObject_GetAttr(module, g_cache_name);
+    if (enabled == nullptr) PyErr_Clear();
+    const bool cache = enabled == Py_True;
+    Py_XDECREF(enabled);
+    PyObject *ind_obj = cache ? THPVariable_Wrap(Ind) : nullptr;
+    if (ind_obj == nullptr) { PyErr_Clear(); return Tensor(); }
+    const Tensor table = table_state(ind_obj, Ind, p, true).table;
+    Py_DECREF(ind_obj);
+    return table;
+}
+
 // ------------------------------------------------------------------------------ autograd
-// Same contract as the Python Functions of hip_kernels.py: what is saved is the inputs (and the routing table that was
-// valid in the forward); the scatter mode is the forward's; both gradients are always computed.
+// Same contract as the Python Functions of hip_kernels.py: what is saved is the inputs; the scatter mode is the forward's; both
+// gradients are always computed.
 struct ExpertGatherFunctionNative : public torch::autograd::Function<ExpertGatherFunctionNative> {
     static Tensor forward(AutogradContext *ctx, const Tensor &X, const Tensor &W, const Tensor &Ind, const std::optional<Tensor> &bias,
-                          const std::optional<Tensor> &table, bool build, int64_t mode)
+                          const std::optional<Tensor> &build, int64_t mode)
     {
-        ctx->save_for_backward({X, W, Ind, table.value_or(Tensor())});
+        ctx->save_for_backward({X, W, Ind});
         ctx->saved_data["mode"] = mode;
         ctx->saved_data["bias"] = bias.has_value();
-        return gather_forward(problem_of(X, W, Ind, true, true, 0), X, W, Ind, build ? *table : Tensor(), EGS_ACT_NONE, bias.value_or(Tensor()));
+        return gather_forward(problem_of(X, W, Ind, true, true, 0), X, W, Ind, build.value_or(Tensor()), EGS_ACT_NONE, bias.value_or(Tensor()));
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
@@ -308,8 +340,8 @@ struct ExpertGatherFunctionNative : public torch::autograd::Function<ExpertGathe
         const Problem p = problem_of(X, W, Ind, true, true, 0);
         TORCH_CHECK(p.ok && plain(grads[0]) && grads[0].scalar_type() == X.scalar_type(), "expert_gather_backward: unexpected operands");
         at::AutoDispatchBelowADInplaceOrView below;
-        Grads g = gather_backward(p, X, W, Ind, saved[3], grads[0], (int)ctx->saved_data["mode"].toInt(), ctx->saved_data["bias"].toBool());
-        return {g.in, g.W, Tensor(), g.bias, Tensor(), Tensor(), Tensor()};
+        Grads g = gather_backward(p, X, W, Ind, table_of_backward(Ind, p), grads[0], (int)ctx->saved_data["mode"].toInt(), ctx->saved_data["bias"].toBool());
+        return {g.in, g.W, Tensor(), g.bias, Tensor(), Tensor()};
     }
 };
 
@@ -395,15 +427,15 @@ PyObject *py_gather_forward(PyObject *, PyObject *const *a, Py_ssize_t n)
         if (!bias_fits(bias, W, p.d.E, p.d.J)) Py_RETURN_NONE;
     }
     if (record && (has_tangent(X) || has_tangent(W) || (bias.defined() && has_tangent(bias)))) Py_RETURN_NONE;
-    TableState ts = table_state(a[2], Ind, p, flag(a[5]));
-    Tensor table = ts.table, Y;
+    const TableState ts = table_state(a[2], Ind, p, flag(a[5]));
+    Tensor table, Y;
     const int64_t mode = PyLong_AsLong(a[4]);
-    const bool build = ts.applies && !table.defined();      // first sight of these indices: built in this launch
+    const bool build = ts.applies && !ts.table.defined();   // first sight of these indices: built in this launch
     {
         NoGil nogil;
         if (build) table = empty_gpu({(int64_t)ts.bytes}, at::kByte, p);
-        if (record && records(X, W, bias)) Y = ExpertGatherFunctionNative::apply(X, W, Ind, some(bias), some(table), build, mode);
-        else Y = gather_forward(p, X, W, Ind, build ? table : Tensor(), EGS_ACT_NONE, bias);
+        if (record && records(X, W, bias)) Y = ExpertGatherFunctionNative::apply(X, W, Ind, some(bias), some(table), mode);
+        else Y = gather_forward(p, X, W, Ind, table, EGS_ACT_NONE, bias);
     }
     if (build) keep_table(a[2], ts.key, table);
     return THPVariable_Wrap(std::move(Y));
@@ -580,6 +612,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_egs_torch", "launchers and autogr
 PyMODINIT_FUNC PyInit__egs_torch(void)
 {
     g_table_attr = PyUnicode_InternFromString("_egs_routing_table");
-    if (g_table_attr == nullptr) return nullptr;
+    g_owner_name = PyUnicode_InternFromString("expertscattergather_amd.hip_kernels");
+    g_cache_name = PyUnicode_InternFromString("_table_cache");
+    if (g_table_attr == nullptr || g_owner_name == nullptr || g_cache_name == nullptr) return nullptr;
     return PyModule_Create(&module);
 }

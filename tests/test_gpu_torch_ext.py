@@ -75,6 +75,61 @@ def test_biases_and_their_gradients(shape, dtype, mode, monkeypatch):
         assert (a.float() - b.float()).abs().max() <= tol * b.float().abs().max(), name
 
 
+def _fresh_table_case():
+    shape = B, T, E, K, I, J = 8, 64, 16, 16, 128, 64       # (the smallest E whose gather backward reads the table)
+    case = make_case(21, *shape, torch.bfloat16)
+    x, W = case["X"].to(DEV).requires_grad_(True), case["Wg"].to(DEV).requires_grad_(True)
+    Ind, other = case["Ind"].to(DEV), make_case(22, *shape, torch.bfloat16)["Ind"].to(DEV)
+    dY = case["Y"].to(DEV)
+    return x, W, Ind, other, dY, torch.autograd.grad(hk.expert_gather(x, W, other.clone()), (x, W), dY)
+
+
+@pytest.mark.parametrize("remedy", ["invalidate", "switch off", "none"])
+def test_gather_backward_uses_no_table_that_was_taken_back(remedy):
+    """A write that the version counter does not see, between forward and backward, with either documented remedy: both gradients
+    follow the indices as they are now.  (Without one the scatter in the backward still reads the table: it is in use.)"""
+    x, W, Ind, other, dY, want = _fresh_table_case()
+    y = hk.expert_gather(x, W, Ind)
+    if remedy == "none":
+        want = torch.autograd.grad(y, x, dY, retain_graph=True) + want[1:]
+    assert hk._TABLE_ATTR in Ind.__dict__
+    Ind.data.copy_(other)
+    try:
+        if remedy == "invalidate":
+            hk.invalidate_routing_table(Ind)
+        elif remedy == "switch off":
+            hk.set_routing_table_cache(False)
+        got = torch.autograd.grad(y, (x, W), dY)
+    finally:
+        hk.set_routing_table_cache(True)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+def test_captured_gather_backward_does_not_use_an_eager_table():
+    """Forward eager, backward alone captured, indices rewritten between replays: every replay sorts what they then hold."""
+    x, W, Ind, other, dY, want = _fresh_table_case()
+    first = Ind.clone()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        torch.autograd.grad(hk.expert_gather(x, W, Ind.clone()), (x, W), dY)                # (library loading before the capture)
+        y = hk.expert_gather(x, W, Ind)
+        before = torch.autograd.grad(y, (x, W), dY, retain_graph=True)
+    s.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        got = torch.autograd.grad(y, (x, W), dY, retain_graph=True)
+    for ind, ref in ((first, before), (other, want), (first, before), (other, want)):
+        Ind.data.copy_(ind)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(got, ref):
+            assert torch.equal(a, b)
+        (x.detach() * 2).sum().item()                                                       # other work between the replays
+
+
 def test_autograd_contract_of_the_native_nodes():
     shape = B, T, E, K, I, J = 4, 64, 8, 16, 128, 64
     case = make_case(9, *shape, torch.bfloat16)
