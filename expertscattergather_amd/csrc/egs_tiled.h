@@ -45,7 +45,7 @@ struct TiledRowsParams {
     char *C;                    // [B,E,K,ldc] rows, element type or fp32
     const float *w_scale;       // [E,N] or nullptr
     const char *bias;           // [E,N] in the element type, or nullptr
-    int64_t a_bytes, w_bytes;   // extents of A and W, at least 16
+    int64_t a_bytes, w_bytes;   // extents of A and W; tiled_rows_kernel: A and an expert's matrix are at least 16 bytes
     int64_t lda_b, lda_t;       // element strides of the source (gather)
     int32_t B, T, E, K, R, N, ldc;
     int32_t ind_dtype, gather, out_f32;
@@ -116,7 +116,8 @@ __global__ __launch_bounds__(kThreads, TN <= 2 ? 4 : 3) void tiled_rows_kernel(T
     }
 
     // ---------------- weight side: byte offsets from the expert's matrix.  A chunk may lie past the reduction length, past the last
-    // column or past the matrix: those values are cleared, never stored, or read early (`w_last`: the last 16 bytes of W)
+    // column or past the matrix: those values are cleared, never stored, or read early (`w_last`: the last 16 bytes of W, which do
+    // not start before this expert's matrix, see launch_tiled)
     const char *We = p.W + (int64_t)e * R * N * WES;
     const int64_t to_end = p.w_bytes - 16 - (int64_t)e * R * N * WES;
     const uint32_t w_last = to_end > 0xffffff00ll ? 0xffffff00u : (uint32_t)to_end;
@@ -356,7 +357,7 @@ __global__ __launch_bounds__(kThreads, TN <= 2 ? 4 : 3) void tiled_rows_kernel(T
     }
 }
 
-// Operands of less than 16 bytes: one thread per product, element by element.
+// Rows or experts of less than 16 bytes in all: one thread per product, element by element.
 template <class TT, int WES, bool W_TRANS>
 __global__ __launch_bounds__(kThreads) void tiny_rows_kernel(TiledRowsParams p)
 {

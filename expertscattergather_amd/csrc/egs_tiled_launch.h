@@ -26,7 +26,9 @@ int launch_tiled(TiledRowsParams &p, hipStream_t s)
 {
     // (offsets inside an expert's matrix are 32-bit, the slab past its end included)
     const bool huge = (uint64_t)p.R * p.N * WES + 128ull * p.N * WES + 4096 > 0xff000000ull;
-    if (p.a_bytes < 16 || p.w_bytes < 16 || huge) {
+    // Every 16-byte read of A stays inside A, and every one of W between the start of an expert's matrix and the end of W: the last
+    // expert's own matrix has to hold one (all others' then do)
+    if (p.a_bytes < 16 || (uint64_t)p.R * p.N * WES < 16 || huge) {
         hipLaunchKernelGGL((tiny_rows_kernel<TT, WES, W_TRANS>), dim3(grid_1d((size_t)p.B * p.E * p.K * p.N)), dim3(kThreads), 0, s, p);
         EGS_CHECK_LAUNCH("tiny_rows_kernel");
         return EGS_OK;

@@ -50,6 +50,23 @@ def test_any_size_matches_the_oracle(shape, dtype, mode):
             assert_close(got[name], ref, dtype, f"{name} {shape} {dtype} {mode}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("dims", [(1, 1), (3, 1), (1, 4), (1, 5), (7, 1), (1, 7), (2, 4), (8, 1), (3, 3)], ids=lambda d: "x".join(map(str, d)))
+def test_experts_of_a_few_bytes(dims, dtype):
+    """16-byte reads of a matrix of less than 16 bytes could not stay inside W: element by element there, by tiles from 16 on."""
+    I, J = dims
+    B, T, E, K = 3, 30, 5, 6
+    case = make_case(40 + I + 9 * J, B, T, E, K, I, J, dtype)
+    X, Wg, Ws, Y, Ind = (dev(case[k]) for k in ("X", "Wg", "Ws", "Y", "Ind"))
+    with _abi.launch_log() as log:
+        got = hk.expert_gather_forward_call(X, Wg, Ind, torch.float32)
+        out = hk.expert_scatter_forward_call(Y, Ws, Ind, T, torch.float32)
+    rows = [k for k in log.kernels if "rows" in k]
+    assert rows == ["tiled_rows_kernel" if I * J * X.element_size() >= 16 else "tiny_rows_kernel"] * 2, log.kernels
+    assert_close(got, O.gather_forward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy()), dtype, "Y")
+    assert_close(out, O.scatter_forward(np64(case["Y"]), np64(case["Ws"]), case["Ind"].numpy(), T), dtype, "out")
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 def test_odd_views_and_values_that_are_not_finite_stay_where_they_are(dtype):
     """X as a view with odd strides that ends at its storage's last element, W and Y off the 16-byte grid (through the C ABI's
