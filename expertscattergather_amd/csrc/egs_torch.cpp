@@ -94,6 +94,12 @@ Problem problem_of(const Tensor &A, const Tensor &W, const Tensor &Ind, bool row
     return p;
 }
 
+// the gradient of an output of these sizes, in the operands' type
+bool grad_fits(const Tensor &g, const Tensor &A, at::IntArrayRef sizes)
+{
+    return plain(g) && g.scalar_type() == A.scalar_type() && g.device() == A.device() && g.sizes().equals(sizes);
+}
+
 Tensor empty_gpu(at::IntArrayRef sizes, at::ScalarType type, const Problem &p)
 {
     return at::detail::empty_cuda(sizes, type, c10::Device(c10::DeviceType::CUDA, p.dev), std::nullopt);
@@ -321,6 +327,34 @@ Tensor table_of_backward(const Tensor &Ind, const Problem &p)
     return table;
 }
 
+// A backward whose operands are not for this way - saved-tensor hooks may hand back another type, layout, alignment or kind of
+// tensor than was saved - by the function `name` of hip_kernels.py, with the saved tensors, the gradient, `option` and whether
+// there is a bias; returns (gradient of the input, of W, of the bias or None).
+Grads backward_in_python(const char *name, const variable_list &saved, const Tensor &grad, int option, bool with_bias)
+{
+    auto fail = [] {
+        python_error err;
+        err.persist();
+        throw err;
+    };
+    Gil gil;
+    PyObject *module = owner();
+    TORCH_CHECK(module != nullptr, name, ": expertscattergather_amd.hip_kernels is not loaded");
+    PyObject *args[4] = {THPVariable_Wrap(saved[0]), THPVariable_Wrap(saved[1]), THPVariable_Wrap(saved[2]), THPVariable_Wrap(grad)};
+    PyObject *res = nullptr;
+    if (args[0] != nullptr && args[1] != nullptr && args[2] != nullptr && args[3] != nullptr)
+        res = PyObject_CallMethod(module, name, "OOOOiO", args[0], args[1], args[2], args[3], option, with_bias ? Py_True : Py_False);
+    for (PyObject *a : args) Py_XDECREF(a);
+    if (res == nullptr) fail();
+    Grads g;
+    Tensor *out[3] = {&g.in, &g.W, &g.bias};
+    if (PyTuple_Check(res) && PyTuple_GET_SIZE(res) == 3)
+        for (int i = 0; i < 3; ++i)
+            if (THPVariable_Check(PyTuple_GET_ITEM(res, i))) *out[i] = THPVariable_Unpack(PyTuple_GET_ITEM(res, i));
+    Py_DECREF(res);
+    return g;
+}
+
 // ------------------------------------------------------------------------------ autograd
 // Same contract as the Python Functions of hip_kernels.py: what is saved is the inputs; the scatter mode is the forward's; both
 // gradients are always computed.
@@ -337,10 +371,16 @@ struct ExpertGatherFunctionNative : public torch::autograd::Function<ExpertGathe
     {
         const auto saved = ctx->get_saved_variables();
         const Tensor &X = saved[0], &W = saved[1], &Ind = saved[2];
+        const int mode = (int)ctx->saved_data["mode"].toInt();
+        const bool bias = ctx->saved_data["bias"].toBool();
         const Problem p = problem_of(X, W, Ind, true, true, 0);
-        TORCH_CHECK(p.ok && plain(grads[0]) && grads[0].scalar_type() == X.scalar_type(), "expert_gather_backward: unexpected operands");
-        at::AutoDispatchBelowADInplaceOrView below;
-        Grads g = gather_backward(p, X, W, Ind, table_of_backward(Ind, p), grads[0], (int)ctx->saved_data["mode"].toInt(), ctx->saved_data["bias"].toBool());
+        Grads g;
+        if (p.ok && grad_fits(grads[0], X, {p.d.B, p.d.E, p.d.K, p.d.J})) {
+            at::AutoDispatchBelowADInplaceOrView below;
+            g = gather_backward(p, X, W, Ind, table_of_backward(Ind, p), grads[0], mode, bias);
+        } else {
+            g = backward_in_python("_gather_backward_of_node", saved, grads[0], mode, bias);
+        }
         return {g.in, g.W, Tensor(), g.bias, Tensor(), Tensor()};
     }
 };
@@ -358,10 +398,15 @@ struct ExpertScatterFunctionNative : public torch::autograd::Function<ExpertScat
     {
         const auto saved = ctx->get_saved_variables();
         const Tensor &Y = saved[0], &W = saved[1], &Ind = saved[2];
+        const bool bias = ctx->saved_data["bias"].toBool();
         const Problem p = problem_of(Y, W, Ind, false, false, ctx->saved_data["T"].toInt());
-        TORCH_CHECK(p.ok && plain(grads[0]) && grads[0].scalar_type() == Y.scalar_type(), "expert_scatter_backward: unexpected operands");
-        at::AutoDispatchBelowADInplaceOrView below;
-        Grads g = scatter_backward(p, Y, W, Ind, grads[0], ctx->saved_data["bias"].toBool());
+        Grads g;
+        if (p.ok && grad_fits(grads[0], Y, {p.d.B, p.d.T, p.d.I})) {
+            at::AutoDispatchBelowADInplaceOrView below;
+            g = scatter_backward(p, Y, W, Ind, grads[0], bias);
+        } else {
+            g = backward_in_python("_scatter_backward_of_node", saved, grads[0], 0, bias);
+        }
         return {g.in, g.W, Tensor(), g.bias, Tensor(), Tensor(), Tensor()};
     }
 };

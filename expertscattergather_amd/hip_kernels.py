@@ -732,17 +732,40 @@ def expert_scatter(Y: torch.Tensor, W: torch.Tensor, Ind: torch.Tensor, T: int, 
         with scatter_mode_scope(scatter_mode):
             out = ExpertScatterFunction.apply(Y, W, Ind, T)
     if bias is not None and T > 0 and Ind.numel() > 0:
-        # picks[b,t,e] = how many times expert e selected token t; each adds bias[e]
-        # (a pick outside [0,T) contributes nothing, as in the kernels: it is routed to slot 0 with weight 0)
-        B, E, K = Ind.shape
-        picks = torch.zeros(B, T, E, device=out.device, dtype=torch.float32)
-        e_ids = torch.arange(E, device=out.device).view(1, E, 1).expand(B, E, K).reshape(B, E * K)
-        ind = Ind.to(torch.int64).reshape(B, E * K)
-        valid = (ind >= 0) & (ind < T)
-        flat = torch.where(valid, ind * E + e_ids, torch.zeros_like(ind))
-        picks.view(B, T * E).scatter_add_(1, flat, valid.to(torch.float32))
-        out = out + (picks @ bias[:, 0, :].float()).to(out.dtype)
+        out = out + (_pick_counts(Ind, T) @ bias[:, 0, :].float()).to(out.dtype)    # each pick adds bias[e]
     return out
+
+
+def _pick_counts(Ind: torch.Tensor, T: int) -> torch.Tensor:
+    """[B,T,E] fp32: how many times expert e selected token t (a pick outside [0,T) contributes nothing, as in the kernels: it
+    is routed to slot 0 with weight 0)."""
+    B, E, K = Ind.shape
+    picks = torch.zeros(B, T, E, device=Ind.device, dtype=torch.float32)
+    e_ids = torch.arange(E, device=Ind.device).view(1, E, 1).expand(B, E, K).reshape(B, E * K)
+    ind = Ind.to(torch.int64).reshape(B, E * K)
+    valid = (ind >= 0) & (ind < T)
+    flat = torch.where(valid, ind * E + e_ids, torch.zeros_like(ind))
+    picks.view(B, T * E).scatter_add_(1, flat, valid.to(torch.float32))
+    return picks
+
+
+# The backward of the two C++ nodes (csrc/egs_torch.cpp) for saved tensors that came back as something those do not take:
+# what the Functions above and the bias's composition from torch operations compute.
+def _gather_backward_of_node(X, W, Ind, grad_output, mode, with_bias):
+    create_kernels()
+    with scatter_mode_scope(next(name for name, m in _MODES.items() if m == mode)):
+        grad_X, grad_W = expert_gather_backward_call(X, W, Ind, grad_output, torch.float32)
+    return grad_X, grad_W, grad_output.sum_to_size(W.shape[0], 1, W.shape[2]) if with_bias else None
+
+
+def _scatter_backward_of_node(Y, W, Ind, grad_X, _, with_bias):
+    create_kernels()
+    grad_Y, grad_W = expert_scatter_backward_call(Y, W, Ind, grad_X, torch.float32)
+    if not with_bias:
+        return grad_Y, grad_W, None
+    T, E = grad_X.shape[1], W.shape[0]
+    grad_bias = _pick_counts(Ind, T).view(-1, E).t() @ grad_X.float().reshape(-1, W.shape[2])
+    return grad_Y, grad_W, grad_bias[:, None].to(grad_X.dtype)
 
 
 # ------------------------------------------------------------------------------ extras (not in the reference)

@@ -130,6 +130,40 @@ def test_captured_gather_backward_does_not_use_an_eager_table():
         (x.detach() * 2).sum().item()                                                       # other work between the replays
 
 
+UNPACK = {"same": lambda t: t, "fp32": lambda t: t.float() if t.is_floating_point() else t.int(),
+          "layout": lambda t: t.transpose(0, 1).contiguous().transpose(0, 1), "copy": lambda t: t.clone(),
+          "alignment": lambda t: torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape).copy_(t)}
+
+
+@pytest.mark.parametrize("bias", [False, True], ids=["plain", "bias"])
+@pytest.mark.parametrize("unpack", list(UNPACK))
+def test_saved_tensors_that_come_back_changed(unpack, bias, monkeypatch):
+    """Saved-tensor hooks may hand back another type, layout or alignment: what the native nodes do not take goes the Python way."""
+    shape = B, T, E, K, I, J = 4, 64, 8, 16, 128, 64
+    case = dict(make_case(31, *shape, torch.bfloat16), shape=shape)
+    case["Ind"][0, 0, 0], case["Ind"][-1, -1, -1] = T, -1
+
+    def run():
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, UNPACK[unpack]):
+            return step(case, torch.bfloat16, case["Ind"].to(DEV), lambda out: case["dOut"].to(DEV), None, bias)
+    fast = run()
+    monkeypatch.setattr(_abi, "_pycall", None)
+    for name, a, b in zip(("out", "dX", "dWg", "dWs", "db_gather", "db_scatter"), fast, run()):
+        assert a.dtype == b.dtype and a.shape == b.shape, name
+        if bias:        # added in fp32 within a launch, or by torch to the rounded result
+            assert (a.float() - b.float()).abs().max() <= 3e-2 * b.float().abs().max(), name
+        else:
+            assert torch.equal(a, b), name
+
+
+def test_saved_tensors_that_come_back_on_the_cpu_are_refused_on_both_routes(monkeypatch):
+    case = dict(make_case(32, 2, 20, 3, 4, 32, 32, torch.bfloat16), shape=(2, 20, 3, 4, 32, 32))
+    for _ in range(2):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.cpu()), pytest.raises(RuntimeError, match="no CPU fallback"):
+            step(case, torch.bfloat16, case["Ind"].to(DEV), lambda out: case["dOut"].to(DEV), None)
+        monkeypatch.setattr(_abi, "_pycall", None)
+
+
 def test_autograd_contract_of_the_native_nodes():
     shape = B, T, E, K, I, J = 4, 64, 8, 16, 128, 64
     case = make_case(9, *shape, torch.bfloat16)
