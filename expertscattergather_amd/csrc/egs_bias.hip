@@ -67,18 +67,19 @@ template <class TT> __global__ __launch_bounds__(kThreads) void bias_rows_kernel
 
 // A workgroup owns tb tokens of a batch element: it counts, in LDS, how often each expert picked each of them (integer
 // additions: their order does not matter), then a wavefront per token adds the rows of the experts that did, in expert order.
+// An output gets one fp32 sum and is rounded once: where the counters do not hold all experts, they are counted again, ec at a
+// time, for every four tokens and 256 columns (E6400 K2 I40 otherwise came out rounded three times).
 template <class TT> __global__ __launch_bounds__(kThreads) void bias_scatter_kernel(BiasParams p)
 {
     extern __shared__ int32_t sh_picks[];               // [tb][ec]
     const int t_blocks = (p.T + p.tb - 1) / p.tb;
     const int b = (int)blockIdx.x / t_blocks, t0 = ((int)blockIdx.x - b * t_blocks) * p.tb;
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int e0 = 0; e0 < p.E; e0 += p.ec) {
-        const int ne = min(p.ec, p.E - e0);
+    auto count = [&](int e0) {
         __syncthreads();
         for (int i = tid; i < p.tb * p.ec; i += kThreads) sh_picks[i] = 0;
         __syncthreads();
-        const int64_t first = ((int64_t)b * p.E + e0) * p.K, n = (int64_t)ne * p.K;
+        const int64_t first = ((int64_t)b * p.E + e0) * p.K, n = (int64_t)min(p.ec, p.E - e0) * p.K;
         for (int64_t q0 = 0; q0 < n; q0 += 4 * kThreads) {
             uint64_t w[4];
 #pragma unroll
@@ -91,12 +92,19 @@ template <class TT> __global__ __launch_bounds__(kThreads) void bias_scatter_ker
             }
         }
         __syncthreads();
-        for (int tl = wave; tl < p.tb && t0 + tl < p.T; tl += kThreads / 64) {
-            char *row = p.out + ((int64_t)b * p.T + t0 + tl) * p.N * TT::ES;
-            for (int c0 = 0; c0 < p.N; c0 += 256) {
-                const int col = c0 + lane * 4, live = min(4, p.N - col);
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                bool any = false;
+    };
+    int counted = -1;                                   // first of the experts whose counts are in LDS
+    for (int tl0 = 0; tl0 < p.tb; tl0 += kThreads / 64) {       // (tb is a multiple of the wavefronts)
+        const int tl = tl0 + wave;
+        const bool exists = t0 + tl < p.T;
+        char *row = p.out + ((int64_t)b * p.T + t0 + tl) * p.N * TT::ES;
+        for (int c0 = 0; c0 < p.N; c0 += 256) {
+            const int col = c0 + lane * 4, live = min(4, p.N - col);
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            bool any = false;
+            for (int e0 = 0; e0 < p.E; e0 += p.ec) {
+                if (counted != e0) { count(e0); counted = e0; }
+                const int ne = exists ? min(p.ec, p.E - e0) : 0;
                 for (int i0 = 0; i0 < ne; i0 += 64) {
                     const int mine = i0 + lane < ne ? sh_picks[tl * p.ec + i0 + lane] : 0;
                     uint64_t who = __ballot(mine != 0);
@@ -110,10 +118,10 @@ template <class TT> __global__ __launch_bounds__(kThreads) void bias_scatter_ker
                         for (int x = 0; x < 4; ++x) acc[x] += c * v[x];
                     }
                 }
-                if (any && live > 0) {
-                    const f32x4 old = elems4<TT>(row, col, live);
-                    for (int x = 0; x < live; ++x) put_elem<TT>(row, col + x, old[x] + acc[x]);
-                }
+            }
+            if (any && live > 0) {
+                const f32x4 old = elems4<TT>(row, col, live);
+                for (int x = 0; x < live; ++x) put_elem<TT>(row, col + x, old[x] + acc[x]);
             }
         }
     }

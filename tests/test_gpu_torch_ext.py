@@ -75,6 +75,21 @@ def test_biases_and_their_gradients(shape, dtype, mode, monkeypatch):
         assert (a.float() - b.float()).abs().max() <= tol * b.float().abs().max(), name
 
 
+@pytest.mark.parametrize("E", [3072, 3073, 6400])
+def test_scatter_bias_is_rounded_once_for_any_number_of_experts(E):
+    """bias_scatter_kernel counts the picks of 3072 experts at a time; what it adds to an output is still one fp32 sum."""
+    B, T, K, I, J = 1, 3, 2, 40, 32
+    gen = torch.Generator().manual_seed(E)
+    Ind, bias = torch.randint(0, T, (B, E, K), generator=gen), (torch.rand(E, 1, I, generator=gen) + 0.5).bfloat16()
+    Y, W = torch.zeros(B, E, K, J, dtype=torch.bfloat16), torch.zeros(E, J, I, dtype=torch.bfloat16)
+    with _abi.launch_log() as log:
+        out = hk.expert_scatter(Y.to(DEV), W.to(DEV), Ind.to(DEV), T, "deterministic", bias.to(DEV)).cpu().double()
+    assert "bias_scatter_kernel" in log.kernels, log.kernels
+    want = torch.zeros(T, I, dtype=torch.float64).index_add_(0, Ind.reshape(-1), bias[:, 0].double().repeat_interleave(K, 0))
+    half_ulp = torch.exp2(torch.floor(torch.log2(want)) - 8)                     # 8 bits of significand
+    assert ((out[0] - want).abs() <= half_ulp + E * K * 2.0 ** -24 * want).all()  # and an fp32 sum of E * K positive terms
+
+
 def _fresh_table_case():
     shape = B, T, E, K, I, J = 8, 64, 16, 16, 128, 64       # (the smallest E whose gather backward reads the table)
     case = make_case(21, *shape, torch.bfloat16)
