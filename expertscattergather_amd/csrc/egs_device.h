@@ -182,30 +182,17 @@ __device__ __forceinline__ int32_t load_token(const void *ind, int ind_dtype, in
 }
 
 // ---------------------------------------------------------------------------- guarded chunk loads
-// `row` points at element 0 of a source row (nullptr => the row reads as zeros), `k0` is the
+// Four fp32 elements.  `row` points at element 0 of a source row (nullptr => the row reads as zeros), `k0` is the
 // first element wanted and `klim` the number of valid elements in the row.  `vec_ok` says the
-// row start is 16-byte aligned and k0 is a multiple of VEC, so an in-range chunk is one load.
-template <int ES>
-__device__ __forceinline__ u32x4 load_chunk(const char *row, int k0, int klim, bool vec_ok)
+// row start is 16-byte aligned and k0 is a multiple of 4, so an in-range chunk is one load.
+__device__ __forceinline__ u32x4 load_chunk_f32(const char *row, int k0, int klim, bool vec_ok)
 {
     u32x4 v = {0u, 0u, 0u, 0u};
     if (row == nullptr || k0 >= klim) return v;
-    constexpr int VEC = 16 / ES;
-    if (vec_ok && k0 + VEC <= klim) {
-        return *reinterpret_cast<const u32x4 *>(row + (size_t)k0 * ES);
-    }
-    if constexpr (ES == 2) {
-        const uint16_t *p = reinterpret_cast<const uint16_t *>(row) + k0;
+    const uint32_t *p = reinterpret_cast<const uint32_t *>(row) + k0;
+    if (vec_ok && k0 + 4 <= klim) return *reinterpret_cast<const u32x4 *>(p);
 #pragma unroll
-        for (int x = 0; x < 8; ++x) {
-            uint32_t h = (k0 + x < klim) ? (uint32_t)p[x] : 0u;
-            v[x >> 1] |= h << (16 * (x & 1));
-        }
-    } else {
-        const uint32_t *p = reinterpret_cast<const uint32_t *>(row) + k0;
-#pragma unroll
-        for (int x = 0; x < 4; ++x) v[x] = (k0 + x < klim) ? p[x] : 0u;
-    }
+    for (int x = 0; x < 4; ++x) v[x] = (k0 + x < klim) ? p[x] : 0u;
     return v;
 }
 
@@ -221,61 +208,6 @@ __device__ __forceinline__ u32x4 fp8x8_to_bf16_chunk(uint32_t lo, uint32_t hi)
     v[1] = (f32_bits(b[0]) >> 16) | (f32_bits(b[1]) & 0xffff0000u);
     v[2] = (f32_bits(c[0]) >> 16) | (f32_bits(c[1]) & 0xffff0000u);
     v[3] = (f32_bits(d[0]) >> 16) | (f32_bits(d[1]) & 0xffff0000u);
-    return v;
-}
-// fp8 source row, result is a bf16 chunk (8 elements); same guards as load_chunk.
-__device__ __forceinline__ u32x4 load_chunk_fp8_as_bf16(const char *row, int k0, int klim, bool vec_ok)
-{
-    u32x4 z = {0u, 0u, 0u, 0u};
-    if (row == nullptr || k0 >= klim) return z;
-    uint32_t lo = 0, hi = 0;
-    if (vec_ok && k0 + 8 <= klim) {
-        u32x2 w = *reinterpret_cast<const u32x2 *>(row + k0);
-        lo = w[0]; hi = w[1];
-    } else {
-        const uint8_t *p = reinterpret_cast<const uint8_t *>(row) + k0;
-#pragma unroll
-        for (int x = 0; x < 8; ++x) {
-            uint32_t b = (k0 + x < klim) ? (uint32_t)p[x] : 0u;
-            if (x < 4) lo |= b << (8 * x); else hi |= b << (8 * (x - 4));
-        }
-    }
-    return fp8x8_to_bf16_chunk(lo, hi);
-}
-
-// 4 consecutive 16-bit elements (8 bytes) with the same guards as load_chunk; `vec_ok` = the row
-// start is 8-byte aligned and k0 is a multiple of 4.
-__device__ __forceinline__ u32x2 load_half_chunk16(const char *row, int k0, int klim, bool vec_ok)
-{
-    u32x2 v = {0u, 0u};
-    if (row == nullptr || k0 >= klim) return v;
-    if (vec_ok && k0 + 4 <= klim) return *reinterpret_cast<const u32x2 *>(row + (size_t)k0 * 2);
-    const uint16_t *p = reinterpret_cast<const uint16_t *>(row) + k0;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-        uint32_t h = (k0 + x < klim) ? (uint32_t)p[x] : 0u;
-        v[x >> 1] |= h << (16 * (x & 1));
-    }
-    return v;
-}
-// 4 consecutive fp8 (e4m3fn) bytes -> 4 bf16; `vec_ok` = 4-byte aligned row start, k0 % 4 == 0.
-__device__ __forceinline__ u32x2 load_half_chunk_fp8_as_bf16(const char *row, int k0, int klim, bool vec_ok)
-{
-    u32x2 z = {0u, 0u};
-    if (row == nullptr || k0 >= klim) return z;
-    uint32_t w = 0;
-    if (vec_ok && k0 + 4 <= klim) {
-        w = *reinterpret_cast<const uint32_t *>(row + k0);
-    } else {
-        const uint8_t *p = reinterpret_cast<const uint8_t *>(row) + k0;
-#pragma unroll
-        for (int x = 0; x < 4; ++x) w |= ((k0 + x < klim) ? (uint32_t)p[x] : 0u) << (8 * x);
-    }
-    auto a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, false);
-    auto b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true);
-    u32x2 v;
-    v[0] = (f32_bits(a[0]) >> 16) | (f32_bits(a[1]) & 0xffff0000u);
-    v[1] = (f32_bits(b[0]) >> 16) | (f32_bits(b[1]) & 0xffff0000u);
     return v;
 }
 
@@ -375,14 +307,6 @@ __device__ __forceinline__ void transpose8x4_16b(const u32x2 (&in)[8], u32x4 (&o
             uint32_t lo = in[2 * p][c >> 1], hi = in[2 * p + 1][c >> 1];
             out[c][p] = (c & 1) ? __builtin_amdgcn_perm(hi, lo, 0x07060302u) : __builtin_amdgcn_perm(hi, lo, 0x05040100u);
         }
-}
-
-__device__ __forceinline__ void transpose4x4_32b(const u32x4 (&in)[4], u32x4 (&out)[4])
-{
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) out[c][r] = in[r][c];
 }
 
 // Lane transposition 16 x 4 -> 4 x 16: lane 16 g + a receives what lane 4 a + g holds.  A global load in

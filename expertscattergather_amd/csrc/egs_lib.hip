@@ -1025,8 +1025,7 @@ int gather_gemm_impl(const void *X, const void *W, const void *Ind, void *Y, con
     const bool w_trans = (w_layout == EGS_W_EIJ);       // [E,I,J]: the reduction index selects the row
     p.a_vec = aligned_to(X, 16) && (ldx_b * ES) % 16 == 0 && (ldx_t * ES) % 16 == 0;
     const int64_t w_row = w_trans ? d->J : d->I;
-    p.w_vec = WES == 1 ? (aligned_to(W, 8) && w_row % 8 == 0) : (aligned_to(W, 16) && (w_row * WES) % 16 == 0);   // stricter than the 8-byte blocks of the transposed loader need
-    p.c_vec = aligned_to(Y, 16) && d->J % 4 == 0;
+    p.w_vec = WES == 1 ? (aligned_to(W, 8) && w_row % 8 == 0) : (aligned_to(W, 16) && (w_row * WES) % 16 == 0);
     {
         const uint64_t span = d->B > 0 && d->T > 0
             ? ((uint64_t)(d->B - 1) * (uint64_t)ldx_b + (uint64_t)(d->T - 1) * (uint64_t)ldx_t + (uint64_t)d->I) * ES : 0;
@@ -1086,7 +1085,6 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
                            (int)aligned_to(acc32, 16));
         EGS_CHECK_LAUNCH("fill_zero_f32_kernel");
         p.C = (char *)acc32;
-        p.c_vec = 0;
         return rows_gemm_scatter(p, act_dtype, w_trans, EPI_ATOMIC_F32, s);
     }
 
@@ -1139,7 +1137,6 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
             }
         }
         p.C = (char *)rows;
-        p.c_vec = d->I % 4 == 0;
         p.seg_off = seg_off; p.perm = perm; p.rank_tmp = rank_tmp; p.long_tab = long_tab;
         // Whether the rows come with the bias is each group's own answer: a last group with fewer rows per expert than the large
         // product kernel takes runs the tiled one, which adds it.  Consecutive groups without it get it in one launch.

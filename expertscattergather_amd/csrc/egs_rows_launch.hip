@@ -1,5 +1,5 @@
-// Launch side of the rows x weight products: rows_gemm_dl_kernel for large well-formed 16-bit shapes, rows_gemm_kernel for
-// fp32 atomics on the output, else the tiled kernels of egs_tiled.h.
+// Launch side of the rows x weight products: rows_gemm_dl_kernel for large well-formed 16-bit shapes, rows_atomic_f32_kernel
+// for fp32 atomics on the output, else the tiled kernels of egs_tiled.h.
 #include "egs_host.h"
 #include "egs_rows_gemm_dl.h"
 
@@ -17,10 +17,10 @@ int launch_rows_atomic(RowsGemmParams &p, hipStream_t s)
     const int64_t grid = (int64_t)8 * ceil_div(p.E, 8) * p.m_tiles * p.n_tiles;
     if (grid > INT32_MAX) return EGS_ERR_BAD_SHAPE;
     if (p.N <= 64)
-        hipLaunchKernelGGL((rows_gemm_kernel<ElemF32, 4, 128, 64, 32, 4, 1, false, W_TRANS, EPI_ATOMIC_F32>), dim3((unsigned)grid), dim3(256), 0, s, p);
+        hipLaunchKernelGGL((rows_atomic_f32_kernel<128, 64, 32, 4, 1, W_TRANS>), dim3((unsigned)grid), dim3(256), 0, s, p);
     else
-        hipLaunchKernelGGL((rows_gemm_kernel<ElemF32, 4, 128, 128, 32, 2, 2, false, W_TRANS, EPI_ATOMIC_F32>), dim3((unsigned)grid), dim3(256), 0, s, p);
-    EGS_CHECK_LAUNCH("rows_gemm_kernel");
+        hipLaunchKernelGGL((rows_atomic_f32_kernel<128, 128, 32, 2, 2, W_TRANS>), dim3((unsigned)grid), dim3(256), 0, s, p);
+    EGS_CHECK_LAUNCH("rows_atomic_f32_kernel");
     return EGS_OK;
 }
 
