@@ -190,6 +190,35 @@ def test_bias_of_a_scatter_cut_into_batch_groups(dims, kernels, dtype):
         assert_close(out[b:b + 1], ref + (picks.numpy() @ np64(bias[:, 0]))[None], dtype, f"out[{b}]")
 
 
+# Numbers of experts that are not a multiple of the eight XCDs, last row tiles of 232 / 240 rows and last column tiles of 8 columns
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("dims", [
+    (8, 512, 67, 61, 2056, 128),        # 269 MB of fp32 rows in one launch, which leave as whole lines past the caches; no table
+    (8, 512, 67, 62, 2056, 128),        # the same with the workgroups of the routing table first in the launch
+    (8, 512, 67, 61, 1032, 128),        # 135 MB: 670 tiles, a workgroup per compute unit goes from one to the next
+    (8, 300, 5, 700, 1032, 192),        # 22 row tiles of each of five experts: some workgroups have one tile more, three XCDs none
+    ], ids=lambda d: "x".join(map(str, d)))
+def test_large_product_rows_with_ragged_tiles(dims, dtype):
+    B, T, E, K, I, J = dims
+    gen = torch.Generator().manual_seed(sum(dims))
+    Y, Ind = torch.randn(B, E, K, J, generator=gen).to(dtype), torch.randint(0, T, (B, E, K), generator=gen)
+    W = (torch.randn(E, J, I, generator=gen) / J ** 0.5).to(dtype)
+    Ind[0, 0, 0], Ind[-1, -1, -1] = T, -1
+    keep = ((Ind >= 0) & (Ind < T)).numpy()[..., None]
+    Yd, Wd, Id = Y.to(DEV), W.to(DEV), Ind.to(DEV)
+    with _abi.launch_log() as log:
+        out = hk.expert_scatter_forward_call(Yd, Wd, Id, T, torch.float32)
+    assert log.kernels[0] == "rows_gemm_dl_kernel" and log.kernels.count("rows_gemm_dl_kernel") == 1, log.kernels
+    assert torch.equal(out, hk.expert_scatter_forward_call(Yd, Wd, Id, T, torch.float32))
+    # the same products with the weights the other way round: grad_X of a gather
+    dX = hk.expert_gather_backward_call(torch.zeros(B, T, I, dtype=dtype, device=DEV), Wd.transpose(1, 2).contiguous(), Id, Yd, torch.float32)[0]
+    safe = Ind.clamp(0, T - 1).numpy()
+    for b in (0, B - 1):
+        ref = O.scatter_forward(np64(Y[b:b + 1]) * keep[b:b + 1], np64(W), safe[b:b + 1], T, acc=np.float64)
+        assert_close(out[b:b + 1], ref, dtype, f"out[{b}]")
+        assert_close(dX[b:b + 1], ref, dtype, f"dX[{b}]")
+
+
 def test_c5_fp8_weights_forward():
     cfg = wl.CONFIGS["C5"]
     B, T, E, K, I, J = cfg.dims
