@@ -1155,29 +1155,29 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
             p.B = sub.B;
             const uint64_t span = (uint64_t)sub.B * N * d->J * ES;
             p.a_bytes = span < (1ull << 31) ? (uint32_t)span : 0;
-            // the routing table may ride along with the (first) product launch (large shapes); otherwise it is a
-            // launch of its own
-            const bool no_table = N >= 1 && N <= kTokenSumPicks && !(dw != nullptr && dw->done && dw->q.S > 1);
-            p.csr_blocks = (b0 == 0 && N > 0 && !no_table) ? d->B : 0; p.csr_done = 0;
+            // the routing table may ride along with the (first) product launch (large shapes); otherwise it is a launch of its own
+            p.csr_blocks = b0 == 0 && N > 0 ? d->B : 0; p.csr_done = 0;
             p.bias = bias; p.bias_done = 0;
             rc = rows_gemm_scatter(p, act_dtype, w_trans, rows_f32 ? EPI_STORE_F32 : EPI_STORE, s);
             if (rc == EGS_OK && p.bias_done) {
                 rc = add_bias_up_to(b0);
                 bare = b0 + sub.B;
             }
-            if (rc == EGS_OK && no_table) {
-                rc = launch_token_sum(rows, rows_f32, (const char *)Ind + (size_t)b0 * N * ind_size(ind_dtype), ind_dtype,
-                                      (char *)Out + (size_t)b0 * d->T * d->I * ES, &sub, act_dtype, s);
-                if (rc != EGS_OK) return rc;
-                continue;
+            // Few picks, and the table would be a launch of its own for one launch of sums: sums that do without it.  us, product and
+            // sums with the table riding along / without a table: bf16 B54 T1123 E15 K23 I192 J320 33 / 40, B14 T2048 E64 K60 I512 J128
+            // 50 / 57, B16 T512 E16 K64 I256 J256 24.5 / 26.9, B8 T2048 E32 K100 I512 J256 38.0 / 36.3; three groups of f16 B61 T1657
+            // E78 K45 I384 J384 234 / 272.  With a launch for the table: B53 T97 E29 K41 I111 J75 fp32 54 / 35.
+            if (rc == EGS_OK && G == d->B && !p.csr_done && N >= 1 && N <= kTokenSumPicks && !(dw != nullptr && dw->done && dw->q.S > 1)) {
+                rc = launch_token_sum(rows, rows_f32, Ind, ind_dtype, Out, d, act_dtype, s);
+            } else {
+                if (rc == EGS_OK && b0 == 0 && !p.csr_done)
+                    rc = launch_routing_table(Ind, ind_dtype, d, seg_off, perm, rank_tmp, cnt, long_tab, s);
+                if (rc == EGS_OK)
+                    rc = launch_segment_sum(rows, rows_f32, seg_off + (size_t)b0 * (d->T + 1), perm + (size_t)b0 * N,
+                                            long_tab + (size_t)b0 * long_tab_stride(N), long_part + (size_t)b0 * long_max_slots(N) * d->I,
+                                            (char *)Out + (size_t)b0 * d->T * d->I * ES, &sub, act_dtype,
+                                            b0 + G >= d->B ? dw : nullptr, s);
             }
-            if (rc == EGS_OK && b0 == 0 && !p.csr_done)
-                rc = launch_routing_table(Ind, ind_dtype, d, seg_off, perm, rank_tmp, cnt, long_tab, s);
-            if (rc != EGS_OK) return rc;
-            rc = launch_segment_sum(rows, rows_f32, seg_off + (size_t)b0 * (d->T + 1), perm + (size_t)b0 * N,
-                                    long_tab + (size_t)b0 * long_tab_stride(N), long_part + (size_t)b0 * long_max_slots(N) * d->I,
-                                    (char *)Out + (size_t)b0 * d->T * d->I * ES, &sub, act_dtype,
-                                    b0 + G >= d->B ? dw : nullptr, s);
             if (rc != EGS_OK) return rc;
         }
         bias_done = true;

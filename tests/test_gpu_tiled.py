@@ -110,3 +110,18 @@ def test_weight_gradient_of_experts_with_few_picks(shape, dtype):
     Yk[0, 0, 0] = Yk[-1, -1, -1] = 0
     assert_close(dWg, O.gather_backward(np64(case["X"]), np64(case["Wg"]), safe, Yk)[1], dtype, "dWg")
     assert_close(dWs, O.scatter_backward(Yk, np64(case["Ws"]), safe, np64(case["dOut"]))[1], dtype, "dWs")
+
+
+@pytest.mark.parametrize("dims, sums", [((6, 200, 16, 64, 256, 192), ["rows_gemm_dl_kernel", "segment_sum_kernel"]),     # the table rides along
+                                        ((6, 200, 16, 64, 256, 120), ["tiled_rows_kernel", "token_sum_kernel"]),         # it would be a launch
+                                        ((6, 200, 33, 125, 256, 120), ["tiled_rows_kernel", "csr_count_kernel", "segment_sum_kernel"]),  # 4125 picks
+                                        ((20, 120, 8, 500, 800, 24), ["tiled_rows_kernel", "csr_count_kernel", "segment_sum_kernel", "tiled_rows_kernel",
+                                                                      "segment_sum_kernel"])],                           # two batch groups
+                         ids=["rides", "few", "many", "groups"])
+def test_which_sums_follow_the_product_rows(dims, sums):
+    B, T, E, K, I, J = dims
+    case = make_case(sum(dims), *dims, torch.bfloat16)
+    with _abi.launch_log() as log:
+        out = hk.expert_scatter_forward_call(dev(case["Y"]), dev(case["Ws"]), dev(case["Ind"]), T, torch.float32)
+    assert log.kernels == sums, log.kernels
+    assert_close(out, O.scatter_forward(np64(case["Y"]), np64(case["Ws"]), case["Ind"].numpy(), T), torch.bfloat16, "out")
