@@ -38,8 +38,16 @@ int launch_rows_tiled(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans
     q.ldc = gather ? p.N : product_ld(p.N);
     q.ind_dtype = p.ind_dtype; q.gather = gather; q.out_f32 = epi == EPI_STORE_F32; q.act = p.act; q.bias = (const char *)p.bias;
     p.bias_done = p.bias != nullptr;
-    // which operand to keep in one XCD's L2: source rows that several experts pick, or the experts' weights
-    q.rows_major = gather && (double)p.B * p.T * p.R * ES > (double)p.E * p.R * p.N * WES;
+    // Which operand to keep in one XCD's L2 (4 MB each), by the bytes that then come from beyond it.  Row tiles outermost: the source
+    // once and the weights again for every row tile (for every XCD, if they fit).  Experts outermost: the weights once and a source
+    // row for every pick.  us, row tiles / experts outermost: bf16 R672 N96 Me2262 E99 106 / 69, f16 R1744 N104 Me2380 E70 235 / 204,
+    // f16 R896 N64 Me2405 E215 183 / 151; the other way bf16 R768 N64 Me2048 E32 18.5 / 19.7.  A source that fits is kept by either:
+    // f16 R64 N256 Me13157 E29 132 / 121.
+    if (gather) {
+        const double fits = 3.5e6, x = (double)p.B * p.T * p.R * ES, w = (double)p.E * p.R * p.N * WES;
+        const double picked = (double)p.E * p.B * p.K * p.R * ES, row_tiles = ((double)p.B * p.K + 63) / 64;
+        q.rows_major = x > fits && (x < picked ? x : picked) + w * (w <= fits ? 8 : row_tiles) < 1.05 * (picked + w);
+    }
     if (fp8_w) return tiled_rows_fp8w(q, w_trans, s);
     return act_dtype == EGS_F32 ? tiled_rows_f32(q, w_trans, s) : act_dtype == EGS_F16 ? tiled_rows_f16(q, w_trans, s) : tiled_rows_bf16(q, w_trans, s);
 }
