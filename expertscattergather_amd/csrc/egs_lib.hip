@@ -1148,6 +1148,7 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
             return bias_scatter((char *)Out + (size_t)bare * d->T * d->I * ES, bias, (const char *)Ind + (size_t)bare * N * ind_size(ind_dtype),
                                 &part, act_dtype, ind_dtype, s);
         };
+        bool token_sums = false;
         for (int b0 = 0; b0 < d->B; b0 += G) {
             egs_dims sub = *d;
             sub.B = d->B - b0 < G ? d->B - b0 : G;
@@ -1166,9 +1167,13 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
             // Few picks, and the table would be a launch of its own for one launch of sums: sums that do without it.  us, product and
             // sums with the table riding along / without a table: bf16 B54 T1123 E15 K23 I192 J320 33 / 40, B14 T2048 E64 K60 I512 J128
             // 50 / 57, B16 T512 E16 K64 I256 J256 24.5 / 26.9, B8 T2048 E32 K100 I512 J256 38.0 / 36.3; three groups of f16 B61 T1657
-            // E78 K45 I384 J384 234 / 272.  With a launch for the table: B53 T97 E29 K41 I111 J75 fp32 54 / 35.
-            if (rc == EGS_OK && G == d->B && !p.csr_done && N >= 1 && N <= kTokenSumPicks && !(dw != nullptr && dw->done && dw->q.S > 1)) {
-                rc = launch_token_sum(rows, rows_f32, Ind, ind_dtype, Out, d, act_dtype, s);
+            // E78 K45 I384 J384 234 / 272.  With a launch for the table: B53 T97 E29 K41 I111 J75 fp32 54 / 35; two groups of rows that
+            // the sums with the table read element by element, bf16 B58 T986 E28 K72 I443 J40 178 / 130.
+            if (b0 == 0)
+                token_sums = (G == d->B || d->I % 4 != 0) && !p.csr_done && N >= 1 && N <= kTokenSumPicks && !(dw != nullptr && dw->done && dw->q.S > 1);
+            if (rc == EGS_OK && token_sums) {
+                rc = launch_token_sum(rows, rows_f32, (const char *)Ind + (size_t)b0 * N * ind_size(ind_dtype), ind_dtype,
+                                      (char *)Out + (size_t)b0 * d->T * d->I * ES, &sub, act_dtype, s);
             } else {
                 if (rc == EGS_OK && b0 == 0 && !p.csr_done)
                     rc = launch_routing_table(Ind, ind_dtype, d, seg_off, perm, rank_tmp, cnt, long_tab, s);
