@@ -42,11 +42,12 @@ int launch_rows_tiled(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans
     // once and the weights again for every row tile (for every XCD, if they fit).  Experts outermost: the weights once and a source
     // row for every pick.  us, row tiles / experts outermost: bf16 R672 N96 Me2262 E99 106 / 69, f16 R1744 N104 Me2380 E70 235 / 204,
     // f16 R896 N64 Me2405 E215 183 / 151; the other way bf16 R768 N64 Me2048 E32 18.5 / 19.7.  A source that fits is kept by either:
-    // f16 R64 N256 Me13157 E29 132 / 121.
+    // f16 R64 N256 Me13157 E29 132 / 121; and where the weights are the larger operand the count promises more than row tiles
+    // outermost keep: f16 R1408 N32 Me140 E165 15.7 / 13.4.
     if (gather) {
         const double fits = 3.5e6, x = (double)p.B * p.T * p.R * ES, w = (double)p.E * p.R * p.N * WES;
         const double picked = (double)p.E * p.B * p.K * p.R * ES, row_tiles = ((double)p.B * p.K + 63) / 64;
-        q.rows_major = x > fits && (x < picked ? x : picked) + w * (w <= fits ? 8 : row_tiles) < 1.05 * (picked + w);
+        q.rows_major = x > fits && x > w && (x < picked ? x : picked) + w * (w <= fits ? 8 : row_tiles) < 1.05 * (picked + w);
     }
     if (fp8_w) return tiled_rows_fp8w(q, w_trans, s);
     return act_dtype == EGS_F32 ? tiled_rows_f32(q, w_trans, s) : act_dtype == EGS_F16 ? tiled_rows_f16(q, w_trans, s) : tiled_rows_bf16(q, w_trans, s);
