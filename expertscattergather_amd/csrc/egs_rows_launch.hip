@@ -1,5 +1,5 @@
-// Launch side of the rows x weight products: rows_gemm_dl_kernel for large well-formed 16-bit shapes, rows_atomic_f32_kernel
-// for fp32 atomics on the output, else the tiled kernels of egs_tiled.h.
+// Launch side of the rows x weight products: rows_gemm_dl_kernel for large well-formed 16-bit shapes, rows_gemm_kernel for other
+// 16-bit shapes that fill its tiles, rows_atomic_f32_kernel for fp32 atomics on the output, else the tiled kernels of egs_tiled.h.
 #include "egs_host.h"
 #include "egs_rows_gemm_dl.h"
 
@@ -51,6 +51,35 @@ int launch_rows_tiled(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans
     }
     if (fp8_w) return tiled_rows_fp8w(q, w_trans, s);
     return act_dtype == EGS_F32 ? tiled_rows_f32(q, w_trans, s) : act_dtype == EGS_F16 ? tiled_rows_f16(q, w_trans, s) : tiled_rows_bf16(q, w_trans, s);
+}
+
+// Large 16-bit products that are not for the direct-to-LDS loads (reduction not a multiple of 64, or shorter than 128); `used`: they
+// are taken here.  Worth it where 128 x 128 or 256 x 256 tiles are filled: by rows and columns, by the experts on each XCD and in the
+// last round of workgroups.  At 110 shapes the product of the three separated what these tiles win (the 32 above the line: 0.98 to
+// 1.51 times, 1.31 on average) from what the small ones do (up to 1.8 times); fp32 rows are bound by their stores more, so that the
+// line lies lower.
+template <class TT, bool GATHER, bool W_TRANS, int EPI>
+int launch_rows_large(RowsGemmParams &p, bool &used, hipStream_t s)
+{
+    used = false;
+    const int64_t Me = (int64_t)p.B * p.K;
+    if (g_force_generic || Me < 512 || p.N < 96 || p.R % 8 != 0 || p.N % 8 != 0 || !p.a_vec || !p.w_vec || !aligned_to(p.C, 16) ||
+        p.act != ACT_NONE || p.bias != nullptr || p.w_scale != nullptr)
+        return EGS_OK;
+    const bool big = p.N >= 192 && p.R >= 128;
+    const int tile = big ? 256 : 128;
+    const int64_t m_tiles = (Me + tile - 1) / tile, n_tiles = ceil_div(p.N, tile), grid = 8 * ceil_div(p.E, 8) * m_tiles * n_tiles;
+    if (grid > INT32_MAX / 2) return EGS_OK;
+    const int64_t tiles = p.E * m_tiles * n_tiles, round = big ? 256 : 512;         // workgroups that run at once
+    const double filled = (double)Me * p.N / ((double)m_tiles * n_tiles * tile * tile) * p.E / (8 * ceil_div(p.E, 8)) *
+                          tiles / ((tiles + round - 1) / round * round);
+    if (filled < (EPI == EPI_STORE_F32 ? 0.7 : 0.75)) return EGS_OK;
+    p.m_tiles = (int)m_tiles; p.n_tiles = (int)n_tiles;
+    if (big) hipLaunchKernelGGL((rows_gemm_kernel<TT, 256, 256, 2, 4, GATHER, W_TRANS, EPI>), dim3((unsigned)grid), dim3(512), 0, s, p);
+    else hipLaunchKernelGGL((rows_gemm_kernel<TT, 128, 128, 2, 2, GATHER, W_TRANS, EPI>), dim3((unsigned)grid), dim3(256), 0, s, p);
+    EGS_CHECK_LAUNCH("rows_gemm_kernel");
+    used = true;
+    return EGS_OK;
 }
 
 // The direct-to-LDS pipeline for large, well-formed 16-bit products; `used`: it takes this one
@@ -123,10 +152,19 @@ int launch_rows_dl(RowsGemmParams &p, bool &used, hipStream_t s)
     return EGS_OK;
 }
 
-template <class TT, bool GATHER, int EPI>
-int launch_rows_dl_w(RowsGemmParams &p, bool w_trans, bool &used, hipStream_t s)
+// the two for 16-bit operands, in this order
+template <class TT, bool GATHER, bool W_TRANS, int EPI>
+int launch_rows_16(RowsGemmParams &p, bool &used, hipStream_t s)
 {
-    return w_trans ? launch_rows_dl<TT, 2, GATHER, true, EPI>(p, used, s) : launch_rows_dl<TT, 2, GATHER, false, EPI>(p, used, s);
+    const int rc = launch_rows_dl<TT, 2, GATHER, W_TRANS, EPI>(p, used, s);
+    if (used || rc != EGS_OK) return rc;
+    p.csr_blocks = 0; p.csr_done = 0;
+    return launch_rows_large<TT, GATHER, W_TRANS, EPI>(p, used, s);
+}
+template <class TT, bool GATHER, int EPI>
+int launch_rows_16_w(RowsGemmParams &p, bool w_trans, bool &used, hipStream_t s)
+{
+    return w_trans ? launch_rows_16<TT, GATHER, true, EPI>(p, used, s) : launch_rows_16<TT, GATHER, false, EPI>(p, used, s);
 }
 
 }  // namespace
@@ -137,8 +175,8 @@ int rows_gemm_gather(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans,
     bool used = false;
     int rc = EGS_OK;
     if (fp8_w) { if (w_trans) rc = launch_rows_dl<ElemBF16, 1, true, true, EPI_STORE>(p, used, s); }
-    else if (act_dtype == EGS_F16) rc = launch_rows_dl_w<ElemF16, true, EPI_STORE>(p, w_trans, used, s);
-    else if (act_dtype == EGS_BF16) rc = launch_rows_dl_w<ElemBF16, true, EPI_STORE>(p, w_trans, used, s);
+    else if (act_dtype == EGS_F16) rc = launch_rows_16_w<ElemF16, true, EPI_STORE>(p, w_trans, used, s);
+    else if (act_dtype == EGS_BF16) rc = launch_rows_16_w<ElemBF16, true, EPI_STORE>(p, w_trans, used, s);
     if (used || rc != EGS_OK) return rc;
     return launch_rows_tiled(p, act_dtype, fp8_w, w_trans, true, EPI_STORE, s);
 }
@@ -150,9 +188,9 @@ int rows_gemm_scatter(RowsGemmParams &p, int act_dtype, bool w_trans, int epi, h
     bool used = false;
     int rc = EGS_OK;
     if (act_dtype == EGS_F16)
-        rc = epi == EPI_STORE ? launch_rows_dl_w<ElemF16, false, EPI_STORE>(p, w_trans, used, s) : launch_rows_dl_w<ElemF16, false, EPI_STORE_F32>(p, w_trans, used, s);
+        rc = epi == EPI_STORE ? launch_rows_16_w<ElemF16, false, EPI_STORE>(p, w_trans, used, s) : launch_rows_16_w<ElemF16, false, EPI_STORE_F32>(p, w_trans, used, s);
     else if (act_dtype == EGS_BF16)
-        rc = epi == EPI_STORE ? launch_rows_dl_w<ElemBF16, false, EPI_STORE>(p, w_trans, used, s) : launch_rows_dl_w<ElemBF16, false, EPI_STORE_F32>(p, w_trans, used, s);
+        rc = epi == EPI_STORE ? launch_rows_16_w<ElemBF16, false, EPI_STORE>(p, w_trans, used, s) : launch_rows_16_w<ElemBF16, false, EPI_STORE_F32>(p, w_trans, used, s);
     if (used || rc != EGS_OK) return rc;
     p.csr_blocks = 0; p.csr_done = 0;
     return launch_rows_tiled(p, act_dtype, false, w_trans, false, epi, s);

@@ -126,3 +126,45 @@ def test_which_sums_follow_the_product_rows(dims, sums):
         out = hk.expert_scatter_forward_call(dev(case["Y"]), dev(case["Ws"]), dev(case["Ind"]), T, torch.float32)
     assert log.kernels == sums, log.kernels
     assert_close(out, O.scatter_forward(np64(case["Y"]), np64(case["Ws"]), case["Ind"].numpy(), T), torch.bfloat16, "out")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("dims, tiles", [((10, 150, 64, 100, 248, 248), "both"),      # 256 x 256, the last row tile 232 rows, the last slab 56 deep
+                                         ((11, 150, 63, 93, 232, 504), "both"),       # 1023 picks; one expert short of eight per XCD
+                                         ((10, 150, 32, 100, 40, 248), "gather"),     # 128 x 128, less than one slab
+                                         ((10, 150, 32, 100, 248, 8), "scatter"),     # one chunk of reduction
+                                         ((8, 150, 32, 125, 72, 256), "gather"),      # a whole slab and one chunk
+                                         ((8, 150, 32, 125, 256, 120), "scatter")], ids=lambda d: "x".join(map(str, d)) if isinstance(d, tuple) else d)
+def test_large_products_off_the_direct_to_lds_loads(dims, tiles, dtype):
+    """rows_gemm_kernel with partial tiles and slabs, both weight layouts, both result types, picks that do not exist."""
+    B, T, E, K, I, J = dims
+    case = make_case(sum(dims), *dims, dtype)
+    Ind = case["Ind"].clone()
+    Ind[0, 0, 0], Ind[-1, -1, -1], Ind[1, 2, 3] = T, -1, -30000
+    keep = ((Ind >= 0) & (Ind < T)).numpy()[..., None]
+    safe = Ind.clamp(0, T - 1).numpy()
+    X, Wg, Ws, Y, dOut, Id = (dev(t) for t in (case["X"], case["Wg"], case["Ws"], case["Y"], case["dOut"], Ind))
+    x, wg, ws, y, do = (np64(case[k]) for k in ("X", "Wg", "Ws", "Y", "dOut"))
+
+    def launch(call, runs):
+        with _abi.launch_log() as log:
+            r = call()
+        assert (log.kernels[0] == "rows_gemm_kernel") == runs, log.kernels
+        return r
+    got = launch(lambda: hk.expert_gather_forward_call(X, Wg, Id, torch.float32), tiles != "scatter")
+    assert_close(got, O.gather_forward(x, wg, safe) * keep, dtype, "Y")
+    wide = torch.full((B, T + 1, I + 8), float("nan"), dtype=dtype, device="cuda")
+    wide[:, :T, :I] = X                                                          # a view with strides of its own, other index types
+    assert torch.equal(launch(lambda: hk.expert_gather_forward_call(wide[:, :T, :I], Wg, Id.int(), torch.float32), tiles != "scatter"), got)
+    dY, _ = launch(lambda: hk.expert_scatter_backward_call(Y, Ws, Id, dOut, torch.float32), tiles != "scatter")
+    assert_close(dY, O.gather_forward(do, ws.transpose(0, 2, 1), safe) * keep, dtype, "dY")
+    want = O.scatter_forward(y * keep, ws, safe, T)
+    for mode in ("deterministic", "atomic"):
+        with hk.scatter_mode_scope(mode):
+            out = launch(lambda: hk.expert_scatter_forward_call(Y, Ws, Id, T, torch.float32), tiles != "gather")
+            dX, _ = launch(lambda: hk.expert_gather_backward_call(X, Ws.transpose(1, 2).contiguous(), Id, Y, torch.float32), tiles != "gather")
+        for name, r in (("out", out), ("dX", dX)):
+            if mode == "atomic":        # one more rounding per pick
+                assert abs(np64(r) - want).max() <= 2 ** (-6 if dtype is torch.bfloat16 else -9) * abs(want).max(), name
+            else:
+                assert_close(r, want, dtype, name)
