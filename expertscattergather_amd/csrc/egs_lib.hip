@@ -521,6 +521,12 @@ template <class TT, bool W_NMAJOR, int KS, int TN, bool GATHER, bool OUT_F32>
 int launch_rows_small_one(SmallRowsJob &j, SmallDwJob *dw, DwTileJob *dwt, hipStream_t s)
 {
     if constexpr (GATHER) {
+        if (j.p.act != ACT_NONE) {
+            if (dw != nullptr || dwt != nullptr) return EGS_ERR_UNSUPPORTED;        // (backward products have no activation)
+            hipLaunchKernelGGL((rows_small_kernel<TT, W_NMAJOR, KS, TN, GATHER, OUT_F32, true>), dim3(j.blocks), dim3(kThreads), j.lds, s, j.p);
+            EGS_CHECK_LAUNCH("rows_small_kernel");
+            return EGS_OK;
+        }
         if (dwt != nullptr) {       // dwt->wide, and j regridded for 8 wavefronts per workgroup (see pair_gather_with_dw_tile)
             static LdsGrant told;
             const size_t tile_lds = dw_tile_lds(kDwWideThreads / 64, 64);
