@@ -55,15 +55,15 @@ int launch_rows_tiled(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans
 
 // Large 16-bit products that are not for the direct-to-LDS loads (reduction not a multiple of 64, or shorter than 128); `used`: they
 // are taken here.  Worth it where 128 x 128 or 256 x 256 tiles are filled: by rows and columns, by the experts on each XCD and in the
-// last round of workgroups.  At 110 shapes the product of the three separated what these tiles win (the 32 above the line: 0.98 to
-// 1.51 times, 1.31 on average) from what the small ones do (up to 1.8 times); fp32 rows are bound by their stores more, so that the
-// line lies lower.
+// last round of workgroups.  At 212 shapes the product of the three separated what these tiles win (the 102 above the lines: 0.94 to
+// 1.67 times, 1.26 on average) from what the small ones do (the others: 0.55 to 1.39, 0.95 on average); fp32 rows are bound by their
+// stores more, so that their line lies lower.
 template <class TT, bool GATHER, bool W_TRANS, int EPI>
 int launch_rows_large(RowsGemmParams &p, bool &used, hipStream_t s)
 {
     used = false;
     const int64_t Me = (int64_t)p.B * p.K;
-    if (g_force_generic || Me < 512 || p.N < 96 || p.R % 8 != 0 || p.N % 8 != 0 || !p.a_vec || !p.w_vec || !aligned_to(p.C, 16) ||
+    if (g_force_generic || Me < 192 || p.N < 96 || p.R % 8 != 0 || p.N % 8 != 0 || !p.a_vec || !p.w_vec || !aligned_to(p.C, 16) ||
         p.act != ACT_NONE || p.bias != nullptr || p.w_scale != nullptr)
         return EGS_OK;
     const bool big = p.N >= 192 && p.R >= 128;
@@ -73,7 +73,7 @@ int launch_rows_large(RowsGemmParams &p, bool &used, hipStream_t s)
     const int64_t tiles = p.E * m_tiles * n_tiles, round = big ? 256 : 512;         // workgroups that run at once
     const double filled = (double)Me * p.N / ((double)m_tiles * n_tiles * tile * tile) * p.E / (8 * ceil_div(p.E, 8)) *
                           tiles / ((tiles + round - 1) / round * round);
-    if (filled < (EPI == EPI_STORE_F32 ? 0.7 : 0.75)) return EGS_OK;
+    if (filled < (EPI == EPI_STORE_F32 ? 0.6 : 0.7)) return EGS_OK;
     p.m_tiles = (int)m_tiles; p.n_tiles = (int)n_tiles;
     if (big) hipLaunchKernelGGL((rows_gemm_kernel<TT, 256, 256, 2, 4, GATHER, W_TRANS, EPI>), dim3((unsigned)grid), dim3(512), 0, s, p);
     else hipLaunchKernelGGL((rows_gemm_kernel<TT, 128, 128, 2, 2, GATHER, W_TRANS, EPI>), dim3((unsigned)grid), dim3(256), 0, s, p);
@@ -117,9 +117,10 @@ int launch_rows_dl(RowsGemmParams &p, bool &used, hipStream_t s)
         }
         p.tile_blocks = (int)grid;
         p.stream_rows = !GATHER && EPI == EPI_STORE_F32 && (uint64_t)Me * p.E * p.N * 4 > (256ull << 20);
-        // A workgroup per CU goes through its share of the tiles without refilling its pipeline between them (C3: 41 -> 37 us per
-        // group); where table workgroups come first the shares would end at different times (C4: 36 -> 40 us), and rows that are
-        // streamed need the LDS for that.
+        // A workgroup per CU goes through its share of the tiles without refilling its pipeline between them (bf16 B1 T4096 E128 K256
+        // I1024 J256, a group of the long-sequence configuration: 37.8 -> 36.5 us in a kernel trace); where table workgroups come first
+        // the shares would end at different times (B8 T1024 E64 K128 I512 J128: 36 -> 40 us), and rows that are streamed need the LDS
+        // for that.
         if (!GATHER && EPI == EPI_STORE_F32 && p.csr_blocks == 0 && !p.stream_rows && grid > 256) grid = 256;
         grid += p.csr_blocks;
         if (grid > INT32_MAX) return EGS_ERR_BAD_SHAPE;

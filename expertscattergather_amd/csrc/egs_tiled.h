@@ -1,14 +1,14 @@
 // Tiled rows x weight products and weight gradients for operands of ANY size and alignment: odd row lengths, views that
-// start anywhere, few picks, few experts.  The specialised kernels (egs_small*.h, egs_rows_gemm_dl.h, egs_dw_tile.h,
-// egs_dw_dl.h) take the shapes they are made for; everything else runs here.
+// start anywhere, few picks, few experts.  The specialised kernels (egs_small*.h, egs_rows_gemm_dl.h, egs_rows_gemm.h,
+// egs_dw_tile.h, egs_dw_dl.h) take the shapes they are made for; everything else runs here.
 //
 // What such calls are bound by is not arithmetic but the chain  index -> row -> LDS -> matrix instruction  and the number of
 // workgroups: a 95 x 65 expert with 74 picks is one 128 x 128 tile, and the kernel this replaces walked its three 32-deep
 // slabs one memory round trip after the other, reading rows that do not start on 16 bytes element by element.  Hence:
 //   * every operand is read 16 bytes at a time wherever a row starts (global memory takes any alignment); the one chunk per
 //     tensor that would reach past its end is read a little earlier and shifted, row tails are masked in the last slab;
-//   * up to four slabs are requested before the first is used, and the LDS tile is double-buffered: one barrier per slab;
-//   * tiles come in 64 or 128 rows x 32 .. 128 columns, so that a ragged width wastes little and a small problem still has
+//   * two slabs are in flight in registers and the LDS tile is double-buffered: one barrier per slab;
+//   * tiles are 64 rows x 32 .. 96 columns, so that a ragged width wastes little and a small problem still has
 //     many workgroups; workgroups are dealt to the XCDs evenly for any number of experts.
 #pragma once
 #include "egs_device.h"
@@ -69,8 +69,9 @@ struct TiledLds {
 
 // 64 rows x 16 * TN columns per workgroup of four wavefronts, each 16 rows x all columns, two slabs in flight in registers.  What
 // hides one workgroup's round trips is the others of its compute unit, so the registers are bounded for three or four.
-// (128-row tiles were level or slower at all of 42 shapes but where they left fewer columns over; four slabs in flight gave
-// 4% at R1000 and a few tiles, and cost occupancy elsewhere.)
+// (128-row tiles of this kernel were level or slower at all of 42 small and ragged shapes but where they left fewer columns over;
+// large 16-bit products are another matter, see rows_gemm_kernel.  Four slabs in flight gave 4% at R1000 and a few tiles, and cost
+// occupancy elsewhere.)
 template <class TT, int WES, bool W_TRANS, int TN>
 __global__ __launch_bounds__(kThreads, TN <= 2 ? 4 : 3) void tiled_rows_kernel(TiledRowsParams p)
 {

@@ -879,10 +879,13 @@ def _mlp_forward_impl(X: torch.Tensor, W_gather: torch.Tensor, W_scatter: torch.
     Y [B,E,K,J] between the two products never exist in memory; every other case, and every case where the one
     kernel is known to lose (more workgroups than one round of the device, or an expensive activation on many
     experts: its four slice workgroups per batch element each repeat the gather product), runs the two forward
-    launchers with torch's activation in between (on the GPU all the same).  ``force_block=True`` takes the one
-    kernel whenever it can run.  ``activation``: "none", "relu",
-    "gelu", "gelu_tanh", "silu".  The activation is applied to the fp32 product and rounded to the element
-    type once, exactly where a stored Y would have been rounded."""
+    launchers: dense 16-bit operands with the activation in the gather's launch, other operands (fp32, views, mixed
+    types) with torch's activation in between.  ``force_block=True`` takes the one kernel whenever it can run.
+    ``activation``: "none", "relu", "gelu", "gelu_tanh", "silu".
+
+    Rounding of 16-bit rows: the one kernel, and the two launchers at the sizes where `_mlp_block_pays`, apply the activation to
+    the fp32 product and round once; elsewhere the product is rounded first, as a stored Y would be, and the activation's
+    result again.  "gelu" in these launches uses an erf with an absolute error below 1.5e-7, far below that rounding."""
     if activation not in _ACTIVATIONS:
         raise ValueError(f"activation must be one of {sorted(k for k in _ACTIVATIONS if k)}, got {activation!r}")
     act = _ACTIVATIONS[activation]

@@ -17,9 +17,9 @@ SHAPES = [
     (3, 9, 2, 5, 5, 3),                 # rows shorter than a chunk on both sides
     (2, 40, 9, 33, 63, 65), (2, 40, 3, 32, 65, 63),                 # one element off a slab and a tile
     (4, 50, 5, 16, 520, 17),            # nine slabs, a column tile with one column in its second 16
-    (2, 70, 7, 65, 129, 81),            # 130 picks per expert: one row tile and two rows; widths of 80 and 144
+    (2, 70, 7, 65, 129, 81),            # 130 picks per expert: two row tiles and two rows; one column past 128 and 80
     (6, 30, 11, 29, 97, 131),           # tokens picked tens of times
-    (40, 33, 13, 64, 72, 100),          # 2560 picks per expert: 128-row tiles, splits of the weight gradient
+    (40, 33, 13, 64, 72, 100),          # 2560 picks per expert: 40 row tiles, the weight gradient in three splits
 ]
 
 
@@ -113,8 +113,8 @@ def test_weight_gradient_of_experts_with_few_picks(shape, dtype):
 
 
 @pytest.mark.parametrize("dims, sums", [((6, 200, 16, 64, 256, 192), ["rows_gemm_dl_kernel", "segment_sum_kernel"]),     # the table rides along
-                                        ((6, 200, 16, 64, 256, 120), ["tiled_rows_kernel", "token_sum_kernel"]),         # it would be a launch
-                                        ((6, 200, 33, 125, 256, 120), ["tiled_rows_kernel", "csr_count_kernel", "segment_sum_kernel"]),  # 4125 picks
+                                        ((6, 200, 16, 64, 256, 121), ["tiled_rows_kernel", "token_sum_kernel"]),         # it would be a launch
+                                        ((6, 200, 33, 125, 256, 121), ["tiled_rows_kernel", "csr_count_kernel", "segment_sum_kernel"]),  # 4125 picks
                                         ((20, 120, 7, 500, 844, 25), ["tiled_rows_kernel", "csr_count_kernel", "segment_sum_kernel", "tiled_rows_kernel",
                                                                       "segment_sum_kernel"]),                            # two batch groups
                                         ((20, 120, 8, 500, 801, 24), ["tiled_rows_kernel", "token_sum_kernel"] * 2)],    # of rows read by elements
