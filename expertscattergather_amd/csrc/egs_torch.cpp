@@ -26,7 +26,9 @@
 #include <torch/csrc/jit/frontend/tracer.h>
 
 #include <algorithm>
+#include <atomic>
 #include <tuple>
+#include <vector>
 
 #include "egs_hip.h"
 
@@ -224,7 +226,7 @@ struct TableKey {
     uint64_t ptr, version, stream, capture;
     PyObject *dtype;            // borrowed
     egs_dims d;
-    int dt;
+    int dt, ind;
 };
 
 bool same_int(PyObject *o, uint64_t v)
@@ -272,7 +274,7 @@ TableState table_state(PyObject *ind_obj, const Tensor &Ind, const Problem &p, b
     s.key.ptr = (uint64_t)(uintptr_t)Ind.const_data_ptr();
     s.key.version = (uint64_t)Ind._version();
     s.key.dtype = (PyObject *)torch::getTHPDtype(Ind.scalar_type());
-    s.key.d = p.d; s.key.dt = p.dt;
+    s.key.d = p.d; s.key.dt = p.dt; s.key.ind = p.ind;
     s.applies = true;
     PyObject **dict = _PyObject_GetDictPtr(ind_obj);
     if (dict == nullptr || *dict == nullptr) return s;
@@ -295,8 +297,40 @@ void keep_table(PyObject *ind_obj, const TableKey &k, const Tensor &table)
     if (rc != 0) throw python_error();
 }
 
-// hip_kernels.py, which owns the switch of set_routing_table_cache (borrowed; null: gone, or not imported under its name)
-PyObject *g_owner_name = nullptr, *g_cache_name = nullptr;      // "expertscattergather_amd.hip_kernels", "_table_cache"
+// What a gather's backward needs to know to use the routing table of its forward: everything that the entry above is checked by
+// in any other call, and what the entry's owner may do to it meanwhile.  No interpreter lock is taken for it (looking the entry
+// up again in the backward was 4 us of an 87 us training step):
+//   - the indices: the memory, the version, the sizes and the type, against the ones the node now sees (saved-tensor hooks may hand back
+//     another tensor);
+//   - the stream and the capture that the backward runs in;
+//   - invalidate_routing_table(Ind), which counts up the version of the table tensor, and set_routing_table_cache(False).
+// What no longer holds is not used: the indices are sorted.
+std::atomic<bool> g_tables_allowed{true};       // set_routing_table_cache's word (a forward is told with the call)
+
+constexpr size_t kTableKey = 13;        // numbers of a table's key, at the end of the node's "numbers"
+void save_table(AutogradContext *ctx, std::vector<int64_t> &numbers, const TableKey &k, const Tensor &table)
+{
+    ctx->saved_data["table"] = table;
+    const int64_t key[kTableKey] = {(int64_t)k.ptr, (int64_t)k.version, (int64_t)k.stream, (int64_t)k.capture, k.d.B, k.d.T, k.d.E,
+                                    k.d.K, k.d.I, k.d.J, k.dt, k.ind, (int64_t)table._version()};
+    numbers.insert(numbers.end(), key, key + kTableKey);
+}
+
+Tensor table_of_backward(AutogradContext *ctx, const std::vector<int64_t> &numbers, const Tensor &Ind, const Problem &p)
+{
+    const auto it = ctx->saved_data.find("table");
+    if (it == ctx->saved_data.end() || !g_tables_allowed.load(std::memory_order_acquire) || Ind.is_inference()) return Tensor();
+    const Tensor table = it->second.toTensor();
+    const uint64_t stream = (uint64_t)(uintptr_t)stream_of(Ind);
+    unsigned long long capture = 0;
+    if (egs_stream_capture_id((void *)(uintptr_t)stream, &capture) != EGS_OK) return Tensor();
+    const int64_t now[kTableKey] = {(int64_t)(uintptr_t)Ind.const_data_ptr(), (int64_t)Ind._version(), (int64_t)stream, (int64_t)capture, p.d.B, p.d.T,
+                                    p.d.E, p.d.K, p.d.I, p.d.J, p.dt, p.ind, (int64_t)table._version()};
+    return numbers.size() >= kTableKey && std::equal(now, now + kTableKey, numbers.end() - kTableKey) ? table : Tensor();
+}
+
+// hip_kernels.py (borrowed; null: not imported under its name)
+PyObject *g_owner_name = nullptr;       // "expertscattergather_amd.hip_kernels"
 PyObject *owner()
 {
     PyObject *modules = PyImport_GetModuleDict();
@@ -308,24 +342,6 @@ struct Gil {                    // for the autograd engine's threads, which have
     Gil() : state(PyGILState_Ensure()) {}
     ~Gil() { PyGILState_Release(state); }
 };
-
-// The table that a backward may use: the one kept with Ind NOW, under the same conditions as in any other call.  (One remembered
-// from the forward would outlive a capture, invalidate_routing_table and set_routing_table_cache(False).)  `Ind` as the node
-// saved it is the caller's object; what saved-tensor hooks made of it has no table, and the indices are sorted.
-Tensor table_of_backward(const Tensor &Ind, const Problem &p)
-{
-    if (egs_routing_table_bytes(&p.d, p.dt) == 0) return Tensor();
-    Gil gil;
-    PyObject *module = owner(), *enabled = module == nullptr ? nullptr : PyObject_GetAttr(module, g_cache_name);
-    if (enabled == nullptr) PyErr_Clear();
-    const bool cache = enabled == Py_True;
-    Py_XDECREF(enabled);
-    PyObject *ind_obj = cache ? THPVariable_Wrap(Ind) : nullptr;
-    if (ind_obj == nullptr) { PyErr_Clear(); return Tensor(); }
-    const Tensor table = table_state(ind_obj, Ind, p, true).table;
-    Py_DECREF(ind_obj);
-    return table;
-}
 
 // A backward whose operands are not for this way - saved-tensor hooks may hand back another type, layout, alignment or kind of
 // tensor than was saved - by the function `name` of hip_kernels.py, with the saved tensors, the gradient, `option` and whether
@@ -356,32 +372,35 @@ Grads backward_in_python(const char *name, const variable_list &saved, const Ten
 }
 
 // ------------------------------------------------------------------------------ autograd
-// Same contract as the Python Functions of hip_kernels.py: what is saved is the inputs; the scatter mode is the forward's; both
-// gradients are always computed.
+// Same contract as the Python Functions of hip_kernels.py: what is saved is the inputs (and the routing table that was valid in the
+// forward, with what it was valid for); the scatter mode is the forward's; both gradients are always computed.
 struct ExpertGatherFunctionNative : public torch::autograd::Function<ExpertGatherFunctionNative> {
     static Tensor forward(AutogradContext *ctx, const Tensor &X, const Tensor &W, const Tensor &Ind, const std::optional<Tensor> &bias,
-                          const std::optional<Tensor> &build, int64_t mode)
+                          const TableState &ts, const std::optional<Tensor> &build, int64_t mode)
     {
         ctx->save_for_backward({X, W, Ind});
-        ctx->saved_data["mode"] = mode;
-        ctx->saved_data["bias"] = bias.has_value();
+        std::vector<int64_t> numbers = {mode, (int64_t)bias.has_value()};
+        const Tensor &table = build.has_value() ? *build : ts.table;
+        if (table.defined() && !table.is_inference()) save_table(ctx, numbers, ts.key, table);      // (one made there has no version)
+        ctx->saved_data["numbers"] = std::move(numbers);
         return gather_forward(problem_of(X, W, Ind, true, true, 0), X, W, Ind, build.value_or(Tensor()), EGS_ACT_NONE, bias.value_or(Tensor()));
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
         const auto saved = ctx->get_saved_variables();
         const Tensor &X = saved[0], &W = saved[1], &Ind = saved[2];
-        const int mode = (int)ctx->saved_data["mode"].toInt();
-        const bool bias = ctx->saved_data["bias"].toBool();
+        const std::vector<int64_t> numbers = ctx->saved_data.at("numbers").toIntVector();
+        const int mode = (int)numbers[0];
+        const bool bias = numbers[1] != 0;
         const Problem p = problem_of(X, W, Ind, true, true, 0);
         Grads g;
         if (p.ok && grad_fits(grads[0], X, {p.d.B, p.d.E, p.d.K, p.d.J})) {
             at::AutoDispatchBelowADInplaceOrView below;
-            g = gather_backward(p, X, W, Ind, table_of_backward(Ind, p), grads[0], mode, bias);
+            g = gather_backward(p, X, W, Ind, table_of_backward(ctx, numbers, Ind, p), grads[0], mode, bias);
         } else {
             g = backward_in_python("_gather_backward_of_node", saved, grads[0], mode, bias);
         }
-        return {g.in, g.W, Tensor(), g.bias, Tensor(), Tensor()};
+        return {g.in, g.W, Tensor(), g.bias, Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -479,7 +498,7 @@ PyObject *py_gather_forward(PyObject *, PyObject *const *a, Py_ssize_t n)
     {
         NoGil nogil;
         if (build) table = empty_gpu({(int64_t)ts.bytes}, at::kByte, p);
-        if (record && records(X, W, bias)) Y = ExpertGatherFunctionNative::apply(X, W, Ind, some(bias), some(table), mode);
+        if (record && records(X, W, bias)) Y = ExpertGatherFunctionNative::apply(X, W, Ind, some(bias), ts, some(table), mode);
         else Y = gather_forward(p, X, W, Ind, table, EGS_ACT_NONE, bias);
     }
     if (build) keep_table(a[2], ts.key, table);
@@ -637,6 +656,13 @@ PyObject *py_mlp_forward(PyObject *, PyObject *const *a, Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
+// set_table_cache(allowed): from now on, also for the backward of calls made before
+PyObject *py_set_table_cache(PyObject *, PyObject *on)
+{
+    g_tables_allowed.store(flag(on), std::memory_order_release);
+    Py_RETURN_NONE;
+}
+
 PyObject *py_abi_version(PyObject *, PyObject *) { return PyLong_FromLong(egs_abi_version()); }
 
 PyMethodDef methods[] = {
@@ -646,6 +672,7 @@ PyMethodDef methods[] = {
     {"scatter_backward", (PyCFunction)(void (*)(void))py_scatter_backward, METH_FASTCALL, "(grad_Y, grad_W), or None: not for this way"},
     {"router", (PyCFunction)(void (*)(void))py_router, METH_FASTCALL, "(Ind, scores), or None: not for this way"},
     {"mlp_forward", (PyCFunction)(void (*)(void))py_mlp_forward, METH_FASTCALL, "out, or None: not for this way"},
+    {"set_table_cache", py_set_table_cache, METH_O, "whether routing tables may be read from now on"},
     {"abi_version", py_abi_version, METH_NOARGS, "ABI version of the library this module is linked to"},
     {nullptr, nullptr, 0, nullptr}};
 
@@ -658,7 +685,6 @@ PyMODINIT_FUNC PyInit__egs_torch(void)
 {
     g_table_attr = PyUnicode_InternFromString("_egs_routing_table");
     g_owner_name = PyUnicode_InternFromString("expertscattergather_amd.hip_kernels");
-    g_cache_name = PyUnicode_InternFromString("_table_cache");
-    if (g_table_attr == nullptr || g_owner_name == nullptr || g_cache_name == nullptr) return nullptr;
+    if (g_table_attr == nullptr || g_owner_name == nullptr) return nullptr;
     return PyModule_Create(&module);
 }

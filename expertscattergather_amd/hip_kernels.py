@@ -289,11 +289,15 @@ def set_routing_table_cache(enabled: bool) -> None:
     EGS_ROUTING_TABLE_CACHE=0 turns it off); results are bit-identical either way."""
     global _table_cache
     _table_cache = bool(enabled)
+    if _abi._torch_ext:                 # loaded: there may be nodes of its own that hold a table
+        _abi._torch_ext.set_table_cache(_table_cache)
 
 
 def invalidate_routing_table(Ind: torch.Tensor) -> None:
     """Forget the routing table kept with `Ind` (after writing into it through a channel its version counter does not see)."""
-    Ind.__dict__.pop(_TABLE_ATTR, None)
+    entry = Ind.__dict__.pop(_TABLE_ATTR, None)
+    if entry is not None and not entry[1].is_inference():
+        torch.autograd.graph.increment_version(entry[1])       # a C++ autograd node that holds the table sees that it was taken back
 
 
 def _capture_id(stream: int) -> int:

@@ -121,6 +121,20 @@ def test_gather_backward_uses_no_table_that_was_taken_back(remedy):
         assert torch.equal(a, b)
 
 
+def test_a_table_made_in_inference_mode():
+    """It has no version to count up: no node holds it, taking it back works, and the gradients are the same."""
+    x, W, Ind, other, dY, want = _fresh_table_case()
+    with torch.inference_mode():
+        hk.expert_gather(x, W, other)
+    assert other.__dict__[hk._TABLE_ATTR][1].is_inference()
+    y = hk.expert_gather(x, W, other)
+    for a, b in zip(torch.autograd.grad(y, (x, W), dY, retain_graph=True), want):
+        assert torch.equal(a, b)
+    hk.invalidate_routing_table(other)
+    for a, b in zip(torch.autograd.grad(y, (x, W), dY), want):
+        assert torch.equal(a, b)
+
+
 def test_captured_gather_backward_does_not_use_an_eager_table():
     """Forward eager, backward alone captured, indices rewritten between replays: every replay sorts what they then hold."""
     x, W, Ind, other, dY, want = _fresh_table_case()
