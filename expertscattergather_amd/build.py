@@ -16,7 +16,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libegs_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
-SOURCES = ["egs_lib.hip", "egs_rows_launch.hip", "egs_dw_launch.hip", "egs_f8_launch.hip", "egs_mlp_launch.hip", "egs_pass_launch.hip", "egs_router.hip", "egs_bias.hip",
+SOURCES = ["egs_lib.hip", "egs_rows_launch.hip", "egs_dw_launch.hip", "egs_f8_launch.hip", "egs_mlp_launch.hip", "egs_pass_launch.hip", "egs_sum_launch.hip",
+           "egs_router.hip", "egs_bias.hip",
+           "egs_small_f16.hip", "egs_small_bf16.hip", "egs_fused_f32.hip", "egs_fused_f16.hip", "egs_fused_bf16.hip",
            "egs_tiled_f32.hip", "egs_tiled_f16.hip", "egs_tiled_bf16.hip", "egs_tiled_fp8.hip"]
 
 HIPCC_FLAGS = [
@@ -56,7 +58,7 @@ def build(verbose: bool = False, extra_flags=()) -> str:
     inc = ["-I", os.path.join(os.path.dirname(HERE), "include")]
     objs = [os.path.join(obj_dir, s.replace(".hip", ".o")) for s in SOURCES]
     cmds = [[hipcc(), *HIPCC_FLAGS, *extra_flags, *inc, "-c", os.path.join(CSRC, s), "-o", o] for s, o in zip(SOURCES, objs)]
-    with ThreadPoolExecutor(max_workers=len(cmds)) as pool:
+    with ThreadPoolExecutor(max_workers=min(len(cmds), max(2, (os.cpu_count() or 8)))) as pool:
         list(pool.map(lambda c: _run(c, verbose), cmds))
     _run([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", LIB_PATH], verbose)
     build_pycall(verbose)

@@ -116,6 +116,15 @@ int tiled_dw_f32(TiledDwParams &p, hipStream_t s);
 int tiled_dw_f16(TiledDwParams &p, hipStream_t s);
 int tiled_dw_bf16(TiledDwParams &p, hipStream_t s);
 
+// ---- egs_sum_launch.hip: sums over product rows, and the routing table as a launch of its own
+// second pass of a weight gradient's split form that may share the launch of the sums; `done`: it did
+struct DwSecondPass { const float *part; char *dW; int S, out_dtype; size_t w_elems; bool done; };
+int launch_routing_table(const void *Ind, int ind_dtype, const egs_dims *d, int32_t *seg_off, int32_t *perm, int32_t *rank_tmp, int32_t *cnt,
+                         int32_t *long_tab, hipStream_t s);
+int launch_segment_sum(const void *rows, bool rows_f32, const int32_t *seg_off, const int32_t *perm, int32_t *long_tab, float *long_part,
+                       void *Out, const egs_dims *d, int act_dtype, DwSecondPass *reduce, hipStream_t s);
+int launch_token_sum(const void *rows, bool rows_f32, const void *Ind, int ind_dtype, void *Out, const egs_dims *d, int act_dtype, hipStream_t s);
+
 // ---- egs_bias.hip: biases added in place, for launches that did not take them along
 int bias_rows(void *Y, const void *bias, const egs_dims *d, int act_dtype, hipStream_t s);
 int bias_scatter(void *Out, const void *bias, const void *Ind, const egs_dims *d, int act_dtype, int ind_dtype, hipStream_t s);

@@ -4,11 +4,8 @@
 #include "egs_host.h"
 #include "../../include/egs_hip_testing.h"
 #include "egs_device.h"
-#include "egs_scatter_aux.h"
-#include "egs_small.h"
-#include "egs_dw_tile.h"
+#include "egs_jobs.h"
 #include "egs_small_f32.h"
-#include "egs_scatter_fused.h"
 
 #include <atomic>
 #include <mutex>
@@ -222,29 +219,6 @@ bool small_shape_ok(int act_dtype, int R, int N)
 {
     return act_dtype != EGS_F32 && (R == 32 || R == 64 || R == 128) && N % 8 == 0 && N >= 8 && N <= 128;
 }
-
-// one launch of rows_small_kernel, or its share of a heterogeneous launch
-struct SmallRowsJob {
-    SmallRowsParams p;
-    int R, act_dtype, blocks;
-    bool nmajor, gather, out_f32;
-    size_t lds;
-};
-// one launch of dw_small_kernel (or its share of a heterogeneous launch) plus the second pass
-struct SmallDwJob {
-    SmallDwParams q;
-    int blocks, act_dtype;
-    size_t w_elems;
-    bool done;          // set once the first pass has been enqueued
-};
-
-// one launch of dw_tile_kernel (or its share of a heterogeneous launch): the whole weight gradient, no second pass
-struct DwTileJob {
-    DwTileParams q;
-    int blocks, act_dtype;
-    bool wide;          // 32 x 64 tiles and 8 wavefronts (dw_tile_wide_kernel) instead of 32 x 32 and 4
-    bool done;          // set once it has been enqueued
-};
 
 // A routing table in caller-owned memory (egs_routing_table_bytes): seg [B][T+1], perm [B][E*K], the picks of each batch
 // element in a stable order by token.  Built once per Ind by a gather forward, read by the one-kernel scatters that follow.
@@ -515,74 +489,10 @@ int gather_small_f32(const void *X, const void *W, const void *Ind, void *Y, con
     }
 }
 
-// ---- launch of a rows job, alone or sharing the launch with a weight gradient of the same call (its one-pass form,
-// or the first pass of its split form)
-template <class TT, bool W_NMAJOR, int KS, int TN, bool GATHER, bool OUT_F32>
-int launch_rows_small_one(SmallRowsJob &j, SmallDwJob *dw, DwTileJob *dwt, hipStream_t s)
-{
-    if constexpr (GATHER) {
-        if (j.p.act != ACT_NONE) {
-            if (dw != nullptr || dwt != nullptr) return EGS_ERR_UNSUPPORTED;        // (backward products have no activation)
-            hipLaunchKernelGGL((rows_small_kernel<TT, W_NMAJOR, KS, TN, GATHER, OUT_F32, true>), dim3(j.blocks), dim3(kThreads), j.lds, s, j.p);
-            EGS_CHECK_LAUNCH("rows_small_kernel");
-            return EGS_OK;
-        }
-        if (dwt != nullptr) {       // dwt->wide, and j regridded for 8 wavefronts per workgroup (see pair_gather_with_dw_tile)
-            static LdsGrant told;
-            const size_t tile_lds = dw_tile_lds(kDwWideThreads / 64, 64);
-            const int rc = allow_large_lds((const void *)rows_dw_tile_kernel<TT, W_NMAJOR, KS, TN>, told, tile_lds,
-                                           "hipFuncSetAttribute(rows_dw_tile_kernel)");
-            if (rc != EGS_OK) return rc;
-            hipLaunchKernelGGL((rows_dw_tile_kernel<TT, W_NMAJOR, KS, TN>), dim3(j.blocks + dwt->blocks), dim3(kDwWideThreads),
-                               tile_lds, s, j.p, dwt->q, j.blocks);
-            EGS_CHECK_LAUNCH("rows_dw_tile_kernel");
-            dwt->done = true;
-            return EGS_OK;
-        }
-    }
-    if (dw != nullptr) {
-        hipLaunchKernelGGL((rows_dw_small_kernel<TT, W_NMAJOR, KS, TN, GATHER, OUT_F32>), dim3(j.blocks + dw->blocks),
-                           dim3(kThreads), j.lds, s, j.p, dw->q, j.blocks);
-        dw->done = true;
-    } else {
-        hipLaunchKernelGGL((rows_small_kernel<TT, W_NMAJOR, KS, TN, GATHER, OUT_F32>), dim3(j.blocks), dim3(kThreads),
-                           j.lds, s, j.p);
-    }
-    EGS_CHECK_LAUNCH(dw != nullptr ? "rows_dw_small_kernel" : "rows_small_kernel");
-    return EGS_OK;
-}
-
-template <class TT, bool W_NMAJOR, int TN, bool GATHER, bool OUT_F32>
-int launch_rows_small_ks(SmallRowsJob &j, SmallDwJob *dw, DwTileJob *dwt, hipStream_t s)
-{
-    switch (j.R) {
-    case 32: return launch_rows_small_one<TT, W_NMAJOR, 1, TN, GATHER, OUT_F32>(j, dw, dwt, s);
-    case 64: return launch_rows_small_one<TT, W_NMAJOR, 2, TN, GATHER, OUT_F32>(j, dw, dwt, s);
-    default: return launch_rows_small_one<TT, W_NMAJOR, 4, TN, GATHER, OUT_F32>(j, dw, dwt, s);
-    }
-}
-
-template <class TT, bool GATHER, bool OUT_F32>
-int launch_rows_small_tn(SmallRowsJob &j, SmallDwJob *dw, DwTileJob *dwt, hipStream_t s)
-{
-    if (j.p.N <= 64)
-        return j.nmajor ? launch_rows_small_ks<TT, true, 4, GATHER, OUT_F32>(j, dw, dwt, s)
-                        : launch_rows_small_ks<TT, false, 4, GATHER, OUT_F32>(j, dw, dwt, s);
-    return j.nmajor ? launch_rows_small_ks<TT, true, 8, GATHER, OUT_F32>(j, dw, dwt, s)
-                    : launch_rows_small_ks<TT, false, 8, GATHER, OUT_F32>(j, dw, dwt, s);
-}
-
-template <class TT>
-int launch_rows_small_tt(SmallRowsJob &j, SmallDwJob *dw, DwTileJob *dwt, hipStream_t s)
-{
-    if (j.gather) return launch_rows_small_tn<TT, true, false>(j, dw, dwt, s);
-    return j.out_f32 ? launch_rows_small_tn<TT, false, true>(j, dw, dwt, s) : launch_rows_small_tn<TT, false, false>(j, dw, dwt, s);
-}
-
 // `dwt` (one-pass weight gradient) shares the launch of a gather only; `dw` (first pass of the split form) any rows job
 int launch_rows_small_job(SmallRowsJob &j, SmallDwJob *dw, DwTileJob *dwt, hipStream_t s)
 {
-    return j.act_dtype == EGS_BF16 ? launch_rows_small_tt<ElemBF16>(j, dw, dwt, s) : launch_rows_small_tt<ElemF16>(j, dw, dwt, s);
+    return j.act_dtype == EGS_BF16 ? launch_rows_small_bf16(j, dw, dwt, s) : launch_rows_small_f16(j, dw, dwt, s);
 }
 
 int launch_dw_small_alone(SmallDwJob &j, hipStream_t s)
@@ -603,222 +513,19 @@ int launch_dw_reduce4(const SmallDwJob &j, hipStream_t s)
     return EGS_OK;
 }
 
-// routing table of the deterministic scatter as a launch of its own: counting sort with
-// per-wavefront histograms when they fit in LDS, bitonic sort in LDS for long sequences, else
-// the one-wavefront counting sort
-int launch_routing_table(const void *Ind, int ind_dtype, const egs_dims *d, int32_t *seg_off, int32_t *perm,
-                         int32_t *rank_tmp, int32_t *cnt, int32_t *long_tab, hipStream_t s)
+// sums over product rows; the second pass of the weight gradient `dw`, where it waits for one, shares the launch if it can
+int segment_sum_with(const void *rows, bool rows_f32, const int32_t *seg_off, const int32_t *perm, int32_t *long_tab, float *long_part,
+                     void *Out, const egs_dims *d, int act_dtype, SmallDwJob *dw, hipStream_t s)
 {
-    const int64_t N = (int64_t)d->E * d->K;
-    if (N >= 1) {
-        // as many wavefronts as the per-wavefront histograms leave room for (up to 148 KB of LDS)
-        const size_t budget = 148 * 1024;
-        int nw = (int)((N + 63) / 64);
-        if (nw > 16) nw = 16;
-        while (nw > 1 && csr_count_lds(d->T, nw) > budget) nw >>= 1;
-        const size_t lds = csr_count_lds(d->T, nw);
-        if (lds <= budget) {
-            static LdsGrant told;
-            const int rc_lds = allow_large_lds((const void *)csr_count_kernel, told, lds, "hipFuncSetAttribute(csr_count_kernel)");
-            if (rc_lds != EGS_OK) return rc_lds;
-            hipLaunchKernelGGL(csr_count_kernel, dim3(d->B), dim3(64 * nw), lds, s, Ind, ind_dtype, d->T, (int32_t)N, seg_off, perm, rank_tmp, long_tab);
-            EGS_CHECK_LAUNCH("csr_count_kernel");
-            return EGS_OK;
-        }
-    }
-    int NP = 1, QB = 0;
-    while (NP < N) { NP <<= 1; ++QB; }
-    const bool sortable = N >= 1 && NP <= 32768 && (((uint64_t)d->T << QB) <= 0xFFFFFFFFull);
-    if (sortable) {
-        const size_t lds = (size_t)NP * 4;
-        static LdsGrant told;
-        const int rc_lds = allow_large_lds((const void *)csr_sort_kernel, told, lds, "hipFuncSetAttribute(csr_sort_kernel)");
-        if (rc_lds != EGS_OK) return rc_lds;
-        int threads = NP / 2;
-        if (threads < 64) threads = 64;
-        if (threads > 1024) threads = 1024;
-        hipLaunchKernelGGL(csr_sort_kernel, dim3(d->B), dim3(threads), lds, s, Ind, ind_dtype, d->T, (int32_t)N, NP, QB, seg_off, perm, long_tab);
-        EGS_CHECK_LAUNCH("csr_sort_kernel");
-        return EGS_OK;
-    }
-    const size_t lds = d->T > kCsrLdsTokens ? 0 : (size_t)d->T * 4;
-    hipLaunchKernelGGL(csr_build_kernel, dim3(d->B), dim3(kWave), lds, s, Ind, ind_dtype, d->T, (int32_t)N, seg_off, perm, cnt, long_tab);
-    EGS_CHECK_LAUNCH("csr_build_kernel");
-    return EGS_OK;
-}
-
-template <class TT, class PT>
-void launch_segment_sum8(const SegSumParams &sp, int seg_blocks, hipStream_t s)
-{
-    hipLaunchKernelGGL((segment_sum_kernel<TT, PT, 8>), dim3(seg_blocks), dim3(kThreads), 0, s, sp);
-}
-
-// fixed-order reduction of the product rows per token; when `reduce` is given (and qualifies) the
-// second pass of that weight gradient shares the launch
-int launch_segment_sum(const void *rows, bool rows_f32, const int32_t *seg_off, const int32_t *perm, int32_t *long_tab,
-                       float *long_part, void *Out, const egs_dims *d, int act_dtype, SmallDwJob *reduce, hipStream_t s)
-{
-    const int N = d->E * d->K;
-    const bool vw4 = d->I % 4 == 0 && aligned_to(Out, 16);
-    // eight elements of a row per thread (16 bytes of a 16-bit row, two 16-byte loads of an fp32 row): half the threads,
-    // table look-ups and address arithmetic per row
-    const bool vw8 = vw4 && d->I % 8 == 0 && aligned_to(rows, 16) &&
-                     !(reduce != nullptr && reduce->done && reduce->q.S > 1);
-    const int iv = vw8 ? d->I / 8 : vw4 ? d->I / 4 : d->I;
-    SegSumParams sp;
-    memset(&sp, 0, sizeof(sp));
-    sp.P = rows; sp.seg_off = seg_off; sp.perm = perm; sp.out = (char *)Out;
-    sp.B = d->B; sp.T = d->T; sp.N = N; sp.I = d->I; sp.ldp = product_ld(d->I);
-    while ((1 << sp.tpr_log2) < iv && sp.tpr_log2 < 8) ++sp.tpr_log2;      // threads sharing an output row (<= 256)
-    sp.gx = ceil_div(d->T, kThreads >> sp.tpr_log2);
-    sp.gy = d->B;
-    while ((int64_t)sp.gx * sp.gy > (1 << 22)) sp.gy = (sp.gy + 1) / 2;     // stride loop over batch elements beyond that
-    sp.long_tab = long_tab; sp.long_part = long_part;
-    const int64_t all_seg_blocks = (int64_t)sp.gx * sp.gy + (int64_t)d->B * long_max_slots(N);
-    if (all_seg_blocks > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
-    const int seg_blocks = (int)all_seg_blocks;
-    const bool fuse = reduce != nullptr && reduce->done && reduce->q.S > 1 && vw4;
-    const int red_blocks = fuse ? grid_1d(reduce->w_elems / 4, 1024) : 0;
-#define EGS_SEGSUM(TT, PT)                                                                                                  \
-    do {                                                                                                                    \
-        if (fuse) hipLaunchKernelGGL((segsum_dwreduce_kernel<TT, PT, 4>), dim3(seg_blocks + red_blocks), dim3(kThreads), 0, \
-                                     s, sp, seg_blocks, (const float *)reduce->q.part, reduce->q.dW, reduce->q.S,           \
-                                     reduce->w_elems / 4, reduce->q.out_dtype);                                             \
-        else if (vw8) launch_segment_sum8<TT, PT>(sp, seg_blocks, s);                                                       \
-        else if (vw4) hipLaunchKernelGGL((segment_sum_kernel<TT, PT, 4>), dim3(seg_blocks), dim3(kThreads), 0, s, sp);      \
-        else hipLaunchKernelGGL((segment_sum_kernel<TT, PT, 1>), dim3(seg_blocks), dim3(kThreads), 0, s, sp);               \
-    } while (0)
-    if (act_dtype == EGS_F32) EGS_SEGSUM(ElemF32, float);
-    else if (act_dtype == EGS_F16) { if (rows_f32) EGS_SEGSUM(ElemF16, float); else EGS_SEGSUM(ElemF16, uint16_t); }
-    else { if (rows_f32) EGS_SEGSUM(ElemBF16, float); else EGS_SEGSUM(ElemBF16, uint16_t); }
-#undef EGS_SEGSUM
-    EGS_CHECK_LAUNCH(fuse ? "segsum_dwreduce_kernel" : "segment_sum_kernel");
-    if (fuse) reduce->q.S = 1;              // second pass done
-    return EGS_OK;
-}
-
-// the same without a routing table, for up to kTokenSumPicks picks per batch element
-int launch_token_sum(const void *rows, bool rows_f32, const void *Ind, int ind_dtype, void *Out, const egs_dims *d, int act_dtype, hipStream_t s)
-{
-    TokenSumParams p;
-    memset(&p, 0, sizeof(p));
-    p.P = rows; p.Ind = Ind; p.out = (char *)Out;
-    p.B = d->B; p.T = d->T; p.N = d->E * d->K; p.I = d->I; p.ldp = product_ld(d->I);
-    p.ind_dtype = ind_dtype;
-    // at most 64 threads (256 columns) per row, so that a hot token's segment has at least four groups of threads to share it
-    p.tpr_log2 = 3;
-    while ((4 << p.tpr_log2) < d->I && p.tpr_log2 < 6) ++p.tpr_log2;
-    p.c_blocks = ceil_div(d->I, 4 << p.tpr_log2);
-    // tokens per workgroup: one per group of threads, more (each workgroup reads all indices of its batch element) once that
-    // alone makes a thousand workgroups
-    const int groups = kThreads >> p.tpr_log2;
-    p.tb = groups;
-    while (p.tb < kTokenSumTokens && (int64_t)d->B * ceil_div(d->T, p.tb) * p.c_blocks > 1024) p.tb *= 2;
-    p.t_blocks = ceil_div(d->T, p.tb);
-    const int64_t grid = (int64_t)d->B * p.t_blocks * p.c_blocks;
-    if (grid > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
-    const size_t lds = token_sum_lds(p.N);
-    if (act_dtype == EGS_F32) hipLaunchKernelGGL((token_sum_kernel<ElemF32, float>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
-    else if (act_dtype == EGS_F16 && rows_f32) hipLaunchKernelGGL((token_sum_kernel<ElemF16, float>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
-    else if (act_dtype == EGS_F16) hipLaunchKernelGGL((token_sum_kernel<ElemF16, uint16_t>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
-    else if (rows_f32) hipLaunchKernelGGL((token_sum_kernel<ElemBF16, float>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
-    else hipLaunchKernelGGL((token_sum_kernel<ElemBF16, uint16_t>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
-    EGS_CHECK_LAUNCH("token_sum_kernel");
-    return EGS_OK;
+    const bool waits = dw != nullptr && dw->done && dw->q.S > 1;
+    DwSecondPass second = {};
+    if (waits) second = {(const float *)dw->q.part, dw->q.dW, dw->q.S, dw->q.out_dtype, dw->w_elems, false};
+    const int rc = launch_segment_sum(rows, rows_f32, seg_off, perm, long_tab, long_part, Out, d, act_dtype, waits ? &second : nullptr, s);
+    if (second.done) dw->q.S = 1;
+    return rc;
 }
 
 // ------------------------------------------------------------------------------ fused small-expert scatter
-template <class TT, bool W_NMAJOR, int KS>
-int launch_scatter_fused_one(const ScatterFusedParams &p, size_t lds, int blocks, SmallDwJob *dw, DwTileJob *dwt, hipStream_t s)
-{
-    static LdsGrant told_plain, told_dw, told_dwt, told_multi;      // one set per template instantiation
-    if constexpr (TT::ES != 2) { dw = nullptr; dwt = nullptr; }     // the small weight gradients exist for 16-bit types only
-    const char *name = "scatter_fused_kernel";
-    if (p.experts_per_pass < p.E && p.tab_seg != nullptr) {
-        name = "scatter_fused_multi_table_kernel";
-        static LdsGrant told_multi_tab;
-        const int rc_lds = allow_large_lds((const void *)scatter_fused_multi_table_kernel<TT, W_NMAJOR, KS>, told_multi_tab, lds,
-                                           "hipFuncSetAttribute(scatter_fused_multi_table_kernel)");
-        if (rc_lds != EGS_OK) return rc_lds;
-        hipLaunchKernelGGL((scatter_fused_multi_table_kernel<TT, W_NMAJOR, KS>), dim3(blocks), dim3(kFusedThreads), lds, s, p);
-    } else if (p.experts_per_pass < p.E) {
-        // several passes over groups of experts: a launch of its own (a weight gradient of the same call follows alone)
-        name = "scatter_fused_multi_kernel";
-        const int rc_lds = allow_large_lds((const void *)scatter_fused_multi_kernel<TT, W_NMAJOR, KS>, told_multi, lds,
-                                           "hipFuncSetAttribute(scatter_fused_multi_kernel)");
-        if (rc_lds != EGS_OK) return rc_lds;
-        hipLaunchKernelGGL((scatter_fused_multi_kernel<TT, W_NMAJOR, KS>), dim3(blocks), dim3(kFusedThreads), lds, s, p);
-    } else if (p.run > 1) {             // (a weight gradient of the same call follows alone)
-        name = "scatter_fused_runs_kernel";
-        static LdsGrant told_runs;
-        const int rc_lds = allow_large_lds((const void *)scatter_fused_runs_kernel<TT, W_NMAJOR, KS>, told_runs, lds,
-                                           "hipFuncSetAttribute(scatter_fused_runs_kernel)");
-        if (rc_lds != EGS_OK) return rc_lds;
-        hipLaunchKernelGGL((scatter_fused_runs_kernel<TT, W_NMAJOR, KS>), dim3(blocks), dim3(kFusedThreads), lds, s, p);
-    } else if (p.tab_seg != nullptr && dwt != nullptr && !dwt->wide && TT::ES == 2) {
-      if constexpr (TT::ES == 2) {
-        name = "scatter_fused_dwtile_table_kernel";
-        static LdsGrant told_dwt_tab;
-        const size_t tile_lds = dw_tile_lds(kFusedThreads / 64);
-        const size_t need = lds > tile_lds ? lds : tile_lds;
-        const int rc_lds = allow_large_lds((const void *)scatter_fused_dwtile_table_kernel<TT, W_NMAJOR, KS>, told_dwt_tab, need,
-                                           "hipFuncSetAttribute(scatter_fused_dwtile_table_kernel)");
-        if (rc_lds != EGS_OK) return rc_lds;
-        hipLaunchKernelGGL((scatter_fused_dwtile_table_kernel<TT, W_NMAJOR, KS>), dim3(blocks + dwt->blocks), dim3(kFusedThreads), need,
-                           s, p, dwt->q, blocks);
-        dwt->done = true;
-      }
-    } else if (p.tab_seg != nullptr && dw == nullptr && (dwt == nullptr || dwt->wide || TT::ES != 2)) {
-        name = "scatter_fused_table_kernel";
-        static LdsGrant told_tab;
-        const int rc_lds = allow_large_lds((const void *)scatter_fused_table_kernel<TT, W_NMAJOR, KS>, told_tab, lds,
-                                           "hipFuncSetAttribute(scatter_fused_table_kernel)");
-        if (rc_lds != EGS_OK) return rc_lds;
-        hipLaunchKernelGGL((scatter_fused_table_kernel<TT, W_NMAJOR, KS>), dim3(blocks), dim3(kFusedThreads), lds, s, p);
-    } else if (dwt != nullptr && !dwt->wide) {
-      if constexpr (TT::ES == 2) {
-        name = "scatter_fused_dwtile_kernel";
-        const size_t tile_lds = dw_tile_lds(kFusedThreads / 64);
-        const size_t need = lds > tile_lds ? lds : tile_lds;
-        const int rc_lds = allow_large_lds((const void *)scatter_fused_dwtile_kernel<TT, W_NMAJOR, KS>, told_dwt, need,
-                                           "hipFuncSetAttribute(scatter_fused_dwtile_kernel)");
-        if (rc_lds != EGS_OK) return rc_lds;
-        hipLaunchKernelGGL((scatter_fused_dwtile_kernel<TT, W_NMAJOR, KS>), dim3(blocks + dwt->blocks), dim3(kFusedThreads), need,
-                           s, p, dwt->q, blocks);
-        dwt->done = true;
-      }
-    } else if (dw != nullptr) {
-      if constexpr (TT::ES == 2) {
-        name = "scatter_fused_dw_kernel";
-        const size_t dw_lds = (size_t)kDwSmallLdsBytes * (kFusedThreads / kThreads);       // one 16 KB tile per wavefront
-        const size_t need = lds > dw_lds ? lds : dw_lds;
-        const int rc_lds = allow_large_lds((const void *)scatter_fused_dw_kernel<TT, W_NMAJOR, KS>, told_dw, need,
-                                           "hipFuncSetAttribute(scatter_fused_dw_kernel)");
-        if (rc_lds != EGS_OK) return rc_lds;
-        hipLaunchKernelGGL((scatter_fused_dw_kernel<TT, W_NMAJOR, KS>), dim3(blocks + dw->blocks), dim3(kFusedThreads), need, s, p,
-                           dw->q, blocks);
-        dw->done = true;
-      }
-    } else {
-        const int rc_lds = allow_large_lds((const void *)scatter_fused_kernel<TT, W_NMAJOR, KS>, told_plain, lds,
-                                           "hipFuncSetAttribute(scatter_fused_kernel)");
-        if (rc_lds != EGS_OK) return rc_lds;
-        hipLaunchKernelGGL((scatter_fused_kernel<TT, W_NMAJOR, KS>), dim3(blocks), dim3(kFusedThreads), lds, s, p);
-    }
-    EGS_CHECK_LAUNCH(name);
-    return EGS_OK;
-}
-
-template <class TT, bool W_NMAJOR>
-int launch_scatter_fused_ks(const ScatterFusedParams &p, int R, size_t lds, int blocks, SmallDwJob *dw, DwTileJob *dwt, hipStream_t s)
-{
-    switch (R / (4 * TT::VEC)) {        // MFMA steps of four 16-byte chunks
-    case 1: return launch_scatter_fused_one<TT, W_NMAJOR, 1>(p, lds, blocks, dw, dwt, s);
-    case 2: return launch_scatter_fused_one<TT, W_NMAJOR, 2>(p, lds, blocks, dw, dwt, s);
-    default: return launch_scatter_fused_one<TT, W_NMAJOR, 4>(p, lds, blocks, dw, dwt, s);
-    }
-}
-
 // Does the one-kernel scatter of small experts (product rows stay in LDS, no workspace) take this problem, and in how
 // many passes over groups of experts?  experts_per_pass == E: one pass.
 struct FusedPlan { bool ok; int experts_per_pass; size_t lds; };
@@ -918,14 +625,8 @@ int scatter_fused(const void *Y, const void *W, const void *Ind, void *Out, cons
     // batch elements of one of its row tiles - 256 / K of them - were written on one XCD
     p.xcd_batch = (d->K == 32 || d->K == 64 || d->K == 128 || d->K == 256) ? 256 / d->K : 2;
     const bool nmajor = (w_layout == EGS_W_EJI);        // [E,J,I] = [E,R,N]
-    if (act_dtype == EGS_F32)
-        return nmajor ? launch_scatter_fused_ks<ElemF32, true>(p, R, lds, (int)blocks, nullptr, nullptr, s)
-                      : launch_scatter_fused_ks<ElemF32, false>(p, R, lds, (int)blocks, nullptr, nullptr, s);
-    if (act_dtype == EGS_F16)
-        return nmajor ? launch_scatter_fused_ks<ElemF16, true>(p, R, lds, (int)blocks, dw, dwt, s)
-                      : launch_scatter_fused_ks<ElemF16, false>(p, R, lds, (int)blocks, dw, dwt, s);
-    return nmajor ? launch_scatter_fused_ks<ElemBF16, true>(p, R, lds, (int)blocks, dw, dwt, s)
-                  : launch_scatter_fused_ks<ElemBF16, false>(p, R, lds, (int)blocks, dw, dwt, s);
+    return act_dtype == EGS_F32 ? launch_fused_f32(p, nmajor, R, lds, (int)blocks, nullptr, nullptr, s)
+         : act_dtype == EGS_F16 ? launch_fused_f16(p, nmajor, R, lds, (int)blocks, dw, dwt, s) : launch_fused_bf16(p, nmajor, R, lds, (int)blocks, dw, dwt, s);
 }
 
 // Which weight-gradient kernel takes these operands, and the workspace it needs.  egs_workspace_bytes asks with
@@ -1184,10 +885,9 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
                 if (rc == EGS_OK && b0 == 0 && !p.csr_done)
                     rc = launch_routing_table(Ind, ind_dtype, d, seg_off, perm, rank_tmp, cnt, long_tab, s);
                 if (rc == EGS_OK)
-                    rc = launch_segment_sum(rows, rows_f32, seg_off + (size_t)b0 * (d->T + 1), perm + (size_t)b0 * N,
-                                            long_tab + (size_t)b0 * long_tab_stride(N), long_part + (size_t)b0 * long_max_slots(N) * d->I,
-                                            (char *)Out + (size_t)b0 * d->T * d->I * ES, &sub, act_dtype,
-                                            b0 + G >= d->B ? dw : nullptr, s);
+                    rc = segment_sum_with(rows, rows_f32, seg_off + (size_t)b0 * (d->T + 1), perm + (size_t)b0 * N,
+                                          long_tab + (size_t)b0 * long_tab_stride(N), long_part + (size_t)b0 * long_max_slots(N) * d->I,
+                                          (char *)Out + (size_t)b0 * d->T * d->I * ES, &sub, act_dtype, b0 + G >= d->B ? dw : nullptr, s);
             }
             if (rc != EGS_OK) return rc;
         }
@@ -1195,7 +895,7 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
         return add_bias_up_to(d->B);
     }
     if (rc != EGS_OK) return rc;
-    return launch_segment_sum(rows, rows_f32, seg_off, perm, long_tab, long_part, Out, d, act_dtype, dw, s);
+    return segment_sum_with(rows, rows_f32, seg_off, perm, long_tab, long_part, Out, d, act_dtype, dw, s);
 }
 
 int dw_impl(const void *Xs, const void *Ys, const void *Ind, void *dW, void *workspace, const egs_dims *d,
