@@ -55,7 +55,7 @@ int dw_general(const void *Xs, const void *Ys, const void *Ind, void *dW, void *
     q.B = d->B; q.T = d->T; q.E = d->E; q.K = d->K; q.I = d->I; q.J = d->J;
     q.ind_dtype = ind_dtype; q.out_dtype = out_dtype; q.eji = dw_layout != 0;
     q.i_tiles = pl.i_tiles; q.j_tiles = pl.j_tiles; q.S = pl.S; q.picks_per_split = pl.picks_per_split;
-    q.wide = pl.wide;
+    q.wide = pl.wide; q.split32 = pl.split32;
     q.edges = (d->I * ES) % 16 != 0 || (d->J * ES) % 16 != 0;
     const int rc = act_dtype == EGS_F32 ? tiled_dw_f32(q, s) : act_dtype == EGS_F16 ? tiled_dw_f16(q, s) : tiled_dw_bf16(q, s);
     if (rc != EGS_OK || pl.S <= 1) return rc;

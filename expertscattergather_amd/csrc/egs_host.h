@@ -84,6 +84,7 @@ struct DwPlan {
     bool big_ok;                                            // shape admits the direct-to-LDS kernel (256 x BQ tiles)
     int b_bq, b_i_tiles, b_j_tiles, b_S, b_rows_per_split;  // its plan
     bool wide;                                              // tiled_dw_wide_kernel, in one pass
+    bool split32;                                           // fp32: tiled_dw_split_kernel, 64 x 64 tiles
     size_t bytes_general, bytes_small, bytes_big;           // workspace of each of the three split kernels (0: no splits)
 };
 

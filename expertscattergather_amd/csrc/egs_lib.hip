@@ -152,6 +152,16 @@ int64_t dw_wide_tiles(const egs_dims *d, int act_dtype)
 }
 bool dw_few_picks(const egs_dims *d, int act_dtype) { return (int64_t)d->B * d->K <= 256 && dw_wide_tiles(d, act_dtype) >= 256; }
 
+// fp32: 32-pick slabs that the 64 x 64 tiles of tiled_dw_split_kernel go through in all.  It is the faster one above some hundred: us, it and
+// the fp32 instruction, by slabs: 42 (B6 T3171 E5 K31 I28 J249) 8.6 / 7.8, 294 (E42 of 196 picks, I32 J116) 9.2 / 7.7, 288 (E9 of 98, I96 J224) 7.4 / 8.2,
+// 660 (B1 T712 E125 K155 I369 J128) 28.4 / 34.5, 2352 (B9 T484 E98 K28 I160 J32) 14.5 / 17.5, 55000 135 / 202.  Few tiles of many picks gain at any
+// number (8 tiles, 774 picks 11.3 / 15.1).  Against the aligned tiles of dw_tile_body, which are narrower: 4096 (B64 T256 E32 K32 I128 J64) 21 / 20,
+// 9450 (B16 T61 E14 K45 I960 J96) 30 / 50, 16384 43 / 66 and 46 / 60; with 32 columns of a tile empty (I32 J96, 7676) 41 / 30.
+int64_t dw_split32_slabs(const egs_dims *d)
+{
+    return (int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, 64) * (((int64_t)d->B * d->K + 31) / 32);
+}
+
 DwPlan plan_dw(const egs_dims *d, int act_dtype)
 {
     DwPlan pl;
@@ -164,8 +174,16 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
     const int64_t base = (int64_t)d->E * pl.i_tiles * pl.j_tiles;
     int64_t S = base > 0 ? 512 / base : 1;
     if (S > (Me + 1023) / 1024) S = (Me + 1023) / 1024;
+    pl.split32 = act_dtype == EGS_F32 && (Me >= 512 || dw_split32_slabs(d) >= 600);
+    if (pl.split32) {
+        // two workgroups per CU where that leaves four slabs or more to each
+        const int64_t tiles = (int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, 64);
+        S = tiles > 0 ? 512 / tiles : 1;
+        if (S > Me / 128) S = Me / 128;
+    }
     if (S < 1) S = 1;
-    int64_t rows = Me > 0 ? ((Me + S - 1) / S + 127) / 128 * 128 : 128;
+    const int64_t grain = pl.split32 ? 32 : 128;
+    int64_t rows = Me > 0 ? ((Me + S - 1) / S + grain - 1) / grain * grain : 128;
     S = Me > 0 ? (Me + rows - 1) / rows : 1;
     pl.S = (int)S;
     pl.picks_per_split = (int)(rows < INT32_MAX ? rows : INT32_MAX);
@@ -349,6 +367,7 @@ bool make_dw_tile(const void *Xs, const void *Ys, const void *Ind, void *dW, con
 {
     if (g_force_generic) return false;
     const int ES = elem_size(act_dtype);
+    if (ES == 4 && d->I > 32 && d->J > 32 && dw_split32_slabs(d) >= 8192) return false;
     if (d->I % 8 || d->J % 8 || d->I < 8 || d->J < 8 || d->I > 2048 || d->J > 128) return false;
     const int64_t Me = (int64_t)d->B * d->K;
     if (Me == 0 || d->E == 0 || d->T == 0) return false;

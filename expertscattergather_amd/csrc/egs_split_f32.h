@@ -1,0 +1,280 @@
+// fp32 products on the bf16 matrix instruction.
+//
+// An fp32 value is the sum of three bf16 values exactly: h = bf16(x), m = bf16(x - h), l = x - h - m (8 bits of the 24 each; the
+// subtractions are exact).  Of the nine products of two such sums six are taken, the smallest first,
+//   x y = lh + hl + mm + mh + hm + hh   (the others are below 2^-25 of it),
+// each exact in the fp32 accumulator's input, so that what is rounded is the accumulator, as with the fp32 matrix instruction -
+// fewer times: 16x16x32 adds 32 products at a time where 16x16x4 adds four.  Measured against 64 bits, 64 problems of N(0,1) data:
+// reduction 32 3.8e-8 (the fp32 instruction 1.0e-7), 64 0.94e-7 (1.44e-7), 128 1.5e-7 (2.0e-7), 1024 4.9e-7 (5.7e-7), 4096 1.00e-6
+// (1.14e-6) of the result's root mean square.  Six instructions of 16 cycles stand for eight of 32, and at a higher clock:
+// 358 TFLOP/s of fp32 work against 138 (an instruction-only loop over all CUs).
+//
+// Limits: the pieces of a value below 2^-109 fall below bf16's smallest number, which leaves them with an absolute error of up to 2^-134.
+// An infinity has no such pieces (inf - inf), nor has a value that rounds up to one in bf16 (above 3.39e38): such products
+// arrive as NaN or infinity, so a wavefront whose results are not all finite takes its tile again with the fp32 instruction.
+#pragma once
+#include "egs_tiled.h"
+
+namespace egs {
+
+// the three pieces of two floats, packed in pairs
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t (&piece)[3])
+{
+    piece[0] = pack2<ElemBF16>(x, y);
+    const float rx = x - bits_f32(piece[0] << 16), ry = y - bits_f32(piece[0] & 0xffff0000u);
+    piece[1] = pack2<ElemBF16>(rx, ry);
+    piece[2] = pack2<ElemBF16>(rx - bits_f32(piece[1] << 16), ry - bits_f32(piece[1] & 0xffff0000u));
+}
+// ... and of four
+__device__ __forceinline__ void split_chunk(const u32x4 &v, u32x2 (&piece)[3])
+{
+    uint32_t lo[3], hi[3];
+    split_pair(bits_f32(v[0]), bits_f32(v[1]), lo);
+    split_pair(bits_f32(v[2]), bits_f32(v[3]), hi);
+#pragma unroll
+    for (int x = 0; x < 3; ++x) piece[x] = u32x2{lo[x], hi[x]};
+}
+// 0 if every element is finite, else NaN
+template <int M, int N> __device__ __forceinline__ float not_finite(const f32x4 (&acc)[M][N])
+{
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) t = fmaf(acc[i][j][x], 0.f, t);
+    return t;
+}
+
+// ------------------------------------------------------------------------------ weight gradient
+// LDS: three planes of 32 picks x 64 columns of both operands, 32-byte units XOR-swizzled by bits 1 and 3 of
+// the pick so that the 16 row pieces of a transpose read fall two deep on every bank; byte offsets of the rows of TAB picks
+struct SplitDwLds {
+    static constexpr int T = 64, PL = 32 * T * 2, STAGE = 6 * PL;
+    static constexpr int RS = T + 4;                                    // floats per row of the results
+    static_assert(T * RS * 4 <= STAGE, "the results fit");
+    static constexpr int TAB = 512, BYTES = STAGE + TAB * 8;
+};
+
+// tiled_dw_wide_kernel (egs_tiled.h) for fp32 with the picks split over workgroups where there are few tiles: a 64 x 64 tile of dW(e)
+// per workgroup, wavefronts 2 x 2; slabs of 32 picks, fetched two ahead.  A slab's fragments go into registers as soon as it is in LDS;
+// one barrier later the next slab is split and written under the matrix instructions of this one.
+// What bounds it is instruction issue: per slab and wavefront 24 matrix instructions (384 cycles) and 110 vector instructions of two to
+// four, 88 of which split; hence buffer loads (a pick that does not exist needs no masks) and 32-bit offsets (with 64-bit
+// ones and masks 180 vector instructions, 151 us for 135).  us against the fp32 instruction: B30 T46 E73 K44 I384 J169 202 -> 135, B53 T97 E29
+// K41 I111 J75 42.7 -> 30, B16 T512 E64 K64 I256 J128 66 -> 43, B33 T1697 E37 K79 I64 J256 73 -> 38.
+// (The products rows x weights gain less, 1.05 to 1.18 times above 12000 slabs and lose below: not taken there.)
+static __global__ __launch_bounds__(kThreads, 3) void tiled_dw_split_kernel(TiledDwParams p)
+{
+    typedef SplitDwLds L;
+    constexpr int ES = 4, TI = L::T, TJ = L::T, XL = 16, NX = 32 * XL / kThreads;         // 16 chunks of four columns per pick
+    extern __shared__ __attribute__((aligned(16))) char smem_split_dw[];
+    u32x2 *tab = reinterpret_cast<u32x2 *>(smem_split_dw + L::STAGE);                     // [TAB] byte offsets of a pick's X and Y rows
+    const int per_e = p.i_tiles * p.j_tiles * p.S;
+    const int lin = balanced_tile((int)blockIdx.x, p.E * per_e);
+    if (lin < 0) return;
+    const int e = lin / per_e;
+    int rest = lin - e * per_e;
+    const int split = rest / (p.i_tiles * p.j_tiles);
+    rest -= split * (p.i_tiles * p.j_tiles);
+    const int i0 = (rest / p.j_tiles) * TI, j0 = (rest % p.j_tiles) * TJ;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int a = lane & 15, g = lane >> 4;
+    const int wi0 = (wave >> 1) * 32, wj0 = (wave & 1) * 32;
+    const int Me = p.B * p.K;
+    const int lo = split * p.picks_per_split, hi = min(Me, lo + p.picks_per_split), nslabs = max(0, (hi - lo + 31) >> 5);
+    const int xp = tid / XL, xc = tid % XL;
+    const int x_last = (int)(p.x_bytes - 16), y_last = (int)(p.y_bytes - 16);
+    const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(p.Xs), 0, (int)p.x_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs_y = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(p.Ys), 0, (int)p.y_bytes, 0x00020000);
+
+    auto pick_of = [&](int m, int &b) -> int64_t {
+        b = m / p.K;
+        return ((int64_t)b * p.E + e) * p.K + (m - b * p.K);
+    };
+    auto make_tab = [&](int s) {                                        // from slab s on (two slabs beyond the last are looked up)
+        for (int at = tid; at < L::TAB && lo + s * 32 + at < hi + 96; at += kThreads) {
+            const int m = lo + s * 32 + at;
+            int b;
+            const int64_t pick = pick_of(min(m, Me - 1), b);
+            const int64_t t = decode_index_word(load_index_word(p.Ind, p.ind_dtype, pick), p.Ind, p.ind_dtype, pick);
+            const bool ok = m < hi && t >= 0 && t < (int64_t)p.T;
+            tab[at] = ok ? u32x2{(uint32_t)(((int64_t)b * p.ldx_b + t * p.ldx_t) * ES), (uint32_t)(pick * p.J * ES)} : u32x2{kVoffInvalid, kVoffInvalid};
+        }
+    };
+    // Picks that do not exist have an offset outside the descriptors and arrive as zeros on both sides.  Columns past a row are the next
+    // row's: they reach only results that are not stored.  A chunk that would pass the end of its operand is read early and shifted.
+    u32x4 rx[2][NX], ry[2][NX];
+    int shift_x[2][NX], shift_y[2][NX];
+    const int xcol = (i0 + xc * 4) * ES, ycol = (j0 + xc * 4) * ES;
+    auto issue = [&](int s, int q) {
+        auto fetch = [&](__amdgpu_buffer_rsrc_t rsrc, int at, int last, int &shift) -> u32x4 {
+            const int from = min(at, last);                             // (signed: what does not exist stays outside)
+            shift = at - from;
+            return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, from, 0, 0));
+        };
+        const u32x2 *row = tab + s % (L::TAB / 32) * 32;
+#pragma unroll
+        for (int h = 0; h < NX; ++h) {
+            const u32x2 at = row[h * (kThreads / XL) + xp];
+            rx[q][h] = fetch(rs_x, (int)(at[0] + (uint32_t)xcol), x_last, shift_x[q][h]);
+            ry[q][h] = fetch(rs_y, (int)(at[1] + (uint32_t)ycol), y_last, shift_y[q][h]);
+        }
+    };
+    auto at = [](int pick, int unit) -> int { return pick * 128 + ((unit ^ (((pick >> 1) & 1) | ((pick >> 2) & 2))) << 5); };
+    auto put_chunk = [&](int q, int c) {                                // chunk c < 2 NX of this thread's
+        auto one = [&](char *plane0, int r, const u32x4 &v) {
+            u32x2 piece[3];
+            split_chunk(v, piece);
+#pragma unroll
+            for (int x = 0; x < 3; ++x) *reinterpret_cast<u32x2 *>(plane0 + x * L::PL + at(r, xc >> 2) + (xc & 3) * 8) = piece[x];
+        };
+        if (c < NX) one(smem_split_dw, c * (kThreads / XL) + xp, rx[q][c]);
+        else one(smem_split_dw + 3 * L::PL, (c - NX) * (kThreads / XL) + xp, ry[q][c - NX]);
+    };
+    auto settle = [&](int q) {
+        if (!p.edges) return;
+        int any = 0;
+#pragma unroll
+        for (int h = 0; h < NX; ++h) any |= shift_x[q][h] | shift_y[q][h];
+        if (__any(any)) {
+#pragma unroll
+            for (int h = 0; h < NX; ++h) { rx[q][h] = shift_right_bytes(rx[q][h], min(shift_x[q][h], 15)); ry[q][h] = shift_right_bytes(ry[q][h], min(shift_y[q][h], 15)); }
+        }
+    };
+    f32x4 acc[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 xf[2][3], yf[2][3];
+    auto read = [&]() {
+        // transpose reads: lane (a, g) points at pick 8 g + 4 h + a / 4, columns 4 (a % 4) .. + 3
+        auto frag = [&](const char *plane, int unit) -> u32x4 {
+            const char *from = plane + at(g * 8 + (a >> 2), unit) + (a & 3) * 8;
+            const u32x2 l = lds_read_tr16(from), h = lds_read_tr16(from + 4 * 128);
+            return u32x4{l[0], l[1], h[0], h[1]};
+        };
+#pragma unroll
+        for (int x = 0; x < 3; ++x)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                xf[i][x] = frag(smem_split_dw + x * L::PL, (wi0 >> 4) + i);
+                yf[i][x] = frag(smem_split_dw + (3 + x) * L::PL, (wj0 >> 4) + i);
+            }
+    };
+    // Piece by piece over all accumulators, the smallest first; `between(t)` is issued behind the matrix instructions of product t < 6.
+    auto multiply = [&](auto between) {
+        constexpr int P[6] = {2, 0, 1, 1, 0, 0}, Q[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int t = 0; t < 6; ++t) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y) mma_chunk<ElemBF16>(acc[x][y], yf[y][P[t]], xf[x][Q[t]]);
+            between(t);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    if (nslabs > 0) {
+        make_tab(0);
+        __syncthreads();
+        issue(0, 0);
+        issue(1, 1);
+        settle(0);
+#pragma unroll
+        for (int c = 0; c < 2 * NX; ++c) put_chunk(0, c);
+        issue(2, 0);
+    }
+    for (int s0 = 0; s0 < nslabs; s0 += 2) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {                                   // (a last odd round's second slab is zeros)
+            const int s = s0 + q;
+            __syncthreads();
+            read();
+            __syncthreads();
+            if ((s + 3) % (L::TAB / 32) == 0) { make_tab(s + 3); __syncthreads(); }
+            settle(q ^ 1);
+            multiply([&](int t) {
+                if (t < 2 * NX) put_chunk(q ^ 1, t);                    // (past the last slab: zeros, which nobody reads)
+                if (t == 5) issue(s + 3, q ^ 1);
+            });
+            if (s + 1 >= nslabs) break;
+        }
+    }
+
+    // ---------------- not all finite: the wavefront's part again, by the fp32 instruction, straight from memory
+    const float odd = not_finite(acc);
+    if (__any(odd != 0.f || odd != odd)) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int m0 = lo; m0 < hi; m0 += 4) {
+            int b;
+            const int m = m0 + g;
+            const int64_t pick = pick_of(min(m, Me - 1), b);
+            const int32_t t = load_token(p.Ind, p.ind_dtype, pick, p.T);
+            const bool ok = m < hi && t >= 0;
+            const float *xr = reinterpret_cast<const float *>(p.Xs) + (ok ? (int64_t)b * p.ldx_b + (int64_t)t * p.ldx_t : 0);
+            const float *yr = reinterpret_cast<const float *>(p.Ys) + pick * p.J;
+            float xv[2], yv[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int i = i0 + wi0 + h * 16 + a, j = j0 + wj0 + h * 16 + a;
+                xv[h] = ok && i < p.I ? xr[min(i, p.I - 1)] : 0.f;
+                yv[h] = ok && j < p.J ? yr[min(j, p.J - 1)] : 0.f;
+            }
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(yv[y], xv[x], acc[x][y], 0, 0, 0);
+        }
+    }
+
+    // ---------------- lane (a, g) holds rows i0 + wi0 + 16 x + a, columns j0 + wj0 + 16 y + 4 g .. + 3; through LDS, so that whole
+    // row (or, [E,J,I], column) segments leave
+    __syncthreads();
+    float *red = reinterpret_cast<float *>(smem_split_dw);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) *reinterpret_cast<f32x4 *>(red + (wi0 + x * 16 + a) * L::RS + wj0 + y * 16 + g * 4) = acc[x][y];
+    __syncthreads();
+    const bool eji = p.eji != 0;
+    const int out_dtype = p.S > 1 ? 0 : p.out_dtype;
+    const int oes = out_dtype == 0 ? 4 : 2;
+    const int64_t part = p.S > 1 ? (int64_t)split * p.E * p.I * p.J : 0;
+    auto pack = [&](float x, float y) -> uint32_t { return out_dtype == 1 ? pack2<ElemF16>(x, y) : pack2<ElemBF16>(x, y); };
+#pragma unroll 1
+    for (int v = tid; v < TI * TJ / 4; v += kThreads) {
+        int gi, gj;
+        f32x4 r;
+        if (eji) {
+            const int il = (v & 15) * 4, jl = v >> 4;
+            const float *from = red + il * L::RS + jl;
+            gi = i0 + il; gj = j0 + jl;
+            r = f32x4{from[0], from[L::RS], from[2 * L::RS], from[3 * L::RS]};
+        } else {
+            const int il = v >> 4, jl = (v & 15) * 4;
+            gi = i0 + il; gj = j0 + jl;
+            r = *reinterpret_cast<const f32x4 *>(red + il * L::RS + jl);
+        }
+        if (gi >= p.I || gj >= p.J) continue;
+        const int live = min(4, eji ? p.I - gi : p.J - gj);
+        char *dst = p.dW + (part + (eji ? ((int64_t)e * p.J + gj) * p.I + gi : ((int64_t)e * p.I + gi) * p.J + gj)) * oes;
+        if (live == 4) {
+            if (oes == 4) *reinterpret_cast<f32x4_any *>(dst) = r;
+            else *reinterpret_cast<u32x2_any *>(dst) = u32x2{pack(r[0], r[1]), pack(r[2], r[3])};
+        } else {
+            for (int x = 0; x < live; ++x) {
+                if (oes == 4) reinterpret_cast<float *>(dst)[x] = r[x];
+                else reinterpret_cast<uint16_t *>(dst)[x] = (uint16_t)(pack(r[x], 0.f) & 0xffffu);
+            }
+        }
+    }
+}
+
+}  // namespace egs

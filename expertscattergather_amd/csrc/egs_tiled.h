@@ -403,6 +403,7 @@ struct TiledDwParams {
     int32_t ind_dtype, out_dtype, eji;
     int32_t i_tiles, j_tiles, S, picks_per_split;
     int32_t wide;               // tiled_dw_wide_kernel (S = 1)
+    int32_t split32;            // fp32: tiled_dw_split_kernel (egs_split_f32.h), for operands below 2 GiB
     int32_t edges;              // some row is not a whole number of chunks: chunks may have to be read early and shifted
 };
 // what a pick that does not exist reads instead of a row
@@ -816,7 +817,15 @@ static __global__ __launch_bounds__(kThreads) void tiled_dw_sum_kernel(const flo
         const int64_t at = i * 4 + 4 <= n ? i * 4 : n >= 4 ? n - 4 : 0;      // the last thread redoes a few sums rather than go element by element
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
         const int live = n >= 4 ? 4 : (int)n;
-        for (int s = 0; s < S; ++s) {
+        int s = 0;
+        for (; live == 4 && s + 4 <= S; s += 4) {                            // four parts in flight
+            f32x4 u[4];
+#pragma unroll
+            for (int x = 0; x < 4; ++x) u[x] = *reinterpret_cast<const f32x4_any *>(part + (int64_t)(s + x) * n + at);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) { v[0] += u[x][0]; v[1] += u[x][1]; v[2] += u[x][2]; v[3] += u[x][3]; }
+        }
+        for (; s < S; ++s) {
             const float *src = part + (int64_t)s * n + at;
             if (live == 4) { const f32x4 u = *reinterpret_cast<const f32x4_any *>(src); v[0] += u[0]; v[1] += u[1]; v[2] += u[2]; v[3] += u[3]; }
             else for (int x = 0; x < live; ++x) v[x] += src[x];

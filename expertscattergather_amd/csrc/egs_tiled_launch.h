@@ -1,6 +1,7 @@
 // Launch side of egs_tiled.h for one element type; included by egs_tiled_<type>.hip, which each instantiate their share.
 #pragma once
 #include "egs_host.h"
+#include "egs_split_f32.h"
 
 namespace egs {
 namespace host {
@@ -60,7 +61,18 @@ int launch_tiled_dw(TiledDwParams &p, hipStream_t s)
         EGS_CHECK_LAUNCH("tiny_dw_kernel");
         return EGS_OK;
     }
-    if (p.wide) {
+    if constexpr (TT::ES == 4) {
+        if (p.split32 && p.x_bytes < (int64_t)1 << 31 && p.y_bytes < (int64_t)1 << 31) {
+            p.i_tiles = ceil_div(p.I, SplitDwLds::T); p.j_tiles = ceil_div(p.J, SplitDwLds::T);
+            const int64_t tiles = (int64_t)p.E * p.i_tiles * p.j_tiles * p.S;
+            if (tiles > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
+            static_assert(SplitDwLds::BYTES <= 64 * 1024, "no grant needed");
+            hipLaunchKernelGGL(tiled_dw_split_kernel, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(kThreads), SplitDwLds::BYTES, s, p);
+            EGS_CHECK_LAUNCH("tiled_dw_wide_kernel");                   // (of which it is the fp32 form)
+            return EGS_OK;
+        }
+    }
+    if (p.wide && p.S == 1) {
         typedef TiledDwWide<TT> L;
         p.i_tiles = ceil_div(p.I, L::TI); p.j_tiles = ceil_div(p.J, L::TJ);
         const int64_t wide = (int64_t)p.E * p.i_tiles * p.j_tiles;

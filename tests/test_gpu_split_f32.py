@@ -1,0 +1,80 @@
+"""The fp32 weight gradient on the bf16 matrix instruction (csrc/egs_split_f32.h): edges of its tiles, slabs and splits, operands that end
+in the middle of a chunk, values that three bf16 pieces cannot hold, and its error against the fp32 instruction's; against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import egs_oracle as O
+from tests._util import assert_close, make_case, np64
+from tests.test_gpu_parity import dev
+
+pytestmark = pytest.mark.gpu
+
+from expertscattergather_amd import _abi
+from expertscattergather_amd import hip_kernels as hk
+
+
+def gradients(case, Ind, X, Y):
+    with _abi.launch_log() as log:
+        _, dWg = hk.expert_gather_backward_call(X, dev(case["Wg"]), Ind, Y, torch.float32)
+        _, dWs = hk.expert_scatter_backward_call(Y, dev(case["Ws"]), Ind, dev(case["dOut"]), torch.float32)
+    return dWg, dWs, log.kernels
+
+
+@pytest.mark.parametrize("shape, splits", [((8, 40, 2, 64, 64, 64), True),          # whole tiles and slabs; 512 picks
+                                           ((8, 40, 3, 65, 65, 63), True),          # one past a tile, one short of one; 520 picks
+                                           ((5, 30, 2, 103, 129, 1), True),         # 515 picks, a column tile of one column
+                                           ((3, 50, 150, 33, 70, 130), False),      # 99 picks: four slabs, the last of three; 900 tiles
+                                           ((1, 9, 640, 1, 3, 5), False),           # one pick per expert; rows shorter than a chunk
+                                           ((26, 33, 64, 20, 66, 64), True)], ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else None)
+def test_weight_gradient_of_split_floats(shape, splits):
+    B, T, E, K, I, J = shape
+    case = make_case(sum(shape), *shape, torch.float32)
+    Ind, Y = case["Ind"].clone(), case["Y"].clone()
+    if B * K > 1:
+        Ind[0, 0, 0], Ind[-1, -1, -1] = T, -1
+        Y[0, 0, 0] = Y[-1, -1, -1] = float("nan")               # picks that do not exist do not count, whatever their rows hold
+    dWg, dWs, kernels = gradients(case, dev(Ind), dev(case["X"]), dev(Y))
+    assert kernels.count("tiled_dw_wide_kernel") == 2 and ("tiled_dw_sum_kernel" in kernels) == splits, kernels
+    safe, Yk = Ind.clamp(0, T - 1).numpy(), np64(Y)
+    if B * K > 1:
+        Yk[0, 0, 0] = Yk[-1, -1, -1] = 0
+    for got, want, what in ((dWg, O.gather_backward(np64(case["X"]), np64(case["Wg"]), safe, Yk)[1], "dWg"),
+                            (dWs, O.scatter_backward(Yk, np64(case["Ws"]), safe, np64(case["dOut"]))[1], "dWs")):
+        assert_close(got, want, torch.float32, what)
+        # no worse than one rounding of the sum per product of a pick: 2^-24 sqrt(picks) of the result, times four
+        assert np.sqrt(((np64(got) - want) ** 2).mean()) <= 4 * 2.0 ** -24 * max(1, B * K) ** 0.5 * np.sqrt((want ** 2).mean()), what
+
+
+def test_views_that_end_in_the_middle_of_a_chunk():
+    B, T, E, K, I, J = 9, 21, 6, 60, 37, 29
+    case = make_case(5, B, T, E, K, I, J, torch.float32)
+    wide = torch.full((B * T * 41,), float("nan"), device="cuda")
+    X = wide[wide.numel() - ((B - 1) * T * 41 + (T - 1) * 41 + I):].as_strided((B, T, I), (T * 41, 41, 1))
+    X.copy_(case["X"])
+    dWg, dWs, kernels = gradients(case, dev(case["Ind"]), X, dev(case["Y"]))
+    assert kernels.count("tiled_dw_wide_kernel") == 2, kernels
+    assert_close(dWg, O.gather_backward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy(), np64(case["Y"]))[1], torch.float32, "dWg")
+    assert_close(dWs, O.scatter_backward(np64(case["Y"]), np64(case["Ws"]), case["Ind"].numpy(), np64(case["dOut"]))[1], torch.float32, "dWs")
+
+
+def test_values_that_have_no_three_pieces():
+    """Infinities, NaN and values that round to infinity in bf16 give what the fp32 instruction gives, and stay with their results."""
+    B, T, E, K, I, J = 4, 50, 3, 130, 70, 66
+    case = make_case(6, B, T, E, K, I, J, torch.float32)
+    X, Y = case["X"].clone(), case["Y"].clone()
+    Ind = case["Ind"] % (T - 3)
+    Ind[1, 0, 7], Ind[2, 1, 9], Ind[3, 2, 11] = T - 1, T - 2, T - 3     # picked once each
+    X[1, T - 1, 5] = float("inf")
+    X[2, T - 2, 69] = float("nan")
+    X[3, T - 3, 64] = 3.4e38
+    Y[3, 2, 11] *= 1e-3
+    got = gradients(case, dev(Ind), dev(X), dev(Y))[0].cpu().double()
+    bi = torch.arange(B)[:, None, None]
+    want = torch.einsum("beki,bekj->eij", X.double()[bi, Ind], Y.double())
+    assert torch.equal(got.isnan(), want.isnan()) and want.isnan().sum() == J
+    assert torch.equal(got.isinf(), want.isinf()) and want.isinf().sum() == J and torch.equal(got[want.isinf()], want[want.isinf()])
+    big = want.abs() > 1e30
+    fine = want.isfinite() & ~big
+    assert (big & want.isfinite()).sum() == J and torch.allclose(got[big], want[big], rtol=1e-5)
+    assert (got[fine] - want[fine]).abs().max() <= 1e-4 * want[fine].abs().max()
