@@ -16,8 +16,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libegs_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
-SOURCES = ["egs_lib.hip", "egs_rows_launch.hip", "egs_dw_launch.hip", "egs_f8_launch.hip", "egs_mlp_launch.hip", "egs_pass_launch.hip", "egs_sum_launch.hip",
-           "egs_router.hip", "egs_bias.hip",
+SOURCES = ["egs_lib.hip", "egs_rows_launch.hip", "egs_dw_launch.hip", "egs_f8_launch.hip", "egs_mlp_launch.hip", "egs_pass_launch.hip",
+           "egs_sum_launch.hip", "egs_stream_launch.hip", "egs_router.hip", "egs_bias.hip",
            "egs_small_f16.hip", "egs_small_bf16.hip", "egs_fused_f32.hip", "egs_fused_f16.hip", "egs_fused_bf16.hip",
            "egs_tiled_f32.hip", "egs_tiled_f16.hip", "egs_tiled_bf16.hip", "egs_tiled_fp8.hip"]
 

@@ -170,6 +170,9 @@ int launch_rows_16_w(RowsGemmParams &p, bool w_trans, bool &used, hipStream_t s)
 
 }  // namespace
 
+// `used`: rows_stream_kernel takes this product
+int rows_stream(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans, bool gather, int epi, bool &used, hipStream_t s);
+
 int rows_gemm_gather(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans, hipStream_t s)
 {
     if (p.B * p.K == 0 || p.E == 0 || p.N == 0) return EGS_OK;
@@ -178,6 +181,8 @@ int rows_gemm_gather(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans,
     if (fp8_w) { if (w_trans) rc = launch_rows_dl<ElemBF16, 1, true, true, EPI_STORE>(p, used, s); }
     else if (act_dtype == EGS_F16) rc = launch_rows_16_w<ElemF16, true, EPI_STORE>(p, w_trans, used, s);
     else if (act_dtype == EGS_BF16) rc = launch_rows_16_w<ElemBF16, true, EPI_STORE>(p, w_trans, used, s);
+    if (used || rc != EGS_OK) return rc;
+    rc = rows_stream(p, act_dtype, fp8_w, w_trans, true, EPI_STORE, used, s);
     if (used || rc != EGS_OK) return rc;
     return launch_rows_tiled(p, act_dtype, fp8_w, w_trans, true, EPI_STORE, s);
 }
@@ -194,6 +199,8 @@ int rows_gemm_scatter(RowsGemmParams &p, int act_dtype, bool w_trans, int epi, h
         rc = epi == EPI_STORE ? launch_rows_16_w<ElemBF16, false, EPI_STORE>(p, w_trans, used, s) : launch_rows_16_w<ElemBF16, false, EPI_STORE_F32>(p, w_trans, used, s);
     if (used || rc != EGS_OK) return rc;
     p.csr_blocks = 0; p.csr_done = 0;
+    rc = rows_stream(p, act_dtype, false, w_trans, false, epi, used, s);
+    if (used || rc != EGS_OK) return rc;
     return launch_rows_tiled(p, act_dtype, false, w_trans, false, epi, s);
 }
 
