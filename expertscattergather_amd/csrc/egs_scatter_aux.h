@@ -469,11 +469,12 @@ __device__ __forceinline__ void csr_count_half_body(int32_t *sh, int b, int h, i
 
 static __global__ __launch_bounds__(1024) void csr_count_kernel(const void *Ind, int32_t ind_dtype, int32_t T, int32_t N,
                                                          int32_t *seg_off, int32_t *perm, int32_t *rank_tmp,
-                                                         int32_t *long_tab)
+                                                         int32_t *long_tab, int32_t parts)
 {
     extern __shared__ int32_t sh_cnt_dyn[];
-    csr_count_body(sh_cnt_dyn, (int)blockIdx.x, (int)blockIdx.x, (int)threadIdx.x, (int)blockDim.x, Ind, ind_dtype, T, N, seg_off, perm,
-                   rank_tmp, long_tab);
+    const int b = (int)blockIdx.x / parts;
+    csr_count_body(sh_cnt_dyn, b, b, (int)threadIdx.x, (int)blockDim.x, Ind, ind_dtype, T, N, seg_off, perm,
+                   rank_tmp, long_tab, NoPrefetch(), (int)blockIdx.x - b * parts, parts);
 }
 
 // Fast version for N <= 32768 picks whose (token, pick) pair fits 32 bits: one workgroup per
@@ -542,7 +543,9 @@ struct SegSumParams {
     float *long_part;           // [B, long_max_slots(N), I] fp32 partial rows
 };
 
-template <class TT, class PT, int VW>
+// STREAM: more rows than the memory-side cache holds are read past it (a read of 2 GB runs at 6.3 TB/s, so at 7.1; rows that are still
+// in the caches come slower that way: B8 T4096 E128 K256 I1024 J256, 134 MB at a time, 498 -> 530 us for the scatter)
+template <class TT, class PT, int VW, bool STREAM = false>
 __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const int bx, const int by)
 {
     static_assert(VW == 1 || VW == 4 || VW == 8, "a thread takes 1, 4 or 8 elements of a row");
@@ -590,10 +593,12 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
             }
         };
         const int32_t *pb = perm + (size_t)b * N;
-        const PT *Pb = P + (size_t)b * N * sp.ldp + (size_t)iv * VW;
+        // fp32 rows, VW = 8: four columns in each half of the row, so that a wavefront's 16-byte loads are contiguous
+        constexpr bool HALVES = sizeof(PT) == 4 && VW == 8;
+        const PT *Pb = P + (size_t)b * N * sp.ldp + (size_t)iv * (HALVES ? 4 : VW);
         int s = s0;
         if constexpr (VW >= 4) {
-            struct alignas(16) F32x8 { f32x4 lo, hi; };
+            struct F32x8 { f32x4 lo, hi; };
             typedef typename std::conditional<sizeof(PT) == 4, typename std::conditional<VW == 8, F32x8, f32x4>::type,
                                               typename std::conditional<VW == 8, u32x4, u32x2>::type>::type vec_t;
             auto add_vec = [&](const vec_t &v) {
@@ -611,6 +616,11 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
                     }
                 }
             };
+            auto load_vec = [&](const PT *src) -> vec_t {
+                auto one = [](auto *at) { if constexpr (STREAM) return __builtin_nontemporal_load(at); else return *at; };
+                if constexpr (HALVES) return vec_t{one(reinterpret_cast<const f32x4 *>(src)), one(reinterpret_cast<const f32x4 *>(src + I / 2))};
+                else return one(reinterpret_cast<const vec_t *>(src));
+            };
             // long segments (hot tokens): 16 rows (256 bytes) in flight per thread; added in table order all the same
             constexpr int LB = sizeof(vec_t) == 32 ? 8 : 16;
             for (; s + LB <= s1; s += LB) {
@@ -619,7 +629,7 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
 #pragma unroll
                 for (int u = 0; u < LB; ++u) q[u] = pb[s + u];
 #pragma unroll
-                for (int u = 0; u < LB; ++u) v[u] = *reinterpret_cast<const vec_t *>(Pb + (size_t)q[u] * sp.ldp);
+                for (int u = 0; u < LB; ++u) v[u] = load_vec(Pb + (size_t)q[u] * sp.ldp);
 #pragma unroll
                 for (int u = 0; u < LB; ++u) add_vec(v[u]);
             }
@@ -632,7 +642,7 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
 #pragma unroll
                 for (int u = 0; u < RB; ++u) q[u] = pb[min(s + u, s1 - 1)];
 #pragma unroll
-                for (int u = 0; u < RB; ++u) v[u] = *reinterpret_cast<const vec_t *>(Pb + (size_t)q[u] * sp.ldp);
+                for (int u = 0; u < RB; ++u) v[u] = load_vec(Pb + (size_t)q[u] * sp.ldp);
 #pragma unroll
                 for (int u = 0; u < RB; ++u)
                     if (u < nb) add_vec(v[u]);
@@ -640,15 +650,18 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
         } else {
             for (; s < s1; ++s) add_row(Pb + (size_t)pb[s] * sp.ldp);
         }
-        size_t at = row * I + (size_t)iv * VW;
+        size_t at = row * I + (size_t)iv * (HALVES ? 4 : VW);
         if constexpr (TT::ES == 4) {
             float *dst = reinterpret_cast<float *>(out) + at;
             if constexpr (VW >= 4) *reinterpret_cast<f32x4 *>(dst) = f32x4{acc[0], acc[1], acc[2], acc[3]};
             else dst[0] = acc[0];
-            if constexpr (VW == 8) *reinterpret_cast<f32x4 *>(dst + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
+            if constexpr (VW == 8) *reinterpret_cast<f32x4 *>(dst + I / 2) = f32x4{acc[4], acc[5], acc[6], acc[7]};
         } else {
             uint16_t *dst = reinterpret_cast<uint16_t *>(out) + at;
-            if constexpr (VW == 8) {
+            if constexpr (HALVES) {
+                *reinterpret_cast<u32x2 *>(dst) = u32x2{pack2<TT>(acc[0], acc[1]), pack2<TT>(acc[2], acc[3])};
+                *reinterpret_cast<u32x2 *>(dst + I / 2) = u32x2{pack2<TT>(acc[4], acc[5]), pack2<TT>(acc[6], acc[7])};
+            } else if constexpr (VW == 8) {
                 u32x4 w;
 #pragma unroll
                 for (int x = 0; x < 4; ++x) w[x] = pack2<TT>(acc[2 * x], acc[2 * x + 1]);
@@ -810,7 +823,7 @@ __device__ __forceinline__ void segment_sum_long_body(const SegSumParams &sp, co
 
 // workgroups [0, B * long_max_slots(N)): chunks of long segments (first, because they are the longest
 // dependent chains of the launch); then gx * gy workgroups for the ordinary rows
-template <class TT, class PT, int VW>
+template <class TT, class PT, int VW, bool STREAM = false>
 __device__ __forceinline__ void segment_sum_dispatch(const SegSumParams &sp, const int block)
 {
     const int slots = long_max_slots(sp.N);
@@ -819,14 +832,14 @@ __device__ __forceinline__ void segment_sum_dispatch(const SegSumParams &sp, con
         segment_sum_long_body<TT, PT, (VW == 8 ? 4 : VW)>(sp, block / slots, block % slots);   // its partial rows are laid out for 4
     } else {
         const int sb = block - long_blocks;
-        segment_sum_body<TT, PT, VW>(sp, sb % sp.gx, sb / sp.gx);
+        segment_sum_body<TT, PT, VW, STREAM>(sp, sb % sp.gx, sb / sp.gx);
     }
 }
 
-template <class TT, class PT, int VW>
+template <class TT, class PT, int VW, bool STREAM = false>
 __global__ __launch_bounds__(kThreads) void segment_sum_kernel(SegSumParams sp)
 {
-    segment_sum_dispatch<TT, PT, VW>(sp, (int)blockIdx.x);
+    segment_sum_dispatch<TT, PT, VW, STREAM>(sp, (int)blockIdx.x);
 }
 
 // zero n floats (the atomic mode's accumulator).  A kernel rather than a memset so that the

@@ -25,7 +25,13 @@ int launch_routing_table(const void *Ind, int ind_dtype, const egs_dims *d, int3
             static LdsGrant told;
             const int rc_lds = allow_large_lds((const void *)csr_count_kernel, told, lds, "hipFuncSetAttribute(csr_count_kernel)");
             if (rc_lds != EGS_OK) return rc_lds;
-            hipLaunchKernelGGL(csr_count_kernel, dim3(d->B), dim3(64 * nw), lds, s, Ind, ind_dtype, d->T, (int32_t)N, seg_off, perm, rank_tmp, long_tab);
+            // Several workgroups per table: a wavefront ranks its picks 64 at a time, one chunk after the other, 16 us for the
+            // 18 chunks of 17670 picks (B2 T1917 E95 K186 I416 J32, scatter with a table of one workgroup 75 us, of three 58, of five 56, of eight 53.5;
+            // B1 T4096 E100 K256 89 and 55; level below 2000 picks), and every part counts all picks.
+            const int64_t per = (int64_t)nw * 128, want = (N + per - 1) / per;
+            const int parts = (int)(want > 8 ? 8 : want);
+            if ((int64_t)d->B * parts > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
+            hipLaunchKernelGGL(csr_count_kernel, dim3(d->B * parts), dim3(64 * nw), lds, s, Ind, ind_dtype, d->T, (int32_t)N, seg_off, perm, rank_tmp, long_tab, parts);
             EGS_CHECK_LAUNCH("csr_count_kernel");
             return EGS_OK;
         }
@@ -51,10 +57,14 @@ int launch_routing_table(const void *Ind, int ind_dtype, const egs_dims *d, int3
     return EGS_OK;
 }
 
+// more product rows than the memory-side cache (256 MB) holds until they are read
+static bool rows_stream_by(const egs_dims *d, size_t row_bytes) { return (uint64_t)d->B * d->E * d->K * row_bytes > (256ull << 20); }
+
 template <class TT, class PT>
-void launch_segment_sum8(const SegSumParams &sp, int seg_blocks, hipStream_t s)
+void launch_segment_sum8(const SegSumParams &sp, int seg_blocks, bool stream, hipStream_t s)
 {
-    hipLaunchKernelGGL((segment_sum_kernel<TT, PT, 8>), dim3(seg_blocks), dim3(kThreads), 0, s, sp);
+    if (stream) hipLaunchKernelGGL((segment_sum_kernel<TT, PT, 8, true>), dim3(seg_blocks), dim3(kThreads), 0, s, sp);
+    else hipLaunchKernelGGL((segment_sum_kernel<TT, PT, 8>), dim3(seg_blocks), dim3(kThreads), 0, s, sp);
 }
 
 // fixed-order reduction of the product rows per token; when `reduce` is given (and qualifies) the
@@ -87,7 +97,7 @@ int launch_segment_sum(const void *rows, bool rows_f32, const int32_t *seg_off, 
         if (fuse) hipLaunchKernelGGL((segsum_dwreduce_kernel<TT, PT, 4>), dim3(seg_blocks + red_blocks), dim3(kThreads), 0, \
                                      s, sp, seg_blocks, reduce->part, reduce->dW, reduce->S, reduce->w_elems / 4,           \
                                      reduce->out_dtype);                                                                    \
-        else if (vw8) launch_segment_sum8<TT, PT>(sp, seg_blocks, s);                                                       \
+        else if (vw8) launch_segment_sum8<TT, PT>(sp, seg_blocks, rows_stream_by(d, (size_t)sp.ldp * sizeof(PT)), s);       \
         else if (vw4) hipLaunchKernelGGL((segment_sum_kernel<TT, PT, 4>), dim3(seg_blocks), dim3(kThreads), 0, s, sp);      \
         else hipLaunchKernelGGL((segment_sum_kernel<TT, PT, 1>), dim3(seg_blocks), dim3(kThreads), 0, s, sp);               \
     } while (0)
@@ -121,11 +131,16 @@ int launch_token_sum(const void *rows, bool rows_f32, const void *Ind, int ind_d
     const int64_t grid = (int64_t)d->B * p.t_blocks * p.c_blocks;
     if (grid > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
     const size_t lds = token_sum_lds(p.N);
-    if (act_dtype == EGS_F32) hipLaunchKernelGGL((token_sum_kernel<ElemF32, float>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
-    else if (act_dtype == EGS_F16 && rows_f32) hipLaunchKernelGGL((token_sum_kernel<ElemF16, float>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
-    else if (act_dtype == EGS_F16) hipLaunchKernelGGL((token_sum_kernel<ElemF16, uint16_t>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
-    else if (rows_f32) hipLaunchKernelGGL((token_sum_kernel<ElemBF16, float>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
-    else hipLaunchKernelGGL((token_sum_kernel<ElemBF16, uint16_t>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);
+    const bool stream = rows_stream_by(d, (size_t)p.ldp * (rows_f32 ? 4 : 2));
+#define EGS_TOKSUM(TT, PT)                                                                                              \
+    do {                                                                                                                \
+        if (stream) hipLaunchKernelGGL((token_sum_kernel<TT, PT, true>), dim3((unsigned)grid), dim3(kThreads), lds, s, p); \
+        else hipLaunchKernelGGL((token_sum_kernel<TT, PT>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);           \
+    } while (0)
+    if (act_dtype == EGS_F32) EGS_TOKSUM(ElemF32, float);
+    else if (act_dtype == EGS_F16) { if (rows_f32) EGS_TOKSUM(ElemF16, float); else EGS_TOKSUM(ElemF16, uint16_t); }
+    else { if (rows_f32) EGS_TOKSUM(ElemBF16, float); else EGS_TOKSUM(ElemBF16, uint16_t); }
+#undef EGS_TOKSUM
     EGS_CHECK_LAUNCH("token_sum_kernel");
     return EGS_OK;
 }

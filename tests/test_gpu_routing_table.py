@@ -274,3 +274,40 @@ def test_a_table_of_garbage_gives_wrong_sums_but_ends():
             assert rc == 0
             torch.cuda.synchronize()
             assert torch.isfinite(out.float()).all()
+
+
+@pytest.mark.parametrize("shape", [(2, 300, 33, 125, 64, 24),      # 4125 picks of 16 wavefronts: three workgroups, the last with 29 picks
+                                   (1, 2300, 90, 200, 40, 24),     # 18000 picks of 15 wavefronts (histograms of 2300 tokens): eight
+                                   (3, 20, 41, 100, 36, 24)],      # 4100 picks of 20 tokens, all of them hot
+                         ids=lambda s: "x".join(map(str, s)))
+def test_table_of_its_own_launch_by_several_workgroups(shape):
+    B, T, E, K, I, J = shape
+    case = make_case(sum(shape), *shape, torch.bfloat16)
+    Ind = case["Ind"].clone()
+    Ind[0, 0, 0], Ind[-1, -1, -1], Ind[0, E // 2, :], Ind[-1, 3, 7] = T, -1, 7, -30000
+    keep = ((Ind >= 0) & (Ind < T)).numpy()[..., None]
+    with _abi.launch_log() as log:
+        out = hk.expert_scatter_forward_call(case["Y"].to(DEV), case["Ws"].to(DEV), Ind.to(DEV), T, torch.float32)
+    assert "csr_count_kernel" in log.kernels and "segment_sum_kernel" in log.kernels, log.kernels
+    assert_close(out, O.scatter_forward(np64(case["Y"]) * keep, np64(case["Ws"]), Ind.clamp(0, T - 1).numpy(), T), torch.bfloat16, "out")
+    again = hk.expert_scatter_forward_call(case["Y"].to(DEV), case["Ws"].to(DEV), Ind.to(DEV), T, torch.float32)
+    assert torch.equal(out, again)
+
+
+@pytest.mark.parametrize("shape, sums", [((20, 64, 256, 16, 1024, 24), "token_sum_kernel"),         # 336 MB of product rows, 4096 picks
+                                         ((4, 600, 64, 300, 1024, 32), "segment_sum_kernel"),       # 315 MB, with a table
+                                         ((4, 600, 64, 300, 1028, 32), "segment_sum_kernel")],      # rows that are added four columns at a time
+                         ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else s)
+def test_sums_of_more_rows_than_the_caches_hold(shape, sums):
+    B, T, E, K, I, J = shape
+    g = torch.Generator(device=DEV).manual_seed(3)
+    Y, W = (torch.randn(*s, device=DEV, generator=g).bfloat16() for s in ((B, E, K, J), (E, J, I)))
+    Ind = torch.randint(0, T, (B, E, K), device=DEV, generator=g)
+    with _abi.launch_log() as log:
+        out = hk.expert_scatter_forward_call(Y, W, Ind, T, torch.float32)
+    assert log.kernels.count(sums) == 1, log.kernels
+    want = torch.zeros(B, T, I, device=DEV)
+    for e in range(E):
+        rows = Y[:, e].reshape(-1, J).float() @ W[e].float()
+        want.view(B * T, I).index_add_(0, (Ind[:, e] + torch.arange(B, device=DEV)[:, None] * T).reshape(-1), rows)
+    assert (out.float() - want).abs().max() <= 2 * 2.0 ** -8 * want.abs().max()
