@@ -27,11 +27,13 @@ int launch_scatter_fused_one(const ScatterFusedParams &p, size_t lds, int blocks
         hipLaunchKernelGGL((scatter_fused_multi_kernel<TT, W_NMAJOR, KS>), dim3(blocks), dim3(kFusedThreads), lds, s, p);
     } else if (p.run > 1) {             // (a weight gradient of the same call follows alone)
         name = "scatter_fused_runs_kernel";
-        static LdsGrant told_runs;
-        const int rc_lds = allow_large_lds((const void *)scatter_fused_runs_kernel<TT, W_NMAJOR, KS>, told_runs, lds,
-                                           "hipFuncSetAttribute(scatter_fused_runs_kernel)");
+        static LdsGrant told_runs[2];
+        constexpr bool kHolds = KS <= 2;
+        const bool hold = kHolds && p.E * ((p.K + 31) / 32) <= kFusedHeldUnits;
+        const auto kernel = hold ? scatter_fused_runs_kernel<TT, W_NMAJOR, KS, kHolds> : scatter_fused_runs_kernel<TT, W_NMAJOR, KS, false>;
+        const int rc_lds = allow_large_lds((const void *)kernel, told_runs[hold], lds, "hipFuncSetAttribute(scatter_fused_runs_kernel)");
         if (rc_lds != EGS_OK) return rc_lds;
-        hipLaunchKernelGGL((scatter_fused_runs_kernel<TT, W_NMAJOR, KS>), dim3(blocks), dim3(kFusedThreads), lds, s, p);
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kFusedThreads), lds, s, p);
     } else if (p.tab_seg != nullptr && dwt != nullptr && !dwt->wide && TT::ES == 2) {
       if constexpr (TT::ES == 2) {
         name = "scatter_fused_dwtile_table_kernel";

@@ -71,7 +71,9 @@ __host__ __device__ inline size_t scatter_fused_lds(int T, int NP, int rows)
 }
 __host__ __device__ inline size_t scatter_fused_lds(int T, int NP) { return scatter_fused_lds(T, NP, NP); }
 
-template <class TT, bool W_NMAJOR, int KS, bool MULTI = false, bool TABLE = false, bool RUNS = false>
+// HOLD (RUNS, at most kFusedHeldUnits units of 32 picks of one expert): see scatter_fused_runs_kernel
+constexpr int kFusedHeldUnits = 4 * (kFusedThreads / 64);
+template <class TT, bool W_NMAJOR, int KS, bool MULTI = false, bool TABLE = false, bool RUNS = false, bool HOLD = false>
 __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, const int block, char *smem)
 {
     // KS = reduction length in MFMA steps of four 16-byte chunks: 32 elements of a 16-bit type, 16 of fp32
@@ -83,8 +85,9 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
     // [E,R,N] weight; with all four units requested up front a wavefront spent 5000 cycles issuing before it multiplied
     // anything, 8.3 against 9.8 us at B64 T256 E32 K32 I128 J64 together with the summing loop below).  In passes: all.
     constexpr int kAhead = MULTI ? kFusedDepth : 1;
-    // a table that this workgroup parks itself (TABLE, one pass) is parked as row addresses, see (2)
-    constexpr bool kEncoded = TABLE && !MULTI;
+    // a table that this workgroup parks itself (TABLE, one pass) or walks several times is parked as row addresses, see (2)
+    constexpr bool kEncoded = (TABLE && !MULTI) || HOLD;
+    static_assert(!HOLD || kFusedDepth * (kFusedThreads / 64) == kFusedHeldUnits, "every unit has a place in registers");
     // the wavefront index is made known as uniform: units, experts and base addresses derived from it are then
     // scalar work, and the loads take a scalar base with a per-lane 32-bit offset
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -117,11 +120,12 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
     struct Unit { u32x4 y[2][KS]; u32x4 w[2 * KS]; };
     Unit buf[kFusedDepth];
     const uint32_t a_base_b = (uint32_t)b * (uint32_t)NP * R * ES;
-    auto load_unit = [&](Unit &u, int unit, int e0, int ne) {
+    auto load_unit = [&](Unit &u, int unit, int e0, int ne, bool with_rows = true) {
         if (unit >= ne * KT2) return;                   // uniform per wavefront; a unit's own loads are unconditional
         const int el = unit / KT2, rp = unit - el * KT2, e = e0 + el;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
+            if (!with_rows) break;
             // coalesced: lanes 4r .. 4r+3 fetch four consecutive chunks of row r; transposed to operand order at use
             const int k = min(rp * 32 + h * 16 + (lane >> 2), K - 1);
             const char *yrow = p.A + a_base_b + (uint32_t)((e * K + k) * R * ES);
@@ -183,7 +187,7 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
             }
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const u32x4 yf = lanes_4a_g_to_16g_a(u.y[h][ks], lane);
+                const u32x4 yf = HOLD ? u.y[h][ks] : lanes_4a_g_to_16g_a(u.y[h][ks], lane);
                 mma_chunk<TT>(acc[h][0], wf[0], yf);
                 mma_chunk<TT>(acc[h][1], wf[1], yf);
             }
@@ -239,8 +243,18 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
     } else {
     csr_count_body(cnt, b, 0, tid, kFusedThreads, p.Ind, p.ind_dtype, T, NP, nullptr, perm, nullptr, nullptr, [&]() {
 #pragma unroll
-        for (int d = 0; d < kAhead; ++d) load_unit(buf[d], wave + NWV * d, 0, min(EP, E));
+        for (int d = 0; d < (HOLD ? kFusedDepth : kAhead); ++d) load_unit(buf[d], wave + NWV * d, 0, min(EP, E));
     });
+    }
+    if constexpr (HOLD) {
+        __syncthreads();                                // the table is in LDS
+        for (int i = tid; i < NP; i += kFusedThreads) perm[i] = (perm[i] << 7) | ((perm[i] & 7) << 4);
+#pragma unroll
+        for (int d = 0; d < kFusedDepth; ++d)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) buf[d].y[h][ks] = lanes_4a_g_to_16g_a(buf[d].y[h][ks], lane);
     }
 
     const int cc = tid & 7;
@@ -259,6 +273,21 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
     if constexpr (!MULTI) {
         for (int sl = slice; sl < slice_end; ++sl) {
             if (sl > slice) __syncthreads();            // everybody is done with the last slice's rows
+            if constexpr (HOLD) {
+                // a unit's weights of the next slice are requested one unit later: asked for all at once behind the products,
+                // they held up the sums (B64 T256 E32 K32 I768 J64 42 us instead of 38.5)
+                auto reload = [&](int d) {
+                    if (sl + 1 == slice_end) return;
+                    c0 += kFusedCols;
+                    load_unit(buf[d], wave + NWV * d, 0, E, false);
+                    c0 -= kFusedCols;
+                };
+#pragma unroll
+                for (int d = 0; d < kFusedDepth; ++d) {
+                    compute_unit(buf[d], wave + NWV * d, E);
+                    if (d > 0) reload(d - 1);
+                }
+            } else
             for (int u0 = wave; u0 < E * KT2; u0 += NWV * kFusedDepth) {
 #pragma unroll
                 for (int d = 0; d < kFusedDepth; ++d) {
@@ -276,7 +305,7 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
                 c0 += kFusedCols;
                 if (sl + 1 < slice_end) {
 #pragma unroll
-                    for (int d = 0; d < kAhead; ++d) load_unit(buf[d], wave + NWV * d, 0, E);
+                    for (int d = HOLD ? kFusedDepth - 1 : 0; d < (HOLD ? kFusedDepth : kAhead); ++d) load_unit(buf[d], wave + NWV * d, 0, E, !HOLD);
                 }
             }
 
@@ -287,9 +316,8 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
             // chunk 0 of row q in the rows' XOR order: a thread's two chunks are one XOR away each.  (The phase is bound by
             // vector-ALU issue - two wavefronts per SIMD, all in it at once - so it is written for few instructions per pick.)
             const uint32_t c2 = (uint32_t)(tid & 3) << 5, zero_sel = (uint32_t)p.zero_at;
-            for (int t = tid >> 2; t < T; t += kFusedThreads >> 2) {
+            auto sum_of = [&](int t, f32x4 &lo, f32x4 &hi) {
                 const int s0 = seg[t], s1 = seg[t + 1];
-                f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
                 for (int s = s0; s < s1; s += 4) {
                     const int n = s1 - s;
                     uint32_t en[4];
@@ -306,6 +334,8 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
 #pragma unroll
                     for (int x = 0; x < 4; ++x) { lo += v[x][0]; hi += v[x][1]; }
                 }
+            };
+            auto store_of = [&](int t, const f32x4 &lo, const f32x4 &hi) {
                 char *dst = p.out + (((size_t)b * T + t) * N + at0) * ES;
                 if constexpr (ES == 4) {
                     reinterpret_cast<f32x4 *>(dst)[0] = lo;
@@ -316,6 +346,24 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
                     w[2] = pack2<TT>(hi[0], hi[1]); w[3] = pack2<TT>(hi[2], hi[3]);
                     *reinterpret_cast<u32x4 *>(dst) = w;
                 }
+            };
+            int t = tid >> 2;
+            if constexpr (HOLD) {
+                // loads and stores share a counter: the next slice's weights are waited for before the first store, which the
+                // next slice would otherwise have to wait for too
+                f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
+                if (t < T) sum_of(t, lo, hi);
+#pragma unroll
+                for (int d = 0; d < kFusedDepth; ++d)
+#pragma unroll
+                    for (int x = 0; x < 2 * KS; ++x) asm volatile("" : "+v"(buf[d].w[x]));
+                if (t < T) store_of(t, lo, hi);
+                t += kFusedThreads >> 2;
+            }
+            for (; t < T; t += kFusedThreads >> 2) {
+                f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
+                sum_of(t, lo, hi);
+                store_of(t, lo, hi);
             }
         }
     } else {
@@ -386,12 +434,16 @@ __global__ __launch_bounds__(kFusedThreads) void scatter_fused_kernel(ScatterFus
     scatter_fused_body<TT, W_NMAJOR, KS>(p, (int)blockIdx.x, smem_fused);
 }
 
-// more slices than the device has CUs for: a run of them per workgroup, with one sort
-template <class TT, bool W_NMAJOR, int KS>
+// More slices than the device has CUs for: a run of them per workgroup, with one sort.  The slices of a run multiply the same rows,
+// so with HOLD (a reduction of at most two steps, and no more units of 32 picks than the wavefronts have registers for) they are
+// read and brought into operand order once, and only weights travel between slices.  B64 T256 E32 K32 I768 J64, bf16: 48 -> 38.5 us
+// (sort and first operands 11, then 4.6 a slice: 128 KB of weights per CU, which all CUs together take 2.2 us to get out of L2,
+// products 1.1, sums 1.0); B128 T64 E8 K16 I1024 J64 39 -> 33; the same with fp32 and J32 65 -> 59.
+template <class TT, bool W_NMAJOR, int KS, bool HOLD>
 __global__ __launch_bounds__(kFusedThreads) void scatter_fused_runs_kernel(ScatterFusedParams p)
 {
     extern __shared__ __attribute__((aligned(16))) char smem_fused_runs[];
-    scatter_fused_body<TT, W_NMAJOR, KS, false, false, true>(p, (int)blockIdx.x, smem_fused_runs);
+    scatter_fused_body<TT, W_NMAJOR, KS, false, false, true, HOLD>(p, (int)blockIdx.x, smem_fused_runs);
 }
 
 // more picks per batch element than LDS holds product rows for: groups of experts, one after the other
