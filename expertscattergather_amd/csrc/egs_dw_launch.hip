@@ -2,9 +2,32 @@
 // shapes, followed by the fixed-order sum over splits.
 #include "egs_host.h"
 #include "egs_dw_dl.h"
+#include "egs_dw_strip.h"
 
 namespace egs {
 namespace host {
+
+namespace {
+
+template <class TT, int TP>
+int launch_dw_strip(const DwDlParams &q, int grid, hipStream_t s)
+{
+    static LdsGrant told;
+    const int rc = allow_large_lds((const void *)dw_strip_kernel<TT, TP>, told, DwStrip<TP>::BYTES, "hipFuncSetAttribute(dw_strip_kernel)");
+    if (rc != EGS_OK) return rc;
+    hipLaunchKernelGGL((dw_strip_kernel<TT, TP>), dim3((unsigned)grid), dim3(kDlThreads), DwStrip<TP>::BYTES, s, q);
+    return EGS_OK;
+}
+template <class TT>
+int launch_dw_strip(const DwDlParams &q, int tp, int grid, hipStream_t s)
+{
+    const int rc = tp == 2 ? launch_dw_strip<TT, 2>(q, grid, s) : tp == 3 ? launch_dw_strip<TT, 3>(q, grid, s) : launch_dw_strip<TT, 4>(q, grid, s);
+    if (rc != EGS_OK) return rc;
+    EGS_CHECK_LAUNCH("dw_strip_kernel");
+    return EGS_OK;
+}
+
+}  // namespace
 
 int dw_general(const void *Xs, const void *Ys, const void *Ind, void *dW, void *workspace, const egs_dims *d,
                int64_t ldx_b, int64_t ldx_t, int act_dtype, int out_dtype, int ind_dtype, int dw_layout,
@@ -32,14 +55,17 @@ int dw_general(const void *Xs, const void *Ys, const void *Ind, void *dW, void *
         if (grid > INT32_MAX) return EGS_ERR_BAD_SHAPE;
         // 128-column tiles: three 48 KB stages of 64 rows (C4: 42.2 -> 37.9 us per weight gradient with its sum over
         // splits); 256-column tiles: four 32 KB stages of 32 rows (C3: 178 -> 174 us)
-        if (act_dtype == EGS_F16) {
+        if (pl.b_bq == 64) {
+            const int rc = act_dtype == EGS_F16 ? launch_dw_strip<ElemF16>(q, pl.b_tp, (int)grid, s) : launch_dw_strip<ElemBF16>(q, pl.b_tp, (int)grid, s);
+            if (rc != EGS_OK) return rc;
+        } else if (act_dtype == EGS_F16) {
             if (pl.b_bq == 256) hipLaunchKernelGGL((dw_dl_kernel<ElemF16, 256, 4, 32>), dim3((unsigned)grid), dim3(kDlThreads), 0, s, q);
             else hipLaunchKernelGGL((dw_dl_kernel<ElemF16, 128, 3>), dim3((unsigned)grid), dim3(kDlThreads), 0, s, q);
         } else {
             if (pl.b_bq == 256) hipLaunchKernelGGL((dw_dl_kernel<ElemBF16, 256, 4, 32>), dim3((unsigned)grid), dim3(kDlThreads), 0, s, q);
             else hipLaunchKernelGGL((dw_dl_kernel<ElemBF16, 128, 3>), dim3((unsigned)grid), dim3(kDlThreads), 0, s, q);
         }
-        EGS_CHECK_LAUNCH("dw_dl_kernel");
+        if (pl.b_bq != 64) EGS_CHECK_LAUNCH("dw_dl_kernel");
         if (pl.b_S > 1) {       // partials are in the output's layout, I % 8 == 0 and J % 8 == 0: vectorised plain sum
             hipLaunchKernelGGL(dw_reduce4_kernel, dim3(grid_1d(w_elems / 4, 4096)), dim3(kThreads), 0, s,
                                (const float *)workspace, (char *)dW, pl.b_S, w_elems / 4, out_dtype);

@@ -162,6 +162,41 @@ int64_t dw_split32_slabs(const egs_dims *d)
     return (int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, 64) * (((int64_t)d->B * d->K + 31) / 32);
 }
 
+// 16-bit, up to 64 output columns: dw_strip_kernel (tp: tiles of 32 tp x 64, S splits of the picks) where it is expected to beat what there
+// is else.  Both sides are a number of rounds of workgroups over the CUs, each some us and some more for every 1000 picks, fitted to times
+// alone on the device (us, strips / 32 x 64 or 32 x 32 tiles): B64 T256 E32 K32 I768 J64 18.8 / 28.4, B2 T1000 E60 K200 I640 J48 12 / 20,
+// B8 T4096 E128 K256 I1024 J64 95 / 147, B100 T500 E6 K100 I448 J64 28 / 33, B20 T900 E14 K64 I1024 J32 10.4 / 11.6, B7 T500 E80 K64 I192
+// J64 5.6 / 9.2; not taken: B33 T300 E16 K64 I288 J64 12.2 / 11.1, I256 J64 at E32 and 2048 picks 13.2 / 10.0, B40 T400 E16 K40 I640 J24
+// 11.8 / 11.3, B1 T2000 E8 K250 I256 J64 4.7 / 3.7.  Where those tiles are not taken the general ones always lose: B3 T120 E5 K90 I200 J56
+// 4.3 / 8.6, B17 T2218 E4 K63 I224 J32 9.3 / 13.2, B2 T300 E100 K100 I160 J32 5.4 / 10.4, B30 T200 E4 K20 I136 J24 5.6 / 9.3.
+struct DwStripPlan { int tp, S, rows_per_split; };
+
+bool dw_strip_takes(const egs_dims *d, int act_dtype, DwStripPlan *plan = nullptr)
+{
+    const int64_t Me = (int64_t)d->B * d->K;
+    if (act_dtype == EGS_F32 || d->I % 8 || d->J % 8 || d->I <= 128 || d->J > 64 || d->J < 8 || Me < 128 || d->E == 0) return false;
+    constexpr double start[] = {2.4, 3.0, 2.6}, per_pick[] = {5.8e-3, 7.3e-3, 10.3e-3}, second_pass = 4.0;
+    DwStripPlan best = {0, 0, 0};
+    double least = 0;
+    for (int tp = 2; tp <= 4; ++tp) {
+        const int64_t tiles = (int64_t)d->E * ceil_div(d->I, 32 * tp), most = tiles < 256 ? 256 / tiles : 1;
+        for (int64_t n = 1; n <= most; n += most > 1 ? most - 1 : 1) {
+            const int64_t rows = ((Me + n - 1) / n + 127) / 128 * 128, S = (Me + rows - 1) / rows;
+            const double us = (double)((tiles * S + 255) / 256) * (start[tp - 2] + (double)rows * per_pick[tp - 2]) +
+                              (S > 1 ? second_pass + (double)S * d->E * d->I * d->J * 2e-6 : 0.0);
+            if (best.tp != 0 && us >= least) continue;
+            least = us;
+            best = {tp, (int)S, (int)(rows < INT32_MAX ? rows : INT32_MAX)};
+        }
+    }
+    if (plan != nullptr) *plan = best;
+    const int64_t narrow = (int64_t)d->E * ceil_div(d->I, 32) * ceil_div(d->J, 32), wide = (int64_t)d->E * ceil_div(d->I, 32);
+    if (narrow < 128 || d->I > 2048 || dw_few_picks(d, act_dtype)) return true;         // make_dw_tile refuses these
+    const double tile = d->J > 32 && (narrow > 256 || Me >= 4096) ? (double)((wide + 255) / 256) * (2.9 + (double)Me * 3.0e-3)
+                                                                  : (double)((narrow + 511) / 512) * (2.9 + (double)Me * 5.0e-3);
+    return least < 0.95 * tile;
+}
+
 DwPlan plan_dw(const egs_dims *d, int act_dtype)
 {
     DwPlan pl;
@@ -208,6 +243,18 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
         pl.b_S = (int)s3;
         pl.b_rows_per_split = (int)r3;
         pl.bytes_big = s3 > 1 ? align_up((size_t)s3 * d->E * d->I * d->J * 4, 256) : 0;
+    }
+
+    DwStripPlan strip;
+    if (dw_strip_takes(d, act_dtype, &strip)) {
+        pl.big_ok = true;
+        pl.b_bq = 64;
+        pl.b_tp = strip.tp;
+        pl.b_i_tiles = ceil_div(d->I, 32 * strip.tp);
+        pl.b_j_tiles = 1;
+        pl.b_S = strip.S;
+        pl.b_rows_per_split = strip.rows_per_split;
+        pl.bytes_big = strip.S > 1 ? align_up((size_t)strip.S * d->E * d->I * d->J * 4, 256) : 0;
     }
 
     // small experts: 64 x 64 tiles, up to 1024 picks per workgroup, enough workgroups to cover the device
@@ -368,6 +415,7 @@ bool make_dw_tile(const void *Xs, const void *Ys, const void *Ind, void *dW, con
     if (g_force_generic) return false;
     const int ES = elem_size(act_dtype);
     if (ES == 4 && d->I > 32 && d->J > 32 && dw_split32_slabs(d) >= 8192) return false;
+    if (dw_strip_takes(d, act_dtype)) return false;
     if (d->I % 8 || d->J % 8 || d->I < 8 || d->J < 8 || d->I > 2048 || d->J > 128) return false;
     const int64_t Me = (int64_t)d->B * d->K;
     if (Me == 0 || d->E == 0 || d->T == 0) return false;
