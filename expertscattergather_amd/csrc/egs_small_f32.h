@@ -1,31 +1,36 @@
 // Gather-GEMM for small experts in fp32: Y[b,e,k,:] = X[b, Ind[b,e,k], :] . W(e), reduction length 32/64/128, 16..64
 // output columns (the reference's default shape in its own precision: B64 T256 E32 K32 I128 J64 fp32).
 //
-// The fp32 matrix instruction (16x16x4) is the roof here (AI 40 FLOP/B against a ridge of 20), so the kernel is
-// arranged to keep it fed: W(e) - 32 KB at the default shape, too much for registers next to 64 picks - is brought
-// into LDS once per workgroup in [column][reduction] order, so that a lane's four reduction-consecutive weights are
-// one 16-byte LDS read; the gathered rows go global -> registers -> operand order (coalesced 64-byte runs per row,
-// then the 4 x 16 lane transposition).  One wavefront = 32 (or 64) picks of one expert, a workgroup 256; one barrier
-// (W(e) in place).  A wavefront multiplies and stores its 16-pick row tiles one after the other, the first tile's rows
-// requested before the barrier and the others after it.
+// The products go through the bf16 matrix instruction, three pieces per value (egs_split.h).  W(e) is split once per workgroup, into
+// three LDS planes in operand order: a lane's eight weights of 32 reduction steps are 16 bytes, steps 4 g .. + 3 of the first
+// sixteen and then of the second, as the rows' 16-byte chunks give them.  The gathered rows go global -> registers -> operand order
+// (coalesced 64-byte runs per row, then the 4 x 16 lane transposition) and are split there.  One wavefront = 32 picks of one
+// expert, a workgroup 256; one barrier (W(e) in place).  A wavefront multiplies and stores its 16-pick row tiles one after the
+// other, the first tile's rows requested before the barrier and the others after it.
+// us, three pieces / the fp32 instruction, which was the roof with 138 TFLOP/s: B64 T256 E32 K32 I128 J64 14.0 / 16.9 (the matrix
+// instructions take 3, indices, rows and W(e) the rest), E60 20.9 / 26.6, I64 9.8 / 11.2, B160 J48 23 / 30, B8 T100 E16 9.2 / 11.8; level for
+// 16 columns.  (The one-kernel scatter does not gain: it would split every weight once per batch element, 20.0 / 18.8.)
 //
 // Replaces the reference's expert_gather_kernel (egs/triton_kernels.py:49-143) on these shapes.
 #pragma once
 #include "egs_small.h"
+#include "egs_split.h"
 
 namespace egs {
 
-__host__ __device__ constexpr size_t rows_small_f32_lds(int R, int N) { return (size_t)N * (R + 4) * 4; }
+// bytes of a column in a plane: 16 more than the weights take, so that the 16 lanes of a read spread over the banks
+__host__ __device__ constexpr int rows_small_f32_column(int R) { return R * 2 + 16; }
+__host__ __device__ constexpr size_t rows_small_f32_lds(int R, int N) { return (size_t)3 * N * rows_small_f32_column(R); }
 
 // Requirements (checked by the launcher): fp32, R == 16 * KS in {32, 64, 128}, N == 16 * TN <= 64, rows of A, W and C
 // 16-byte aligned, every tensor below 4 GiB.  W is [E,R,N] (W_NMAJOR) or [E,N,R].
 // TQ = 16-pick row tiles per wavefront (4, or 2 with twice the wavefronts: a workgroup covers 256 picks either way)
 template <bool W_NMAJOR, int KS, int TN, int TQ = 4>
-__global__ __launch_bounds__(64 * (16 / TQ)) void rows_small_f32_kernel(SmallRowsParams p)
+__global__ __launch_bounds__(64 * (16 / TQ), 4) void rows_small_f32_kernel(SmallRowsParams p)
 {
-    constexpr int R = 16 * KS, N = 16 * TN, LDW = R + 4;        // LDW: padded so that the 16 lanes of a read spread over the banks
+    constexpr int R = 16 * KS, N = 16 * TN, COL = rows_small_f32_column(R), PLANE = N * COL;
     constexpr int PW = 16 * TQ, NTHREADS = 64 * (256 / PW);     // picks per wavefront, threads per workgroup
-    extern __shared__ __attribute__((aligned(16))) float w_lds[];      // [N][LDW]
+    extern __shared__ __attribute__((aligned(16))) char w_lds[];       // [3][N][COL]
     int e, tile;
     int bid = (int)blockIdx.x;
     // routing-table build of a later scatter riding along (csr_blocks = B, or 0): one workgroup per batch element, first in line
@@ -59,21 +64,19 @@ __global__ __launch_bounds__(64 * (16 / TQ)) void rows_small_f32_kernel(SmallRow
 
     // W(e) -> registers (all loads in flight behind the index load), LDS as [column][reduction] further down
     const char *We = p.W + (size_t)e * R * N * 4;
-    constexpr int W_CHUNKS = R * N / 4, W_IT = (W_CHUNKS + NTHREADS - 1) / NTHREADS;
-    // Which 16-byte chunk a thread takes.  [N][R] (rows copied as they lie): consecutive threads, consecutive chunks.
-    // [R][N] (written to LDS transposed, four single floats per chunk): a wavefront takes 16 reduction rows x 16 columns per
-    // load, lanes 4 q .. 4 q + 3 the four chunks of row q's 64 bytes - as many L1 accesses as consecutive chunks make, and
-    // the 64 floats of one transposed write (columns 16 apart in steps of 4 lanes, rows q = 0..15) fall on 64 different
-    // banks; with consecutive chunks they fell on 16, four lanes deep.
+    constexpr int W_CHUNKS = R * N / 4, W_UNITS = KS / 2 * TN, NWAVES = NTHREADS / 64;
+    constexpr int W_IT = W_NMAJOR ? 2 * ((W_UNITS + NWAVES - 1) / NWAVES) : (W_CHUNKS + NTHREADS - 1) / NTHREADS;
+    // Which 16-byte chunk a thread takes.  [N][R]: consecutive threads, consecutive chunks.  [R][N]: a wavefront takes 32 reduction
+    // rows x 16 columns per two loads, lanes 4 q .. 4 q + 3 the four chunks of rows 2 q and 2 q + 1, whose pieces go to LDS in pairs;
+    // the 64 pairs of one write (columns 16 apart in steps of 4 lanes) fall on 64 different banks.
     auto w_chunk = [&](int i) -> int {
         if constexpr (!W_NMAJOR) {
             const int c = tid + i * NTHREADS;
             return c < W_CHUNKS ? c : -1;
         } else {
-            const int u = wave + i * (NTHREADS / 64);                       // (16-row block, 16-column group) of this load
-            if ((KS * TN) % (NTHREADS / 64) != 0 && u >= KS * TN) return -1;
-            const int r = (u / TN) * 16 + (lane >> 2), n4 = (u % TN) * 4 + (lane & 3);
-            return r * (N / 4) + n4;
+            const int u = wave + (i >> 1) * NWAVES;                         // (32-row block, 16-column group) of these two loads
+            if (W_UNITS % NWAVES != 0 && u >= W_UNITS) return -1;
+            return ((u / TN) * 32 + (lane >> 2) * 2 + (i & 1)) * (N / 4) + (u % TN) * 4 + (lane & 3);
         }
     };
     u32x4 wv[W_IT];
@@ -101,17 +104,26 @@ __global__ __launch_bounds__(64 * (16 / TQ)) void rows_small_f32_kernel(SmallRow
 #pragma unroll
     for (int s = 0; s < KS; ++s) xr[0][s] = *reinterpret_cast<const u32x4 *>(p.A + xo[0] + s * 64);
     __builtin_amdgcn_sched_barrier(0);
+    // reduction step k of a column: 32-step block, its lane group, which of its two sixteens
+    auto w_at = [](int n, int k) -> int { return n * COL + (k >> 5) * 64 + ((k >> 2) & 3) * 16 + ((k >> 4) & 1) * 8 + (k & 3) * 2; };
 #pragma unroll
-    for (int i = 0; i < W_IT; ++i) {
+    for (int i = 0; i < W_IT; i += W_NMAJOR ? 2 : 1) {
         const int c = w_chunk(i);
-        if (W_CHUNKS % NTHREADS == 0 || c >= 0) {
-            if constexpr (!W_NMAJOR) {      // stored [N][R]: rows copied as they are
-                const int n = c / (R / 4), k4 = c - n * (R / 4);
-                *reinterpret_cast<u32x4 *>(w_lds + n * LDW + 4 * k4) = wv[i];
-            } else {                        // stored [R][N]: four columns of one reduction row per thread, written transposed
-                const int r = c / (N / 4), n4 = c - r * (N / 4);
+        if (c < 0) continue;
+        if constexpr (!W_NMAJOR) {
+            const int n = c / (R / 4), k4 = c - n * (R / 4);
+            u32x2 piece[3];
+            split_chunk(wv[i], piece);
 #pragma unroll
-                for (int x = 0; x < 4; ++x) w_lds[(4 * n4 + x) * LDW + r] = bits_f32(wv[i][x]);
+            for (int x = 0; x < 3; ++x) *reinterpret_cast<u32x2 *>(w_lds + x * PLANE + w_at(n, 4 * k4)) = piece[x];
+        } else {
+            const int r = c / (N / 4), n4 = c - r * (N / 4);                // an even row and the next, four columns
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+                uint32_t piece[3];
+                split_pair(bits_f32(wv[i][y]), bits_f32(wv[i + 1][y]), piece);
+#pragma unroll
+                for (int x = 0; x < 3; ++x) *reinterpret_cast<uint32_t *>(w_lds + x * PLANE + w_at(4 * n4 + y, r)) = piece[x];
             }
         }
     }
@@ -127,7 +139,7 @@ __global__ __launch_bounds__(64 * (16 / TQ)) void rows_small_f32_kernel(SmallRow
     // instructions of the next instead of all at the kernel's end - as long as a tile alone keeps four accumulators
     // busy (consecutive matrix instructions on one accumulator would wait for each other); narrower outputs take the
     // row tiles of the wavefront together (TG = TQ).
-    constexpr int TG = TN >= 4 ? 1 : TQ;
+    constexpr int TG = TN >= 3 ? 1 : TQ;
 #pragma unroll
     for (int t0 = 0; t0 < TQ; t0 += TG) {
         f32x4 acc[TG][TN];
@@ -136,23 +148,54 @@ __global__ __launch_bounds__(64 * (16 / TQ)) void rows_small_f32_kernel(SmallRow
 #pragma unroll
             for (int tn = 0; tn < TN; ++tn) acc[t][tn] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            u32x4 xf[TG];
+        for (int s = 0; s < KS; s += 2) {
+            u32x4 xf[TG][3];
 #pragma unroll
-            for (int t = 0; t < TG; ++t) xf[t] = lanes_4a_g_to_16g_a(xr[t0 + t][s], lane);
-            // lane (a, g): weights of column 16 tn + a at reduction 16 s + 4 g .. + 3
-            u32x4 wf[TN];
+            for (int t = 0; t < TG; ++t) {
+                u32x2 lo[3], hi[3];
+                split_chunk(lanes_4a_g_to_16g_a(xr[t0 + t][s], lane), lo);
+                split_chunk(lanes_4a_g_to_16g_a(xr[t0 + t][s + 1], lane), hi);
 #pragma unroll
-            for (int tn = 0; tn < TN; ++tn) wf[tn] = *reinterpret_cast<const u32x4 *>(w_lds + (tn * 16 + a) * LDW + s * 16 + g * 4);
-            // the four reduction elements of a lane outermost: consecutive matrix instructions then go to different
-            // accumulators and none waits for the one before it
+                for (int x = 0; x < 3; ++x) xf[t][x] = u32x4{lo[x][0], lo[x][1], hi[x][0], hi[x][1]};
+            }
+            u32x4 wf[TN][3];
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
+            for (int x = 0; x < 3; ++x)
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn)
+                    wf[tn][x] = *reinterpret_cast<const u32x4 *>(w_lds + x * PLANE + (tn * 16 + a) * COL + s * 32 + g * 16);
+            // piece by piece over all accumulators: consecutive matrix instructions then go to different ones
+#pragma unroll
+            for (int c = 0; c < 6; ++c)
 #pragma unroll
                 for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-                    for (int t = 0; t < TG; ++t)
-                        acc[t][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(bits_f32(wf[tn][c]), bits_f32(xf[t][c]), acc[t][tn], 0, 0, 0);
+                    for (int t = 0; t < TG; ++t) mma_chunk<ElemBF16>(acc[t][tn], wf[tn][kSplitP[c]], xf[t][kSplitQ[c]]);
+        }
+        // not all finite: these row tiles again, by the fp32 instruction, weights straight from memory
+        const float odd = not_finite(acc);
+        if (__any(odd != 0.f || odd != odd)) {
+#pragma unroll
+            for (int t = 0; t < TG; ++t)
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn) acc[t][tn] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+#pragma unroll
+                for (int t = 0; t < TG; ++t) {
+                    const u32x4 x = lanes_4a_g_to_16g_a(xr[t0 + t][s], lane);
+#pragma unroll 1
+                    for (int c = 0; c < 4; ++c) {
+                        const float xc = bits_f32(c == 0 ? x[0] : c == 1 ? x[1] : c == 2 ? x[2] : x[3]);
+                        const int k = s * 16 + g * 4 + c;
+#pragma unroll
+                        for (int tn = 0; tn < TN; ++tn) {
+                            const int n = tn * 16 + a;
+                            const float w = *reinterpret_cast<const float *>(We + (W_NMAJOR ? k * N + n : n * R + k) * 4);
+                            acc[t][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, xc, acc[t][tn], 0, 0, 0);
+                        }
+                    }
+                }
         }
         // lane (a, g) holds, for pick 16 tq + a, columns 16 tn + 4 g .. + 3: the four lanes g of a pick write 64 contiguous bytes
 #pragma unroll

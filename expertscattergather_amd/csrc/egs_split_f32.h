@@ -1,51 +1,9 @@
-// fp32 products on the bf16 matrix instruction.
-//
-// An fp32 value is the sum of three bf16 values exactly: h = bf16(x), m = bf16(x - h), l = x - h - m (8 bits of the 24 each; the
-// subtractions are exact).  Of the nine products of two such sums six are taken, the smallest first,
-//   x y = lh + hl + mm + mh + hm + hh   (the others are below 2^-25 of it),
-// each exact in the fp32 accumulator's input, so that what is rounded is the accumulator, as with the fp32 matrix instruction -
-// fewer times: 16x16x32 adds 32 products at a time where 16x16x4 adds four.  Measured against 64 bits, 64 problems of N(0,1) data:
-// reduction 32 3.8e-8 (the fp32 instruction 1.0e-7), 64 0.94e-7 (1.44e-7), 128 1.5e-7 (2.0e-7), 1024 4.9e-7 (5.7e-7), 4096 1.00e-6
-// (1.14e-6) of the result's root mean square.  Six instructions of 16 cycles stand for eight of 32, and at a higher clock:
-// 358 TFLOP/s of fp32 work against 138 (an instruction-only loop over all CUs).
-//
-// Limits: the pieces of a value below 2^-109 fall below bf16's smallest number, which leaves them with an absolute error of up to 2^-134.
-// An infinity has no such pieces (inf - inf), nor has a value that rounds up to one in bf16 (above 3.39e38): such products
-// arrive as NaN or infinity, so a wavefront whose results are not all finite takes its tile again with the fp32 instruction.
+// The fp32 weight gradient on the bf16 matrix instruction (egs_split.h says how).
 #pragma once
+#include "egs_split.h"
 #include "egs_tiled.h"
 
 namespace egs {
-
-// the three pieces of two floats, packed in pairs
-__device__ __forceinline__ void split_pair(float x, float y, uint32_t (&piece)[3])
-{
-    piece[0] = pack2<ElemBF16>(x, y);
-    const float rx = x - bits_f32(piece[0] << 16), ry = y - bits_f32(piece[0] & 0xffff0000u);
-    piece[1] = pack2<ElemBF16>(rx, ry);
-    piece[2] = pack2<ElemBF16>(rx - bits_f32(piece[1] << 16), ry - bits_f32(piece[1] & 0xffff0000u));
-}
-// ... and of four
-__device__ __forceinline__ void split_chunk(const u32x4 &v, u32x2 (&piece)[3])
-{
-    uint32_t lo[3], hi[3];
-    split_pair(bits_f32(v[0]), bits_f32(v[1]), lo);
-    split_pair(bits_f32(v[2]), bits_f32(v[3]), hi);
-#pragma unroll
-    for (int x = 0; x < 3; ++x) piece[x] = u32x2{lo[x], hi[x]};
-}
-// 0 if every element is finite, else NaN
-template <int M, int N> __device__ __forceinline__ float not_finite(const f32x4 (&acc)[M][N])
-{
-    float t = 0.f;
-#pragma unroll
-    for (int i = 0; i < M; ++i)
-#pragma unroll
-        for (int j = 0; j < N; ++j)
-#pragma unroll
-            for (int x = 0; x < 4; ++x) t = fmaf(acc[i][j][x], 0.f, t);
-    return t;
-}
 
 // ------------------------------------------------------------------------------ weight gradient
 // LDS: three planes of 32 picks x 64 columns of both operands, 32-byte units XOR-swizzled by bits 1 and 3 of
@@ -166,13 +124,12 @@ static __global__ __launch_bounds__(kThreads, 3) void tiled_dw_split_kernel(Tile
     };
     // Piece by piece over all accumulators, the smallest first; `between(t)` is issued behind the matrix instructions of product t < 6.
     auto multiply = [&](auto between) {
-        constexpr int P[6] = {2, 0, 1, 1, 0, 0}, Q[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
         for (int t = 0; t < 6; ++t) {
 #pragma unroll
             for (int x = 0; x < 2; ++x)
 #pragma unroll
-                for (int y = 0; y < 2; ++y) mma_chunk<ElemBF16>(acc[x][y], yf[y][P[t]], xf[x][Q[t]]);
+                for (int y = 0; y < 2; ++y) mma_chunk<ElemBF16>(acc[x][y], yf[y][kSplitP[t]], xf[x][kSplitQ[t]]);
             between(t);
             __builtin_amdgcn_sched_barrier(0);
         }
