@@ -9,22 +9,21 @@ namespace host {
 
 namespace {
 
-template <class TT, int TP>
-int launch_dw_strip(const DwDlParams &q, int grid, hipStream_t s)
+template <class TT, int TP, int BQ>
+int launch_dw_strip_one(const DwDlParams &q, int grid, hipStream_t s)
 {
     static LdsGrant told;
-    const int rc = allow_large_lds((const void *)dw_strip_kernel<TT, TP>, told, DwStrip<TP>::BYTES, "hipFuncSetAttribute(dw_strip_kernel)");
+    const int rc = allow_large_lds((const void *)dw_strip_kernel<TT, TP, BQ>, told, DwStrip<TP, BQ>::BYTES, "hipFuncSetAttribute(dw_strip_kernel)");
     if (rc != EGS_OK) return rc;
-    hipLaunchKernelGGL((dw_strip_kernel<TT, TP>), dim3((unsigned)grid), dim3(kDlThreads), DwStrip<TP>::BYTES, s, q);
+    hipLaunchKernelGGL((dw_strip_kernel<TT, TP, BQ>), dim3((unsigned)grid), dim3(kDlThreads), (DwStrip<TP, BQ>::BYTES), s, q);
+    EGS_CHECK_LAUNCH("dw_strip_kernel");
     return EGS_OK;
 }
 template <class TT>
-int launch_dw_strip(const DwDlParams &q, int tp, int grid, hipStream_t s)
+int launch_dw_strip(const DwDlParams &q, int tp, int bq, int grid, hipStream_t s)
 {
-    const int rc = tp == 2 ? launch_dw_strip<TT, 2>(q, grid, s) : tp == 3 ? launch_dw_strip<TT, 3>(q, grid, s) : launch_dw_strip<TT, 4>(q, grid, s);
-    if (rc != EGS_OK) return rc;
-    EGS_CHECK_LAUNCH("dw_strip_kernel");
-    return EGS_OK;
+    return bq == 128 ? launch_dw_strip_one<TT, 4, 128>(q, grid, s) : tp == 2 ? launch_dw_strip_one<TT, 2, 64>(q, grid, s)
+         : tp == 3 ? launch_dw_strip_one<TT, 3, 64>(q, grid, s) : launch_dw_strip_one<TT, 4, 64>(q, grid, s);
 }
 
 }  // namespace
@@ -51,12 +50,14 @@ int dw_general(const void *Xs, const void *Ys, const void *Ind, void *dW, void *
         q.d = p;
         q.d.i_tiles = pl.b_i_tiles; q.d.j_tiles = pl.b_j_tiles; q.d.S = pl.b_S; q.d.rows_per_split = pl.b_rows_per_split;
         q.x_bytes = (uint32_t)x_span; q.y_bytes = (uint32_t)y_span;
-        const int64_t grid = (int64_t)8 * ceil_div(d->E, 8) * pl.b_i_tiles * pl.b_j_tiles * pl.b_S;
+        const int64_t per_e = (int64_t)pl.b_i_tiles * pl.b_j_tiles * pl.b_S;
+        const int64_t grid = pl.b_tp != 0 ? (d->E * per_e + 7) / 8 * 8 : 8 * ceil_div(d->E, 8) * per_e;
         if (grid > INT32_MAX) return EGS_ERR_BAD_SHAPE;
         // 128-column tiles: three 48 KB stages of 64 rows (C4: 42.2 -> 37.9 us per weight gradient with its sum over
         // splits); 256-column tiles: four 32 KB stages of 32 rows (C3: 178 -> 174 us)
-        if (pl.b_bq == 64) {
-            const int rc = act_dtype == EGS_F16 ? launch_dw_strip<ElemF16>(q, pl.b_tp, (int)grid, s) : launch_dw_strip<ElemBF16>(q, pl.b_tp, (int)grid, s);
+        if (pl.b_tp != 0) {
+            const int rc = act_dtype == EGS_F16 ? launch_dw_strip<ElemF16>(q, pl.b_tp, pl.b_bq, (int)grid, s)
+                                                : launch_dw_strip<ElemBF16>(q, pl.b_tp, pl.b_bq, (int)grid, s);
             if (rc != EGS_OK) return rc;
         } else if (act_dtype == EGS_F16) {
             if (pl.b_bq == 256) hipLaunchKernelGGL((dw_dl_kernel<ElemF16, 256, 4, 32>), dim3((unsigned)grid), dim3(kDlThreads), 0, s, q);
@@ -65,7 +66,7 @@ int dw_general(const void *Xs, const void *Ys, const void *Ind, void *dW, void *
             if (pl.b_bq == 256) hipLaunchKernelGGL((dw_dl_kernel<ElemBF16, 256, 4, 32>), dim3((unsigned)grid), dim3(kDlThreads), 0, s, q);
             else hipLaunchKernelGGL((dw_dl_kernel<ElemBF16, 128, 3>), dim3((unsigned)grid), dim3(kDlThreads), 0, s, q);
         }
-        if (pl.b_bq != 64) EGS_CHECK_LAUNCH("dw_dl_kernel");
+        if (pl.b_tp == 0) EGS_CHECK_LAUNCH("dw_dl_kernel");
         if (pl.b_S > 1) {       // partials are in the output's layout, I % 8 == 0 and J % 8 == 0: vectorised plain sum
             hipLaunchKernelGGL(dw_reduce4_kernel, dim3(grid_1d(w_elems / 4, 4096)), dim3(kThreads), 0, s,
                                (const float *)workspace, (char *)dW, pl.b_S, w_elems / 4, out_dtype);

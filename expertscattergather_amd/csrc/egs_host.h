@@ -82,8 +82,8 @@ struct DwPlan {
     bool small_ok;                                          // shape admits the small-expert kernel
     int s_i_tiles, s_j_tiles, s_S, s_rows_per_split;        // its plan
     bool big_ok;                                            // shape admits the direct-to-LDS kernel (256 x BQ tiles)
-    int b_bq, b_i_tiles, b_j_tiles, b_S, b_rows_per_split;  // its plan; b_bq 64: dw_strip_kernel, tiles of 32 b_tp x 64
-    int b_tp;
+    int b_bq, b_i_tiles, b_j_tiles, b_S, b_rows_per_split;  // its plan
+    int b_tp;                                               // not 0: dw_strip_kernel, tiles of 32 b_tp x b_bq
     bool wide;                                              // tiled_dw_wide_kernel, in one pass
     bool split32;                                           // fp32: tiled_dw_split_kernel, 64 x 64 tiles
     size_t bytes_general, bytes_small, bytes_big;           // workspace of each of the three split kernels (0: no splits)

@@ -162,39 +162,61 @@ int64_t dw_split32_slabs(const egs_dims *d)
     return (int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, 64) * (((int64_t)d->B * d->K + 31) / 32);
 }
 
-// 16-bit, up to 64 output columns: dw_strip_kernel (tp: tiles of 32 tp x 64, S splits of the picks) where it is expected to beat what there
-// is else.  Both sides are a number of rounds of workgroups over the CUs, each some us and some more for every 1000 picks, fitted to times
-// alone on the device (us, strips / 32 x 64 or 32 x 32 tiles): B64 T256 E32 K32 I768 J64 18.8 / 28.4, B2 T1000 E60 K200 I640 J48 12 / 20,
-// B8 T4096 E128 K256 I1024 J64 95 / 147, B100 T500 E6 K100 I448 J64 28 / 33, B20 T900 E14 K64 I1024 J32 10.4 / 11.6, B7 T500 E80 K64 I192
-// J64 5.6 / 9.2; not taken: B33 T300 E16 K64 I288 J64 12.2 / 11.1, I256 J64 at E32 and 2048 picks 13.2 / 10.0, B40 T400 E16 K40 I640 J24
-// 11.8 / 11.3, B1 T2000 E8 K250 I256 J64 4.7 / 3.7.  Where those tiles are not taken the general ones always lose: B3 T120 E5 K90 I200 J56
-// 4.3 / 8.6, B17 T2218 E4 K63 I224 J32 9.3 / 13.2, B2 T300 E100 K100 I160 J32 5.4 / 10.4, B30 T200 E4 K20 I136 J24 5.6 / 9.3.
-struct DwStripPlan { int tp, S, rows_per_split; };
+// 16-bit weight gradients in strips: the tile (32 tp x bq) and the number of splits of the picks that dw_strip_kernel is expected to be
+// the fastest with, and the us that takes: rounds of workgroups over the CUs, each some us and some more for every 1000 picks, fitted to
+// times alone on the device.
+struct DwStripPlan { int tp, bq, S, rows_per_split; double us; };
 
-bool dw_strip_takes(const egs_dims *d, int act_dtype, DwStripPlan *plan = nullptr)
+DwStripPlan dw_strip_plan(const egs_dims *d)
+{
+    struct Width { int tp, bq; double start, per_pick; };
+    static constexpr Width widths[] = {{2, 64, 2.4, 5.8e-3}, {3, 64, 3.0, 7.3e-3}, {4, 64, 2.6, 10.0e-3}, {4, 128, 4.5, 11.7e-3}};
+    constexpr double second_pass = 4.0, per_sum = 2e-6;
+    const int64_t Me = (int64_t)d->B * d->K;
+    DwStripPlan best = {0, 0, 0, 0, 0.0};
+    for (const Width &w : widths) {
+        if (w.bq == 128 && d->J <= 64) continue;
+        const int64_t tiles = (int64_t)d->E * ceil_div(d->I, 32 * w.tp) * ceil_div(d->J, w.bq), most = tiles < 256 ? 256 / tiles : 1;
+        for (int64_t n = 1; n <= most; n += most > 1 ? most - 1 : 1) {
+            const int64_t rows = ((Me + n - 1) / n + 127) / 128 * 128, S = (Me + rows - 1) / rows;
+            const double us = (double)((tiles * S + 255) / 256) * (w.start + (double)rows * w.per_pick) +
+                              (S > 1 ? second_pass + (double)S * d->E * d->I * d->J * per_sum : 0.0);
+            if (best.tp == 0 || us < best.us) best = {w.tp, w.bq, (int)S, (int)(rows < INT32_MAX ? rows : INT32_MAX), us};
+        }
+    }
+    return best;
+}
+
+// Up to 64 output columns, against the 32 x 64 and 32 x 32 tiles of make_dw_tile, modelled the same way.  us, strips / those: B64 T256 E32 K32
+// I768 J64 18.8 / 28.4, B2 T1000 E60 K200 I640 J48 12 / 20, B8 T4096 E128 K256 I1024 J64 95 / 147, B100 T500 E6 K100 I448 J64 18 / 33, B20
+// T900 E14 K64 I1024 J32 10.4 / 11.6, B7 T500 E80 K64 I192 J64 5.6 / 9.2; not taken: I256 J64 at E32 and 2048 picks 13.2 / 10.0, B40 T400
+// E16 K40 I640 J24 11.8 / 11.3, B1 T2000 E8 K250 I256 J64 4.7 / 3.7.  Where those are not taken the general tiles always lose: B3 T120 E5
+// K90 I200 J56 4.3 / 8.6, B17 T2218 E4 K63 I224 J32 9.3 / 13.2, B2 T300 E100 K100 I160 J32 5.4 / 10.4, B30 T200 E4 K20 I136 J24 5.6 / 9.3.
+bool dw_strip_narrow(const egs_dims *d, int act_dtype)
 {
     const int64_t Me = (int64_t)d->B * d->K;
     if (act_dtype == EGS_F32 || d->I % 8 || d->J % 8 || d->I <= 128 || d->J > 64 || d->J < 8 || Me < 128 || d->E == 0) return false;
-    constexpr double start[] = {2.4, 3.0, 2.6}, per_pick[] = {5.8e-3, 7.3e-3, 10.3e-3}, second_pass = 4.0;
-    DwStripPlan best = {0, 0, 0};
-    double least = 0;
-    for (int tp = 2; tp <= 4; ++tp) {
-        const int64_t tiles = (int64_t)d->E * ceil_div(d->I, 32 * tp), most = tiles < 256 ? 256 / tiles : 1;
-        for (int64_t n = 1; n <= most; n += most > 1 ? most - 1 : 1) {
-            const int64_t rows = ((Me + n - 1) / n + 127) / 128 * 128, S = (Me + rows - 1) / rows;
-            const double us = (double)((tiles * S + 255) / 256) * (start[tp - 2] + (double)rows * per_pick[tp - 2]) +
-                              (S > 1 ? second_pass + (double)S * d->E * d->I * d->J * 2e-6 : 0.0);
-            if (best.tp != 0 && us >= least) continue;
-            least = us;
-            best = {tp, (int)S, (int)(rows < INT32_MAX ? rows : INT32_MAX)};
-        }
-    }
-    if (plan != nullptr) *plan = best;
     const int64_t narrow = (int64_t)d->E * ceil_div(d->I, 32) * ceil_div(d->J, 32), wide = (int64_t)d->E * ceil_div(d->I, 32);
     if (narrow < 128 || d->I > 2048 || dw_few_picks(d, act_dtype)) return true;         // make_dw_tile refuses these
     const double tile = d->J > 32 && (narrow > 256 || Me >= 4096) ? (double)((wide + 255) / 256) * (2.9 + (double)Me * 3.0e-3)
                                                                   : (double)((narrow + 511) / 512) * (2.9 + (double)Me * 5.0e-3);
-    return least < 0.95 * tile;
+    return dw_strip_plan(d).us < 0.95 * tile;
+}
+
+// More columns, against the 256-row tiles of dw_dl_kernel and their sum over splits (an XCD takes whole experts there).  us, strips / those:
+// B6 T1100 E20 K150 I328 J136 10.1 / 24.2, B16 T1024 E64 K128 I512 J128 30 / 37, B12 T1000 E5 K100 I1000 J256 12 / 26, B8 T1024 E16 K128
+// I512 J256 13 / 30, B40 T300 E40 K40 I256 J192 17 / 40, B3 T1000 E90 K250 I736 J200 64 / 83; not taken: B8 T4096 E128 K256 I1024 J256
+// 219 / 180.  (With fewer than 256 picks the general tiles are as fast: B1 T4000 E64 K250 I1024 J256 30.3 / 31.6, B1 T700 E120 K150 I384
+// J256 20.5 / 20.0.)  With up to 128 rows and more than 128 columns the general tiles are the alternative: B4 T500 E30 K100 I96 J192
+// 5.8 / 9.7, B20 T400 E12 K50 I64 J256 7.9 / 11.1, B30 T300 E40 K40 I32 J160 9.6 / 15.0, B6 T2000 E3 K200 I128 J224 10.0 / 11.6.
+bool dw_strip_broad(const egs_dims *d, int act_dtype, const DwPlan &pl, const DwStripPlan &strip)
+{
+    if (act_dtype == EGS_F32 || d->I % 8 || d->J % 8 || d->J <= 64 || d->I < 32 || d->E == 0) return false;
+    if (!pl.big_ok) return d->I <= 128 && d->J > 128 && (int64_t)d->B * d->K >= 128;
+    const int64_t on_xcd = (int64_t)ceil_div(d->E, 8) * pl.b_i_tiles * pl.b_j_tiles * pl.b_S;
+    const double per_round = pl.b_bq == 256 ? 9.5 + pl.b_rows_per_split * 39e-3 : 7.0 + pl.b_rows_per_split * 20e-3;
+    const double us = (double)((on_xcd + 31) / 32) * per_round + (pl.b_S > 1 ? 3.5 + (double)pl.b_S * d->E * d->I * d->J * 0.45e-6 : 0.0);
+    return strip.us < 0.95 * us;
 }
 
 DwPlan plan_dw(const egs_dims *d, int act_dtype)
@@ -245,16 +267,18 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
         pl.bytes_big = s3 > 1 ? align_up((size_t)s3 * d->E * d->I * d->J * 4, 256) : 0;
     }
 
-    DwStripPlan strip;
-    if (dw_strip_takes(d, act_dtype, &strip)) {
+    const DwStripPlan strip = Me >= 128 && act_dtype != EGS_F32 && d->E > 0 && d->I > 0 && d->J > 0 ? dw_strip_plan(d) : DwStripPlan{};
+    if (dw_strip_narrow(d, act_dtype) || (strip.tp != 0 && dw_strip_broad(d, act_dtype, pl, strip))) {
         pl.big_ok = true;
-        pl.b_bq = 64;
+        pl.b_bq = strip.bq;
         pl.b_tp = strip.tp;
         pl.b_i_tiles = ceil_div(d->I, 32 * strip.tp);
-        pl.b_j_tiles = 1;
+        pl.b_j_tiles = ceil_div(d->J, strip.bq);
         pl.b_S = strip.S;
         pl.b_rows_per_split = strip.rows_per_split;
-        pl.bytes_big = strip.S > 1 ? align_up((size_t)strip.S * d->E * d->I * d->J * 4, 256) : 0;
+        // never less than the 256-row tiles ask for: which sizes fit a scratch of a given size does not depend on the choice between the two
+        const size_t bytes = strip.S > 1 ? align_up((size_t)strip.S * d->E * d->I * d->J * 4, 256) : 0;
+        if (bytes > pl.bytes_big) pl.bytes_big = bytes;
     }
 
     // small experts: 64 x 64 tiles, up to 1024 picks per workgroup, enough workgroups to cover the device
@@ -415,7 +439,7 @@ bool make_dw_tile(const void *Xs, const void *Ys, const void *Ind, void *dW, con
     if (g_force_generic) return false;
     const int ES = elem_size(act_dtype);
     if (ES == 4 && d->I > 32 && d->J > 32 && dw_split32_slabs(d) >= 8192) return false;
-    if (dw_strip_takes(d, act_dtype)) return false;
+    if (dw_strip_narrow(d, act_dtype)) return false;
     if (d->I % 8 || d->J % 8 || d->I < 8 || d->J < 8 || d->I > 2048 || d->J > 128) return false;
     const int64_t Me = (int64_t)d->B * d->K;
     if (Me == 0 || d->E == 0 || d->T == 0) return false;

@@ -21,6 +21,9 @@ from expertscattergather_amd import hip_kernels as hk
     (41, 64, 64, 50, 384, 64),      # 96 columns, a second table of offsets two picks long
     (17, 140, 64, 130, 488, 64),    # four tiles of 128 columns, the last of 104; three tables of offsets
     (40, 100, 2, 100, 264, 64),     # splits
+    (6, 200, 20, 150, 328, 136),    # 96 columns by three column tiles, the last of eight
+    (18, 80, 60, 115, 512, 120),    # 128 by 128, ragged; slabs of 64, a second table of offsets 22 picks long
+    (5, 300, 3, 200, 120, 200),     # few rows; splits
 ], ids=lambda s: "x".join(map(str, s)))
 def test_strips_match_the_oracle(shape, dtype):
     B, T, E, K, I, J = shape
