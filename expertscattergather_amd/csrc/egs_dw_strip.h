@@ -27,14 +27,6 @@ template <int TP, int BQ_> struct DwStrip {
     static constexpr int ROWS = STAGE > 40 * 1024 ? 1024 : 2048;    // picks whose offsets are in LDS at a time
     static constexpr int BYTES = NST * STAGE + 8 * ROWS;
     static_assert(BYTES <= 160 * 1024, "LDS of a CU");
-    // XORed into the number of a row's 32-byte unit, so that the 16 rows of a transpose read fall two deep on every bank.  Rows of
-    // 192 bytes are on different banks four by four; four lane groups, eight rows apart, are not.
-    template <int COLS> static __device__ __forceinline__ int key(int row)
-    {
-        return COLS == 128 ? tr_swizzle(row) : COLS == 96 ? (row >> 3) & 1 : (row & 3) ^ ((row >> 3) & 3);
-    }
-    static __device__ __forceinline__ int p_key(int row) { return key<BP>(row); }
-    static __device__ __forceinline__ int q_key(int row) { return key<BQ>(row); }
 };
 
 template <class TT, int TP, int BQ>
@@ -65,14 +57,14 @@ __global__ __launch_bounds__(kDlThreads) void dw_strip_kernel(DwDlParams pp)
 #pragma unroll
     for (int jj = 0; jj < PL; ++jj) {
         const int at = (wave * PL + jj) * 64 + lane, row = at / PCR, pc = at - row * PCR;
-        const int col = i0 + ((((pc >> 1) ^ L::p_key(row)) << 1) | (pc & 1)) * 8;
+        const int col = i0 + ((((pc >> 1) ^ tr_key<L::BP>(row)) << 1) | (pc & 1)) * 8;
         p_row[jj] = row;
         p_col[jj] = col < p.I ? (uint32_t)col * 2u : kVoffInvalid;
     }
 #pragma unroll
     for (int jj = 0; jj < QL; ++jj) {
         const int at = (wave * QL + jj) * 64 + lane, row = at / QCR, pc = at - row * QCR;
-        const int col = j0 + ((((pc >> 1) ^ L::q_key(row)) << 1) | (pc & 1)) * 8;
+        const int col = j0 + ((((pc >> 1) ^ tr_key<BQ>(row)) << 1) | (pc & 1)) * 8;
         q_row[jj] = row;
         q_col[jj] = col < p.J ? (uint32_t)col * 2u : kVoffInvalid;
     }
@@ -98,9 +90,9 @@ __global__ __launch_bounds__(kDlThreads) void dw_strip_kernel(DwDlParams pp)
     for (int h = 0; h < 2; ++h) {
         const int row = half * (L::SLAB / 2) + g * 8 + h * 4 + (a >> 2);
 #pragma unroll
-        for (int x = 0; x < TP; ++x) p_at[h][x] = row * (L::BP * 2) + (((wi * TP + x) ^ L::p_key(row)) << 5) + (a & 3) * 8;
+        for (int x = 0; x < TP; ++x) p_at[h][x] = row * (L::BP * 2) + (((wi * TP + x) ^ tr_key<L::BP>(row)) << 5) + (a & 3) * 8;
 #pragma unroll
-        for (int y = 0; y < NQ; ++y) q_at[h][y] = L::P_BYTES + row * (L::BQ * 2) + (((wj * NQ + y) ^ L::q_key(row)) << 5) + (a & 3) * 8;
+        for (int y = 0; y < NQ; ++y) q_at[h][y] = L::P_BYTES + row * (L::BQ * 2) + (((wj * NQ + y) ^ tr_key<BQ>(row)) << 5) + (a & 3) * 8;
     }
     f32x4 acc[TP][NQ];
 #pragma unroll

@@ -192,15 +192,19 @@ DwStripPlan dw_strip_plan(const egs_dims *d)
 // T900 E14 K64 I1024 J32 10.4 / 11.6, B7 T500 E80 K64 I192 J64 5.6 / 9.2; not taken: I256 J64 at E32 and 2048 picks 13.2 / 10.0, B40 T400
 // E16 K40 I640 J24 11.8 / 11.3, B1 T2000 E8 K250 I256 J64 4.7 / 3.7.  Where those are not taken the general tiles always lose: B3 T120 E5
 // K90 I200 J56 4.3 / 8.6, B17 T2218 E4 K63 I224 J32 9.3 / 13.2, B2 T300 E100 K100 I160 J32 5.4 / 10.4, B30 T200 E4 K20 I136 J24 5.6 / 9.3.
-bool dw_strip_narrow(const egs_dims *d, int act_dtype)
+bool dw_strip_narrow(const egs_dims *d, int act_dtype, DwStripPlan *plan = nullptr)
 {
     const int64_t Me = (int64_t)d->B * d->K;
     if (act_dtype == EGS_F32 || d->I % 8 || d->J % 8 || d->I <= 128 || d->J > 64 || d->J < 8 || Me < 128 || d->E == 0) return false;
     const int64_t narrow = (int64_t)d->E * ceil_div(d->I, 32) * ceil_div(d->J, 32), wide = (int64_t)d->E * ceil_div(d->I, 32);
-    if (narrow < 128 || d->I > 2048 || dw_few_picks(d, act_dtype)) return true;         // make_dw_tile refuses these
+    const bool alone = narrow < 128 || d->I > 2048 || dw_few_picks(d, act_dtype);       // make_dw_tile refuses these
+    if (alone && plan == nullptr) return true;
+    const DwStripPlan strip = dw_strip_plan(d);
+    if (plan != nullptr) *plan = strip;
+    if (alone) return true;
     const double tile = d->J > 32 && (narrow > 256 || Me >= 4096) ? (double)((wide + 255) / 256) * (2.9 + (double)Me * 3.0e-3)
                                                                   : (double)((narrow + 511) / 512) * (2.9 + (double)Me * 5.0e-3);
-    return dw_strip_plan(d).us < 0.95 * tile;
+    return strip.us < 0.95 * tile;
 }
 
 // More columns, against the 256-row tiles of dw_dl_kernel and their sum over splits (an XCD takes whole experts there).  us, strips / those:
@@ -209,10 +213,12 @@ bool dw_strip_narrow(const egs_dims *d, int act_dtype)
 // 219 / 180.  (With fewer than 256 picks the general tiles are as fast: B1 T4000 E64 K250 I1024 J256 30.3 / 31.6, B1 T700 E120 K150 I384
 // J256 20.5 / 20.0.)  With up to 128 rows and more than 128 columns the general tiles are the alternative: B4 T500 E30 K100 I96 J192
 // 5.8 / 9.7, B20 T400 E12 K50 I64 J256 7.9 / 11.1, B30 T300 E40 K40 I32 J160 9.6 / 15.0, B6 T2000 E3 K200 I128 J224 10.0 / 11.6.
-bool dw_strip_broad(const egs_dims *d, int act_dtype, const DwPlan &pl, const DwStripPlan &strip)
+bool dw_strip_broad(const egs_dims *d, int act_dtype, const DwPlan &pl, DwStripPlan &strip)
 {
     if (act_dtype == EGS_F32 || d->I % 8 || d->J % 8 || d->J <= 64 || d->I < 32 || d->E == 0) return false;
-    if (!pl.big_ok) return d->I <= 128 && d->J > 128 && (int64_t)d->B * d->K >= 128;
+    if (!pl.big_ok && (d->I > 128 || d->J <= 128 || (int64_t)d->B * d->K < 128)) return false;
+    strip = dw_strip_plan(d);
+    if (!pl.big_ok) return true;
     const int64_t on_xcd = (int64_t)ceil_div(d->E, 8) * pl.b_i_tiles * pl.b_j_tiles * pl.b_S;
     const double per_round = pl.b_bq == 256 ? 9.5 + pl.b_rows_per_split * 39e-3 : 7.0 + pl.b_rows_per_split * 20e-3;
     const double us = (double)((on_xcd + 31) / 32) * per_round + (pl.b_S > 1 ? 3.5 + (double)pl.b_S * d->E * d->I * d->J * 0.45e-6 : 0.0);
@@ -267,8 +273,8 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
         pl.bytes_big = s3 > 1 ? align_up((size_t)s3 * d->E * d->I * d->J * 4, 256) : 0;
     }
 
-    const DwStripPlan strip = Me >= 128 && act_dtype != EGS_F32 && d->E > 0 && d->I > 0 && d->J > 0 ? dw_strip_plan(d) : DwStripPlan{};
-    if (dw_strip_narrow(d, act_dtype) || (strip.tp != 0 && dw_strip_broad(d, act_dtype, pl, strip))) {
+    DwStripPlan strip;
+    if (dw_strip_narrow(d, act_dtype, &strip) || dw_strip_broad(d, act_dtype, pl, strip)) {
         pl.big_ok = true;
         pl.b_bq = strip.bq;
         pl.b_tp = strip.tp;

@@ -52,6 +52,13 @@ __host__ __device__ constexpr int dl_threads(int BM, int BN) { return (BM / 128)
 // swizzle of the [reduction][column] tile: 32-byte units of a row are XORed with bits {0,1,3} of
 // the row number, which spreads the 16 rows one transpose read touches over all banks
 __device__ __forceinline__ int tr_swizzle(int row) { return (row & 3) | (((row >> 3) & 1) << 2); }
+// the same for rows of COLS columns: XORed into the number of a row's 32-byte unit, so that the 16 rows of a transpose read fall two
+// deep on every bank.  Rows of 192 bytes are on different banks four by four; four lane groups, eight rows apart, are not.
+template <int COLS> __device__ __forceinline__ int tr_key(int row)
+{
+    static_assert(COLS == 64 || COLS == 96 || COLS == 128, "units of a row");
+    return COLS == 128 ? tr_swizzle(row) : COLS == 96 ? (row >> 3) & 1 : (row & 3) ^ ((row >> 3) & 3);
+}
 // swizzle key of the K-major tiles (XORed into the 16-byte chunk index of a row of CR chunks), chosen so
 // that the 16 lanes of one fragment read (16 consecutive rows) hit 16 different 16-byte bank groups.
 template <int CR> __device__ __forceinline__ int kmajor_key_rows(int row) { return CR == 8 ? (row & 7) : ((row >> 2) & 3); }

@@ -1,7 +1,8 @@
 // Launch side of the rows x weight products: rows_gemm_dl_kernel for large well-formed 16-bit shapes, rows_gemm_kernel for other
-// 16-bit shapes that fill its tiles, rows_atomic_f32_kernel for fp32 atomics on the output, else the tiled kernels of egs_tiled.h.
+// 16-bit shapes that fill its tiles, rows_strip_kernel for mid-sized ones, rows_atomic_f32_kernel for fp32 atomics on the output, else the tiled kernels of egs_tiled.h.
 #include "egs_host.h"
 #include "egs_rows_gemm_dl.h"
+#include "egs_rows_strip.h"
 
 namespace egs {
 namespace host {
@@ -24,6 +25,19 @@ int launch_rows_atomic(RowsGemmParams &p, hipStream_t s)
     return EGS_OK;
 }
 
+// Which operand to keep in one XCD's L2 (4 MB each), by the bytes that then come from beyond it.  Row tiles outermost: the source
+// once and the weights again for every row tile (for every XCD, if they fit).  Experts outermost: the weights once and a source
+// row for every pick.  us, row tiles / experts outermost: bf16 R672 N96 Me2262 E99 106 / 69, f16 R1744 N104 Me2380 E70 235 / 204,
+// f16 R896 N64 Me2405 E215 183 / 151; the other way bf16 R768 N64 Me2048 E32 18.5 / 19.7.  A source that fits is kept by either:
+// f16 R64 N256 Me13157 E29 132 / 121; and where the weights are the larger operand the count promises more than row tiles
+// outermost keep: f16 R1408 N32 Me140 E165 15.7 / 13.4.
+bool rows_outermost(const RowsGemmParams &p, int ES, int WES)
+{
+    const double fits = 3.5e6, x = (double)p.B * p.T * p.R * ES, w = (double)p.E * p.R * p.N * WES;
+    const double picked = (double)p.E * p.B * p.K * p.R * ES, row_tiles = ((double)p.B * p.K + 63) / 64;
+    return x > fits && x > w && (x < picked ? x : picked) + w * (w <= fits ? 8 : row_tiles) < 1.05 * (picked + w);
+}
+
 // anything the direct-to-LDS kernels do not take
 int launch_rows_tiled(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans, bool gather, int epi, hipStream_t s)
 {
@@ -38,17 +52,7 @@ int launch_rows_tiled(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans
     q.ldc = gather ? p.N : product_ld(p.N);
     q.ind_dtype = p.ind_dtype; q.gather = gather; q.out_f32 = epi == EPI_STORE_F32; q.act = p.act; q.bias = (const char *)p.bias;
     p.bias_done = p.bias != nullptr;
-    // Which operand to keep in one XCD's L2 (4 MB each), by the bytes that then come from beyond it.  Row tiles outermost: the source
-    // once and the weights again for every row tile (for every XCD, if they fit).  Experts outermost: the weights once and a source
-    // row for every pick.  us, row tiles / experts outermost: bf16 R672 N96 Me2262 E99 106 / 69, f16 R1744 N104 Me2380 E70 235 / 204,
-    // f16 R896 N64 Me2405 E215 183 / 151; the other way bf16 R768 N64 Me2048 E32 18.5 / 19.7.  A source that fits is kept by either:
-    // f16 R64 N256 Me13157 E29 132 / 121; and where the weights are the larger operand the count promises more than row tiles
-    // outermost keep: f16 R1408 N32 Me140 E165 15.7 / 13.4.
-    if (gather) {
-        const double fits = 3.5e6, x = (double)p.B * p.T * p.R * ES, w = (double)p.E * p.R * p.N * WES;
-        const double picked = (double)p.E * p.B * p.K * p.R * ES, row_tiles = ((double)p.B * p.K + 63) / 64;
-        q.rows_major = x > fits && x > w && (x < picked ? x : picked) + w * (w <= fits ? 8 : row_tiles) < 1.05 * (picked + w);
-    }
+    q.rows_major = gather && rows_outermost(p, ES, WES);
     if (fp8_w) return tiled_rows_fp8w(q, w_trans, s);
     return act_dtype == EGS_F32 ? tiled_rows_f32(q, w_trans, s) : act_dtype == EGS_F16 ? tiled_rows_f16(q, w_trans, s) : tiled_rows_bf16(q, w_trans, s);
 }
@@ -168,6 +172,50 @@ int launch_rows_16_w(RowsGemmParams &p, bool w_trans, bool &used, hipStream_t s)
     return w_trans ? launch_rows_16<TT, GATHER, true, EPI>(p, used, s) : launch_rows_16<TT, GATHER, false, EPI>(p, used, s);
 }
 
+template <class TT, bool W_TRANS>
+int launch_rows_strip(RowsStripParams &p, hipStream_t s)
+{
+    typedef RowsStripLds L;
+    p.m_tiles = ceil_div(p.B * p.K, L::BM);
+    p.n_tiles = ceil_div(p.N, L::BN);
+    const int64_t total = (int64_t)p.E * p.m_tiles * p.n_tiles;
+    if (total > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
+    static_assert(L::BYTES <= 64 * 1024, "no grant needed");
+    hipLaunchKernelGGL((rows_strip_kernel<TT, W_TRANS>), dim3((unsigned)(8 * ((total + 7) / 8))), dim3(kStripThreads), L::BYTES, s, p);
+    EGS_CHECK_LAUNCH("rows_strip_kernel");
+    return EGS_OK;
+}
+
+// Mid-sized 16-bit products; `used`: rows_strip_kernel takes this one.  Against tiled_rows_kernel, us, strips / that: R768 N64 Me2048 E32 13.8 /
+// 19.3, R328 N136 Me900 E20 10 / 14, R136 N328 13.3 to 16 / 17, R800 N64 Me1628 E34 17 / 22, R64 N576 Me2814 E14 18 to 19 / 25, R896 N128
+// Me232 E83 13.2 / 16.3, R192 N64 Me92 E65 5.0 / 5.7; not with few workgroups (R352 N64 Me252 E18: 36, 6.2 / 5.3) or half empty columns (R896
+// N32 Me119 E53 9.6 / 7.9, R288 N32 Me2080 E35 10.2 / 9.8), unless there are many (R800 N32 Me2146 E116: 1972, 42 / 47).
+int rows_strip(RowsGemmParams &p, int act_dtype, bool w_trans, bool gather, int epi, bool &used, hipStream_t s)
+{
+    used = false;
+    if (g_force_generic || act_dtype == EGS_F32 || !p.a_vec || !p.w_vec || p.a_bytes == 0 || !aligned_to(p.W, 16) || !aligned_to(p.C, 16) ||
+        p.R % 8 != 0 || p.N % 8 != 0 || (uint64_t)p.R * p.N * 2 >= (1ull << 31) || p.w_scale != nullptr)
+        return EGS_OK;
+    if (!gather && p.bias != nullptr) return EGS_OK;        // biased product rows: the general kernel's route is the one that is tested
+    const int64_t Me = (int64_t)p.B * p.K, strips = p.E * ((Me + 127) / 128) * ceil_div(p.N, 64);
+    const bool filled = (double)Me * p.N * p.E >= 0.6 * 128 * 64 * (double)strips;
+    if (strips < (filled ? 64 : 1500)) return EGS_OK;
+    RowsStripParams q;
+    memset(&q, 0, sizeof(q));
+    q.A = p.A; q.W = p.W; q.Ind = p.Ind; q.C = p.C; q.bias = (const char *)p.bias;
+    q.lda_b = p.lda_b; q.lda_t = p.lda_t; q.a_bytes = p.a_bytes;
+    q.B = p.B; q.T = p.T; q.E = p.E; q.K = p.K; q.R = p.R; q.N = p.N; q.ldc = gather ? p.N : product_ld(p.N);
+    q.ind_dtype = p.ind_dtype; q.gather = gather; q.out_f32 = epi == EPI_STORE_F32; q.act = p.act;
+    q.rows_major = gather && rows_outermost(p, 2, 2);
+    const int rc = act_dtype == EGS_BF16 ? (w_trans ? launch_rows_strip<ElemBF16, true>(q, s) : launch_rows_strip<ElemBF16, false>(q, s))
+                                         : (w_trans ? launch_rows_strip<ElemF16, true>(q, s) : launch_rows_strip<ElemF16, false>(q, s));
+    if (rc != EGS_OK) return rc;
+    p.csr_blocks = 0; p.csr_done = 0;
+    p.bias_done = p.bias != nullptr;
+    used = true;
+    return EGS_OK;
+}
+
 }  // namespace
 
 // `used`: rows_stream_kernel takes this product
@@ -177,12 +225,21 @@ int rows_gemm_gather(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans,
 {
     if (p.B * p.K == 0 || p.E == 0 || p.N == 0) return EGS_OK;
     bool used = false;
-    int rc = EGS_OK;
+    int rc = rows_stream(p, act_dtype, fp8_w, w_trans, true, EPI_STORE, used, s);      // (fewer rows than any other but the general kernel)
+    if (used || rc != EGS_OK) return rc;
+    // Too few 256-row tiles for the CUs: us, strips / the direct-to-LDS tiles, R1024 N256 Me1200 E5 (25 of 256 columns) 12 / 26, R512 N256 Me1024
+    // E16 (64) 11.7 / 18, R448 N128 Me600 E50 (150 of 128 columns) 10.8 / 15, R256 N256 Me1600 E20 (140) 15.0 / 15.0, R448 N128 Me936 E71 (284)
+    // 22 / 21
+    const int64_t dl_tiles = p.E * (((int64_t)p.B * p.K + 255) / 256) * ceil_div(p.N, p.N >= 192 ? 256 : 128);
+    if (!fp8_w && p.N > 64 && dl_tiles <= (p.N >= 192 ? 100 : 200)) {
+        rc = rows_strip(p, act_dtype, w_trans, true, EPI_STORE, used, s);
+        if (used || rc != EGS_OK) return rc;
+    }
     if (fp8_w) { if (w_trans) rc = launch_rows_dl<ElemBF16, 1, true, true, EPI_STORE>(p, used, s); }
     else if (act_dtype == EGS_F16) rc = launch_rows_16_w<ElemF16, true, EPI_STORE>(p, w_trans, used, s);
     else if (act_dtype == EGS_BF16) rc = launch_rows_16_w<ElemBF16, true, EPI_STORE>(p, w_trans, used, s);
     if (used || rc != EGS_OK) return rc;
-    rc = rows_stream(p, act_dtype, fp8_w, w_trans, true, EPI_STORE, used, s);
+    if (!fp8_w) rc = rows_strip(p, act_dtype, w_trans, true, EPI_STORE, used, s);
     if (used || rc != EGS_OK) return rc;
     return launch_rows_tiled(p, act_dtype, fp8_w, w_trans, true, EPI_STORE, s);
 }
@@ -200,6 +257,8 @@ int rows_gemm_scatter(RowsGemmParams &p, int act_dtype, bool w_trans, int epi, h
     if (used || rc != EGS_OK) return rc;
     p.csr_blocks = 0; p.csr_done = 0;
     rc = rows_stream(p, act_dtype, false, w_trans, false, epi, used, s);
+    if (used || rc != EGS_OK) return rc;
+    rc = rows_strip(p, act_dtype, w_trans, false, epi, used, s);
     if (used || rc != EGS_OK) return rc;
     return launch_rows_tiled(p, act_dtype, false, w_trans, false, epi, s);
 }
