@@ -132,10 +132,12 @@ int launch_token_sum(const void *rows, bool rows_f32, const void *Ind, int ind_d
     if (grid > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
     const size_t lds = token_sum_lds(p.N);
     const bool stream = rows_stream_by(d, (size_t)p.ldp * (rows_f32 ? 4 : 2));
+    const bool wave = p.tpr_log2 == 6;
 #define EGS_TOKSUM(TT, PT)                                                                                              \
     do {                                                                                                                \
-        if (stream) hipLaunchKernelGGL((token_sum_kernel<TT, PT, true>), dim3((unsigned)grid), dim3(kThreads), lds, s, p); \
-        else hipLaunchKernelGGL((token_sum_kernel<TT, PT>), dim3((unsigned)grid), dim3(kThreads), lds, s, p);           \
+        const auto kernel = wave ? (stream ? token_sum_kernel<TT, PT, true, true> : token_sum_kernel<TT, PT, true, false>)       \
+                                 : (stream ? token_sum_kernel<TT, PT, false, true> : token_sum_kernel<TT, PT, false, false>);    \
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kThreads), lds, s, p);                                    \
     } while (0)
     if (act_dtype == EGS_F32) EGS_TOKSUM(ElemF32, float);
     else if (act_dtype == EGS_F16) { if (rows_f32) EGS_TOKSUM(ElemF16, float); else EGS_TOKSUM(ElemF16, uint16_t); }

@@ -37,7 +37,8 @@ __host__ __device__ inline size_t token_sum_lds(int N)
 }
 
 // STREAM: as for segment_sum_body (B29 T216 E69 K40 I1280 J144, 410 MB of rows: the scatter 222 -> 194 us)
-template <class TT, class PT, bool STREAM = false>
+// WAVE: 2^tpr_log2 is 64.  (A kernel of its own: with both ways in one the other took 12.2 us instead of 11.1 at B53 T97 E29 K41 I111.)
+template <class TT, class PT, bool WAVE, bool STREAM>
 __global__ __launch_bounds__(kThreads) void token_sum_kernel(TokenSumParams p)
 {
     extern __shared__ __attribute__((aligned(16))) char smem_token_sum[];
@@ -190,6 +191,41 @@ __global__ __launch_bounds__(kThreads) void token_sum_kernel(TokenSumParams p)
             }
         }
     };
+    // Where a wavefront is a token's group it takes neighbouring tokens, whose picks follow one another, and has eight rows on their
+    // way, whichever they are for; token by token, of two or three rows each, it waited for memory once for every token.  us, fp32 rows:
+    // B5 T2250 E28 K24 I928 21.9 -> 14.7, B71 T1000 E12 K10 I160 23.6 -> 18.4, B62 T394 E31 K43 I386 37.5 -> 31.6, B4 T512 E256 K8 I2048
+    // 20.0 -> 15.7, B6 T1100 E20 K150 I328 14.4 -> 12.5.
+    const int lens = WAVE && lane < tb ? first[lane + 1] - first[lane] : 0;
+    if (WAVE && __ballot(lens > kTokenSumHot) == 0) {
+        const int each = (tb + groups - 1) / groups, tl1 = min(tb, (wave + 1) * each);
+        int tl = min(tb, wave * each);
+        const int ends = first[min(lane, kTokenSumTokens - 1) + 1];     // of token `lane`
+        int s = __builtin_amdgcn_readfirstlane(first[tl]);
+        const int end = __builtin_amdgcn_readfirstlane(first[tl1]);
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        int here = __builtin_amdgcn_readlane(ends, min(tl, kTokenSumTokens - 1));
+        auto next = [&]() {
+            store(tl, acc);
+            acc = f32x4{0.f, 0.f, 0.f, 0.f};
+            ++tl;
+            here = __builtin_amdgcn_readlane(ends, min(tl, kTokenSumTokens - 1));
+        };
+        constexpr int FB = 8;
+        for (; s < end; s += FB) {
+            const int q = order[min(s + (lane & (FB - 1)), end - 1)];
+            vec_t v[FB];
+#pragma unroll
+            for (int u = 0; u < FB; ++u) v[u] = row(__builtin_amdgcn_readlane(q, u));
+#pragma unroll
+            for (int u = 0; u < FB; ++u) {
+                if (s + u >= end) break;
+                while (s + u >= here) next();
+                add(acc, v[u]);
+            }
+        }
+        while (tl < tl1) next();
+        return;
+    }
     for (int tl = grp; tl < tb; tl += groups) {
         const int s0 = first[tl], s1 = first[tl + 1];
         if (groups > 1 && s1 - s0 > kTokenSumHot) continue;
