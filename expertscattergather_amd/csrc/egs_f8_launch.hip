@@ -26,6 +26,25 @@ F8Plan plan_f8(const egs_dims *d)
     return pl;
 }
 
+int64_t f8_grid(const egs_dims *d, int tile)
+{
+    return (int64_t)8 * ceil_div(d->E, 8) * ceil_div(d->B * d->K, tile) * ceil_div(d->J, tile);
+}
+
+// 256 x 256 tiles (one workgroup to a CU) or 128 x 128 (two, the same bits): whichever needs the fewer turns of the chip, a turn
+// of the large tiles taking as long as two of the small.  On a tie the large ones from a reduction of more than 1024 on, where
+// their half as many bytes from the L2 count.  Both measured, large then small, in us, as (rows of an expert, E, I, J):
+// (195, 22, 1280, 256) 27.0, 11.9; (391, 53, 640, 144) 21.7, 11.0; (32, 256, 2048, 512) 79.4, 53.6;
+// (1024, 48, 2048, 512) 86.0, 65.7; (1280, 64, 2048, 384) 120, 100; ties: (1024, 32, 4096, 512) 72.0, 91.2; (2048, 64, 2048, 512)
+// 173, 188; (2048, 128, 1024, 256) 119, 124; (1024, 64, 1024, 512) 58.3, 59.3; (2048, 64, 512, 512) 86.8, 79.4.
+bool f8_large_tiles(const egs_dims *d)
+{
+    const int64_t n256 = f8_grid(d, 256), n128 = f8_grid(d, 128);
+    if (n128 > INT32_MAX) return true;
+    const int64_t turns256 = 2 * ((n256 + 255) / 256), turns128 = (n128 + 511) / 512;
+    return turns256 < turns128 || (turns256 == turns128 && d->I > 1024);
+}
+
 bool ind_dtype_known(int ind_dtype) { return ind_dtype >= EGS_IND_I16 && ind_dtype <= EGS_IND_U8; }
 
 }  // namespace
@@ -83,12 +102,15 @@ int egs_gather_gemm_fp8act(const void *X, const void *Wq, const float *w_scale, 
     p.Aq = q.Xq; p.a_scale = q.xs; p.W = (const char *)Wq; p.w_scale = w_scale; p.Ind = Ind; p.C = (char *)Y;
     p.B = d->B; p.T = d->T; p.E = d->E; p.K = d->K; p.R = d->I; p.N = d->J;
     p.ind_dtype = ind_dtype;
-    p.m_tiles = ceil_div(d->B * d->K, kF8BM);
-    p.n_tiles = ceil_div(d->J, kF8BN);
     p.a_bytes = (uint32_t)((uint64_t)d->B * d->T * d->I);
-    const int64_t grid = (int64_t)8 * ceil_div(d->E, 8) * p.m_tiles * p.n_tiles;
+    const bool large = f8_large_tiles(d);
+    const int tile = large ? 256 : 128;
+    p.m_tiles = ceil_div(d->B * d->K, tile);
+    p.n_tiles = ceil_div(d->J, tile);
+    const int64_t grid = f8_grid(d, tile);
     if (grid > INT32_MAX) return EGS_ERR_BAD_SHAPE;
-    hipLaunchKernelGGL(rows_gemm_f8_kernel, dim3((unsigned)grid), dim3(kF8Threads), 0, s, p);
+    if (large) hipLaunchKernelGGL((rows_gemm_f8_kernel<256, 256>), dim3((unsigned)grid), dim3(kF8Threads), 0, s, p);
+    else hipLaunchKernelGGL((rows_gemm_f8_kernel<128, 128>), dim3((unsigned)grid), dim3(kF8Threads), 0, s, p);
     EGS_CHECK_LAUNCH("rows_gemm_f8_kernel");
     return EGS_OK;
 }

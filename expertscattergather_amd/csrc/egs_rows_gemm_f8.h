@@ -10,7 +10,9 @@
 //       the gather moves.
 //   rows_gemm_f8_kernel         the direct-to-LDS pipeline of egs_rows_gemm_dl.h at one byte per element:
 //       256 x 256 tile of one expert's product per workgroup (8 wavefronts, 2 x 4, 128 x 64 each), 128-deep
-//       slabs (32 KB of gathered rows + 32 KB of weights), two stages, one barrier per slab.  Rows are K-major
+//       slabs (32 KB of gathered rows + 32 KB of weights), two stages, one barrier per slab; or, where those
+//       leave CUs idle or mostly hold padding, 128 x 128 (4 x 2 wavefronts of 32 x 64, 16 KB + 16 KB), two
+//       workgroups to a CU (the rule and both sides' times are in egs_f8_launch.hip).  Rows are K-major
 //       in LDS and read with 16-byte reads, weights stay [reduction][column] and are read with the 8-bit LDS
 //       transpose read; both operands of one MFMA are 32 bytes per lane and use the same order of reduction
 //       elements within a lane group, which is all the instruction needs.
@@ -101,22 +103,28 @@ struct RowsGemmF8Params {
     uint32_t a_bytes;       // B*T*R, below 2 GiB
 };
 
-constexpr int kF8BM = 256, kF8BN = 256, kF8BK = 128, kF8Stages = 2, kF8Threads = 512;
-constexpr int kF8StageBytes = kF8BM * kF8BK + kF8BK * kF8BN;
+constexpr int kF8BK = 128, kF8Stages = 2, kF8Threads = 512;
 
 // swizzle key of the K-major byte rows (8 chunks of 16 bytes), XORed into the chunk index: the 16-byte
 // fragment reads of consecutive rows spread over the banks
 __device__ __forceinline__ int f8_key_rows(int row) { return row & 7; }
 
-static __global__ __launch_bounds__(kF8Threads) void rows_gemm_f8_kernel(RowsGemmF8Params p)
+// swizzle key of the weight rows (BN / 16 chunks of 16 bytes, one 16-column tile each): the 32 rows of a transpose read, sixteen
+// apart in fours of eight, fall two deep on every bank
+template <int BN> __device__ __forceinline__ int f8_key_weights(int row) { return BN == 256 ? row & 15 : ((row >> 1) & 3) | ((row >> 4) & 1) << 2; }
+
+// Each result is the sum over slabs in order of one 128-deep matrix instruction, whatever the tile: both give the same bits.
+template <int BM, int BN>
+__global__ __launch_bounds__(kF8Threads, BM == 128 ? 4 : 2) void rows_gemm_f8_kernel(RowsGemmF8Params p)
 {
-    constexpr int BM = kF8BM, BN = kF8BN, BK = kF8BK, NSTAGE = kF8Stages;
-    constexpr int NW = kF8Threads / 64, WN = 4;
-    constexpr int TM = 8, TN = 4;                       // 16 x 16 tiles per wavefront: 128 x 64
-    constexpr int P_BYTES = BM * BK, STAGE = kF8StageBytes;
+    static_assert((BM == 256 && BN == 256) || (BM == 128 && BN == 128), "tile shapes");
+    constexpr int BK = kF8BK, NSTAGE = kF8Stages;
+    constexpr int NW = kF8Threads / 64, WN = BN / 64;
+    constexpr int TM = BM / (NW / WN) / 16, TN = 4;     // 16 x 16 tiles per wavefront: 128 x 64 or 32 x 64
+    constexpr int P_BYTES = BM * BK, STAGE = BM * BK + BK * BN;
     constexpr int PL = BM * (BK / 16) / 64 / NW;        // row-side loads per wavefront and slab (1 KB = 8 rows each)
-    constexpr int QL = BK / 4 / NW;                     // weight-side loads (1 KB = 4 reduction rows of 256 bytes)
-    static_assert(PL == 4 && QL == 4, "loads per slab");
+    constexpr int WCR = BN / 16;                        // 16-byte chunks per weight row
+    constexpr int QL = BK * WCR / 64 / NW;              // weight-side loads (1 KB = 4 or 8 reduction rows)
 
     __shared__ __attribute__((aligned(1024))) char smem[NSTAGE * STAGE + BM * 16];
     uint32_t *a_voff = reinterpret_cast<uint32_t *>(smem + NSTAGE * STAGE);
@@ -160,8 +168,8 @@ static __global__ __launch_bounds__(kF8Threads) void rows_gemm_f8_kernel(RowsGem
     const u32x4 rs_w = make_rsrc(p.W + (size_t)e * R * N, (uint32_t)((size_t)R * N));
 
     // ---------------- loaders: lane l of a row-side load lands on row 8 j + l/8, physical chunk l%8 and so
-    // fetches logical chunk (l%8) ^ key(row); lane l of a weight-side load lands on reduction row 4 j + l/16,
-    // physical chunk l%16 and fetches the 16 columns of logical chunk (l%16) ^ (row & 15)
+    // fetches logical chunk (l%8) ^ key(row); lane l of a weight-side load lands on reduction row (64 / WCR) j + l / WCR,
+    // physical chunk l % WCR and fetches the 16 columns of logical chunk (l % WCR) ^ key(row)
     uint32_t pv[PL], qv[QL];
 #pragma unroll
     for (int jj = 0; jj < PL; ++jj) {
@@ -171,8 +179,8 @@ static __global__ __launch_bounds__(kF8Threads) void rows_gemm_f8_kernel(RowsGem
     }
 #pragma unroll
     for (int jj = 0; jj < QL; ++jj) {
-        const int row = (wave * QL + jj) * 4 + (lane >> 4);
-        const int n = n0 + ((lane & 15) ^ (row & 15)) * 16;
+        const int row = (wave * QL + jj) * (64 / WCR) + lane / WCR;
+        const int n = n0 + ((lane % WCR) ^ f8_key_weights<BN>(row)) * 16;
         qv[jj] = n < N ? (uint32_t)row * (uint32_t)N + (uint32_t)n : kVoffInvalid;
     }
     auto issue = [&](int kt, int stage) {
@@ -190,7 +198,7 @@ static __global__ __launch_bounds__(kF8Threads) void rows_gemm_f8_kernel(RowsGem
     // reduction elements 64 u + 16 g + 8 h .. + 7 for (u, h) = (0,0), (0,1), (1,0), (1,1): one 16-byte read per
     // u on the row side (chunk 4 u + g of the row), one transpose read per (u, h) on the weight side
     const int a = lane & 15, g = lane >> 4;
-    const int wave_m0 = (wave / WN) * 128, wave_n0 = (wave % WN) * 64;
+    const int wave_m0 = (wave / WN) * (TM * 16), wave_n0 = (wave % WN) * 64;
     int m_at[2], n_at[4];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -199,7 +207,7 @@ static __global__ __launch_bounds__(kF8Threads) void rows_gemm_f8_kernel(RowsGem
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int kr = u * 64 + g * 16 + h * 8 + (a >> 1);      // the transpose read's row of this lane
-            n_at[2 * u + h] = kr * BN + (((wave_n0 >> 4) ^ (kr & 15)) << 4) + (a & 1) * 8;
+            n_at[2 * u + h] = kr * BN + (((wave_n0 >> 4) ^ f8_key_weights<BN>(kr)) << 4) + (a & 1) * 8;
         }
     }
 
@@ -242,8 +250,8 @@ static __global__ __launch_bounds__(kF8Threads) void rows_gemm_f8_kernel(RowsGem
     }
 
     // ---------------- epilogue.  Lane (a, g) holds, for row 16 i + a, the four columns 16 j + 4 g .. + 3.  Both
-    // scales are applied, the bf16 tile goes through LDS (the slab stages are free now: 256 rows x 512 bytes)
-    // and leaves as whole row segments, 512 contiguous bytes of each of two rows per store instruction.
+    // scales are applied, the bf16 tile goes through LDS (the slab stages are free now)
+    // and leaves as whole row segments, 512 or 256 contiguous bytes of each of two or four rows per store instruction.
     constexpr int ROW_BYTES = BN * 2;
     static_assert(BM * ROW_BYTES <= NSTAGE * STAGE, "staging tile fits the slab stages");
     __syncthreads();
@@ -263,9 +271,10 @@ static __global__ __launch_bounds__(kF8Threads) void rows_gemm_f8_kernel(RowsGem
         }
     }
     __syncthreads();
-    const int lrow = lane >> 5, lchunk = lane & 31;
+    constexpr int CPR = ROW_BYTES / 16, RPI = 64 / CPR;     // chunks per row, rows per store instruction
+    const int lrow = lane / CPR, lchunk = lane % CPR;
     const int n_here = n0 + lchunk * 8;
-    for (int r0 = wave * 2; r0 < BM; r0 += NW * 2) {
+    for (int r0 = wave * RPI; r0 < BM; r0 += NW * RPI) {
         const int row = r0 + lrow;
         const int64_t co = c_off[row];
         const u32x4 v = *reinterpret_cast<const u32x4 *>(smem + row * ROW_BYTES + ((lchunk ^ (row & 15)) << 4));

@@ -1,0 +1,39 @@
+"""rows_gemm_f8_kernel in 128 x 128 tiles (csrc/egs_rows_gemm_f8.h): the edges of rows, columns and slabs against the quantised oracle,
+and the bits of the 256 x 256 tiles."""
+import numpy as np
+import pytest
+import torch
+
+from expertscattergather_amd import hip_kernels as hk
+from expertscattergather_amd import workloads as wl
+from oracle import egs_oracle as O
+from tests._util import assert_close, make_case
+from tests.test_gpu_parity import dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", [(1, 5, 1, 1, 128, 16), (1, 300, 3, 127, 128, 112), (1, 300, 9, 128, 256, 128), (3, 90, 10, 43, 384, 144),
+                                   (2, 200, 17, 129, 1280, 272)], ids=str)
+def test_small_tiles_match_the_quantised_oracle(shape):
+    B, T, E, K, I, J = shape
+    case = make_case(47, B, T, E, K, I, J, torch.bfloat16)
+    case["Ind"][0, 0, 0] = T                                 # contributes a zero row
+    case["Ind"][-1, -1, -1] = -1
+    Wq, scale = wl.quantize_fp8_weights(case["Wg"].float())
+    Y = hk.expert_gather_fp8_forward(dev(case["X"]), dev(Wq), dev(scale), dev(case["Ind"]))
+    ind = case["Ind"].numpy().astype(np.int64)
+    live = (ind >= 0) & (ind < T)
+    ref = O.gather_forward_fp8(case["X"].float().numpy(), Wq.view(torch.uint8).numpy(), scale.numpy(), np.where(live, ind, 0)) * live[..., None]
+    assert_close(Y, ref, torch.bfloat16, "fp8 tiles")
+
+
+def test_small_and_large_tiles_give_the_same_bits():
+    """All 64 experts at once take the 256 x 256 tiles, eight of them at a time the small ones."""
+    case = make_case(48, 20, 300, 64, 50, 1152, 496, torch.bfloat16)
+    Wq, scale = wl.quantize_fp8_weights(case["Wg"].float())
+    X, q, sc, ind = dev(case["X"]), dev(Wq), dev(scale), dev(case["Ind"])
+    Y = hk.expert_gather_fp8_forward(X, q, sc, ind)
+    for e in range(0, 64, 8):
+        part = hk.expert_gather_fp8_forward(X, q[e:e + 8].contiguous(), sc[e:e + 8].contiguous(), ind[:, e:e + 8].contiguous())
+        assert torch.equal(Y[:, e:e + 8], part)
