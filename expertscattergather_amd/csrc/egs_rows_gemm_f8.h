@@ -37,27 +37,57 @@ struct QuantRowsParams {
     int64_t ldx_b, ldx_t;
 };
 
-// one wavefront per row: pass 1 finds max|x|, pass 2 (the row is in the cache by then) scales,
-// clamps and converts with round-to-nearest-even; adjacent lanes write adjacent 8-byte pieces
-static __global__ __launch_bounds__(kThreads) void quantize_rows_e4m3_kernel(QuantRowsParams p)
+// magnitude of a row: the integer maximum of the magnitude bits.  For non-negative floats the bit patterns order like the values,
+// infinities sort above every finite value and NaNs above the infinities, so a NaN anywhere in the row survives the reduction
+// (fmaxf would drop it)
+__device__ __forceinline__ uint32_t amax_bits_of(uint32_t m, u32x4 v)
+{
+#pragma unroll
+    for (int x = 0; x < 4; ++x) m = max(max(m, (v[x] << 16) & 0x7fffffffu), v[x] & 0x7fff0000u);
+    return m;
+}
+
+__device__ __forceinline__ u32x2 quantize_e4m3(u32x4 v, float inv)
+{
+    u32x2 q;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        float f[4];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            f[2 * x] = fminf(fmaxf(bits_f32(v[2 * h + x] << 16) * inv, -kE4M3Max), kE4M3Max);
+            f[2 * x + 1] = fminf(fmaxf(bits_f32(v[2 * h + x] & 0xffff0000u) * inv, -kE4M3Max), kE4M3Max);
+        }
+        int w = 0;
+        w = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], w, false);
+        w = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], w, true);
+        q[h] = (uint32_t)w;
+    }
+    return q;
+}
+
+// One wavefront per row: find max|x|, then scale, clamp and convert with round-to-nearest-even; adjacent lanes write adjacent 8-byte
+// pieces.  Bound by the bytes in flight.  Rows of up to HELD * 512 elements are fetched at once and kept in registers, so a row is one
+// round trip; longer ones (HELD = 0) are read a second time, from the cache by then.
+template <int HELD>
+__global__ __launch_bounds__(kThreads) void quantize_rows_e4m3_kernel(QuantRowsParams p)
 {
     const int lane = (int)threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * (kThreads / 64) + ((int)threadIdx.x >> 6);
-    if (row >= (int64_t)p.B * p.T) return;
-    const int64_t b = row / p.T, t = row - b * p.T;
-    const char *src = p.X + (b * p.ldx_b + t * p.ldx_t) * 2;
+    const uint32_t row = blockIdx.x * (uint32_t)(kThreads / 64) + (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (row >= (uint32_t)p.B * (uint32_t)p.T) return;
+    const uint32_t b = row / (uint32_t)p.T, t = row - b * (uint32_t)p.T;
+    const char *src = p.X + ((int64_t)b * p.ldx_b + (int64_t)t * p.ldx_t) * 2;
     const int chunks = p.I >> 3;
-    // max|x| over the row as an integer maximum of the magnitude bits: for non-negative floats the bit patterns
-    // order like the values, infinities sort above every finite value and NaNs above the infinities, so a NaN
-    // anywhere in the row survives the reduction (fmaxf would drop it)
+    u32x4 v[HELD > 0 ? HELD : 1];
     uint32_t amax_bits = 0u;
-    for (int c = lane; c < chunks; c += 64) {
-        const u32x4 v = *reinterpret_cast<const u32x4 *>(src + (size_t)c * 16);
+    if constexpr (HELD > 0) {
+        // lanes past the row's end fetch its last chunk again
 #pragma unroll
-        for (int x = 0; x < 4; ++x) {
-            amax_bits = max(amax_bits, (v[x] << 16) & 0x7fffffffu);
-            amax_bits = max(amax_bits, v[x] & 0x7fff0000u);
-        }
+        for (int x = 0; x < HELD; ++x) v[x] = *reinterpret_cast<const u32x4 *>(src + (size_t)min(x * 64 + lane, chunks - 1) * 16);
+#pragma unroll
+        for (int x = 0; x < HELD; ++x) amax_bits = amax_bits_of(amax_bits, v[x]);
+    } else {
+        for (int c = lane; c < chunks; c += 64) amax_bits = amax_bits_of(amax_bits, *reinterpret_cast<const u32x4 *>(src + (size_t)c * 16));
     }
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) amax_bits = max(amax_bits, (uint32_t)__shfl_xor((int)amax_bits, m));
@@ -68,24 +98,14 @@ static __global__ __launch_bounds__(kThreads) void quantize_rows_e4m3_kernel(Qua
     const float scale = !finite ? bits_f32(0x7fc00000u) : (amax > 0.f ? amax / kE4M3Max : 1.0f);
     const float inv = finite ? 1.0f / scale : 0.f;
     if (lane == 0) p.xs[row] = scale;
-    char *dst = p.Xq + row * p.I;
-    for (int c = lane; c < chunks; c += 64) {
-        const u32x4 v = *reinterpret_cast<const u32x4 *>(src + (size_t)c * 16);
-        u32x2 q;
+    char *dst = p.Xq + (size_t)row * p.I;
+    if constexpr (HELD > 0) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            float f[4];
-#pragma unroll
-            for (int x = 0; x < 2; ++x) {
-                f[2 * x] = fminf(fmaxf(bits_f32(v[2 * h + x] << 16) * inv, -kE4M3Max), kE4M3Max);
-                f[2 * x + 1] = fminf(fmaxf(bits_f32(v[2 * h + x] & 0xffff0000u) * inv, -kE4M3Max), kE4M3Max);
-            }
-            int w = 0;
-            w = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], w, false);
-            w = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], w, true);
-            q[h] = (uint32_t)w;
-        }
-        *reinterpret_cast<u32x2 *>(dst + (size_t)c * 8) = q;
+        for (int x = 0; x < HELD; ++x)
+            if (x * 64 + lane < chunks) *reinterpret_cast<u32x2 *>(dst + (size_t)(x * 64 + lane) * 8) = quantize_e4m3(v[x], inv);
+    } else {
+        for (int c = lane; c < chunks; c += 64)
+            *reinterpret_cast<u32x2 *>(dst + (size_t)c * 8) = quantize_e4m3(*reinterpret_cast<const u32x4 *>(src + (size_t)c * 16), inv);
     }
 }
 

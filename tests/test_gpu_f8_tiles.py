@@ -37,3 +37,21 @@ def test_small_and_large_tiles_give_the_same_bits():
     for e in range(0, 64, 8):
         part = hk.expert_gather_fp8_forward(X, q[e:e + 8].contiguous(), sc[e:e + 8].contiguous(), ind[:, e:e + 8].contiguous())
         assert torch.equal(Y[:, e:e + 8], part)
+
+
+@pytest.mark.parametrize("width", [128, 512, 640, 1024, 2176, 4096, 4224])
+def test_row_quantiser_at_every_number_of_chunks_a_lane_holds(width):
+    """quantize_rows_e4m3_kernel<1, 2, 4, 8, 0>: bit for bit the oracle's, also for zero rows and rows with a NaN or an infinity."""
+    case = make_case(49, 2, 33, 2, 3, width, 16, torch.bfloat16)
+    X = case["X"]
+    X[0, 0] = 0
+    X[1, 2, width - 1] = 1000                                # the largest value in the last lane's chunk
+    Wq, scale = wl.quantize_fp8_weights(case["Wg"].float())
+    run = lambda x: hk.expert_gather_fp8_forward(dev(x), dev(Wq), dev(scale), dev(case["Ind"]), return_quantised=True)[1:]
+    Xq, xs = run(X)
+    q_o, xs_o = O.quantize_rows_e4m3(X.float().numpy())
+    assert np.array_equal(xs.cpu().numpy(), xs_o)
+    assert np.array_equal(Xq.cpu().view(torch.uint8).numpy(), q_o)
+    X[0, 1, width - 1], X[1, 3, 0] = float("nan"), float("-inf")
+    xs = run(X)[1].cpu().reshape(2, 33)
+    assert xs[0, 1].isnan() and xs[1, 3].isnan() and int(xs.isnan().sum()) == 2
