@@ -225,7 +225,8 @@ __global__ __launch_bounds__(WM * WN * kWave) void rows_gemm_kernel(RowsGemmPara
     }
 }
 
-// fp32 products added to the output with atomics, operands of any size and alignment.
+// fp32 products added to the output with atomics, operands of any size and alignment.  BM x BN: 64 x 64 or 128 x 128 (the rule and
+// both sides' times are in egs_rows_launch.hip).
 template <int BM, int BN, int BK, int WM, int WN, bool W_TRANS>
 __global__ __launch_bounds__(WM * WN * kWave) void rows_atomic_f32_kernel(RowsGemmParams p)
 {
@@ -393,7 +394,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void rows_atomic_f32_kernel(RowsGe
     }
 
     // ---------------- fp32 atomics on the output.  Rows of the tile that land on the same token (a hot token under a skewed router:
-    // tens of the 128 picks of a tile) are first added up inside the workgroup - LDS atomics into one of kSlots
+    // tens of the picks of a tile) are first added up inside the workgroup - LDS atomics into one of kSlots
     // rows of partial sums - so that the token receives one atomic per column from this tile, not one per pick.
     // A tile without such rows (the common case, known since the row bookkeeping) goes straight to memory.
     float *cbase = reinterpret_cast<float *>(p.C);

@@ -9,18 +9,23 @@ namespace host {
 namespace {
 
 // ------------------------------------------------------------------------------ rows-GEMM dispatch
-// fp32 atomics on the output: the one epilogue that the tiled kernels of egs_tiled.h do not have
+// fp32 atomics on the output: the one epilogue that the tiled kernels of egs_tiled.h do not have.  128 x 128 tiles only for long reductions
+// that fill the chip with them, where their half as many operand bytes count; else 64 x 64, of which a CU takes several.  us, 128 then
+// 64: R2048 N1024 Me512 E32 617, 695; R1024 N1024 Me512 E32 374, 387; R2048 N200 Me400 E32 187, 171; R2048 N512 Me256 E16 187, 101; R512
+// N128 Me4000 E16 109, 102; R128 N512 Me2048 E64 390, 304 (Zipf-routed 490, 362); R196 N220 Me51 E15 34, 14.4; R64 N96 Me4800 E60 181, 125
 template <bool W_TRANS>
 int launch_rows_atomic(RowsGemmParams &p, hipStream_t s)
 {
     const int Me = p.B * p.K;
-    p.m_tiles = ceil_div(Me, 128); p.n_tiles = ceil_div(p.N, p.N <= 64 ? 64 : 128);
+    const bool large = p.R >= 1024 && (int64_t)p.E * ceil_div(Me, 128) * ceil_div(p.N, 128) >= 512;
+    const int tile = large ? 128 : 64;
+    p.m_tiles = ceil_div(Me, tile); p.n_tiles = ceil_div(p.N, tile);
     const int64_t grid = (int64_t)8 * ceil_div(p.E, 8) * p.m_tiles * p.n_tiles;
     if (grid > INT32_MAX) return EGS_ERR_BAD_SHAPE;
-    if (p.N <= 64)
-        hipLaunchKernelGGL((rows_atomic_f32_kernel<128, 64, 32, 4, 1, W_TRANS>), dim3((unsigned)grid), dim3(256), 0, s, p);
-    else
+    if (large)
         hipLaunchKernelGGL((rows_atomic_f32_kernel<128, 128, 32, 2, 2, W_TRANS>), dim3((unsigned)grid), dim3(256), 0, s, p);
+    else
+        hipLaunchKernelGGL((rows_atomic_f32_kernel<64, 64, 32, 4, 1, W_TRANS>), dim3((unsigned)grid), dim3(256), 0, s, p);
     EGS_CHECK_LAUNCH("rows_atomic_f32_kernel");
     return EGS_OK;
 }
