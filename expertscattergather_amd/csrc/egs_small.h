@@ -443,6 +443,16 @@ __global__ __launch_bounds__(kThreads) void dw_small_kernel(SmallDwParams p)
     dw_small_body<TT>(p, (int)blockIdx.x, red);
 }
 
+// v += part[s], ..., part[s + N - 1], in that order; the N loads in flight at once
+template <int N> __device__ __forceinline__ void dw_reduce4_add(f32x4 &v, const f32x4 *part, size_t total4)
+{
+    f32x4 u[N];
+#pragma unroll
+    for (int x = 0; x < N; ++x) u[x] = part[(size_t)x * total4];
+#pragma unroll
+    for (int x = 0; x < N; ++x) { v[0] += u[x][0]; v[1] += u[x][1]; v[2] += u[x][2]; v[3] += u[x][3]; }
+}
+
 // dW = sum_s part[s] in increasing s, rounded once; partials already have the output's layout.
 // 4 elements per thread (total % 4 == 0, 16-byte aligned); `block` of `nblocks` workgroups.
 __device__ __forceinline__ void dw_reduce4_body(const float *part, char *dW, int32_t S, size_t total4, int32_t out_dtype,
@@ -450,10 +460,12 @@ __device__ __forceinline__ void dw_reduce4_body(const float *part, char *dW, int
 {
     for (size_t o = (size_t)block * kThreads + threadIdx.x; o < total4; o += (size_t)nblocks * kThreads) {
         f32x4 v = reinterpret_cast<const f32x4 *>(part)[o];
-        for (int s = 1; s < S; ++s) {
-            const f32x4 u = reinterpret_cast<const f32x4 *>(part)[(size_t)s * total4 + o];
-            v[0] += u[0]; v[1] += u[1]; v[2] += u[2]; v[3] += u[3];
-        }
+        const f32x4 *src = reinterpret_cast<const f32x4 *>(part) + total4 + o;
+        int left = S - 1;
+        for (; left >= 8; left -= 8, src += 8 * total4) dw_reduce4_add<8>(v, src, total4);
+        if (left & 4) { dw_reduce4_add<4>(v, src, total4); src += 4 * total4; }
+        if (left & 2) { dw_reduce4_add<2>(v, src, total4); src += 2 * total4; }
+        if (left & 1) dw_reduce4_add<1>(v, src, total4);
         if (out_dtype == 0) {
             reinterpret_cast<f32x4 *>(dW)[o] = v;
         } else {
