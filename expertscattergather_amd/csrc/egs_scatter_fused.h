@@ -316,8 +316,9 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
             // chunk 0 of row q in the rows' XOR order: a thread's two chunks are one XOR away each.  (The phase is bound by
             // vector-ALU issue - two wavefronts per SIMD, all in it at once - so it is written for few instructions per pick.)
             const uint32_t c2 = (uint32_t)(tid & 3) << 5, zero_sel = (uint32_t)p.zero_at;
-            auto sum_of = [&](int t, f32x4 &lo, f32x4 &hi) {
+            for (int t = tid >> 2; t < T; t += kFusedThreads >> 2) {
                 const int s0 = seg[t], s1 = seg[t + 1];
+                f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
                 for (int s = s0; s < s1; s += 4) {
                     const int n = s1 - s;
                     uint32_t en[4];
@@ -334,8 +335,14 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
 #pragma unroll
                     for (int x = 0; x < 4; ++x) { lo += v[x][0]; hi += v[x][1]; }
                 }
-            };
-            auto store_of = [&](int t, const f32x4 &lo, const f32x4 &hi) {
+                if (HOLD && t == tid >> 2) {
+                    // loads and stores share a counter: the next slice's weights are waited for before the first store, which the
+                    // next slice would otherwise have to wait for too
+#pragma unroll
+                    for (int d = 0; d < kFusedDepth; ++d)
+#pragma unroll
+                        for (int x = 0; x < 2 * KS; ++x) asm volatile("" : "+v"(buf[d].w[x]));
+                }
                 char *dst = p.out + (((size_t)b * T + t) * N + at0) * ES;
                 if constexpr (ES == 4) {
                     reinterpret_cast<f32x4 *>(dst)[0] = lo;
@@ -346,24 +353,6 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
                     w[2] = pack2<TT>(hi[0], hi[1]); w[3] = pack2<TT>(hi[2], hi[3]);
                     *reinterpret_cast<u32x4 *>(dst) = w;
                 }
-            };
-            int t = tid >> 2;
-            if constexpr (HOLD) {
-                // loads and stores share a counter: the next slice's weights are waited for before the first store, which the
-                // next slice would otherwise have to wait for too
-                f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
-                if (t < T) sum_of(t, lo, hi);
-#pragma unroll
-                for (int d = 0; d < kFusedDepth; ++d)
-#pragma unroll
-                    for (int x = 0; x < 2 * KS; ++x) asm volatile("" : "+v"(buf[d].w[x]));
-                if (t < T) store_of(t, lo, hi);
-                t += kFusedThreads >> 2;
-            }
-            for (; t < T; t += kFusedThreads >> 2) {
-                f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
-                sum_of(t, lo, hi);
-                store_of(t, lo, hi);
             }
         }
     } else {
