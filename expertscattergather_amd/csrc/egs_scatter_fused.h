@@ -315,8 +315,12 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
             // instead of its own, so that the additions need no condition.  Entry q stands for byte (q << 7) | ((q & 7) << 4),
             // chunk 0 of row q in the rows' XOR order: a thread's two chunks are one XOR away each.  (The phase is bound by
             // vector-ALU issue - two wavefronts per SIMD, all in it at once - so it is written for few instructions per pick.)
+            constexpr int kTokens = kFusedThreads >> 2;
             const uint32_t c2 = (uint32_t)(tid & 3) << 5, zero_sel = (uint32_t)p.zero_at;
-            for (int t = tid >> 2; t < T; t += kFusedThreads >> 2) {
+            // (HOLD: a thread's first token by itself, see below.  Not functions: those made the loop 0.2 to 0.5 us slower without HOLD)
+#pragma unroll
+            for (int part = 0; part < (HOLD ? 2 : 1); ++part)
+            for (int t = (tid >> 2) + part * kTokens; t < (HOLD && part == 0 ? min(T, kTokens) : T); t += kTokens) {
                 const int s0 = seg[t], s1 = seg[t + 1];
                 f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
                 for (int s = s0; s < s1; s += 4) {
@@ -335,7 +339,7 @@ __device__ __forceinline__ void scatter_fused_body(const ScatterFusedParams &p, 
 #pragma unroll
                     for (int x = 0; x < 4; ++x) { lo += v[x][0]; hi += v[x][1]; }
                 }
-                if (HOLD && t == tid >> 2) {
+                if (HOLD && part == 0) {
                     // loads and stores share a counter: the next slice's weights are waited for before the first store, which the
                     // next slice would otherwise have to wait for too
 #pragma unroll
@@ -425,7 +429,7 @@ __global__ __launch_bounds__(kFusedThreads) void scatter_fused_kernel(ScatterFus
 
 // More slices than the device has CUs for: a run of them per workgroup, with one sort.  The slices of a run multiply the same rows,
 // so with HOLD (a reduction of at most two steps, and no more units of 32 picks than the wavefronts have registers for) they are
-// read and brought into operand order once, and only weights travel between slices.  B64 T256 E32 K32 I768 J64, bf16: 48 -> 38.5 us
+// read and brought into operand order once, and only weights travel between slices.  B64 T256 E32 K32 I768 J64, bf16: 47 -> 37 us
 // (sort and first operands 11, then 4.6 a slice: 128 KB of weights per CU, which all CUs together take 2.2 us to get out of L2,
 // products 1.1, sums 1.0); B128 T64 E8 K16 I1024 J64 39 -> 33; the same with fp32 and J32 65 -> 59.
 template <class TT, bool W_NMAJOR, int KS, bool HOLD>
