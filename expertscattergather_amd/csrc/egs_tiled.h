@@ -844,7 +844,7 @@ static __global__ __launch_bounds__(kThreads) void tiled_dw_sum_kernel(const flo
     }
 }
 
-// Operands of less than 16 bytes: one thread per element of dW, pick by pick.
+// Operands of less than 16 bytes: one thread per element of dW, pick by pick, all picks (S = 1).
 template <class TT>
 __global__ __launch_bounds__(kThreads) void tiny_dw_kernel(TiledDwParams p)
 {

@@ -67,6 +67,25 @@ def test_experts_of_a_few_bytes(dims, dtype):
     assert_close(out, O.scatter_forward(np64(case["Y"]), np64(case["Ws"]), case["Ind"].numpy(), T), dtype, "out")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("shape", [(1, 3, 2, 600, 1, 5), (1, 2, 3, 2100, 1, 9), (1, 0, 2, 2100, 3, 5)], ids=lambda s: "x".join(map(str, s)))
+def test_weight_gradient_of_sources_below_16_bytes_with_many_picks(shape, dtype):
+    """More picks than one workgroup usually takes, of a source that holds no 16-byte chunk (or nothing): tiny_dw_kernel sums them all."""
+    B, T, E, K, I, J = shape
+    case = make_case(3, B, max(T, 1), E, K, I, J, dtype)
+    X, Y, Ind = dev(case["X"][:, :T]), dev(case["Y"]), dev(case["Ind"])
+    dW = torch.full((E, I, J), float("nan"), dtype=dtype, device="cuda")
+    dims = _abi.Dims(B, T, E, K, I, J)
+    code, n = hk.dtype_to_type_id(dtype), _abi.lib().egs_workspace_bytes(_abi.OP_DW, 0, dims, hk.dtype_to_type_id(dtype))
+    ws = torch.full((max(n, 256) // 4,), float("nan"), device="cuda")
+    with _abi.launch_log() as log:
+        rc = _abi.lib().egs_dw(X.data_ptr() or Y.data_ptr(), Y.data_ptr(), Ind.data_ptr(), dW.data_ptr(), ws.data_ptr(), n, dims, T * I, I, code, code,
+                               _abi.IND_I64, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and log.kernels == ["tiny_dw_kernel"], (rc, log.kernels)
+    want = O.gather_backward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy(), np64(case["Y"]))[1] if T else torch.zeros(E, I, J).double().numpy()
+    assert_close(dW, want, dtype, "dW")
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 def test_odd_views_and_values_that_are_not_finite_stay_where_they_are(dtype):
     """X as a view with odd strides that ends at its storage's last element, W and Y off the 16-byte grid (through the C ABI's
