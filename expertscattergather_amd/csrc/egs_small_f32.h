@@ -196,6 +196,13 @@ __global__ __launch_bounds__(64 * (16 / TQ), 4) void rows_small_f32_kernel(Small
                         }
                     }
                 }
+        } else {
+#pragma unroll
+            for (int t = 0; t < TG; ++t)
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) acc[t][tn][x] *= kSplitUnscale;
         }
         // lane (a, g) holds, for pick 16 tq + a, columns 16 tn + 4 g .. + 3: the four lanes g of a pick write 64 contiguous bytes
 #pragma unroll

@@ -9,17 +9,22 @@
 // (1.14e-6) of the result's root mean square.  Six instructions of 16 cycles stand for eight of 32, and at a higher clock:
 // 358 TFLOP/s of fp32 work against 138 (an instruction-only loop over all CUs).
 //
-// Limits: the pieces of a value below 2^-109 fall below bf16's smallest number, which leaves them with an absolute error of up to 2^-134.
-// An infinity has no such pieces (inf - inf), nor has a value that rounds up to one in bf16 (above 3.39e38): such products
-// arrive as NaN or infinity, so a wavefront whose results are not all finite takes its tile again with the fp32 instruction.
+// bf16 numbers end at 2^-133 (subnormal ones are kept by the conversion and by the matrix instruction), where an fp32 value may still
+// have bits down to 2^-149.  So both operands are taken times 2^16, which makes the three pieces exact down to the smallest fp32 number,
+// and sums times 2^-32.  What that brings near the other end - values from 2^112 on, sums from 2^96 - arrives as infinity or NaN, as
+// infinities (inf - inf) and NaN do: a wavefront whose results are not all finite takes its tile again with the fp32 instruction.
+// Without the factor the error grew below 2^-110: operands of 2^-115 1.1e-6, 2^-120 3.5e-5, 2^-125 1.1e-3.
 #pragma once
 #include "egs_device.h"
 
 namespace egs {
 
-// the three pieces of two floats, packed in pairs
+constexpr float kSplitScale = 65536.f, kSplitUnscale = 0x1p-32f;       // of a value; of a sum of products of two
+
+// the three pieces of two floats (times kSplitScale), packed in pairs
 __device__ __forceinline__ void split_pair(float x, float y, uint32_t (&piece)[3])
 {
+    x *= kSplitScale; y *= kSplitScale;
     piece[0] = pack2<ElemBF16>(x, y);
     const float rx = x - bits_f32(piece[0] << 16), ry = y - bits_f32(piece[0] & 0xffff0000u);
     piece[1] = pack2<ElemBF16>(rx, ry);

@@ -189,6 +189,13 @@ static __global__ __launch_bounds__(kThreads, 3) void tiled_dw_split_kernel(Tile
 #pragma unroll
                 for (int y = 0; y < 2; ++y) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(yv[y], xv[x], acc[x][y], 0, 0, 0);
         }
+    } else {
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[x][y][r] *= kSplitUnscale;
     }
 
     // ---------------- lane (a, g) holds rows i0 + wi0 + 16 x + a, columns j0 + wj0 + 16 y + 4 g .. + 3; through LDS, so that whole

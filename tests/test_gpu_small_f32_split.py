@@ -59,3 +59,17 @@ def test_values_that_have_no_three_pieces():
     assert big.sum() == J and torch.allclose(got[big], want[big], rtol=1e-5)
     fine = want.isfinite() & ~big
     assert (got[fine] - want[fine]).abs().max() <= 1e-4 * want[fine].abs().max()
+
+
+@pytest.mark.parametrize("x_exp, w_exp", [(-100, 0), (-120, 20), (10, -120), (-140, 40), (-60, -70), (100, -100), (112, -60), (-120, 117), (60, 40)])
+def test_operands_of_any_magnitude(x_exp, w_exp):
+    """Operands down to the smallest subnormal number and up to 2^120: as close to 64 bits as a rounding of each product and sum, of which
+    those below 2^-126 have an absolute one of 2^-150."""
+    B, T, E, K, I, J = 8, 40, 16, 32, 64, 48
+    case = make_case(4, B, T, E, K, I, J, torch.float32)
+    X = (case["X"].double() * 2.0 ** x_exp).float()
+    case["Wg"] = (case["Wg"].double() * 2.0 ** w_exp).float()
+    Y, _ = products(case, dev(case["Ind"]), dev(X), dev(case["dOut"]))
+    want = O.gather_forward(np64(X), np64(case["Wg"]), case["Ind"].numpy())
+    limit = 4 * 2.0 ** -24 * I ** 0.5 * np.sqrt((want ** 2).mean()) + 4 * 2.0 ** -150 * I ** 0.5
+    assert np.sqrt(((np64(Y) - want) ** 2).mean()) <= limit

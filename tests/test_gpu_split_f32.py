@@ -78,3 +78,17 @@ def test_values_that_have_no_three_pieces():
     fine = want.isfinite() & ~big
     assert (big & want.isfinite()).sum() == J and torch.allclose(got[big], want[big], rtol=1e-5)
     assert (got[fine] - want[fine]).abs().max() <= 1e-4 * want[fine].abs().max()
+
+
+@pytest.mark.parametrize("x_exp, y_exp", [(-100, 0), (-120, 20), (10, -120), (-140, 40), (-60, -70), (100, -100), (112, -60), (-120, 117), (60, 40)])
+def test_operands_of_any_magnitude(x_exp, y_exp):
+    """Operands down to the smallest subnormal number and up to 2^120: as close to 64 bits as a rounding of each product and sum, of which
+    those below 2^-126 have an absolute one of 2^-150."""
+    B, T, E, K, I, J = 8, 40, 3, 65, 65, 63
+    case = make_case(11, B, T, E, K, I, J, torch.float32)
+    X, Y = (case["X"].double() * 2.0 ** x_exp).float(), (case["Y"].double() * 2.0 ** y_exp).float()
+    dWg, _, kernels = gradients(case, dev(case["Ind"]), dev(X), dev(Y))
+    want = O.gather_backward(np64(X), np64(case["Wg"]), case["Ind"].numpy(), np64(Y))[1]
+    n = (B * K) ** 0.5
+    limit = 4 * 2.0 ** -24 * n * np.sqrt((want ** 2).mean()) + 4 * 2.0 ** -150 * n
+    assert np.sqrt(((np64(dWg) - want) ** 2).mean()) <= limit
