@@ -157,6 +157,8 @@ bool dw_few_picks(const egs_dims *d, int act_dtype) { return (int64_t)d->B * d->
 // 660 (B1 T712 E125 K155 I369 J128) 28.4 / 34.5, 2352 (B9 T484 E98 K28 I160 J32) 14.5 / 17.5, 55000 135 / 202.  Few tiles of many picks gain at any
 // number (8 tiles, 774 picks 11.3 / 15.1).  Against the aligned tiles of dw_tile_body, which are narrower: 4096 (B64 T256 E32 K32 I128 J64) 21 / 20,
 // 9450 (B16 T61 E14 K45 I960 J96) 30 / 50, 16384 43 / 66 and 46 / 60; with 32 columns of a tile empty (I32 J96, 7676) 41 / 30.
+// Not below four picks, where its six roundings of a product stand against no more of the fp32 instruction's: error of the result, it and that,
+// 1 pick 3.5e-8 / 2.5e-8, 2 3.4e-8 / 3.1e-8, 4 3.3e-8 / 4.0e-8, 32 3.8e-8 / 10.3e-8.
 int64_t dw_split32_slabs(const egs_dims *d)
 {
     return (int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, 64) * (((int64_t)d->B * d->K + 31) / 32);
@@ -237,7 +239,7 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
     const int64_t base = (int64_t)d->E * pl.i_tiles * pl.j_tiles;
     int64_t S = base > 0 ? 512 / base : 1;
     if (S > (Me + 1023) / 1024) S = (Me + 1023) / 1024;
-    pl.split32 = act_dtype == EGS_F32 && (Me >= 512 || dw_split32_slabs(d) >= 600);
+    pl.split32 = act_dtype == EGS_F32 && (Me >= 512 || (Me >= 4 && dw_split32_slabs(d) >= 600));
     if (pl.split32) {
         // two workgroups per CU where that leaves four slabs or more to each
         const int64_t tiles = (int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, 64);

@@ -92,3 +92,14 @@ def test_operands_of_any_magnitude(x_exp, y_exp):
     n = (B * K) ** 0.5
     limit = 4 * 2.0 ** -24 * n * np.sqrt((want ** 2).mean()) + 4 * 2.0 ** -150 * n
     assert np.sqrt(((np64(dWg) - want) ** 2).mean()) <= limit
+
+
+def test_one_pick_is_one_rounding():
+    """The weight gradient of an expert with one pick: each product rounded once, as fp32 gives it."""
+    B, T, E, K, I, J = 1, 9, 640, 1, 67, 35
+    case = make_case(12, B, T, E, K, I, J, torch.float32)
+    dWg, dWs, _ = gradients(case, dev(case["Ind"]), dev(case["X"]), dev(case["Y"]))
+    x, y, do = (t.double()[0] for t in (case["X"], case["Y"], case["dOut"]))
+    token = case["Ind"][0, :, 0]
+    assert torch.equal(dWg.cpu(), (x[token][:, :, None] * y[:, 0][:, None, :]).float())
+    assert torch.equal(dWs.cpu(), (y[:, 0][:, :, None] * do[token][:, None, :]).float())
