@@ -172,9 +172,16 @@ __global__ __launch_bounds__(64 * (16 / TQ), 4) void rows_small_f32_kernel(Small
 #pragma unroll
                     for (int t = 0; t < TG; ++t) mma_chunk<ElemBF16>(acc[t][tn], wf[tn][kSplitP[c]], xf[t][kSplitQ[c]]);
         }
-        // not all finite: these row tiles again, by the fp32 instruction, weights straight from memory
-        const float odd = not_finite(acc);
-        if (__any(odd != 0.f || odd != odd)) {
+        // not all finite: these row tiles again, by the fp32 instruction, weights straight from memory.  (Only what is stored counts:
+        // a pick that does not exist multiplied some row or other.)
+        float odd = 0.f;
+#pragma unroll
+        for (int t = 0; t < TG; ++t) {
+            const int live = __shfl(state, (t0 + t) * 16 + a, kWave) == 1 ? 4 : 0;
+#pragma unroll
+            for (int tn = 0; tn < TN; ++tn) odd = not_finite(acc[t][tn], live, odd);
+        }
+        if (__any(odd != odd)) {
 #pragma unroll
             for (int t = 0; t < TG; ++t)
 #pragma unroll

@@ -12,7 +12,7 @@
 // bf16 numbers end at 2^-133 (subnormal ones are kept by the conversion and by the matrix instruction), where an fp32 value may still
 // have bits down to 2^-149.  So both operands are taken times 2^16, which makes the three pieces exact down to the smallest fp32 number,
 // and sums times 2^-32.  What that brings near the other end - values from 2^112 on, sums from 2^96 - arrives as infinity or NaN, as
-// infinities (inf - inf) and NaN do: a wavefront whose results are not all finite takes its tile again with the fp32 instruction.
+// infinities (inf - inf) and NaN do: a wavefront whose stored results are not all finite takes its tile again with the fp32 instruction.
 // Without the factor the error grew below 2^-110: operands of 2^-115 1.1e-6, 2^-120 3.5e-5, 2^-125 1.1e-3.
 #pragma once
 #include "egs_device.h"
@@ -39,16 +39,11 @@ __device__ __forceinline__ void split_chunk(const u32x4 &v, u32x2 (&piece)[3])
 #pragma unroll
     for (int x = 0; x < 3; ++x) piece[x] = u32x2{lo[x], hi[x]};
 }
-// 0 if every element is finite, else NaN
-template <int M, int N> __device__ __forceinline__ float not_finite(const f32x4 (&acc)[M][N])
+// `t` if the first `live` elements are finite, else NaN
+__device__ __forceinline__ float not_finite(const f32x4 &v, int live, float t)
 {
-    float t = 0.f;
 #pragma unroll
-    for (int i = 0; i < M; ++i)
-#pragma unroll
-        for (int j = 0; j < N; ++j)
-#pragma unroll
-            for (int x = 0; x < 4; ++x) t = fmaf(acc[i][j][x], 0.f, t);
+    for (int x = 0; x < 4; ++x) t = fmaf(x < live ? v[x] : 0.f, 0.f, t);
     return t;
 }
 

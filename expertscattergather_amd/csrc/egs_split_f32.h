@@ -161,9 +161,14 @@ static __global__ __launch_bounds__(kThreads, 3) void tiled_dw_split_kernel(Tile
         }
     }
 
-    // ---------------- not all finite: the wavefront's part again, by the fp32 instruction, straight from memory
-    const float odd = not_finite(acc);
-    if (__any(odd != 0.f || odd != odd)) {
+    // ---------------- not all finite: the wavefront's part again, by the fp32 instruction, straight from memory.  (Only what is stored
+    // counts: columns past a row hold whatever follows it in memory.)
+    float odd = 0.f;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) odd = not_finite(acc[x][y], i0 + wi0 + x * 16 + a < p.I ? p.J - (j0 + wj0 + y * 16 + g * 4) : 0, odd);
+    if (__any(odd != odd)) {
 #pragma unroll
         for (int x = 0; x < 2; ++x)
 #pragma unroll

@@ -73,3 +73,17 @@ def test_operands_of_any_magnitude(x_exp, w_exp):
     want = O.gather_forward(np64(X), np64(case["Wg"]), case["Ind"].numpy())
     limit = 4 * 2.0 ** -24 * I ** 0.5 * np.sqrt((want ** 2).mean()) + 4 * 2.0 ** -150 * I ** 0.5
     assert np.sqrt(((np64(Y) - want) ** 2).mean()) <= limit
+
+
+def test_picks_that_do_not_exist_do_not_count_as_results():
+    """Picks out of range give zeros whatever the first token's row holds, and the picks beside them keep their bits."""
+    B, T, E, K, I, J = 4, 40, 16, 32, 64, 64
+    case = make_case(5, B, T, E, K, I, J, torch.float32)
+    Ind = case["Ind"].clamp(min=1)
+    Ind[:, :, 3], Ind[:, :, 20] = T, -1
+    got = []
+    for first in (0.0, float("nan")):
+        X = case["X"].clone()
+        X[:, 0] = first
+        got.append(products(case, dev(Ind), dev(X), dev(case["dOut"]))[0])
+    assert torch.equal(*got) and got[0][:, :, [3, 20]].eq(0).all()

@@ -103,3 +103,26 @@ def test_one_pick_is_one_rounding():
     token = case["Ind"][0, :, 0]
     assert torch.equal(dWg.cpu(), (x[token][:, :, None] * y[:, 0][:, None, :]).float())
     assert torch.equal(dWs.cpu(), (y[:, 0][:, :, None] * do[token][:, None, :]).float())
+
+
+@pytest.mark.parametrize("I, J", [(37, 29), (70, 66), (129, 1)])
+def test_what_lies_between_the_rows_does_not_count(I, J):
+    """Views whose gaps hold NaN give the bits of views whose gaps hold zeros: no wavefront does its tile again for columns nobody stores."""
+    B, T, E, K = 9, 21, 6, 60
+    case = make_case(13, B, T, E, K, I, J, torch.float32)
+    got = []
+    for gap in (0.0, float("nan")):
+        X = torch.full((B, T, I + 5), gap, device="cuda")
+        X[..., :I] = dev(case["X"])
+        dW = torch.empty(E, I, J, device="cuda")
+        dims = _abi.Dims(B, T, E, K, I, J)
+        n = _abi.lib().egs_workspace_bytes(_abi.OP_DW, 0, dims, _abi.F32)
+        ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+        Y = torch.full((B * E * K * J + 64,), gap, device="cuda")[:B * E * K * J].view(B, E, K, J).copy_(dev(case["Y"]))
+        Ind = dev(case["Ind"])
+        rc = _abi.lib().egs_dw(X.data_ptr(), Y.data_ptr(), Ind.data_ptr(), dW.data_ptr(), ws.data_ptr(), n, dims, X.stride(0), X.stride(1),
+                               _abi.F32, _abi.F32, _abi.IND_I64, 0, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        got.append(dW)
+    assert torch.equal(*got)
+    assert_close(got[0], O.gather_backward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy(), np64(case["Y"]))[1], torch.float32, "dW")
