@@ -46,6 +46,13 @@ __device__ __forceinline__ float not_finite(const f32x4 &v, int live, float t)
     for (int x = 0; x < 4; ++x) t = fmaf(x < live ? v[x] : 0.f, 0.f, t);
     return t;
 }
+// sums of split products out of their scale; where one is not finite, the second take's result instead.  (Element by element: which
+// bits a finite result has does not depend on its neighbours.)
+__device__ __forceinline__ void split_result(f32x4 &v, const f32x4 &second)
+{
+#pragma unroll
+    for (int x = 0; x < 4; ++x) v[x] = fabsf(v[x]) < __builtin_inff() ? v[x] * kSplitUnscale : second[x];
+}
 
 constexpr int kSplitP[6] = {2, 0, 1, 1, 0, 0}, kSplitQ[6] = {0, 2, 1, 0, 1, 0};   // pieces of the six products, the smallest first
 

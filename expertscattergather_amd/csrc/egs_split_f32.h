@@ -168,11 +168,12 @@ static __global__ __launch_bounds__(kThreads, 3) void tiled_dw_split_kernel(Tile
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y) odd = not_finite(acc[x][y], i0 + wi0 + x * 16 + a < p.I ? p.J - (j0 + wj0 + y * 16 + g * 4) : 0, odd);
+    f32x4 again[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) again[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (__any(odd != odd)) {
-#pragma unroll
-        for (int x = 0; x < 2; ++x)
-#pragma unroll
-            for (int y = 0; y < 2; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
         for (int m0 = lo; m0 < hi; m0 += 4) {
             int b;
@@ -192,16 +193,13 @@ static __global__ __launch_bounds__(kThreads, 3) void tiled_dw_split_kernel(Tile
 #pragma unroll
             for (int x = 0; x < 2; ++x)
 #pragma unroll
-                for (int y = 0; y < 2; ++y) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(yv[y], xv[x], acc[x][y], 0, 0, 0);
+                for (int y = 0; y < 2; ++y) again[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(yv[y], xv[x], again[x][y], 0, 0, 0);
         }
-    } else {
-#pragma unroll
-        for (int x = 0; x < 2; ++x)
-#pragma unroll
-            for (int y = 0; y < 2; ++y)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[x][y][r] *= kSplitUnscale;
     }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) split_result(acc[x][y], again[x][y]);
 
     // ---------------- lane (a, g) holds rows i0 + wi0 + 16 x + a, columns j0 + wj0 + 16 y + 4 g .. + 3; through LDS, so that whole
     // row (or, [E,J,I], column) segments leave

@@ -87,3 +87,18 @@ def test_picks_that_do_not_exist_do_not_count_as_results():
         X[:, 0] = first
         got.append(products(case, dev(Ind), dev(X), dev(case["dOut"]))[0])
     assert torch.equal(*got) and got[0][:, :, [3, 20]].eq(0).all()
+
+
+def test_finite_results_keep_their_bits_beside_others():
+    B, T, E, K, I, J = 4, 40, 16, 32, 128, 64
+    case = make_case(6, B, T, E, K, I, J, torch.float32)
+    Ind, dOut = dev(case["Ind"]), dev(case["dOut"])
+    plain = products(case, Ind, dev(case["X"]), dOut)[0]
+    W = case["Wg"].clone()
+    W[:, 5, 7], W[:, 6, 40], W[:, 7, 63] = float("inf"), float("nan"), 2.0 ** 113
+    got = products(dict(case, Wg=W), Ind, dev(case["X"]), dOut)[0]
+    columns = [j for j in range(J) if j not in (7, 40, 63)]
+    assert torch.equal(got[..., columns], plain[..., columns])
+    assert not got[..., [7, 40]].isfinite().any()
+    want = O.gather_forward(np64(case["X"]), np64(W[:, :, 63:]), case["Ind"].numpy())
+    assert_close(got[..., 63:], want, torch.float32, "Y")

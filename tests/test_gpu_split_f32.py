@@ -126,3 +126,18 @@ def test_what_lies_between_the_rows_does_not_count(I, J):
         got.append(dW)
     assert torch.equal(*got)
     assert_close(got[0], O.gather_backward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy(), np64(case["Y"]))[1], torch.float32, "dW")
+
+
+def test_finite_results_keep_their_bits_beside_others():
+    B, T, E, K, I, J = 4, 50, 3, 130, 70, 66
+    case = make_case(14, B, T, E, K, I, J, torch.float32)
+    Ind, Y = dev(case["Ind"]), dev(case["Y"])
+    plain = gradients(case, Ind, dev(case["X"]), Y)[0]
+    X = case["X"].clone()
+    X[:, :, 7], X[:, :, 40], X[:, :, 69] = float("inf"), float("nan"), 2.0 ** 113
+    got = gradients(case, Ind, dev(X), Y)[0]
+    rows = [i for i in range(I) if i not in (7, 40, 69)]
+    assert torch.equal(got[:, rows], plain[:, rows])
+    assert not got[:, [7, 40]].isfinite().any()
+    want = O.gather_backward(np64(X[:, :, 69:]), np64(case["Wg"][:, 69:]), case["Ind"].numpy(), np64(case["Y"]))[1]
+    assert_close(got[:, 69:], want, torch.float32, "dW")
