@@ -181,34 +181,40 @@ __global__ __launch_bounds__(64 * (16 / TQ), 4) void rows_small_f32_kernel(Small
 #pragma unroll
             for (int tn = 0; tn < TN; ++tn) odd = not_finite(acc[t][tn], live, odd);
         }
-        f32x4 again[TG][TN];
-#pragma unroll
-        for (int t = 0; t < TG; ++t)
-#pragma unroll
-            for (int tn = 0; tn < TN; ++tn) again[t][tn] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (__any(odd != odd)) {
+            f32x4 again[TG][TN];
+#pragma unroll
+            for (int t = 0; t < TG; ++t)
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn) again[t][tn] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int s = 0; s < KS; ++s)
 #pragma unroll
                 for (int t = 0; t < TG; ++t) {
                     const u32x4 x = lanes_4a_g_to_16g_a(xr[t0 + t][s], lane);
-#pragma unroll 1
+#pragma unroll
                     for (int c = 0; c < 4; ++c) {
-                        const float xc = bits_f32(c == 0 ? x[0] : c == 1 ? x[1] : c == 2 ? x[2] : x[3]);
                         const int k = s * 16 + g * 4 + c;
 #pragma unroll
                         for (int tn = 0; tn < TN; ++tn) {
                             const int n = tn * 16 + a;
-                            const float w = *reinterpret_cast<const float *>(We + (W_NMAJOR ? k * N + n : n * R + k) * 4);
-                            again[t][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, xc, again[t][tn], 0, 0, 0);
+                            const float w = *reinterpret_cast<const float *>(We + (uint32_t)((W_NMAJOR ? k * N + n : n * R + k) * 4));
+                            again[t][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, bits_f32(x[c]), again[t][tn], 0, 0, 0);
                         }
                     }
                 }
+#pragma unroll
+            for (int t = 0; t < TG; ++t)
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn) split_result(acc[t][tn], again[t][tn]);
+        } else {
+#pragma unroll
+            for (int t = 0; t < TG; ++t)
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) acc[t][tn][x] *= kSplitUnscale;
         }
-#pragma unroll
-        for (int t = 0; t < TG; ++t)
-#pragma unroll
-            for (int tn = 0; tn < TN; ++tn) split_result(acc[t][tn], again[t][tn]);
         // lane (a, g) holds, for pick 16 tq + a, columns 16 tn + 4 g .. + 3: the four lanes g of a pick write 64 contiguous bytes
 #pragma unroll
         for (int t = 0; t < TG; ++t) {
