@@ -75,7 +75,8 @@ int dw_general(const void *Xs, const void *Ys, const void *Ind, void *dW, void *
         return EGS_OK;
     }
     // operands of less than 16 bytes, which tiny_dw_kernel takes: whole sums, however many picks
-    const int S = x_span < 16 || y_span < 16 ? 1 : pl.S;
+    const bool split32 = pl.split32 && x_span < (1ull << 31) && y_span < (1ull << 31);
+    const int S = x_span < 16 || y_span < 16 ? 1 : split32 ? pl.f_S : pl.S;
     TiledDwParams q;
     memset(&q, 0, sizeof(q));
     q.Xs = p.Xs; q.Ys = p.Ys; q.Ind = Ind; q.dW = S > 1 ? (char *)workspace : (char *)dW;
@@ -83,8 +84,8 @@ int dw_general(const void *Xs, const void *Ys, const void *Ind, void *dW, void *
     q.ldx_b = ldx_b; q.ldx_t = ldx_t;
     q.B = d->B; q.T = d->T; q.E = d->E; q.K = d->K; q.I = d->I; q.J = d->J;
     q.ind_dtype = ind_dtype; q.out_dtype = out_dtype; q.eji = dw_layout != 0;
-    q.i_tiles = pl.i_tiles; q.j_tiles = pl.j_tiles; q.S = S; q.picks_per_split = pl.picks_per_split;
-    q.wide = pl.wide; q.split32 = pl.split32;
+    q.i_tiles = pl.i_tiles; q.j_tiles = pl.j_tiles; q.S = S; q.picks_per_split = split32 ? pl.f_picks_per_split : pl.picks_per_split;
+    q.wide = pl.wide; q.split32 = split32;
     q.edges = (d->I * ES) % 16 != 0 || (d->J * ES) % 16 != 0;
     const int rc = act_dtype == EGS_F32 ? tiled_dw_f32(q, s) : act_dtype == EGS_F16 ? tiled_dw_f16(q, s) : tiled_dw_bf16(q, s);
     if (rc != EGS_OK || S <= 1) return rc;

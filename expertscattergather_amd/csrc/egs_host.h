@@ -85,7 +85,8 @@ struct DwPlan {
     int b_bq, b_i_tiles, b_j_tiles, b_S, b_rows_per_split;  // its plan
     int b_tp;                                               // not 0: dw_strip_kernel, tiles of 32 b_tp x b_bq
     bool wide;                                              // tiled_dw_wide_kernel, in one pass
-    bool split32;                                           // fp32: tiled_dw_split_kernel, 64 x 64 tiles
+    bool split32;                                           // fp32: tiled_dw_split_kernel, 64 x 64 tiles, where the operands are below 2 GiB
+    int f_S, f_picks_per_split;                             // its splits
     size_t bytes_general, bytes_small, bytes_big;           // workspace of each of the three split kernels (0: no splits)
 };
 

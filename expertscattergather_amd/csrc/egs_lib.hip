@@ -239,19 +239,23 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
     const int64_t base = (int64_t)d->E * pl.i_tiles * pl.j_tiles;
     int64_t S = base > 0 ? 512 / base : 1;
     if (S > (Me + 1023) / 1024) S = (Me + 1023) / 1024;
+    if (S < 1) S = 1;
+    int64_t rows = Me > 0 ? ((Me + S - 1) / S + 127) / 128 * 128 : 128;
+    S = Me > 0 ? (Me + rows - 1) / rows : 1;
+    pl.S = (int)S;
+    pl.picks_per_split = (int)(rows < INT32_MAX ? rows : INT32_MAX);
     pl.split32 = act_dtype == EGS_F32 && (Me >= 512 || (Me >= 4 && dw_split32_slabs(d) >= 600));
     if (pl.split32) {
         // two workgroups per CU where that leaves four slabs or more to each
         const int64_t tiles = (int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, 64);
-        S = tiles > 0 ? 512 / tiles : 1;
-        if (S > Me / 128) S = Me / 128;
+        int64_t parts = tiles > 0 ? 512 / tiles : 1;
+        if (parts > Me / 128) parts = Me / 128;
+        if (parts < 1) parts = 1;
+        rows = ((Me + parts - 1) / parts + 31) / 32 * 32;
+        pl.f_S = (int)((Me + rows - 1) / rows);
+        pl.f_picks_per_split = (int)(rows < INT32_MAX ? rows : INT32_MAX);
+        if (S < pl.f_S) S = pl.f_S;         // workspace for either
     }
-    if (S < 1) S = 1;
-    const int64_t grain = pl.split32 ? 32 : 128;
-    int64_t rows = Me > 0 ? ((Me + S - 1) / S + grain - 1) / grain * grain : 128;
-    S = Me > 0 ? (Me + rows - 1) / rows : 1;
-    pl.S = (int)S;
-    pl.picks_per_split = (int)(rows < INT32_MAX ? rows : INT32_MAX);
     pl.wide = Me <= 128 || (Me <= 512 && dw_wide_tiles(d, act_dtype) >= 256) || dw_wide_tiles(d, act_dtype) >= 768;
     pl.bytes_general = S > 1 ? align_up((size_t)S * d->E * d->I * d->J * 4, 256) : 256;     // never none: this path always has a workspace
 

@@ -403,7 +403,7 @@ struct TiledDwParams {
     int32_t ind_dtype, out_dtype, eji;
     int32_t i_tiles, j_tiles, S, picks_per_split;
     int32_t wide;               // tiled_dw_wide_kernel (S = 1)
-    int32_t split32;            // fp32: tiled_dw_split_kernel (egs_split_f32.h), for operands below 2 GiB
+    int32_t split32;            // fp32: tiled_dw_split_kernel (egs_split_f32.h); operands below 2 GiB
     int32_t edges;              // some row is not a whole number of chunks: chunks may have to be read early and shifted
 };
 // what a pick that does not exist reads instead of a row

@@ -62,7 +62,7 @@ int launch_tiled_dw(TiledDwParams &p, hipStream_t s)
         return EGS_OK;
     }
     if constexpr (TT::ES == 4) {
-        if (p.split32 && p.x_bytes < (int64_t)1 << 31 && p.y_bytes < (int64_t)1 << 31) {
+        if (p.split32) {
             p.i_tiles = ceil_div(p.I, SplitDwLds::T); p.j_tiles = ceil_div(p.J, SplitDwLds::T);
             const int64_t tiles = (int64_t)p.E * p.i_tiles * p.j_tiles * p.S;
             if (tiles > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
@@ -72,7 +72,7 @@ int launch_tiled_dw(TiledDwParams &p, hipStream_t s)
             return EGS_OK;
         }
     }
-    if (p.wide && p.S == 1) {
+    if (p.wide) {
         typedef TiledDwWide<TT> L;
         p.i_tiles = ceil_div(p.I, L::TI); p.j_tiles = ceil_div(p.J, L::TJ);
         const int64_t wide = (int64_t)p.E * p.i_tiles * p.j_tiles;

@@ -141,3 +141,20 @@ def test_finite_results_keep_their_bits_beside_others():
     assert not got[:, [7, 40]].isfinite().any()
     want = O.gather_backward(np64(X[:, :, 69:]), np64(case["Wg"][:, 69:]), case["Ind"].numpy(), np64(case["Y"]))[1]
     assert_close(got[:, 69:], want, torch.float32, "dW")
+
+
+def test_sources_from_2_gib_on():
+    """A view that spans more than 2 GiB: the fp32 instruction's kernel, in as many parts as that one takes."""
+    B, T, E, K, I, J = 3, 30, 2, 200, 70, 66
+    case = make_case(15, B, T, E, K, I, J, torch.float32)
+    X = torch.empty(2 * (2 ** 28 + 64) + T * I, device="cuda").as_strided((B, T, I), (2 ** 28 + 64, I, 1)).copy_(case["X"])
+    Y, Ind = dev(case["Y"]), dev(case["Ind"])
+    dW = torch.empty(E, I, J, device="cuda")
+    dims = _abi.Dims(B, T, E, K, I, J)
+    n = _abi.lib().egs_workspace_bytes(_abi.OP_DW, 0, dims, _abi.F32)
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    with _abi.launch_log() as log:
+        rc = _abi.lib().egs_dw(X.data_ptr(), Y.data_ptr(), Ind.data_ptr(), dW.data_ptr(), ws.data_ptr(), n, dims, X.stride(0), X.stride(1),
+                               _abi.F32, _abi.F32, _abi.IND_I64, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and log.kernels == ["tiled_dw_kernel"], (rc, log.kernels)
+    assert_close(dW, O.gather_backward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy(), np64(case["Y"]))[1], torch.float32, "dW")
