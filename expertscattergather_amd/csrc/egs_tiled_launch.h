@@ -68,7 +68,7 @@ int launch_tiled_dw(TiledDwParams &p, hipStream_t s)
             if (tiles > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
             static_assert(SplitDwLds::BYTES <= 64 * 1024, "no grant needed");
             hipLaunchKernelGGL(tiled_dw_split_kernel, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(kThreads), SplitDwLds::BYTES, s, p);
-            EGS_CHECK_LAUNCH("tiled_dw_wide_kernel");                   // (of which it is the fp32 form)
+            EGS_CHECK_LAUNCH("tiled_dw_split_kernel");
             return EGS_OK;
         }
     }

@@ -25,7 +25,7 @@ def gradients(case, Ind, X, Y):
                                            ((8, 40, 3, 65, 65, 63), True),          # one past a tile, one short of one; 520 picks
                                            ((5, 30, 2, 103, 129, 1), True),         # 515 picks, a column tile of one column
                                            ((3, 50, 150, 33, 70, 130), False),      # 99 picks: four slabs, the last of three; 900 tiles
-                                           ((1, 9, 640, 1, 3, 5), False),           # one pick per expert; rows shorter than a chunk
+                                           ((1, 9, 640, 4, 3, 5), False),           # four picks per expert; rows shorter than a chunk
                                            ((26, 33, 64, 20, 66, 64), True)], ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else None)
 def test_weight_gradient_of_split_floats(shape, splits):
     B, T, E, K, I, J = shape
@@ -35,7 +35,7 @@ def test_weight_gradient_of_split_floats(shape, splits):
         Ind[0, 0, 0], Ind[-1, -1, -1] = T, -1
         Y[0, 0, 0] = Y[-1, -1, -1] = float("nan")               # picks that do not exist do not count, whatever their rows hold
     dWg, dWs, kernels = gradients(case, dev(Ind), dev(case["X"]), dev(Y))
-    assert kernels.count("tiled_dw_wide_kernel") == 2 and ("tiled_dw_sum_kernel" in kernels) == splits, kernels
+    assert kernels.count("tiled_dw_split_kernel") == 2 and ("tiled_dw_sum_kernel" in kernels) == splits, kernels
     safe, Yk = Ind.clamp(0, T - 1).numpy(), np64(Y)
     if B * K > 1:
         Yk[0, 0, 0] = Yk[-1, -1, -1] = 0
@@ -53,7 +53,7 @@ def test_views_that_end_in_the_middle_of_a_chunk():
     X = wide[wide.numel() - ((B - 1) * T * 41 + (T - 1) * 41 + I):].as_strided((B, T, I), (T * 41, 41, 1))
     X.copy_(case["X"])
     dWg, dWs, kernels = gradients(case, dev(case["Ind"]), X, dev(case["Y"]))
-    assert kernels.count("tiled_dw_wide_kernel") == 2, kernels
+    assert kernels.count("tiled_dw_split_kernel") == 2, kernels
     assert_close(dWg, O.gather_backward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy(), np64(case["Y"]))[1], torch.float32, "dWg")
     assert_close(dWs, O.scatter_backward(np64(case["Y"]), np64(case["Ws"]), case["Ind"].numpy(), np64(case["dOut"]))[1], torch.float32, "dWs")
 
@@ -69,7 +69,9 @@ def test_values_that_have_no_three_pieces():
     X[2, T - 2, 69] = float("nan")
     X[3, T - 3, 64] = 3.4e38
     Y[3, 2, 11] *= 1e-3
-    got = gradients(case, dev(Ind), dev(X), dev(Y))[0].cpu().double()
+    got, _, kernels = gradients(case, dev(Ind), dev(X), dev(Y))
+    assert kernels.count("tiled_dw_split_kernel") == 2, kernels
+    got = got.cpu().double()
     bi = torch.arange(B)[:, None, None]
     want = torch.einsum("beki,bekj->eij", X.double()[bi, Ind], Y.double())
     assert torch.equal(got.isnan(), want.isnan()) and want.isnan().sum() == J
@@ -88,6 +90,7 @@ def test_operands_of_any_magnitude(x_exp, y_exp):
     case = make_case(11, B, T, E, K, I, J, torch.float32)
     X, Y = (case["X"].double() * 2.0 ** x_exp).float(), (case["Y"].double() * 2.0 ** y_exp).float()
     dWg, _, kernels = gradients(case, dev(case["Ind"]), dev(X), dev(Y))
+    assert kernels.count("tiled_dw_split_kernel") == 2, kernels
     want = O.gather_backward(np64(X), np64(case["Wg"]), case["Ind"].numpy(), np64(Y))[1]
     n = (B * K) ** 0.5
     limit = 4 * 2.0 ** -24 * n * np.sqrt((want ** 2).mean()) + 4 * 2.0 ** -150 * n
@@ -98,7 +101,8 @@ def test_one_pick_is_one_rounding():
     """The weight gradient of an expert with one pick: each product rounded once, as fp32 gives it."""
     B, T, E, K, I, J = 1, 9, 640, 1, 67, 35
     case = make_case(12, B, T, E, K, I, J, torch.float32)
-    dWg, dWs, _ = gradients(case, dev(case["Ind"]), dev(case["X"]), dev(case["Y"]))
+    dWg, dWs, kernels = gradients(case, dev(case["Ind"]), dev(case["X"]), dev(case["Y"]))
+    assert kernels.count("tiled_dw_wide_kernel") == 2, kernels
     x, y, do = (t.double()[0] for t in (case["X"], case["Y"], case["dOut"]))
     token = case["Ind"][0, :, 0]
     assert torch.equal(dWg.cpu(), (x[token][:, :, None] * y[:, 0][:, None, :]).float())
@@ -120,9 +124,10 @@ def test_what_lies_between_the_rows_does_not_count(I, J):
         ws = torch.empty(n, dtype=torch.uint8, device="cuda")
         Y = torch.full((B * E * K * J + 64,), gap, device="cuda")[:B * E * K * J].view(B, E, K, J).copy_(dev(case["Y"]))
         Ind = dev(case["Ind"])
-        rc = _abi.lib().egs_dw(X.data_ptr(), Y.data_ptr(), Ind.data_ptr(), dW.data_ptr(), ws.data_ptr(), n, dims, X.stride(0), X.stride(1),
-                               _abi.F32, _abi.F32, _abi.IND_I64, 0, torch.cuda.current_stream().cuda_stream)
-        assert rc == 0
+        with _abi.launch_log() as log:
+            rc = _abi.lib().egs_dw(X.data_ptr(), Y.data_ptr(), Ind.data_ptr(), dW.data_ptr(), ws.data_ptr(), n, dims, X.stride(0), X.stride(1),
+                                   _abi.F32, _abi.F32, _abi.IND_I64, 0, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0 and log.kernels[0] == "tiled_dw_split_kernel", (rc, log.kernels)
         got.append(dW)
     assert torch.equal(*got)
     assert_close(got[0], O.gather_backward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy(), np64(case["Y"]))[1], torch.float32, "dW")
@@ -135,7 +140,8 @@ def test_finite_results_keep_their_bits_beside_others():
     plain = gradients(case, Ind, dev(case["X"]), Y)[0]
     X = case["X"].clone()
     X[:, :, 7], X[:, :, 40], X[:, :, 69] = float("inf"), float("nan"), 2.0 ** 113
-    got = gradients(case, Ind, dev(X), Y)[0]
+    got, _, kernels = gradients(case, Ind, dev(X), Y)
+    assert kernels.count("tiled_dw_split_kernel") == 2, kernels
     rows = [i for i in range(I) if i not in (7, 40, 69)]
     assert torch.equal(got[:, rows], plain[:, rows])
     assert not got[:, [7, 40]].isfinite().any()
