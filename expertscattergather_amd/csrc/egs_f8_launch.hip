@@ -116,7 +116,7 @@ int egs_gather_gemm_fp8act(const void *X, const void *Wq, const float *w_scale, 
     if (grid > INT32_MAX) return EGS_ERR_BAD_SHAPE;
     if (large) hipLaunchKernelGGL((rows_gemm_f8_kernel<256, 256>), dim3((unsigned)grid), dim3(kF8Threads), 0, s, p);
     else hipLaunchKernelGGL((rows_gemm_f8_kernel<128, 128>), dim3((unsigned)grid), dim3(kF8Threads), 0, s, p);
-    EGS_CHECK_LAUNCH("rows_gemm_f8_kernel");
+    EGS_CHECK_LAUNCH(large ? "rows_gemm_f8_kernel<256>" : "rows_gemm_f8_kernel<128>");
     return EGS_OK;
 }
 

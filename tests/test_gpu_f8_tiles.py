@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+from expertscattergather_amd import _abi
 from expertscattergather_amd import hip_kernels as hk
 from expertscattergather_amd import workloads as wl
 from oracle import egs_oracle as O
@@ -21,7 +22,9 @@ def test_small_tiles_match_the_quantised_oracle(shape):
     case["Ind"][0, 0, 0] = T                                 # contributes a zero row
     case["Ind"][-1, -1, -1] = -1
     Wq, scale = wl.quantize_fp8_weights(case["Wg"].float())
-    Y = hk.expert_gather_fp8_forward(dev(case["X"]), dev(Wq), dev(scale), dev(case["Ind"]))
+    with _abi.launch_log() as log:
+        Y = hk.expert_gather_fp8_forward(dev(case["X"]), dev(Wq), dev(scale), dev(case["Ind"]))
+    assert log.kernels[-1] == "rows_gemm_f8_kernel<128>", log.kernels
     ind = case["Ind"].numpy().astype(np.int64)
     live = (ind >= 0) & (ind < T)
     ref = O.gather_forward_fp8(case["X"].float().numpy(), Wq.view(torch.uint8).numpy(), scale.numpy(), np.where(live, ind, 0)) * live[..., None]
@@ -33,9 +36,13 @@ def test_small_and_large_tiles_give_the_same_bits():
     case = make_case(48, 20, 300, 64, 50, 1152, 496, torch.bfloat16)
     Wq, scale = wl.quantize_fp8_weights(case["Wg"].float())
     X, q, sc, ind = dev(case["X"]), dev(Wq), dev(scale), dev(case["Ind"])
-    Y = hk.expert_gather_fp8_forward(X, q, sc, ind)
+    with _abi.launch_log() as log:
+        Y = hk.expert_gather_fp8_forward(X, q, sc, ind)
+    assert log.kernels[-1] == "rows_gemm_f8_kernel<256>", log.kernels
     for e in range(0, 64, 8):
-        part = hk.expert_gather_fp8_forward(X, q[e:e + 8].contiguous(), sc[e:e + 8].contiguous(), ind[:, e:e + 8].contiguous())
+        with _abi.launch_log() as log:
+            part = hk.expert_gather_fp8_forward(X, q[e:e + 8].contiguous(), sc[e:e + 8].contiguous(), ind[:, e:e + 8].contiguous())
+        assert log.kernels[-1] == "rows_gemm_f8_kernel<128>", log.kernels
         assert torch.equal(Y[:, e:e + 8], part)
 
 
