@@ -201,7 +201,6 @@ int rows_strip(RowsGemmParams &p, int act_dtype, bool w_trans, bool gather, int 
     if (g_force_generic || act_dtype == EGS_F32 || !p.a_vec || !p.w_vec || p.a_bytes == 0 || !aligned_to(p.W, 16) || !aligned_to(p.C, 16) ||
         p.R % 8 != 0 || p.N % 8 != 0 || (uint64_t)p.R * p.N * 2 >= (1ull << 31) || p.w_scale != nullptr)
         return EGS_OK;
-    if (!gather && p.bias != nullptr) return EGS_OK;        // biased product rows: the general kernel's route is the one that is tested
     const int64_t Me = (int64_t)p.B * p.K, strips = p.E * ((Me + 127) / 128) * ceil_div(p.N, 64);
     const bool filled = (double)Me * p.N * p.E >= 0.6 * 128 * 64 * (double)strips;
     if (strips < (filled ? 64 : 1500)) return EGS_OK;

@@ -168,12 +168,12 @@ def test_scatter_cut_into_uneven_batch_groups():
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("dims, kernels", [
-    ((10, 256, 128, 64, 1024, 128), ["rows_gemm_dl_kernel", "rows_gemm_dl_kernel", "tiled_rows_kernel"]),       # groups of 4, 4 and 2
-    ((19, 300, 37, 255, 1024, 192), ["rows_gemm_dl_kernel"] * 6 + ["tiled_rows_kernel"]),                       # six of 3 and one of 1
+    ((10, 256, 128, 64, 1024, 128), ["rows_gemm_dl_kernel", "rows_gemm_dl_kernel", "rows_strip_kernel"]),       # groups of 4, 4 and 2
+    ((19, 300, 37, 255, 1024, 192), ["rows_gemm_dl_kernel"] * 6 + ["rows_strip_kernel"]),                       # six of 3 and one of 1
     ((8, 256, 128, 64, 1024, 128), ["rows_gemm_dl_kernel"] * 2)], ids=["4+4+2", "6x3+1", "4+4"])
 def test_bias_of_a_scatter_cut_into_batch_groups(dims, kernels, dtype):
-    """A last group with fewer rows per expert than the large product kernel takes runs the tiled one, which adds the bias to its rows;
-    the other groups' bias is added afterwards.  Elements on both sides of every group boundary against the oracle."""
+    """A last group with fewer rows per expert than the large product kernel takes runs the one for mid-sized experts, which adds the bias to
+    its rows; the other groups' bias is added afterwards.  Elements on both sides of every group boundary against the oracle."""
     B, T, E, K, I, J = dims
     gen = torch.Generator().manual_seed(sum(dims))
     Y, Ws = torch.randn(B, E, K, J, generator=gen).to(dtype), (torch.randn(E, J, I, generator=gen) / J ** 0.5).to(dtype)

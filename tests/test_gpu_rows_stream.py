@@ -85,6 +85,24 @@ def test_bias_and_activation(act):
     assert_close(Y, want.numpy(), torch.bfloat16, act)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_scatter_with_bias(dtype):
+    B, T, E, K, I, J = 3, 40, 7, 11, 136, 448
+    case = make_case(10, B, T, E, K, I, J, dtype)
+    Ind = case["Ind"].clone()
+    Ind[0, 0, 0], Ind[-1, -1, -1] = T, -1
+    bias = torch.randn(E, 1, I, generator=torch.Generator().manual_seed(2)).to(dtype)
+    with _abi.launch_log() as log:
+        out = hk.expert_scatter(dev(case["Y"]), dev(case["Ws"]), dev(Ind), T, "deterministic", dev(bias))
+    assert log.kernels == ["rows_stream_kernel", "token_sum_kernel"], log.kernels
+    keep = (Ind >= 0) & (Ind < T)
+    picks = torch.zeros(B * T, E, dtype=torch.float64)
+    b, e, _ = keep.nonzero(as_tuple=True)
+    picks.index_put_((Ind[keep] + b * T, e), torch.ones((), dtype=torch.float64), accumulate=True)
+    want = O.scatter_forward(np64(case["Y"]) * keep.numpy()[..., None], np64(case["Ws"]), Ind.clamp(0, T - 1).numpy(), T)
+    assert_close(out, want + (picks.numpy() @ np64(bias[:, 0])).reshape(B, T, I), dtype, "out")
+
+
 def test_weights_past_the_caches():
     """More than 128 MB of weights under a single row tile: read past the caches."""
     B, T, E, K, I, J = 1, 64, 131, 20, 1024, 512

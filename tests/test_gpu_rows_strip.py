@@ -89,3 +89,33 @@ def test_bias_and_activation(act):
         want = O.gather_forward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy())
         want = want + np64(bias)[None, :, None, :] if act == "none" else want.clip(0)
         assert_close(got, want, torch.bfloat16, "Y")
+
+
+@pytest.mark.parametrize("mode", ["deterministic", "atomic"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_scatter_with_bias(dtype, mode):
+    """The rows come with their bias, in fp32 or (atomic mode) in the element type: the general kernel's bits."""
+    B, T, E, K, I, J = 3, 400, 24, 70, 120, 200
+    case = make_case(10, B, T, E, K, I, J, dtype)
+    Ind = case["Ind"].clone()
+    Ind[0, 0, 0], Ind[-1, -1, -1] = T, -1
+    bias = torch.randn(E, 1, I, generator=torch.Generator().manual_seed(2)).to(dtype)
+    Y, Ws, Id, bd = (dev(t) for t in (case["Y"], case["Ws"], Ind, bias))
+
+    def run():
+        with _abi.launch_log() as log:
+            out = hk.expert_scatter(Y, Ws, Id, T, mode, bd)
+        return out, log.kernels
+
+    got, kernels = run()
+    assert kernels == ["rows_strip_kernel", "token_sum_kernel"], kernels
+    plain, kernels = in_general(run)
+    assert kernels == ["tiled_rows_kernel", "token_sum_kernel"], kernels
+    assert torch.equal(got, plain)
+    if mode == "deterministic":
+        keep = (Ind >= 0) & (Ind < T)
+        picks = torch.zeros(B * T, E, dtype=torch.float64)
+        b, e, _ = keep.nonzero(as_tuple=True)
+        picks.index_put_((Ind[keep] + b * T, e), torch.ones((), dtype=torch.float64), accumulate=True)
+        want = O.scatter_forward(np64(case["Y"]) * keep.numpy()[..., None], np64(case["Ws"]), Ind.clamp(0, T - 1).numpy(), T)
+        assert_close(got, want + (picks.numpy() @ np64(bias[:, 0])).reshape(B, T, I), dtype, "out")
