@@ -152,16 +152,32 @@ int64_t dw_wide_tiles(const egs_dims *d, int act_dtype)
 }
 bool dw_few_picks(const egs_dims *d, int act_dtype) { return (int64_t)d->B * d->K <= 256 && dw_wide_tiles(d, act_dtype) >= 256; }
 
-// fp32: 32-pick slabs that the 64 x 64 tiles of tiled_dw_split_kernel go through in all.  It is the faster one above some hundred: us, it and
-// the fp32 instruction, by slabs: 42 (B6 T3171 E5 K31 I28 J249) 8.6 / 7.8, 294 (E42 of 196 picks, I32 J116) 9.2 / 7.7, 288 (E9 of 98, I96 J224) 7.4 / 8.2,
-// 660 (B1 T712 E125 K155 I369 J128) 28.4 / 34.5, 2352 (B9 T484 E98 K28 I160 J32) 14.5 / 17.5, 55000 135 / 202.  Few tiles of many picks gain at any
-// number (8 tiles, 774 picks 11.3 / 15.1).  Against the aligned tiles of dw_tile_body, which are narrower: 4096 (B64 T256 E32 K32 I128 J64) 21 / 20,
-// 9450 (B16 T61 E14 K45 I960 J96) 30 / 50, 16384 43 / 66 and 46 / 60; with 32 columns of a tile empty (I32 J96, 7676) 41 / 30.
-// Not below four picks, where its six roundings of a product stand against no more of the fp32 instruction's: error of the result, it and that,
-// 1 pick 3.5e-8 / 2.5e-8, 2 3.4e-8 / 3.1e-8, 4 3.3e-8 / 4.0e-8, 32 3.8e-8 / 10.3e-8.
+// fp32: 32-pick slabs that the 64 x 64 tiles of tiled_dw_split_kernel go through in all
 int64_t dw_split32_slabs(const egs_dims *d)
 {
     return (int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, 64) * (((int64_t)d->B * d->K + 31) / 32);
+}
+
+// Is tiled_dw_split_kernel, in the parts of `pl`, the faster one?  Some hundred slabs are needed in any case.
+// Against tiled_dw_wide_kernel, which has the same tiles: from 64 picks on (us, it / that: 12 picks 19.6 / 16.8, 20 picks 9.4 / 8.5, 34 picks
+// 12.7 / 12.0, 48 level, 99 picks at B3 E150 I70 J130 0.91 of it, 155 picks at B1 T712 E125 I369 J128 28.4 / 34.5).
+// Against the 32 x 32 tiles of tiled_dw_kernel by the time that the fullest CU takes, fitted to 1101 sizes alone on the device: up to three
+// workgroups of it on a CU, two of those, each some us, and some for every 32 picks (128) that a CU's workgroups go through, plus the
+// second pass.  Within 10 and 12 % of the time at 95 % of the sizes; by it 6 sizes are 3 % slower than they could be and none more than
+// 10 %.  us, it / that: B53 T97 E29 K41 I111 J75 30 / 43, B12 T121 E52 K61 I272 J31 (59 % of the tiles empty) 30 / 18.6, B26 T665 E30 K30 I523
+// J32 33 / 23.5, B20 T289 E33 K163 I693 J29 111 / 90.
+bool dw_split32_pays(const egs_dims *d, const DwPlan &pl)
+{
+    const int64_t Me = (int64_t)d->B * d->K;
+    if (Me < 512 && dw_split32_slabs(d) < 600) return false;
+    if (pl.wide) return Me >= 64;
+    const int64_t split = ((int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, 64) * pl.f_S + 255) / 256;
+    const int64_t plain = ((int64_t)d->E * pl.i_tiles * pl.j_tiles * pl.S + 255) / 256;
+    const double elems = (double)d->E * d->I * d->J;
+    const double split_us = 6.2 * (double)((split + 2) / 3) + 0.56 * (double)split * (pl.f_picks_per_split / 32) + (pl.f_S > 1 ? 1.9 + 2.5e-6 * pl.f_S * elems : 0.0);
+    const double plain_us = 2.7 + 3.4 * (double)((plain + 1) / 2) + 1.08 * (double)plain * (((int64_t)pl.picks_per_split + 127) / 128) +
+                            (pl.S > 1 ? 3.0 + 2.8e-6 * pl.S * elems : 0.0);
+    return split_us < 0.97 * plain_us;
 }
 
 // 16-bit weight gradients in strips: the tile (32 tp x bq) and the number of splits of the picks that dw_strip_kernel is expected to be
@@ -244,8 +260,8 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
     S = Me > 0 ? (Me + rows - 1) / rows : 1;
     pl.S = (int)S;
     pl.picks_per_split = (int)(rows < INT32_MAX ? rows : INT32_MAX);
-    pl.split32 = act_dtype == EGS_F32 && (Me >= 512 || (Me >= 4 && dw_split32_slabs(d) >= 600));
-    if (pl.split32) {
+    pl.wide = Me <= 128 || (Me <= 512 && dw_wide_tiles(d, act_dtype) >= 256) || dw_wide_tiles(d, act_dtype) >= 768;
+    if (act_dtype == EGS_F32 && Me > 0) {
         // two workgroups per CU where that leaves four slabs or more to each
         const int64_t tiles = (int64_t)d->E * ceil_div(d->I, 64) * ceil_div(d->J, 64);
         int64_t parts = tiles > 0 ? 512 / tiles : 1;
@@ -254,9 +270,9 @@ DwPlan plan_dw(const egs_dims *d, int act_dtype)
         rows = ((Me + parts - 1) / parts + 31) / 32 * 32;
         pl.f_S = (int)((Me + rows - 1) / rows);
         pl.f_picks_per_split = (int)(rows < INT32_MAX ? rows : INT32_MAX);
-        if (S < pl.f_S) S = pl.f_S;         // workspace for either
+        pl.split32 = dw_split32_pays(d, pl);
+        if (pl.split32 && S < pl.f_S) S = pl.f_S;       // workspace for either
     }
-    pl.wide = Me <= 128 || (Me <= 512 && dw_wide_tiles(d, act_dtype) >= 256) || dw_wide_tiles(d, act_dtype) >= 768;
     pl.bytes_general = S > 1 ? align_up((size_t)S * d->E * d->I * d->J * 4, 256) : 256;     // never none: this path always has a workspace
 
     // large 16-bit shapes: 256 x 256 (or 256 x 128) tiles, 64-row slabs, splits only to give every CU a workgroup
@@ -450,6 +466,8 @@ bool make_dw_tile(const void *Xs, const void *Ys, const void *Ind, void *dW, con
 {
     if (g_force_generic) return false;
     const int ES = elem_size(act_dtype);
+    // (fp32, the bf16 instruction's 64 x 64 tiles / these, us, by slabs: 4096 (B64 T256 E32 K32 I128 J64) 21 / 20, 9450 (B16 T61 E14 K45 I960 J96)
+    // 30 / 50, 16384 43 / 66 and 46 / 60; with 32 columns of a tile empty (I32 J96, 7676) 41 / 30)
     if (ES == 4 && d->I > 32 && d->J > 32 && dw_split32_slabs(d) >= 8192) return false;
     if (dw_strip_narrow(d, act_dtype)) return false;
     if (d->I % 8 || d->J % 8 || d->I < 8 || d->J < 8 || d->I > 2048 || d->J > 128) return false;

@@ -21,12 +21,12 @@ def gradients(case, Ind, X, Y):
     return dWg, dWs, log.kernels
 
 
-@pytest.mark.parametrize("shape, splits", [((8, 40, 2, 64, 64, 64), True),          # whole tiles and slabs; 512 picks
+@pytest.mark.parametrize("shape, splits", [((8, 40, 4, 128, 64, 64), True),         # whole tiles and slabs; 1024 picks
                                            ((8, 40, 3, 65, 65, 63), True),          # one past a tile, one short of one; 520 picks
                                            ((5, 30, 2, 103, 129, 1), True),         # 515 picks, a column tile of one column
                                            ((3, 50, 150, 33, 70, 130), False),      # 99 picks: four slabs, the last of three; 900 tiles
-                                           ((1, 9, 640, 4, 3, 5), False),           # four picks per expert; rows shorter than a chunk
-                                           ((26, 33, 64, 20, 66, 64), True)], ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else None)
+                                           ((16, 9, 320, 4, 3, 5), False),          # 64 picks per expert; rows shorter than a chunk
+                                           ((26, 33, 48, 20, 66, 64), True)], ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else None)
 def test_weight_gradient_of_split_floats(shape, splits):
     B, T, E, K, I, J = shape
     case = make_case(sum(shape), *shape, torch.float32)
@@ -112,7 +112,7 @@ def test_one_pick_is_one_rounding():
 @pytest.mark.parametrize("I, J", [(37, 29), (70, 66), (129, 1)])
 def test_what_lies_between_the_rows_does_not_count(I, J):
     """Views whose gaps hold NaN give the bits of views whose gaps hold zeros: no wavefront does its tile again for columns nobody stores."""
-    B, T, E, K = 9, 21, 6, 60
+    B, T, E, K = 9, 21, 5, 60
     case = make_case(13, B, T, E, K, I, J, torch.float32)
     got = []
     for gap in (0.0, float("nan")):
@@ -164,3 +164,15 @@ def test_sources_from_2_gib_on():
                                _abi.F32, _abi.F32, _abi.IND_I64, 0, torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and log.kernels == ["tiled_dw_kernel"], (rc, log.kernels)
     assert_close(dW, O.gather_backward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy(), np64(case["Y"]))[1], torch.float32, "dW")
+
+
+@pytest.mark.parametrize("shape, kernel", [((12, 121, 52, 61, 272, 31), "tiled_dw_kernel"),         # 59 % of the 64 x 64 tiles empty
+                                           ((26, 60, 30, 30, 523, 32), "tiled_dw_kernel"),
+                                           ((1, 40, 640, 40, 3, 5), "tiled_dw_wide_kernel"),        # fewer than 64 picks
+                                           ((8, 30, 90, 8, 66, 130), "tiled_dw_split_kernel"),      # 64 picks
+                                           ((53, 97, 29, 41, 111, 75), "tiled_dw_split_kernel")], ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else None)
+def test_where_the_split_kernel_is_taken(shape, kernel):
+    case = make_case(16, *shape, torch.float32)
+    dWg, _, kernels = gradients(case, dev(case["Ind"]), dev(case["X"]), dev(case["Y"]))
+    assert kernels.count(kernel) == 2, kernels
+    assert_close(dWg, O.gather_backward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy(), np64(case["Y"]))[1], torch.float32, "dW")
