@@ -467,14 +467,15 @@ __device__ __forceinline__ void csr_count_half_body(int32_t *sh, int b, int h, i
 }
 
 
-static __global__ __launch_bounds__(1024) void csr_count_kernel(const void *Ind, int32_t ind_dtype, int32_t T, int32_t N,
-                                                         int32_t *seg_off, int32_t *perm, int32_t *rank_tmp,
-                                                         int32_t *long_tab, int32_t parts)
+// PARTED: `parts` workgroups share a batch element's table
+template <bool PARTED>
+__global__ __launch_bounds__(1024) void csr_count_kernel(const void *Ind, int32_t ind_dtype, int32_t T, int32_t N, int32_t *seg_off, int32_t *perm,
+                                                         int32_t *rank_tmp, int32_t *long_tab, int32_t parts)
 {
     extern __shared__ int32_t sh_cnt_dyn[];
-    const int b = (int)blockIdx.x / parts;
+    const int b = PARTED ? (int)blockIdx.x / parts : (int)blockIdx.x;
     csr_count_body(sh_cnt_dyn, b, b, (int)threadIdx.x, (int)blockDim.x, Ind, ind_dtype, T, N, seg_off, perm,
-                   rank_tmp, long_tab, NoPrefetch(), (int)blockIdx.x - b * parts, parts);
+                   rank_tmp, long_tab, NoPrefetch(), PARTED ? (int)blockIdx.x - b * parts : 0, PARTED ? parts : 1);
 }
 
 // Fast version for N <= 32768 picks whose (token, pick) pair fits 32 bits: one workgroup per

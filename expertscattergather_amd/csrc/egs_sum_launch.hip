@@ -22,16 +22,18 @@ int launch_routing_table(const void *Ind, int ind_dtype, const egs_dims *d, int3
         while (nw > 1 && csr_count_lds(d->T, nw) > budget) nw >>= 1;
         const size_t lds = csr_count_lds(d->T, nw);
         if (lds <= budget) {
-            static LdsGrant told;
-            const int rc_lds = allow_large_lds((const void *)csr_count_kernel, told, lds, "hipFuncSetAttribute(csr_count_kernel)");
+            // Several workgroups per table where a wavefront has more than four chunks of 64 picks, which it ranks one after the other: 16 us
+            // for the 18 chunks of 17670 picks.  Every part also counts all picks, so not below that (us more with two parts at one to three
+            // chunks: 0.5 to 1.3), and as many as there are CUs for, one workgroup each: scatters at B46 T1359 E128 K84 with one part 94.7, two
+            // 84.5, four 81.8, six 94.0; B99 T1086 E128 K181 314, 306, 314, 328; B1 T1133 E64 K211 41.7, 31.9, 28.3 and with eight 25.8.
+            const int64_t per = (int64_t)nw * 128, want = N <= 2 * per ? 1 : (N + per - 1) / per;
+            const int64_t most = d->B >= 256 ? 1 : 256 / d->B < 8 ? 256 / d->B : 8;
+            const int parts = (int)(want > most ? most : want);
+            const auto kernel = parts > 1 ? csr_count_kernel<true> : csr_count_kernel<false>;
+            static LdsGrant told[2];
+            const int rc_lds = allow_large_lds((const void *)kernel, told[parts > 1], lds, "hipFuncSetAttribute(csr_count_kernel)");
             if (rc_lds != EGS_OK) return rc_lds;
-            // Several workgroups per table: a wavefront ranks its picks 64 at a time, one chunk after the other, 16 us for the
-            // 18 chunks of 17670 picks (B2 T1917 E95 K186 I416 J32, scatter with a table of one workgroup 75 us, of three 58, of five 56, of eight 53.5;
-            // B1 T4096 E100 K256 89 and 55; level below 2000 picks), and every part counts all picks.
-            const int64_t per = (int64_t)nw * 128, want = (N + per - 1) / per;
-            const int parts = (int)(want > 8 ? 8 : want);
-            if ((int64_t)d->B * parts > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
-            hipLaunchKernelGGL(csr_count_kernel, dim3(d->B * parts), dim3(64 * nw), lds, s, Ind, ind_dtype, d->T, (int32_t)N, seg_off, perm, rank_tmp, long_tab, parts);
+            hipLaunchKernelGGL(kernel, dim3(d->B * parts), dim3(64 * nw), lds, s, Ind, ind_dtype, d->T, (int32_t)N, seg_off, perm, rank_tmp, long_tab, parts);
             EGS_CHECK_LAUNCH("csr_count_kernel");
             return EGS_OK;
         }
