@@ -18,7 +18,7 @@ SHAPES = [(1, 9, 3, 1, 384, 384),          # one row, six slabs: three in flight
           (2, 40, 5, 16, 448, 384),        # 32 rows: one tile
           (3, 40, 4, 11, 384, 512),        # 33 rows: two tiles, the second with one row
           (4, 50, 2, 32, 576, 392),        # 128 rows; 392 columns (and a reduction of 392, which is not for this kernel)
-          (2, 33, 66, 17, 1024, 1024)]     # 34 rows and 1056 column tiles: tiles of 64 rows
+          (2, 33, 20, 17, 1024, 1024)]     # 34 rows: two tiles, the second with two rows
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
@@ -52,7 +52,7 @@ def test_products_of_few_rows(shape, dtype):
     assert_close(dX, O.gather_backward(x, wg, safe, y * keep)[0], dtype, "dX")
 
 
-@pytest.mark.parametrize("shape", [(2, 40, 5, 16, 448, 128), (3, 40, 4, 11, 384, 144), (1, 33, 9, 40, 512, 272)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("shape", [(2, 40, 64, 16, 448, 128), (3, 40, 57, 11, 384, 144), (1, 33, 31, 40, 512, 272), (2, 20, 130, 20, 384, 1024)], ids=lambda s: "x".join(map(str, s)))
 def test_fp8_weights(shape):
     B, T, E, K, I, J = shape
     case = make_case(sum(shape), *shape, torch.bfloat16)
@@ -103,9 +103,10 @@ def test_scatter_with_bias(dtype):
     assert_close(out, want + (picks.numpy() @ np64(bias[:, 0])).reshape(B, T, I), dtype, "out")
 
 
-def test_weights_past_the_caches():
-    """More than 128 MB of weights under a single row tile: read past the caches."""
-    B, T, E, K, I, J = 1, 64, 131, 20, 1024, 512
+@pytest.mark.parametrize("rows", [20, 40])
+def test_weights_past_the_caches(rows):
+    """More than 256 MB of weights under a single row tile of 32 or 64 rows: read past the caches."""
+    B, T, E, K, I, J = 1, 64, 340, rows, 1024, 512
     g = torch.Generator(device="cuda").manual_seed(2)
     X, W = (torch.randn(*s, device="cuda", generator=g).bfloat16() for s in ((B, T, I), (E, I, J)))
     Ind = torch.randint(0, T, (B, E, K), device="cuda", generator=g)
@@ -114,3 +115,19 @@ def test_weights_past_the_caches():
     assert log.kernels == ["rows_stream_kernel"], log.kernels
     want = torch.stack([X[0, Ind[0, e]].float() @ W[e].float() for e in range(E)])
     assert (Y[0].float() - want).abs().max() <= 2 * 2.0 ** -8 * want.abs().max()
+
+
+@pytest.mark.parametrize("dims, streamed", [((1, 200, 114, 128, 1984, 256), False),         # four row tiles of many weights
+                                            ((1, 64, 251, 26, 1280, 312), False),           # weight rows of no whole lines, more than a round
+                                            ((2, 64, 88, 58, 1408, 128), True),             # one round
+                                            ((1, 64, 206, 30, 704, 256), True)], ids=lambda d: "x".join(map(str, d)) if isinstance(d, tuple) else None)
+def test_where_weights_stream(dims, streamed):
+    B, T, E, K, I, J = dims
+    g = torch.Generator(device="cuda").manual_seed(3)
+    X, W = (torch.randn(*s, device="cuda", generator=g).bfloat16() for s in ((B, T, I), (E, I, J)))
+    Ind = torch.randint(0, T, (B, E, K), device="cuda", generator=g)
+    with _abi.launch_log() as log:
+        Y = hk.expert_gather_forward_call(X, W, Ind, torch.float32)
+    assert (log.kernels == ["rows_stream_kernel"]) == streamed, log.kernels
+    want = torch.stack([torch.stack([X[b, Ind[b, e]].float() @ W[e].float() for e in range(E)]) for b in range(B)])
+    assert (Y.float() - want).abs().max() <= 2 * 2.0 ** -8 * want.abs().max()
