@@ -193,8 +193,9 @@ int launch_rows_strip(RowsStripParams &p, hipStream_t s)
 
 // Mid-sized 16-bit products; `used`: rows_strip_kernel takes this one.  Against tiled_rows_kernel, us, strips / that: R768 N64 Me2048 E32 13.8 /
 // 19.3, R328 N136 Me900 E20 10 / 14, R136 N328 13.3 to 16 / 17, R800 N64 Me1628 E34 17 / 22, R64 N576 Me2814 E14 18 to 19 / 25, R896 N128
-// Me232 E83 13.2 / 16.3, R192 N64 Me92 E65 5.0 / 5.7; not with few workgroups (R352 N64 Me252 E18: 36, 6.2 / 5.3) or half empty columns (R896
-// N32 Me119 E53 9.6 / 7.9, R288 N32 Me2080 E35 10.2 / 9.8), unless there are many (R800 N32 Me2146 E116: 1972, 42 / 47).
+// Me232 E83 13.2 / 16.3, R192 N64 Me92 E65 5.0 / 5.7; not with little work, counted in full tiles of 128 x 64 (R352 N64 Me252 E18: 35, 6.2 /
+// 5.3, R96 N48 Me576 E13: 44, 5.1 / 4.6, R160 N128 Me468 E8: 58, 5.5 / 4.8), nor with half empty columns (R896 N32 Me119 E53 9.6 / 7.9, R288
+// N32 Me2080 E35 10.2 / 9.8) unless there are many and long ones (1972 strips, R800 N32 Me2146 E116 42 / 47; but R160 N32 Me1920 E103 35.7 / 32.3).
 int rows_strip(RowsGemmParams &p, int act_dtype, bool w_trans, bool gather, int epi, bool &used, hipStream_t s)
 {
     used = false;
@@ -202,8 +203,8 @@ int rows_strip(RowsGemmParams &p, int act_dtype, bool w_trans, bool gather, int 
         p.R % 8 != 0 || p.N % 8 != 0 || (uint64_t)p.R * p.N * 2 >= (1ull << 31) || p.w_scale != nullptr)
         return EGS_OK;
     const int64_t Me = (int64_t)p.B * p.K, strips = p.E * ((Me + 127) / 128) * ceil_div(p.N, 64);
-    const bool filled = (double)Me * p.N * p.E >= 0.6 * 128 * 64 * (double)strips;
-    if (strips < (filled ? 64 : 1500)) return EGS_OK;
+    const double full = (double)Me * p.N * p.E / (128 * 64);
+    if (full < 80 || (full < 0.6 * (double)strips && (strips < 1500 || p.R < 400))) return EGS_OK;
     RowsStripParams q;
     memset(&q, 0, sizeof(q));
     q.A = p.A; q.W = p.W; q.Ind = p.Ind; q.C = p.C; q.bias = (const char *)p.bias;

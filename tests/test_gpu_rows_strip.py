@@ -66,7 +66,7 @@ def test_strips_match_the_oracle_and_the_general_kernel(shape, dtype):
 
 @pytest.mark.parametrize("act", ["none", "relu", "gelu", "silu"])
 def test_bias_and_activation(act):
-    B, T, E, K, I, J = 3, 400, 24, 70, 200, 120
+    B, T, E, K, I, J = 3, 400, 30, 70, 200, 120
     case = make_case(9, B, T, E, K, I, J, torch.bfloat16)
     X, Wg, Ind = dev(case["X"]), dev(case["Wg"]), dev(case["Ind"])
     bias = dev(torch.randn(E, J, generator=torch.Generator().manual_seed(1)).bfloat16()) if act == "none" else None
@@ -95,7 +95,7 @@ def test_bias_and_activation(act):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 def test_scatter_with_bias(dtype, mode):
     """The rows come with their bias, in fp32 or (atomic mode) in the element type: the general kernel's bits."""
-    B, T, E, K, I, J = 3, 400, 24, 70, 120, 200
+    B, T, E, K, I, J = 3, 400, 30, 70, 120, 200
     case = make_case(10, B, T, E, K, I, J, dtype)
     Ind = case["Ind"].clone()
     Ind[0, 0, 0], Ind[-1, -1, -1] = T, -1
@@ -119,3 +119,15 @@ def test_scatter_with_bias(dtype, mode):
         picks.index_put_((Ind[keep] + b * T, e), torch.ones((), dtype=torch.float64), accumulate=True)
         want = O.scatter_forward(np64(case["Y"]) * keep.numpy()[..., None], np64(case["Ws"]), Ind.clamp(0, T - 1).numpy(), T)
         assert_close(got, want + (picks.numpy() @ np64(bias[:, 0])).reshape(B, T, I), dtype, "out")
+
+
+@pytest.mark.parametrize("dims, strips", [((6, 90, 8, 78, 160, 128), False),        # 58 full tiles
+                                          ((10, 90, 30, 25, 144, 96), True),        # 88
+                                          ((16, 120, 103, 120, 160, 32), False),    # 1545 half empty strips of a short reduction
+                                          ((16, 120, 103, 120, 416, 32), True)], ids=lambda d: "x".join(map(str, d)) if isinstance(d, tuple) else None)
+def test_where_strips_are_taken(dims, strips):
+    case = make_case(11, *dims, torch.bfloat16)
+    with _abi.launch_log() as log:
+        Y = hk.expert_gather_forward_call(dev(case["X"]), dev(case["Wg"]), dev(case["Ind"]), torch.float32)
+    assert log.kernels == ["rows_strip_kernel" if strips else "tiled_rows_kernel"], log.kernels
+    assert_close(Y, O.gather_forward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy()), torch.bfloat16, "Y")
