@@ -235,6 +235,8 @@ bool dw_strip_broad(const egs_dims *d, int act_dtype, const DwPlan &pl, DwStripP
 {
     if (act_dtype == EGS_F32 || d->I % 8 || d->J % 8 || d->J <= 64 || d->I < 32 || d->E == 0) return false;
     if (!pl.big_ok && (d->I > 128 || d->J <= 128 || (int64_t)d->B * d->K < 128)) return false;
+    // (half the rows of a strip empty, and CUs enough to fill with less: I32 J192 E46 7568 picks 42 / 32, J144 E117 1204 picks 18.4 / 16.8)
+    if (d->I <= 32 && (int64_t)d->E * ceil_div(d->J, 64) >= 128 && (int64_t)d->B * d->K >= 384) return false;
     strip = dw_strip_plan(d);
     if (!pl.big_ok) return true;
     const int64_t on_xcd = (int64_t)ceil_div(d->E, 8) * pl.b_i_tiles * pl.b_j_tiles * pl.b_S;
@@ -461,15 +463,18 @@ bool make_dw_small(const void *Xs, const void *Ys, const void *Ind, void *dW, vo
 
 // The one-pass weight gradient (32 x 32 tiles of dW(e), every workgroup reduces all picks of its expert) is taken
 // when its tiles alone fill the device; with fewer tiles the picks are split instead (dw_small_kernel + second pass).
+// `shared`: in the launch of a scatter, where strips would be one or two launches of their own (gather's backward, us, with strips / shared:
+// B50 T45 E16 K45 I160 J64 28.5 / 19.8, B12 T1243 E15 K21 I192 J64 17.6 / 13.6, B20 T396 E10 K85 I256 J64 20.9 / 18.5, B26 T165 E5 K121 I608 J64
+// 36.2 / 37.4).
 bool make_dw_tile(const void *Xs, const void *Ys, const void *Ind, void *dW, const egs_dims *d, int64_t ldx_b, int64_t ldx_t,
-                  int act_dtype, int out_dtype, int ind_dtype, int dw_layout, DwTileJob &j, bool wide = false)
+                  int act_dtype, int out_dtype, int ind_dtype, int dw_layout, DwTileJob &j, bool wide = false, bool shared = false)
 {
     if (g_force_generic) return false;
     const int ES = elem_size(act_dtype);
     // (fp32, the bf16 instruction's 64 x 64 tiles / these, us, by slabs: 4096 (B64 T256 E32 K32 I128 J64) 21 / 20, 9450 (B16 T61 E14 K45 I960 J96)
     // 30 / 50, 16384 43 / 66 and 46 / 60; with 32 columns of a tile empty (I32 J96, 7676) 41 / 30)
     if (ES == 4 && d->I > 32 && d->J > 32 && dw_split32_slabs(d) >= 8192) return false;
-    if (dw_strip_narrow(d, act_dtype)) return false;
+    if (!shared && dw_strip_narrow(d, act_dtype)) return false;
     if (d->I % 8 || d->J % 8 || d->I < 8 || d->J < 8 || d->I > 2048 || d->J > 128) return false;
     const int64_t Me = (int64_t)d->B * d->K;
     if (Me == 0 || d->E == 0 || d->T == 0) return false;
@@ -707,6 +712,23 @@ ScatterPath scatter_choose(const void *Y, const void *W, const void *Out, const 
     return SCATTER_ROWS;
 }
 
+// More slices than CUs: runs of slices with one sort.  A CU does its workgroups' slices one after the other, however many fit
+// its LDS, and a sort takes 0.6 of a slice's time; the run with the shortest rounds was the fastest at 12 of 12 sizes (B64
+// T256 E32 K32 I768 J64: runs of 6, 61 -> 47 us; B128 T64 E8 K16 I1024 J64: 16, 73 -> 37).
+int fused_run(const FusedPlan &fp, const egs_dims *d)
+{
+    const int slices = d->I / kFusedCols;
+    int run = 1;
+    if (fp.experts_per_pass == d->E) {
+        double least = 0;
+        for (int r = 1; r <= slices; ++r) {
+            const double cost = (double)(((int64_t)d->B * ceil_div(slices, r) + 255) / 256) * (r + 0.6);
+            if (r == 1 || cost < least) { least = cost; run = r; }
+        }
+    }
+    return run;
+}
+
 // GEMM-scatter of small experts in one kernel; the caller has checked scatter_fused_takes().  Both scatter modes
 // take it: it is bitwise reproducible and needs no workspace.
 int scatter_fused(const void *Y, const void *W, const void *Ind, void *Out, const egs_dims *d, int act_dtype, int ind_dtype,
@@ -718,17 +740,7 @@ int scatter_fused(const void *Y, const void *W, const void *Ind, void *Out, cons
     if (!fp.ok) return EGS_ERR_UNSUPPORTED;
     const size_t lds = fp.lds;
     const int slices = N / kFusedCols;
-    // More slices than CUs: runs of slices with one sort.  A CU does its workgroups' slices one after the other, however many fit
-    // its LDS, and a sort takes 0.6 of a slice's time; the run with the shortest rounds was the fastest at 12 of 12 sizes (B64
-    // T256 E32 K32 I768 J64: runs of 6, 61 -> 47 us; B128 T64 E8 K16 I1024 J64: 16, 73 -> 37).
-    int run = 1;
-    if (fp.experts_per_pass == d->E) {
-        double least = 0;
-        for (int r = 1; r <= slices; ++r) {
-            const double cost = (double)(((int64_t)d->B * ceil_div(slices, r) + 255) / 256) * (r + 0.6);
-            if (r == 1 || cost < least) { least = cost; run = r; }
-        }
-    }
+    const int run = fused_run(fp, d);
     const int64_t blocks = (int64_t)8 * ceil_div(d->B, 8) * ceil_div(slices, run);
     ScatterFusedParams p;
     memset(&p, 0, sizeof(p));
@@ -1273,10 +1285,10 @@ static int gather_backward_impl(const void *X, const void *W, const void *Ind, c
     // 32 x 32 tiles when they can share the launch of the one-kernel scatter (one pass) and come after it in one round of
     // workgroups, else what suits a launch of its own (I = 256: 42.9 us sharing, 37 us as two launches with 32 x 64 tiles)
     const FusedPlan fpl = scatter_fused_plan(grad_Y, W, grad_X, d, dtype);
-    const bool shares_launch = dtype != EGS_F32 && fpl.ok && fpl.experts_per_pass == d->E &&
+    const bool shares_launch = dtype != EGS_F32 && fpl.ok && fpl.experts_per_pass == d->E && fused_run(fpl, d) == 1 &&
                                (int64_t)d->E * ceil_div(d->I, 32) * ceil_div(d->J, 32) <= 256;
     const bool dw_tile = w_elems > 0 && make_dw_tile(X, grad_Y, Ind, grad_W, d, ldx_b, ldx_t, dtype, dtype, ind_dtype, EGS_W_EIJ, dwt,
-                                                     !shares_launch && dw_tile_wide_alone(d, dtype));
+                                                     !shares_launch && dw_tile_wide_alone(d, dtype), shares_launch);
     const bool dw_small = !dw_tile && w_elems > 0 && make_dw_small(X, grad_Y, Ind, grad_W, ws2, d, ldx_b, ldx_t, dtype, dtype,
                                                                    ind_dtype, EGS_W_EIJ, dpl, dwj);
     rc = gemm_scatter_impl(grad_Y, W, Ind, grad_X, workspace, d, dtype, ind_dtype, EGS_W_EIJ, mode, dw_small ? &dwj : nullptr,

@@ -42,3 +42,16 @@ def test_strips_match_the_oracle(shape, dtype):
     Y = np64(case["Y"]) * keep
     assert_close(dWg, O.gather_backward(np64(case["X"]), np64(case["Wg"]), safe, Y)[1], dtype, "dW of the gather")
     assert_close(dWs, O.scatter_backward(Y, np64(case["Ws"]), safe, np64(case["dOut"]))[1], dtype, "dW of the scatter")
+
+
+@pytest.mark.parametrize("shape, kernels", [((12, 300, 15, 21, 192, 64), ["scatter_fused_dwtile_kernel"]),                      # 180 tiles of 32 x 32 in the scatter's launch
+                                            ((50, 45, 16, 45, 160, 64), ["scatter_fused_dwtile_kernel"]),
+                                            ((64, 60, 30, 32, 768, 64), ["scatter_fused_runs_kernel", "dw_strip_kernel"]),      # a scatter in runs shares none
+                                            ((44, 60, 46, 80, 32, 192), ["tiled_dw_kernel", "tiled_dw_sum_kernel"])], ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else None)
+def test_where_strips_are_not_taken(shape, kernels):
+    B, T, E, K, I, J = shape
+    case = make_case(sum(shape), *shape, torch.bfloat16)
+    with _abi.launch_log() as log:
+        _, dW = hk.expert_gather_backward_call(dev(case["X"]), dev(case["Wg"]), dev(case["Ind"]), dev(case["Y"]), torch.float32)
+    assert log.kernels[-len(kernels):] == kernels, log.kernels
+    assert_close(dW, O.gather_backward(np64(case["X"]), np64(case["Wg"]), case["Ind"].numpy(), np64(case["Y"]))[1], torch.bfloat16, "dW")
