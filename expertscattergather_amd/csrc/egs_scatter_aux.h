@@ -594,9 +594,7 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
             }
         };
         const int32_t *pb = perm + (size_t)b * N;
-        // fp32 rows, VW = 8: four columns in each half of the row, so that a wavefront's 16-byte loads are contiguous
-        constexpr bool HALVES = sizeof(PT) == 4 && VW == 8;
-        const PT *Pb = P + (size_t)b * N * sp.ldp + (size_t)iv * (HALVES ? 4 : VW);
+        const PT *Pb = P + (size_t)b * N * sp.ldp + (size_t)iv * VW;
         int s = s0;
         if constexpr (VW >= 4) {
             struct F32x8 { f32x4 lo, hi; };
@@ -619,7 +617,7 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
             };
             auto load_vec = [&](const PT *src) -> vec_t {
                 auto one = [](auto *at) { if constexpr (STREAM) return __builtin_nontemporal_load(at); else return *at; };
-                if constexpr (HALVES) return vec_t{one(reinterpret_cast<const f32x4 *>(src)), one(reinterpret_cast<const f32x4 *>(src + I / 2))};
+                if constexpr (sizeof(vec_t) == 32) return vec_t{one(reinterpret_cast<const f32x4 *>(src)), one(reinterpret_cast<const f32x4 *>(src) + 1)};
                 else return one(reinterpret_cast<const vec_t *>(src));
             };
             // long segments (hot tokens): 16 rows (256 bytes) in flight per thread; added in table order all the same
@@ -651,18 +649,15 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
         } else {
             for (; s < s1; ++s) add_row(Pb + (size_t)pb[s] * sp.ldp);
         }
-        size_t at = row * I + (size_t)iv * (HALVES ? 4 : VW);
+        size_t at = row * I + (size_t)iv * VW;
         if constexpr (TT::ES == 4) {
             float *dst = reinterpret_cast<float *>(out) + at;
             if constexpr (VW >= 4) *reinterpret_cast<f32x4 *>(dst) = f32x4{acc[0], acc[1], acc[2], acc[3]};
             else dst[0] = acc[0];
-            if constexpr (VW == 8) *reinterpret_cast<f32x4 *>(dst + I / 2) = f32x4{acc[4], acc[5], acc[6], acc[7]};
+            if constexpr (VW == 8) *reinterpret_cast<f32x4 *>(dst + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
         } else {
             uint16_t *dst = reinterpret_cast<uint16_t *>(out) + at;
-            if constexpr (HALVES) {
-                *reinterpret_cast<u32x2 *>(dst) = u32x2{pack2<TT>(acc[0], acc[1]), pack2<TT>(acc[2], acc[3])};
-                *reinterpret_cast<u32x2 *>(dst + I / 2) = u32x2{pack2<TT>(acc[4], acc[5]), pack2<TT>(acc[6], acc[7])};
-            } else if constexpr (VW == 8) {
+            if constexpr (VW == 8) {
                 u32x4 w;
 #pragma unroll
                 for (int x = 0; x < 4; ++x) w[x] = pack2<TT>(acc[2 * x], acc[2 * x + 1]);
