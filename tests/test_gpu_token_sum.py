@@ -1,5 +1,6 @@
 """token_sum_kernel (csrc/egs_token_sum.h) with a wavefront per token: tokens nobody picked first, last and in a row, tokens of one to
-sixty-four picks (nine: one more than are on their way at a time) and of more, fewer tokens than wavefronts; against the oracle."""
+thirty-two picks (nine: one more than are on their way at a time), of more, and of more than sixty-four, fewer tokens than wavefronts;
+against the oracle."""
 import pytest
 import torch
 
@@ -15,8 +16,8 @@ from expertscattergather_amd import hip_kernels as hk
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
 @pytest.mark.parametrize("mode", ["deterministic", "atomic"])
-@pytest.mark.parametrize("T, counts", [(60, [0, 0, 9, 1, 8, 0, 0, 0, 0, 17, 16, 64, 0, 3]), (60, [0, 65, 0, 7, 130]), (3, [0, 2, 0]), (2, [40, 0])],
-                         ids=["few", "hot", "three", "two"])
+@pytest.mark.parametrize("T, counts", [(60, [0, 0, 9, 1, 8, 0, 0, 0, 0, 17, 16, 32, 0, 3]), (60, [0, 33, 5, 64, 1]), (60, [0, 65, 0, 7, 130]), (3, [0, 2, 0]), (2, [40, 0])],
+                         ids=["few", "some", "hot", "three", "two"])
 def test_sums_of_neighbouring_tokens(T, counts, mode, dtype):
     E, I, J = 5, 261, 24
     picks = [t for t, n in enumerate(counts) for _ in range(n)]
