@@ -32,17 +32,18 @@ int64_t f8_grid(const egs_dims *d, int tile)
 }
 
 // 256 x 256 tiles (one workgroup to a CU) or 128 x 128 (two, the same bits): whichever needs the fewer turns of the chip, a turn
-// of the large tiles taking as long as two of the small.  On a tie the large ones from a reduction of more than 1024 on, where
-// their half as many bytes from the L2 count.  Both measured, large then small, in us, as (rows of an expert, E, I, J):
+// of the large tiles taking as long as two of the small.  From a reduction of more than 1024 on, where their half as many bytes from
+// the L2 count, the large ones on a tie and for up to 15 % more turns.  Both measured, large then small, in us, as (rows of an expert, E, I, J):
 // (195, 22, 1280, 256) 27.0, 11.9; (391, 53, 640, 144) 21.7, 11.0; (32, 256, 2048, 512) 79.4, 53.6;
 // (1024, 48, 2048, 512) 86.0, 65.7; (1280, 64, 2048, 384) 120, 100; ties: (1024, 32, 4096, 512) 72.0, 91.2; (2048, 64, 2048, 512)
-// 173, 188; (2048, 128, 1024, 256) 119, 124; (1024, 64, 1024, 512) 58.3, 59.3; (2048, 64, 512, 512) 86.8, 79.4.
+// 173, 188; (2048, 128, 1024, 256) 119, 124; (1024, 64, 1024, 512) 58.3, 59.3; (2048, 64, 512, 512) 86.8, 79.4; eight turns and seven:
+// (510, 204, 1536, 432) 148, 159 with the quantisation.
 bool f8_large_tiles(const egs_dims *d)
 {
     const int64_t n256 = f8_grid(d, 256), n128 = f8_grid(d, 128);
     if (n128 > INT32_MAX) return true;
     const int64_t turns256 = 2 * ((n256 + 255) / 256), turns128 = (n128 + 511) / 512;
-    return turns256 < turns128 || (turns256 == turns128 && d->I > 1024);
+    return d->I > 1024 ? 20 * turns256 <= 23 * turns128 : turns256 < turns128;
 }
 
 bool ind_dtype_known(int ind_dtype) { return ind_dtype >= EGS_IND_I16 && ind_dtype <= EGS_IND_U8; }

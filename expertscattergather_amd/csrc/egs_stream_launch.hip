@@ -53,8 +53,12 @@ int rows_stream(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans, bool
     // weights come from memory in any case (R2048 N512 Me64 E256 121 / 139; 102 such sizes 0.85 to 1.04 of the other's time).
     const int64_t tiles = (int64_t)p.E * ceil_div(p.N, cols), row_tiles = (Me + 31) / 32;
     if (fp8_w) {
-        // half as many bytes: also in more rounds, up to 64 rows; not with few workgroups (R1920 N144 Me28 E30 16.2 / 14.0, R640 N144 Me41 E24 8.5 / 7.4)
-        if ((int64_t)p.E * p.N < 64 * cols || (Me > 64 && row_tiles * tiles > 1536)) return EGS_OK;
+        // half as many bytes: also in more rounds, up to 64 rows; not with few workgroups (R1920 N144 Me28 E30 16.2 / 14.0, R640 N144 Me41 E24 8.5 / 7.4),
+        // nor several row tiles of columns that are a quarter empty (R1024 N288 Me54 E47 12.2 / 11.2, R1408 N144 Me50 E70 14.9 / 13.5) or come in little
+        // more than a round (R384 N304 Me102 E69 12.4 / 11.1, R1664 N464 Me49 E100 31.6 / 27.9)
+        const bool filled = 4 * (int64_t)p.N > 3 * (int64_t)cols * ceil_div(p.N, cols);
+        const int64_t all = row_tiles * tiles;
+        if ((int64_t)p.E * p.N < 64 * cols || (Me > 32 && (!filled || (all > 768 && all <= 1024))) || (Me > 64 && all > 1536)) return EGS_OK;
     } else {
         const bool lines = !w_trans || p.N % 64 == 0;
         const bool from_memory = Me <= 64 && tiles >= 1024 && (uint64_t)p.E * p.R * p.N * 2 > (320ull << 20);

@@ -52,7 +52,7 @@ def test_products_of_few_rows(shape, dtype):
     assert_close(dX, O.gather_backward(x, wg, safe, y * keep)[0], dtype, "dX")
 
 
-@pytest.mark.parametrize("shape", [(2, 40, 64, 16, 448, 128), (3, 40, 57, 11, 384, 144), (1, 33, 31, 40, 512, 272), (2, 20, 130, 20, 384, 1024)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("shape", [(2, 40, 64, 16, 448, 128), (3, 40, 57, 10, 384, 144), (1, 33, 31, 40, 512, 304), (2, 20, 130, 20, 384, 1024)], ids=lambda s: "x".join(map(str, s)))
 def test_fp8_weights(shape):
     B, T, E, K, I, J = shape
     case = make_case(sum(shape), *shape, torch.bfloat16)
