@@ -124,7 +124,8 @@ def test_scatter_with_bias(dtype, mode):
 @pytest.mark.parametrize("dims, strips", [((6, 90, 8, 78, 160, 128), False),        # 58 full tiles
                                           ((10, 90, 30, 25, 144, 96), True),        # 88
                                           ((16, 120, 103, 120, 160, 32), False),    # 1545 half empty strips of a short reduction
-                                          ((16, 120, 103, 120, 416, 32), True)], ids=lambda d: "x".join(map(str, d)) if isinstance(d, tuple) else None)
+                                          ((16, 120, 103, 120, 416, 32), True),
+                                          ((2, 120, 150, 12, 456, 1024), False)], ids=lambda d: "x".join(map(str, d)) if isinstance(d, tuple) else None)
 def test_where_strips_are_taken(dims, strips):
     case = make_case(11, *dims, torch.bfloat16)
     with _abi.launch_log() as log:
