@@ -17,7 +17,8 @@ template <bool W_TRANS>
 int launch_rows_atomic(RowsGemmParams &p, hipStream_t s)
 {
     const int Me = p.B * p.K;
-    const bool large = p.R >= 1024 && (int64_t)p.E * ceil_div(Me, 128) * ceil_div(p.N, 128) >= 512;
+    const bool large = (p.R >= 1024 && (int64_t)p.E * ceil_div(Me, 128) * ceil_div(p.N, 128) >= 512) ||
+                       (int64_t)8 * ceil_div(p.E, 8) * ceil_div(Me, 64) * ceil_div(p.N, 64) > INT32_MAX;       // (more than a grid holds)
     const int tile = large ? 128 : 64;
     p.m_tiles = ceil_div(Me, tile); p.n_tiles = ceil_div(p.N, tile);
     const int64_t grid = (int64_t)8 * ceil_div(p.E, 8) * p.m_tiles * p.n_tiles;

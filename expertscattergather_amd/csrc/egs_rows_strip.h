@@ -48,7 +48,7 @@ __global__ __launch_bounds__(kStripThreads, 6) void rows_strip_kernel(RowsStripP
     static_assert(TT::ES == 2, "16-bit element types");
     typedef RowsStripLds L;
     constexpr int BM = L::BM, BN = L::BN, WM = 4, WN = 8 / WM, TM = BM / WM / 16, TN = BN / WN / 16;   // wavefront grid, 16 x 16 tiles of a wavefront
-    constexpr int PL = BM / 64, QL = BN / 64, NL = PL + QL;             // loads (1 KB) per wavefront and slab: rows, weights
+    constexpr int PL = BM / 64, QL = BN / 64;                           // loads (1 KB) per wavefront and slab: rows, weights
     extern __shared__ __attribute__((aligned(1024))) char smem_rows_strip[];
 
     const int lin = balanced_tile((int)blockIdx.x, p.E * p.m_tiles * p.n_tiles);
@@ -102,8 +102,8 @@ __global__ __launch_bounds__(kStripThreads, 6) void rows_strip_kernel(RowsStripP
 #pragma unroll
         for (int j = 0; j < QL; ++j) direct_load16(rs_w, qk[j] < left ? qv[j] : kVoffInvalid, so, smem_rows_strip + stage * L::STAGE + L::A + (wave * QL + j) * 1024);
     };
-    constexpr int AHEAD = L::NST - 1;
-    for (int s = 0; s < min(AHEAD, nk); ++s) issue_w(s, s);
+    static_assert(L::NST == 2, "one slab on its way under the one being multiplied");
+    if (nk > 0) issue_w(0, 0);
     const u32x4 rs_a = make_rsrc(p.A, p.a_bytes);
     uint32_t pv[PL];
 #pragma unroll
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(kStripThreads, 6) void rows_strip_kernel(RowsStripP
 #pragma unroll
         for (int j = 0; j < PL; ++j) direct_load16(rs_a, ac < left ? pv[j] : kVoffInvalid, (uint32_t)kt * 128, smem_rows_strip + stage * L::STAGE + (wave * PL + j) * 1024);
     };
-    for (int s = 0; s < min(AHEAD, nk); ++s) issue_a(s, s);
+    if (nk > 0) issue_a(0, 0);
     int64_t *const c_row = reinterpret_cast<int64_t *>(smem_rows_strip + L::NST * L::STAGE);
     if (tid < BM) {
         int b;
@@ -137,17 +137,11 @@ __global__ __launch_bounds__(kStripThreads, 6) void rows_strip_kernel(RowsStripP
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     int stage = 0;
     for (int kt = 0; kt < nk; ++kt) {
-        // what may still be on its way: the slabs requested after this one (of the first AHEAD the weights came before any rows)
-        if (kt + AHEAD > nk) wait_vmem<0>();
-        else if (kt == 0) wait_vmem<(AHEAD - 1) * PL>();
-        else if (AHEAD >= 3 && kt == 1) wait_vmem<(AHEAD - 2) * PL + NL>();
-        else wait_vmem<(AHEAD - 1) * NL>();
+        wait_vmem<0>();             // slab kt, the only one on its way
         __syncthreads();            // slab kt is everybody's; nobody reads the stage that is filled next
-        if (kt + AHEAD < nk) {
-            int fill = stage + AHEAD;
-            if (fill >= L::NST) fill -= L::NST;
-            issue_a(kt + AHEAD, fill);
-            issue_w(kt + AHEAD, fill);
+        if (kt + 1 < nk) {
+            issue_a(kt + 1, stage ^ 1);
+            issue_w(kt + 1, stage ^ 1);
         }
         const char *ta = smem_rows_strip + stage * L::STAGE, *tw = ta + L::A;
 #pragma unroll
@@ -172,7 +166,7 @@ __global__ __launch_bounds__(kStripThreads, 6) void rows_strip_kernel(RowsStripP
 #pragma unroll
                 for (int j = 0; j < TN; ++j) mma_chunk<TT>(acc[i][j], nf[j], mf[i]);
         }
-        if (++stage == L::NST) stage = 0;
+        stage ^= 1;
     }
 
     // ---------------- results through LDS, out as whole row segments; lane (a, g) holds columns 4 g .. + 3 of row a of a tile
