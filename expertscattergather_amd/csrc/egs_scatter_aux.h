@@ -594,7 +594,11 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
             }
         };
         const int32_t *pb = perm + (size_t)b * N;
-        const PT *Pb = P + (size_t)b * N * sp.ldp + (size_t)iv * VW;
+        // fp32 rows past the caches, VW = 8: four columns in each half of the row, so that a wavefront's 16-byte loads are whole lines (side by
+        // side every line comes twice: B10 T1373 E98 K214 I448, 376 MB, 187 -> 207 us; from the caches one address per row is worth more: B2 T58
+        // E95 K23 I32 19.2, in halves 20.2)
+        constexpr bool HALVES = STREAM && sizeof(PT) == 4 && VW == 8;
+        const PT *Pb = P + (size_t)b * N * sp.ldp + (size_t)iv * (HALVES ? 4 : VW);
         int s = s0;
         if constexpr (VW >= 4) {
             struct F32x8 { f32x4 lo, hi; };
@@ -617,7 +621,7 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
             };
             auto load_vec = [&](const PT *src) -> vec_t {
                 auto one = [](auto *at) { if constexpr (STREAM) return __builtin_nontemporal_load(at); else return *at; };
-                if constexpr (sizeof(vec_t) == 32) return vec_t{one(reinterpret_cast<const f32x4 *>(src)), one(reinterpret_cast<const f32x4 *>(src) + 1)};
+                if constexpr (sizeof(vec_t) == 32) return vec_t{one(reinterpret_cast<const f32x4 *>(src)), one(reinterpret_cast<const f32x4 *>(src + (HALVES ? I / 2 : 4)))};
                 else return one(reinterpret_cast<const vec_t *>(src));
             };
             // long segments (hot tokens): 16 rows (256 bytes) in flight per thread; added in table order all the same
@@ -649,15 +653,18 @@ __device__ __forceinline__ void segment_sum_body(const SegSumParams &sp, const i
         } else {
             for (; s < s1; ++s) add_row(Pb + (size_t)pb[s] * sp.ldp);
         }
-        size_t at = row * I + (size_t)iv * VW;
+        size_t at = row * I + (size_t)iv * (HALVES ? 4 : VW);
         if constexpr (TT::ES == 4) {
             float *dst = reinterpret_cast<float *>(out) + at;
             if constexpr (VW >= 4) *reinterpret_cast<f32x4 *>(dst) = f32x4{acc[0], acc[1], acc[2], acc[3]};
             else dst[0] = acc[0];
-            if constexpr (VW == 8) *reinterpret_cast<f32x4 *>(dst + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
+            if constexpr (VW == 8) *reinterpret_cast<f32x4 *>(dst + (HALVES ? I / 2 : 4)) = f32x4{acc[4], acc[5], acc[6], acc[7]};
         } else {
             uint16_t *dst = reinterpret_cast<uint16_t *>(out) + at;
-            if constexpr (VW == 8) {
+            if constexpr (HALVES) {
+                *reinterpret_cast<u32x2 *>(dst) = u32x2{pack2<TT>(acc[0], acc[1]), pack2<TT>(acc[2], acc[3])};
+                *reinterpret_cast<u32x2 *>(dst + I / 2) = u32x2{pack2<TT>(acc[4], acc[5]), pack2<TT>(acc[6], acc[7])};
+            } else if constexpr (VW == 8) {
                 u32x4 w;
 #pragma unroll
                 for (int x = 0; x < 4; ++x) w[x] = pack2<TT>(acc[2 * x], acc[2 * x + 1]);
