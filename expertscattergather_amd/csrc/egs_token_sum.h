@@ -17,7 +17,7 @@ namespace egs {
 constexpr int kTokenSumPicks = 4096;        // most picks per batch element
 constexpr int kTokenSumTokens = 32;         // most tokens per workgroup
 constexpr int kTokenSumHot = 64;            // longer segments are shared by the whole workgroup
-constexpr int kTokenSumRun = 32;            // up to here a wavefront adds neighbouring tokens in one run of rows
+constexpr int kTokenSumOne = 32;            // a wavefront's only token: longer segments go sixteen rows at a time
 
 struct TokenSumParams {
     const void *P;              // product rows [B, N, ldp], fp32 or the 16-bit element type
@@ -195,11 +195,12 @@ __global__ __launch_bounds__(kThreads) void token_sum_kernel(TokenSumParams p)
     // Where a wavefront is a token's group it takes neighbouring tokens, whose picks follow one another, and has eight rows on their
     // way, whichever they are for; token by token, of two or three rows each, it waited for memory once for every token.  us, fp32 rows:
     // B5 T2250 E28 K24 I928 21.9 -> 14.7, B71 T1000 E12 K10 I160 23.6 -> 18.4, B62 T394 E31 K43 I386 37.5 -> 31.6, B4 T512 E256 K8 I2048
-    // 20.0 -> 15.7, B6 T1100 E20 K150 I328 14.4 -> 12.5.  Not with a token of more than 32 picks, whose sixteen rows on their way (a share for
-    // each group from 64 on) are worth more than its neighbours' trips: scatters under Zipf routing B1 T315 E4 K44 I576 12.1 for 10.9, B10 T58 E7
-    // K22 I672 15.6 for 14.9; with the line at 64, 16 or 8 picks more sizes lose.
+    // 20.0 -> 15.7, B6 T1100 E20 K150 I328 14.4 -> 12.5.  Not with a token of more than kTokenSumHot
+    // picks, nor, where a wavefront has one token only, of more than kTokenSumOne: sixteen rows on their way are worth more there (scatters under
+    // Zipf routing, one token at a time / in runs, B1 T315 E4 K44 I576 10.9 / 12.1, B10 T58 E7 K22 I672 14.9 / 15.6; with eight tokens to a
+    // wavefront B6 T3346 E60 K5 I427 25.7 / 23.7).
     const int lens = WAVE && lane < tb ? first[lane + 1] - first[lane] : 0;
-    if (WAVE && __ballot(lens > kTokenSumRun) == 0) {
+    if (WAVE && __ballot(lens > (p.tb > groups ? kTokenSumHot : kTokenSumOne)) == 0) {
         const int each = (tb + groups - 1) / groups, tl1 = min(tb, (wave + 1) * each);
         int tl = min(tb, wave * each);
         const int ends = first[min(lane, kTokenSumTokens - 1) + 1];     // of token `lane`

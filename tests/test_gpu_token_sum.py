@@ -1,6 +1,6 @@
 """token_sum_kernel (csrc/egs_token_sum.h) with a wavefront per token: tokens nobody picked first, last and in a row, tokens of one to
-thirty-two picks (nine: one more than are on their way at a time), of more, and of more than sixty-four, fewer tokens than wavefronts;
-against the oracle."""
+thirty-two picks (nine: one more than are on their way at a time), of more, and of more than sixty-four, fewer tokens than wavefronts,
+one token to a wavefront and several; against the oracle."""
 import pytest
 import torch
 
@@ -38,3 +38,15 @@ def test_sums_of_neighbouring_tokens(T, counts, mode, dtype):
     if mode == "atomic" and dtype != torch.float32:     # product rows in the element type
         return assert_close(out.float(), O.scatter_forward(Y, np64(case["Ws"]), Ind.clamp(max=T - 1).numpy(), T), torch.bfloat16, "out")
     assert_close(out, O.scatter_forward(Y, np64(case["Ws"]), Ind.clamp(max=T - 1).numpy(), T), dtype, "out")
+
+
+def test_several_tokens_to_a_wavefront():
+    """1536 workgroups of four tokens would be more than a thousand: eight to a workgroup, two to a wavefront, of up to 64 picks."""
+    B, T, E, K, I, J = 64, 96, 5, 40, 261, 24
+    case = make_case(4, B, T, E, K, I, J, torch.float32)
+    Ind = case["Ind"].clone()
+    Ind[:, 0, :], Ind[:, 1, :20], Ind[1::2, 2, :] = 7, 7, 7              # 60 picks of a token, or a hundred
+    with _abi.launch_log() as log:
+        out = hk.expert_scatter_forward_call(dev(case["Y"]), dev(case["Ws"]), dev(Ind), T, torch.float32)
+    assert log.kernels[-1] == "token_sum_kernel", log.kernels
+    assert_close(out, O.scatter_forward(np64(case["Y"]), np64(case["Ws"]), Ind.numpy(), T), torch.float32, "out")
