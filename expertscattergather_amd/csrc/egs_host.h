@@ -71,6 +71,22 @@ inline int grid_1d(size_t items, int cap = 8192)
     return (int)(g > (size_t)cap ? (size_t)cap : g);
 }
 
+// tiled_rows_kernel's columns per tile, in sixteens: what takes the fewest rounds of the 256 CUs, each as long as the tile's matrix instructions
+// and the fixed part of a tile (fetching 64 rows, and what a slab's barriers cost) let it be, measured at 42 shapes.  80 columns only where
+// the matrix instructions are the larger part (fp32: E35 of 6000 picks, R185 N67 71 us, 78 with 96 columns; 16-bit 35 and 33).
+inline int tiled_columns(int64_t E, int64_t Me, int N, bool f32)
+{
+    const int64_t row_tiles = E * ((Me + 63) / 64);
+    int tn = 0;
+    double least = 0;
+    for (const int c : {6, 5, 4, 2}) {
+        if (c == 5 && !f32) continue;
+        const double cost = (double)((row_tiles * ceil_div(N, 16 * c) + 255) / 256) * (c + (f32 ? 1.0 : 1.5));
+        if (tn == 0 || cost < least) { least = cost; tn = c; }
+    }
+    return tn;
+}
+
 // row stride (elements) of product rows in the workspace: whole 16-byte (fp32) or 8-byte pieces for token_sum / segment_sum
 inline int product_ld(int I) { return (I + 3) & ~3; }
 

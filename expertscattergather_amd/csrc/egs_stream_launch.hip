@@ -31,6 +31,23 @@ int launch_stream(RowsStreamParams &p, int mt, hipStream_t s)
     return mt == 2 ? launch_stream<TT, WES, W_TRANS, 2>(p, s) : launch_stream<TT, WES, W_TRANS, 4>(p, s);
 }
 
+// fp8 weights: is this kernel faster than tiled_rows_kernel?  Both by the time of the fullest CU, fitted to 1565
+// sizes of up to 128 rows: a fixed part, and for every 64 reduction elements what a CU's workgroups take side by side, three of this kernel's
+// or two of the other's.  By it 23 sizes are 3 % slower than they could be, none 15 %.  us, it / that: R1792 N352 Me84 E236 64 / 90, R640
+// N480 Me70 E165 27 / 37; not taken: R384 N304 Me102 E69 12.4 / 11.1, R1408 N144 Me50 E70 14.9 / 13.5, R1920 N144 Me28 E30 16.2 / 14.0.
+bool stream_fp8_pays(int64_t E, int64_t Me, int R, int N)
+{
+    const auto rounds = [](int64_t n, int per, double alone, double each) {
+        const int64_t rest = n % per;
+        const auto round = [&](int64_t k) { return (double)k * each > alone ? (double)k * each : alone; };
+        return (double)(n / per) * round(per) + (rest ? round(rest) : 0.0);
+    };
+    const int tn = tiled_columns(E, Me, N, false);
+    const int64_t stream = (E * ((Me + 31) / 32) * ceil_div(N, 128) + 255) / 256, tiled = (E * ((Me + 63) / 64) * ceil_div(N, 16 * tn) + 255) / 256;
+    const double slabs = R / 64;
+    return 2.5 + 1.3 * (double)((stream + 2) / 3) + slabs * rounds(stream, 3, 0.37, 0.25) < 4.8 + slabs * rounds(tiled, 2, 0.14 + 0.064 * tn, 0.06 + 0.062 * tn);
+}
+
 }  // namespace
 
 int rows_stream(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans, bool gather, int epi, bool &used, hipStream_t s)
@@ -53,12 +70,7 @@ int rows_stream(RowsGemmParams &p, int act_dtype, bool fp8_w, bool w_trans, bool
     // weights come from memory in any case (R2048 N512 Me64 E256 121 / 139; 102 such sizes 0.85 to 1.04 of the other's time).
     const int64_t tiles = (int64_t)p.E * ceil_div(p.N, cols), row_tiles = (Me + 31) / 32;
     if (fp8_w) {
-        // half as many bytes: also in more rounds, up to 64 rows; not with few workgroups (R1920 N144 Me28 E30 16.2 / 14.0, R640 N144 Me41 E24 8.5 / 7.4),
-        // nor several row tiles of columns that are a quarter empty (R1024 N288 Me54 E47 12.2 / 11.2, R1408 N144 Me50 E70 14.9 / 13.5) or come in little
-        // more than a round (R384 N304 Me102 E69 12.4 / 11.1, R1664 N464 Me49 E100 31.6 / 27.9)
-        const bool filled = 4 * (int64_t)p.N > 3 * (int64_t)cols * ceil_div(p.N, cols);
-        const int64_t all = row_tiles * tiles;
-        if ((int64_t)p.E * p.N < 64 * cols || (Me > 32 && (!filled || (all > 768 && all <= 1024))) || (Me > 64 && all > 1536)) return EGS_OK;
+        if (!(tiles >= 1024 && Me <= 64) && !stream_fp8_pays(p.E, Me, p.R, p.N)) return EGS_OK;
     } else {
         const bool lines = !w_trans || p.N % 64 == 0;
         const bool from_memory = Me <= 64 && tiles >= 1024 && (uint64_t)p.E * p.R * p.N * 2 > (320ull << 20);

@@ -34,17 +34,7 @@ int launch_tiled(TiledRowsParams &p, hipStream_t s)
         EGS_CHECK_LAUNCH("tiny_rows_kernel");
         return EGS_OK;
     }
-    // Columns per tile: what takes the fewest rounds of the 256 CUs, each as long as the tile's matrix instructions and the fixed
-    // part of a tile (fetching 64 rows, and what a slab's barriers cost) let it be, measured at 42 shapes.  80 columns only where
-    // the matrix instructions are the larger part (fp32: E35 of 6000 picks, R185 N67 71 us, 78 with 96 columns; 16-bit 35 and 33).
-    const int64_t Me = (int64_t)p.B * p.K, row_tiles = p.E * ((Me + 63) / 64);
-    int tn = 0;
-    double least = 0;
-    for (const int c : {6, 5, 4, 2}) {
-        if (c == 5 && TT::ES == 2) continue;
-        const double cost = (double)((row_tiles * ceil_div(p.N, 16 * c) + 255) / 256) * (c + (TT::ES == 2 ? 1.5 : 1.0));
-        if (tn == 0 || cost < least) { least = cost; tn = c; }
-    }
+    const int tn = tiled_columns(p.E, (int64_t)p.B * p.K, p.N, TT::ES == 4);
     if constexpr (TT::ES == 4) {
         if (tn == 5) return launch_tiled_one<TT, WES, W_TRANS, 5>(p, s);
     }
