@@ -163,8 +163,8 @@ int64_t dw_split32_slabs(const egs_dims *d)
 // 12.7 / 12.0, 48 level, 99 picks at B3 E150 I70 J130 0.91 of it, 155 picks at B1 T712 E125 I369 J128 28.4 / 34.5).
 // Against the 32 x 32 tiles of tiled_dw_kernel by the time that the fullest CU takes, fitted to 1101 sizes alone on the device: up to three
 // workgroups of it on a CU, two of those, each some us, and some for every 32 picks (128) that a CU's workgroups go through, plus the
-// second pass.  Within 10 and 12 % of the time at 95 % of the sizes; by it 6 sizes are 3 % slower than they could be and none more than
-// 10 %.  us, it / that: B53 T97 E29 K41 I111 J75 30 / 43, B12 T121 E52 K61 I272 J31 (59 % of the tiles empty) 30 / 18.6, B26 T665 E30 K30 I523
+// second pass.  Within 10 and 12 % of the time at 95 % of the sizes; by it 13 sizes are 3 % slower than on the fp32 instruction and none more
+// than 10 %.  us, it / that: B53 T97 E29 K41 I111 J75 30 / 43, B12 T121 E52 K61 I272 J31 (59 % of the tiles empty) 30 / 18.6, B26 T665 E30 K30 I523
 // J32 33 / 23.5, B20 T289 E33 K163 I693 J29 111 / 90.
 bool dw_split32_pays(const egs_dims *d, const DwPlan &pl)
 {
@@ -177,7 +177,7 @@ bool dw_split32_pays(const egs_dims *d, const DwPlan &pl)
     const double split_us = 6.2 * (double)((split + 2) / 3) + 0.56 * (double)split * (pl.f_picks_per_split / 32) + (pl.f_S > 1 ? 1.9 + 2.5e-6 * pl.f_S * elems : 0.0);
     const double plain_us = 2.7 + 3.4 * (double)((plain + 1) / 2) + 1.08 * (double)plain * (((int64_t)pl.picks_per_split + 127) / 128) +
                             (pl.S > 1 ? 3.0 + 2.8e-6 * pl.S * elems : 0.0);
-    return split_us < 0.97 * plain_us;
+    return split_us < plain_us;
 }
 
 // 16-bit weight gradients in strips: the tile (32 tp x bq) and the number of splits of the picks that dw_strip_kernel is expected to be
