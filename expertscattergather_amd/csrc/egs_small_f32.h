@@ -177,9 +177,10 @@ __global__ __launch_bounds__(64 * (16 / TQ), 4) void rows_small_f32_kernel(Small
         float odd = 0.f;
 #pragma unroll
         for (int t = 0; t < TG; ++t) {
-            const int live = __shfl(state, (t0 + t) * 16 + a, kWave) == 1 ? 4 : 0;
+            float one = 0.f;
 #pragma unroll
-            for (int tn = 0; tn < TN; ++tn) odd = not_finite(acc[t][tn], live, odd);
+            for (int tn = 0; tn < TN; ++tn) one = not_finite(acc[t][tn], 4, one);
+            if (__shfl(state, (t0 + t) * 16 + a, kWave) == 1) odd += one;
         }
         if (__any(odd != odd)) {
             f32x4 again[TG][TN];
