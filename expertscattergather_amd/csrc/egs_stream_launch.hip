@@ -16,10 +16,12 @@ int launch_stream(RowsStreamParams &p, hipStream_t s)
     if (total > INT32_MAX / 2) return EGS_ERR_BAD_SHAPE;
     static_assert(L::BYTES <= 64 * 1024, "no grant needed");
     const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
-    // Weights that the memory-side cache (256 MB) does not hold until the next call go past the caches; below that they may still be there: us, past
-    // them / not, R1856 N440 Me32 E88 (143 MB) 39.0 / 28.5, R3072 N256 Me8 E131 (206 MB) 46.6 / 40.8.  (16-bit weights by 64 rows are always more.)
+    // Weights of which two - a layer has a gather's and a scatter's - do not stay in the memory-side cache (256 MB) go past the caches.  Over 157 sizes,
+    // past them against not, two weights in turn: 90 to 130 MB 1.07 to 1.13 of the time, to 150 MB 1.00 to 1.02, from there on 0.91 to 0.96
+    // (B4 T512 E256 K8 I2048 J512, fp8, a gather and a scatter: 181 us and 188).  A call repeated by itself with the same weights finds them there
+    // up to 256 MB, and loses 12 %: no layer does that.  (16-bit weights by 64 rows are always more.)
     constexpr bool kAlways = WES == 2 && MT == 4;
-    const bool once = kAlways || (p.m_tiles == 1 && (uint64_t)p.E * p.R * p.N * WES > (256ull << 20));
+    const bool once = kAlways || (p.m_tiles == 1 && (uint64_t)p.E * p.R * p.N * WES > (128ull << 20));
     if (once) hipLaunchKernelGGL((rows_stream_kernel<TT, WES, W_TRANS, MT, true>), grid, dim3(kThreads), L::BYTES, s, p);
     else hipLaunchKernelGGL((rows_stream_kernel<TT, WES, W_TRANS, MT, kAlways>), grid, dim3(kThreads), L::BYTES, s, p);
     EGS_CHECK_LAUNCH("rows_stream_kernel");

@@ -105,7 +105,7 @@ def test_scatter_with_bias(dtype):
 
 @pytest.mark.parametrize("rows", [20, 40])
 def test_weights_past_the_caches(rows):
-    """More than 256 MB of weights under a single row tile of 32 or 64 rows: read past the caches."""
+    """More weights than the line (128 MB), under a single row tile of 32 or 64 rows: read past the caches."""
     B, T, E, K, I, J = 1, 64, 340, rows, 1024, 512
     g = torch.Generator(device="cuda").manual_seed(2)
     X, W = (torch.randn(*s, device="cuda", generator=g).bfloat16() for s in ((B, T, I), (E, I, J)))
