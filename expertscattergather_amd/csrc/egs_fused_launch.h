@@ -29,7 +29,11 @@ int launch_scatter_fused_one(const ScatterFusedParams &p, size_t lds, int blocks
         name = "scatter_fused_runs_kernel";
         static LdsGrant told_runs[2];
         constexpr bool kHolds = KS <= 2;
-        const bool hold = kHolds && p.E * ((p.K + 31) / 32) <= kFusedHeldUnits;
+        // Rows stay in registers where that saves a workgroup ten units' loads or more; bringing them into operand order ahead of the first slice
+        // and a pass over the table are its price.  Of 507 sizes, us, held / not: B18 T76 E2 K3 I896 J64 two units in runs of two 13.9 / 11.7, B85
+        // T286 E4 K48 I160 J64 eight in runs of two 15.8 / 13.6; from this line on 4 of 361 are more than 3 % slower, on average 0.90 of it.
+        const int units = p.E * ((p.K + 31) / 32);
+        const bool hold = kHolds && units <= kFusedHeldUnits && units * (p.run - 1) >= 10;
         const auto kernel = hold ? scatter_fused_runs_kernel<TT, W_NMAJOR, KS, kHolds> : scatter_fused_runs_kernel<TT, W_NMAJOR, KS, false>;
         const int rc_lds = allow_large_lds((const void *)kernel, told_runs[hold], lds, "hipFuncSetAttribute(scatter_fused_runs_kernel)");
         if (rc_lds != EGS_OK) return rc_lds;

@@ -15,7 +15,8 @@ from expertscattergather_amd import hip_kernels as hk
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
 @pytest.mark.parametrize("shape", [
-    (90, 5, 1, 3, 128, 32),         # one unit, fewer tokens than a wavefront sums at a time
+    (90, 5, 1, 3, 128, 32),         # one unit, fewer tokens than a wavefront sums at a time; in a run of two, not held
+    (128, 5, 1, 3, 704, 32),        # in a run of eleven, held
     (33, 300, 16, 64, 288, 64),     # every register taken, three rounds of tokens, a short last run
     (33, 130, 33, 17, 288, 64),     # one unit more than there are registers for
     (40, 129, 31, 33, 256, 32),     # two units per expert, the second of one pick: too many
