@@ -8,8 +8,8 @@
 // slab's picks by a 2 x 2 grid of the tile; the halves' sums meet in LDS at the end, in that order.  Rows that do not exist get an
 // offset outside the buffer descriptor and arrive as zeros.  Consecutive tiles of an expert share an XCD, and every XCD gets as many.
 //
-// What bounds it is the rows' way from the memory-side cache into the eight L2s, which the gather makes 90 MB long at B64 T256 E32 K32
-// I768 J64: 18.8 us there, of which 4 before the first slab, with 256 workgroups of 96 columns; tiles of 32 columns, a wavefront-private
+// What bounds it is the rows' way from the memory-side cache into the eight L2s, which the gather makes 88 MB long at B64 T256 E32 K32
+// I768 J64: 18.9 us there, of which 4 before the first slab, with 256 workgroups of 96 columns; tiles of 32 columns, a wavefront-private
 // stage each and the wavefronts' sums met in LDS took 28.4 us.  Wider tiles read less and fill fewer CUs, so the host picks the width by
 // the rounds it makes (dw_strip_plan); 256 x 256 tiles with the picks split to fill the CUs took 24 us at B6 T1100 E20 K150 I328 J136,
 // strips of 96 take 10.

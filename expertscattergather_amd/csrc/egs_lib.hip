@@ -1,6 +1,8 @@
 // Host side of the library: argument validation, workspace plans, kernel selection and the C ABI
-// declared in include/egs_hip.h.  The two template-heavy launch families (tiled rows products,
-// tiled weight gradients) live in egs_rows_launch.hip and egs_dw_launch.hip.
+// declared in include/egs_hip.h.  The launches of kernels that are templates live in units of their own, so that
+// they build side by side: egs_rows_launch.hip (products), egs_stream_launch.hip (few rows), egs_f8_launch.hip, egs_dw_launch.hip
+// (weight gradients), egs_tiled_*.hip (any size), egs_small_*.hip and egs_fused_*.hip (small experts), egs_sum_launch.hip (tables and
+// sums), egs_pass_launch.hip, egs_mlp_launch.hip, egs_bias.hip, egs_router.hip.
 #include "egs_host.h"
 #include "../../include/egs_hip_testing.h"
 #include "egs_device.h"

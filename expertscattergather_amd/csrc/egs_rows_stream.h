@@ -1,11 +1,12 @@
 // Rows x weight products of experts with few rows: what takes the time is that every weight has to come from memory once.
 //
 // A workgroup of four wavefronts owns 16 MT rows (32 or 64) x 128 bytes of weight columns of one expert and goes through the whole
-// reduction.  What bounds such a product is the number of bytes on their way: a request beyond the L2 takes about 2.4 us under load,
-// so 256 CUs move B / 2.4 us x 256 of weights for B bytes in flight on each.  tiled_rows_kernel keeps two slabs of two operands in
+// reduction.  What bounds such a product is the number of bytes on their way: a request beyond the L2 takes about 4 us under load (3.9 at
+// 4.9 TB/s), so 256 CUs move B / 4 us x 256 of weights for B bytes in flight on each.  tiled_rows_kernel keeps two slabs of two operands in
 // registers, 24 KB a workgroup of which 8 KB fp8 weights.  Here slabs of 64 reduction elements (8 KB of weights and 4 KB
 // of rows, at MT = 2) go from memory to LDS without passing through registers, three of them in flight and one being multiplied,
-// three workgroups to a CU: 72 KB of weights.  Weight pieces are whole 128-byte lines.
+// three workgroups to a CU: 72 KB of weights.  Weight pieces are whole 128-byte lines.  A gather's first rows are requested once the first
+// weights are there: the index words are the compiler's loads, and it waits for everything before it uses one, also what it does not count.
 //
 // 16-bit rows, 16-bit or (with [reduction][column] weights) fp8 weights, R a multiple of 64, 16-byte aligned rows, operands below 2 GiB.
 #pragma once

@@ -6,7 +6,7 @@
 // slab of direct 16-byte loads in flight under the one being multiplied, one barrier per slab.  Chunks past the reduction length, rows
 // that do not exist and columns past the last get an offset outside the buffer descriptors and arrive as zeros.
 //
-// What bounds such a product is a chain of round trips (index, rows, slabs, results), so three workgroups share a CU: two stages of 24 KB
+// What bounds such a product is a chain of round trips (index, with which the compiler waits for the first weights too, rows, slabs, results), so three workgroups share a CU: two stages of 24 KB
 // (three stages and two workgroups: level where one round of those is enough, else slower, 27.7 us for 23.5 at R256 N136 Me2400 E40).
 // 128 x 128 tiles took 1.8 times as long at R328 N136 Me900 E20, 64 x 64 tiles 1.2 times.  Against the general kernel's 64 rows through
 // registers: R768 N64 Me2048 E32 (150 MB through the L2s instead of 200) 19.3 -> 13.8 us, R328 N136 Me900 E20 14 -> 10.

@@ -7,8 +7,8 @@
 // (coalesced 64-byte runs per row, then the 4 x 16 lane transposition) and are split there.  One wavefront = 32 picks of one
 // expert, a workgroup 256; one barrier (W(e) in place).  A wavefront multiplies and stores its 16-pick row tiles one after the
 // other, the first tile's rows requested before the barrier and the others after it.
-// us, three pieces / the fp32 instruction, which was the roof with 138 TFLOP/s: B64 T256 E32 K32 I128 J64 14.0 / 16.9 (the matrix
-// instructions take 3, indices, rows and W(e) the rest), E60 20.9 / 26.6, I64 9.8 / 11.2, B160 J48 23 / 30, B8 T100 E16 9.2 / 11.8; level for
+// us in a graph, three pieces / the fp32 instruction, which was the roof with 138 TFLOP/s: B64 T256 E32 K32 I128 J64 13.4 / 15.5 (the matrix
+// instructions take 3, indices, rows and W(e) the rest), E60 21.7 / 26.7, I64 9.2 / 10.3, B160 J48 22.4 / 28.4, B8 T100 E16 9.4 / 11.5; level for
 // 16 columns.  (The one-kernel scatter does not gain: it would split every weight once per batch element, 20.0 / 18.8.)
 //
 // Replaces the reference's expert_gather_kernel (egs/triton_kernels.py:49-143) on these shapes.

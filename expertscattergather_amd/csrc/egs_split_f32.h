@@ -18,10 +18,11 @@ struct SplitDwLds {
 // tiled_dw_wide_kernel (egs_tiled.h) for fp32 with the picks split over workgroups where there are few tiles: a 64 x 64 tile of dW(e)
 // per workgroup, wavefronts 2 x 2; slabs of 32 picks, fetched two ahead.  A slab's fragments go into registers as soon as it is in LDS;
 // one barrier later the next slab is split and written under the matrix instructions of this one.
-// What bounds it is instruction issue: per slab and wavefront 24 matrix instructions (384 cycles) and 110 vector instructions of two to
-// four, 88 of which split; hence buffer loads (a pick that does not exist needs no masks) and 32-bit offsets (with 64-bit
-// ones and masks 180 vector instructions, 151 us for 135).  us against the fp32 instruction: B30 T46 E73 K44 I384 J169 202 -> 135, B53 T97 E29
-// K41 I111 J75 42.7 -> 30, B16 T512 E64 K64 I256 J128 66 -> 43, B33 T1697 E37 K79 I64 J256 73 -> 38.
+// What bounds it is instruction issue: per slab and wavefront 24 matrix instructions (384 cycles) and 126 vector instructions of two to
+// four, 104 of which split (16 of them the factor: B53 T97 E29 K41 I111 J75 26.3 us without, 27.5 with, in a trace); hence buffer loads (a pick
+// that does not exist needs no masks) and 32-bit offsets (with 64-bit ones and masks 70 vector instructions more, 151 us for 135 at the first of
+// these).  us in a graph, the fp32 instruction / this: B30 T46 E73 K44 I384 J169 182 / 130, B53 T97 E29 K41 I111 J75 40.7 / 29.6, B16 T512
+// E64 K64 I256 J128 61 / 42, B33 T1697 E37 K79 I64 J256 71 / 40.
 // (The products rows x weights gain less, 1.05 to 1.18 times above 12000 slabs and lose below: not taken there.)
 static __global__ __launch_bounds__(kThreads, 3) void tiled_dw_split_kernel(TiledDwParams p)
 {
