@@ -430,7 +430,7 @@ __global__ __launch_bounds__(kFusedThreads) void scatter_fused_kernel(ScatterFus
 // More slices than the device has CUs for: a run of them per workgroup, with one sort.  The slices of a run multiply the same rows,
 // so with HOLD (a reduction of at most two steps, and no more units of 32 picks than the wavefronts have registers for) they are
 // read and brought into operand order once, and only weights travel between slices.  B64 T256 E32 K32 I768 J64, bf16: 47 -> 37 us
-// (sort and first operands 11, then 4.6 a slice: 128 KB of weights per CU, which all CUs together take 2.2 us to get out of L2,
+// (sort and first operands 7, then 4.9 a slice: 128 KB of weights per CU, which all CUs together take 2.2 us to get out of L2,
 // products 1.1, sums 1.0); B128 T64 E8 K16 I1024 J64 39 -> 33; the same with fp32 and J32 65 -> 59.
 template <class TT, bool W_NMAJOR, int KS, bool HOLD>
 __global__ __launch_bounds__(kFusedThreads) void scatter_fused_runs_kernel(ScatterFusedParams p)
