@@ -13,15 +13,35 @@ SHAPES = [(1, 1, 1, 1), (3, 17, 5, 4), (2, 64, 9, 64), (2, 65, 64, 33), (64, 256
 LARGE = [(1, 1024, 70, 100), (1, 700, 140, 30), (2, 3000, 40, 130), (64, 800, 129, 9)]
 
 
+def kernels_of(B, T, E):
+    """What a call launches: the rows' sums ahead of the router where it asks for a workspace to put them."""
+    return ["router_stats_kernel", "router_kernel"] if _abi.lib().egs_expert_choice_router_workspace_bytes(B, T, E) > 0 else ["router_kernel"]
+
+
+def without_workspace(logits, K, ind_dtype):
+    """The router as one launch: every workgroup computes the rows' sums."""
+    B, T, E = logits.shape
+    Ind, scores = torch.empty(B, E, K, dtype=ind_dtype, device="cuda"), torch.empty(B, E, K, device="cuda")
+    codes = {torch.float32: _abi.F32, torch.float16: _abi.F16, torch.bfloat16: _abi.BF16}, {torch.int16: _abi.IND_I16, torch.int64: _abi.IND_I64}
+    with _abi.launch_log() as log:
+        rc = _abi.lib().egs_expert_choice_router(logits.data_ptr(), Ind.data_ptr(), scores.data_ptr(), None, 0, B, T, E, K, codes[0][logits.dtype],
+                                                 codes[1][ind_dtype], torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and log.kernels == ["router_kernel"], (rc, log.kernels)
+    return Ind, scores
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
 @pytest.mark.parametrize("B,T,E,K", SHAPES, ids=lambda v: str(v))
 def test_router_matches_topk(B, T, E, K, dtype):
     gen = torch.Generator().manual_seed(B + T + E + K)
     logits = torch.randn(B, T, E, generator=gen).to(dtype)
     ind_dtype = torch.int16 if dtype is torch.float16 else torch.int64
+    on_device = logits.cuda()
     with _abi.launch_log() as log:
-        Ind, scores = expert_choice_router(logits.cuda(), K, ind_dtype)
-    assert log.kernels == ["router_kernel"] and Ind.dtype is ind_dtype and scores.dtype is torch.float32
+        Ind, scores = expert_choice_router(on_device, K, ind_dtype)
+    assert log.kernels == kernels_of(B, T, E) and Ind.dtype is ind_dtype and scores.dtype is torch.float32
+    if len(log.kernels) > 1:                            # one launch, whatever the library prefers: the same bits
+        assert all(torch.equal(a, b) for a, b in zip((Ind, scores), without_workspace(on_device, K, ind_dtype)))
     aff = torch.softmax(logits.double(), -1).transpose(1, 2)
     want = aff.topk(K, -1)[0]
     Ind, scores = Ind.cpu().long(), scores.cpu()
@@ -73,10 +93,16 @@ def test_row_sums_first_or_by_every_workgroup(B, T, E, K):
     L, stream = _abi.lib(), torch.cuda.current_stream().cuda_stream
     need = L.egs_expert_choice_router_workspace_bytes(B, T, E)
     assert need in (0, B * T * 8)
-    Ind, scores = expert_choice_router(logits, K)
-    own_Ind, own = torch.empty_like(Ind), torch.empty_like(scores)
-    rc = L.egs_expert_choice_router(logits.data_ptr(), own_Ind.data_ptr(), own.data_ptr(), None, 0, B, T, E, K, _abi.BF16, _abi.IND_I64, stream)
-    assert rc == 0
+    with _abi.launch_log() as log:
+        Ind, scores = expert_choice_router(logits, K)
+    assert log.kernels == kernels_of(B, T, E), log.kernels
+    own_Ind, own = without_workspace(logits, K, torch.int64)
+    if need == 0:                                       # a workspace that is not asked for changes nothing
+        ws, more_Ind, more = torch.empty(B * T * 8, dtype=torch.uint8, device="cuda"), torch.empty_like(Ind), torch.empty_like(scores)
+        with _abi.launch_log() as log:
+            assert L.egs_expert_choice_router(logits.data_ptr(), more_Ind.data_ptr(), more.data_ptr(), ws.data_ptr(), ws.numel(), B, T, E, K, _abi.BF16,
+                                              _abi.IND_I64, stream) == 0
+        assert log.kernels == ["router_kernel"] and torch.equal(more_Ind, own_Ind)
     assert torch.equal(Ind, own_Ind) and torch.equal(scores.view(torch.int32), own.view(torch.int32))
     aff = torch.softmax(logits.cpu().double(), -1).transpose(1, 2).nan_to_num(9.0)
     scores = scores.cpu().double().nan_to_num(9.0)
