@@ -381,8 +381,10 @@ __device__ __forceinline__ void tiled_rows_body(const TiledRowsParams &p, const 
     }
 }
 
+// Two slabs of fp32 rows times 80 columns of weights [N][R] take 104 registers: bound to the 96 of five wavefronts they put two away in memory (120 such
+// gathers 1.011 of the time; two of them, of 46 us and more, 0.97).
 template <class TT, int WES, bool W_TRANS, int TN, int SLABS>
-__global__ __launch_bounds__(kThreads, SLABS == 1 ? 6 : SLABS == 2 ? 5 : SLABS > 0 || TN <= 2 ? 4 : 3) void tiled_rows_kernel(TiledRowsParams p)
+__global__ __launch_bounds__(kThreads, SLABS == 1 ? 6 : SLABS == 2 && !(TT::ES == 4 && !W_TRANS && TN == 5) ? 5 : SLABS > 0 || TN <= 2 ? 4 : 3) void tiled_rows_kernel(TiledRowsParams p)
 {
     tiled_rows_body<TT, WES, W_TRANS, TN, SLABS>(p, (int)blockIdx.x);
 }

@@ -40,3 +40,9 @@ def test_two_of_the_routers_workgroups_of_1024_threads_share_a_compute_unit(kern
         assert k["sgpr_count"] <= 80, (name, k)
         if "ELi0E" in name:                         # the rows' sums from a launch before it
             assert k["vgpr_count"] <= 64, (name, k)
+
+
+def test_no_kernel_puts_registers_away_in_memory(kernels):
+    known = {"_ZN3egs21rows_small_f32_kernelILb1ELi8ELi4ELi2EEEvNS_15SmallRowsParamsE"}      # 128 x 64 weights in registers: four of them, once per tile
+    spilled = [(n, k["vgpr_spill_count"], k["private_segment_fixed_size"]) for n, k in kernels if n not in known and (k["vgpr_spill_count"] or k["private_segment_fixed_size"])]
+    assert not spilled, spilled
