@@ -11,6 +11,8 @@
 //   * tiles are 64 rows x 32 .. 96 columns, so that a ragged width wastes little and a small problem still has
 //     many workgroups; workgroups are dealt to the XCDs evenly for any number of experts.
 #pragma once
+#include <type_traits>
+
 #include "egs_device.h"
 
 namespace egs {
@@ -79,8 +81,13 @@ struct TiledLds {
 // 76 to 156.  Products alone, us, loop / written out: f16 B70 T302 E52 K143 I32 J93 56 / 37, bf16 B114 T627 E44 K33 I64 J167 42 / 30, f32 B13 T243 E104
 // K48 I49 J224 40 / 34, bf16 B81 T155 E72 K82 I192 J35 54 / 45; of 2200 with their sums 10 are more than 3 % slower.  The loop in one stage had to
 // spill (73 -> 248 us at worst).
+// The parameters: by value where the compiler then keeps a second slab's loads ahead (fp8 weights, 32 columns, the loop: 114 registers; by
+// reference 92, and 1.014 of the time over 84 sizes, 9 of them more than 3 % slower), else by reference (by value 158 registers and not 126 with
+// 96 columns).
+template <int WES, int TN, int SLABS>
+using TiledRowsBy = typename std::conditional<WES == 1 && TN == 2 && SLABS == 0, const TiledRowsParams, const TiledRowsParams &>::type;
 template <class TT, int WES, bool W_TRANS, int TN, int SLABS = 0>
-__device__ __forceinline__ void tiled_rows_body(const TiledRowsParams &p, const int block)
+__device__ __forceinline__ void tiled_rows_body(TiledRowsBy<WES, TN, SLABS> p, const int block)
 {
     constexpr int ES = TT::ES, VEC = TT::VEC;
     constexpr bool W_FP8 = WES == 1;

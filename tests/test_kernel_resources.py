@@ -46,3 +46,10 @@ def test_no_kernel_puts_registers_away_in_memory(kernels):
     known = {"_ZN3egs21rows_small_f32_kernelILb1ELi8ELi4ELi2EEEvNS_15SmallRowsParamsE"}      # 128 x 64 weights in registers: four of them, once per tile
     spilled = [(n, k["vgpr_spill_count"], k["private_segment_fixed_size"]) for n, k in kernels if n not in known and (k["vgpr_spill_count"] or k["private_segment_fixed_size"])]
     assert not spilled, spilled
+
+
+def test_the_fp8_loop_of_32_columns_keeps_two_slabs_ahead(kernels):
+    """Two slabs of 64 rows and of 32 columns' weights on their way are 16 + 8 registers, the addresses 24; with fewer than a hundred in all the compiler waits
+    for one slab before it asks for the next."""
+    (loop,) = [k for n, k in kernels if "tiled_rows_kernelINS_8ElemBF16ELi1ELb1ELi2ELi0E" in n]
+    assert loop["vgpr_count"] > 100, loop
