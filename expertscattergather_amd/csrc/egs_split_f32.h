@@ -262,9 +262,9 @@ static __global__ __launch_bounds__(kThreads, 3) void tiled_dw_split_kernel(Tile
 // ------------------------------------------------------------------------------ product and weight gradient of a backward call in one launch
 // dY or dX's product rows and the weight gradient do not depend on each other, and at most sizes that come here neither fills the device: each
 // is a chain of round trips of 5 to 15 us with a launch of its own.  The workgroups with the longer chains come
-// first (launch_tiled_pair); the bodies are those of the kernels alone (the same bits) and take about the same LDS and registers, so nothing
-// is lost where both do fill it: of 769 backward calls of random sizes up to 1 ms none is more than 1.6 % slower, and they take 0.775 of
-// the time on average (0.68 of 10 to 15 us, 0.80 of 20 to 30, 0.87 of 50 to 100, 0.90 beyond).
+// first (launch_tiled_pair); the bodies are those of the kernels alone (the same bits; the product's the loop, also for the short reductions that are
+// written out where it is alone, and then sometimes faster apart: tiled_apart).  Against two launches with the kernels as they are, 393 scatter backward
+// calls of random sizes take 0.73 of the time and 389 gather backward calls, sums and all, 0.84; none is more than 1.6 % slower.
 // us in a graph, two launches / one: bf16 B3 T607 E7 K90 I768 J19 dY and dW 15.3 / 8.3, B4 T201 E17 K6 I352 J31 11.3 / 6.3, f32 B66 T52 E5 K5 I431 J27
 // 19.3 / 10.8, f32 B30 T706 E66 K21 I866 J192 253 / 248.
 enum TiledDwKind { TILED_DW, TILED_DW_WIDE, TILED_DW_SPLIT };

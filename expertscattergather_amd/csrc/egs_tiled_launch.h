@@ -31,6 +31,21 @@ bool tiled_dw_grid(TiledDwParams &p, TiledDwGrid &g)
     return true;
 }
 
+// Two launches where the product's written-out kernel (one or two slabs), which more workgroups of a CU run side by side than the shared launch's loop,
+// gains more than the sharing saves: many tiles of product, enough of the weight gradient's to fill the device on their own, in chains that are
+// not long against the product.  us, one launch / two: bf16 dY and dW B41 T1715 E119 K224 I32 J25 90 / 74, B90 T1835 E94 K138 I32 J25 100 / 84, f32 B113
+// T319 E117 K63 I32 J55 158 / 135, f32 dX and dW B98 T555 E63 K217 I32 J64 323 / 276; not bf16 B43 T1534 E102 K139 I39 J160 191 / 189.  Of 1542 backward
+// calls (most of them of short reductions and large) 56 go this way, 6 of them more than 3 % slower for it (1.05); of 1045 others of that kind 7 are left that
+// two launches would run more than 3 % faster (at worst 1.14), where one in 37 was (1.21).
+template <class TT>
+bool tiled_apart(const TiledRowsParams &p, int blocks, const TiledDwParams &q, const TiledDwGrid &g)
+{
+    const int slabs = ceil_div(p.R, 8 * TT::VEC);
+    if (g.kind != TILED_DW || slabs > 2 || g.blocks < 400) return false;
+    const double tiles = blocks * (TT::ES == 4 ? 2.0 : 1.0), steps = (double)q.B * q.K / q.S / 128;        // fp32 tiles take twice as long
+    return tiles >= 4096 * (2 * slabs - 1) && tiles >= 0.6 * g.blocks * steps;
+}
+
 template <class TT, int TN, int KIND>
 int launch_tiled_pair(const TiledRowsParams &p, int blocks, size_t lds, const TiledDwParams &q, const TiledDwGrid &g, hipStream_t s)
 {
@@ -59,7 +74,8 @@ int launch_tiled_one(TiledRowsParams &p, TiledDwJob *dw, hipStream_t s)
     const int blocks = (int)(8 * ((total + 7) / 8));
     if constexpr (!W_TRANS && WES == TT::ES) {
         TiledDwGrid g;
-        if (dw != nullptr && !dw->done && tiled_dw_grid<TT>(dw->q, g) && (int64_t)g.blocks + blocks <= INT32_MAX / 2) {
+        if (dw != nullptr && !dw->done && tiled_dw_grid<TT>(dw->q, g) && (int64_t)g.blocks + blocks <= INT32_MAX / 2 &&
+            !tiled_apart<TT>(p, blocks, dw->q, g)) {
             int rc;
             if (TT::ES == 4 && g.kind == TILED_DW_SPLIT) rc = launch_tiled_pair<TT, TN, TT::ES == 4 ? TILED_DW_SPLIT : TILED_DW>(p, blocks, lds, dw->q, g, s);
             else if (g.kind == TILED_DW_WIDE) rc = launch_tiled_pair<TT, TN, TILED_DW_WIDE>(p, blocks, lds, dw->q, g, s);

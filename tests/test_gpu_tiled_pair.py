@@ -5,7 +5,8 @@ import ctypes
 import pytest
 import torch
 
-from tests._util import make_case
+from oracle import egs_oracle as O
+from tests._util import assert_close, make_case, np64
 from tests.test_gpu_parity import dev
 
 pytestmark = pytest.mark.gpu
@@ -56,3 +57,26 @@ def test_one_launch_has_the_bits_of_two(shape, dtype):
     assert "tiled_pair_kernel" not in log.kernels, log.kernels
     for name, a, b in zip(("dX", "dW of the gather", "dY", "dW of the scatter"), (dX, dWg, dY, dWs), want):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("shape, dtype, gather, scatter", [
+    ((30, 50, 70, 70, 65, 31), torch.float32, False, True),     # one slab of 31 columns, three of 65: dX's rows written out, dY's in the loop
+    ((62, 204, 58, 131, 51, 32), torch.float32, False, False),  # two slabs of 51
+    ((30, 50, 64, 70, 31, 33), torch.float32, True, True),      # a weight gradient in bf16 pieces always shares
+    ((60, 50, 64, 70, 31, 33), torch.bfloat16, True, True),     # half as many tiles as the line asks for
+], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v).replace("torch.", ""))
+def test_large_products_of_short_reductions_stay_apart(shape, dtype, gather, scatter):
+    B, T, E, K, I, J = shape
+    case = make_case(sum(shape), *shape, dtype)
+    X, Wg, Ws, Y, dOut, Ind = (dev(case[k]) for k in ("X", "Wg", "Ws", "Y", "dOut", "Ind"))
+    with _abi.launch_log() as log:
+        dX, dWg = hk.expert_gather_backward_call(X, Wg, Ind, Y, torch.float32)
+    assert ("tiled_pair_kernel" in log.kernels) == gather and "tiled_rows_kernel" in log.kernels, log.kernels
+    with _abi.launch_log() as log:
+        dY, dWs = hk.expert_scatter_backward_call(Y, Ws, Ind, dOut, torch.float32)
+    assert ("tiled_pair_kernel" in log.kernels) == scatter and "tiled_rows_kernel" in log.kernels, log.kernels
+    ind = case["Ind"].numpy()
+    wX, wWg = O.gather_backward(np64(case["X"]), np64(case["Wg"]), ind, np64(case["Y"]))
+    wY, wWs = O.scatter_backward(np64(case["Y"]), np64(case["Ws"]), ind, np64(case["dOut"]))
+    for name, got, want in (("dX", dX, wX), ("dW of the gather", dWg, wWg), ("dY", dY, wY), ("dW of the scatter", dWs, wWs)):
+        assert_close(got, want, dtype, name)
