@@ -783,14 +783,15 @@ size_t dw_bytes_planned(const egs_dims *d, int act_dtype)
 // (within 14 and 9 % of most): the turns that its workgroups take at the CUs, each a sort of the picks and then, for every slice, units of 32
 // picks of one expert, empty places included, and sums of all tokens; against the rows written and read, the tiles they are made in,
 // the weights, the output, and the indices that every group of 32 tokens looks through.  What it loses are many experts of few picks (units
-// mostly empty: bf16 B1 T2127 E83 K5 I640 J128 33 us, 14 as rows; f32 B91 T338 E64 K5 I192 J64 99 / 35), few batch elements with many tokens
-// (f32 B9 T454 E28 K5 I96 J64 16.6 / 10.8) and slices by the hundred (f16 B80 T269 E43 K23 I928 J64 227 / 98); of 1319 calls that this is asked
-// for 381 go by rows and 4 are more than 3 % slower for it, and scatters (gather backward calls) take 0.95 (0.94) of the time they took in
-// 16 bits, 0.87 (0.84) in fp32.  A weight gradient that shares a launch with either counts 3 or 4 us for it.  Zipf-distributed picks,
-// whose hot tokens one group of threads adds up here and many there, make it lose 1.1 to 1.4 times as often; a call can't know.
-// In passes (more than 1024 picks) it loses to the rows by 1.2 on average (1.5 to 1.6 in fp32) and by 2 to 3 with Zipf-distributed picks; the
-// model keeps 103 of 293 scatters there (0.97 of the rows' time; bf16 B78 T43 E49 K25 I96 J32 16.7 / 28.3) and one whose table comes with the
-// gather's launch, and the others take 0.70 of the time they took.
+// mostly empty: bf16 B1 T2127 E83 K5 I640 J128 34 us, 13 as rows; f32 B91 T338 E64 K5 I192 J64 82 / 30), few batch elements with many tokens
+// (f32 B9 T454 E28 K5 I96 J64 16.3 / 10.3) and slices by the hundred of few picks (f16 B21 T416 E125 K5 I896 J128 94 / 32; not of full units: f16 B80
+// T269 E43 K23 I928 J64 85 / 126).  Of 2481 other calls that either takes 507 go by rows, 4 of them more than 3 % slower for it (1.11), and all
+// take 0.93 of the one kernel's time in 16 bits and 0.83 in fp32 (0.89 and 0.77 are the least: the margin is on its side, for it needs no workspace).
+// A weight gradient that shares a launch with either counts 3 or 4 us for it.  Zipf-distributed picks, whose hot tokens one group of threads adds up
+// here and many there, make it lose more (its time 1.0 to 1.5 of the rows' on average in one pass); a call can't know.
+// In passes (more than 1024 picks) it loses to the rows by 1.3 on average (1.85 in fp32) and by 3 with Zipf-distributed picks; the
+// model keeps 184 of 379 scatters there (1.18 of the rows' time; bf16 B78 T43 E49 K25 I96 J32 17.8 / 28.7) and one whose table comes with the
+// gather's launch, and the others take 0.55 of the time they took.
 bool fused_model_pays(const FusedPlan &fp, const egs_dims *d, int act_dtype, double extra_us, double margin = 1.15)
 {
     const bool f32 = act_dtype == EGS_F32, passes = fp.experts_per_pass != d->E;
@@ -815,8 +816,8 @@ bool fused_model_pays(const FusedPlan &fp, const egs_dims *d, int act_dtype, dou
     return fused_us + extra_us < margin * rows_us;
 }
 
-// Layout of a caller-owned routing table, for the sizes whose one-kernel scatter can read one (16-bit types, one pass,
-// T + 1 <= 2048 table offsets per batch element); `ok` false: a table would not be used; `worth` false: none is asked for, and one that is given is
+// Layout of a caller-owned routing table, for the sizes whose one-kernel scatter can read one (fused_reads_table: one pass of any type, or 16-bit types in
+// passes); `ok` false: a table would not be used; `worth` false: none is asked for, and one that is given is
 // built, and read where the one-kernel scatter runs.
 struct TableLayout { bool ok, worth; size_t perm_at, bytes; };
 TableLayout routing_table_layout(const egs_dims *d, int act_dtype)

@@ -252,3 +252,22 @@ def test_planning_functions_survive_arbitrary_sizes(lib):
             assert lib.egs_routing_table_bytes(d, dt) % 256 == 0
         assert lib.egs_gather_gemm_fp8act_workspace_bytes(d) % 256 == 0
     assert lib.egs_workspace_bytes(1, 0, None, _abi.BF16) == 0 and lib.egs_expert_mlp_supported(None, _abi.BF16) == 0
+
+
+@pytest.mark.parametrize("dtype, dims, rows", [
+    (_abi.BF16, (1, 2127, 83, 5, 640, 128), True),      # units of 32 picks mostly empty: 34 us in one kernel, 13 as rows
+    (_abi.F32, (91, 338, 64, 5, 192, 64), True),        # 82 / 30
+    (_abi.F32, (9, 454, 28, 5, 96, 64), True),          # many tokens, few batch elements: 16.3 / 10.3
+    (_abi.F16, (21, 416, 125, 5, 896, 128), True),      # slices by the hundred, of few picks: 94 / 32
+    (_abi.F16, (80, 269, 43, 23, 928, 64), False),      # and of full units: 85 / 126
+    (_abi.BF16, (78, 43, 49, 25, 96, 32), False),       # in passes, short rows: 17.8 / 28.7
+    (_abi.BF16, (64, 256, 32, 32, 768, 64), False),     # runs of slices: 38 / 74
+], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_which_scatter_is_planned(lib, dtype, dims, rows):
+    """The product rows are in the workspace, the one kernel needs none: the sizes that the rule's figures name go the way they say."""
+    d = _abi.Dims(*dims)
+    B, T, E, K, I, J = dims
+    need = lib.egs_workspace_bytes(_abi.OP_GEMM_SCATTER, 0, d, dtype)
+    assert (need >= B * E * K * I * 4) if rows else need == 0, need
+    both = lib.egs_workspace_bytes(_abi.OP_GATHER_BACKWARD, 0, d, dtype)
+    assert both == need + lib.egs_workspace_bytes(_abi.OP_DW, 0, d, dtype)
