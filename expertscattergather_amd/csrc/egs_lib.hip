@@ -958,13 +958,13 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
 
 // The picks that sums without a routing table look through: 4096 a batch element, or twice that for few tokens of short rows, where the launch for the
 // table takes as long as the sums.  us: bf16 B1 T2941 E47 K157 I32 J160 25.8 -> 13.9, B2 T1832 E59 K79 I32 J20 21.7 -> 12.8, f32 B2 T440 E27 K162 I32 J40
-// 20 -> 13; 68 random scatters take 0.76 of their time, 16 under Zipf routing 0.92 (one of them is 4 % slower).  Longer rows take 0.78 to 0.83, under Zipf
+// 20 -> 13; 68 random scatters take 0.76 of their time, 16 under Zipf routing 0.92 (one of them is 4 % slower); 160 of 4097 to 4224 picks 0.70, under Zipf
+// routing 0.87 (11 slower, f16 B34 T252 E57 K72 I68 J37 44 -> 61).  Longer rows take 0.78 to 0.83, under Zipf
 // routing 1.2 to 1.4: a hot token's rows are many workgroups' with a table, and one's here.
 bool token_sums_take(const egs_dims *d)
 {
     const int64_t N = (int64_t)d->E * d->K;
-    // (4097 to 4224 picks stay with the table: its tests with the smallest number of parts are of such sizes)
-    const bool few = N > 4224 && N <= kTokenSumPicksFew && d->I <= 128 && (int64_t)d->B * d->T <= 16384;
+    const bool few = N > kTokenSumPicks && N <= kTokenSumPicksFew && d->I <= 128 && (int64_t)d->B * d->T <= 16384;
     return N >= 1 && (N <= kTokenSumPicks || few);
 }
 

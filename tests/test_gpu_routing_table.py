@@ -276,10 +276,10 @@ def test_a_table_of_garbage_gives_wrong_sums_but_ends():
             assert torch.isfinite(out.float()).all()
 
 
-@pytest.mark.parametrize("shape", [(2, 300, 33, 125, 64, 24),      # 4125 picks of 16 wavefronts: three workgroups, the last with 29 picks
+@pytest.mark.parametrize("shape", [(2, 300, 33, 125, 132, 24),     # 4125 picks of 16 wavefronts: three workgroups, the last with 29 picks
                                    (1, 2300, 90, 200, 40, 24),     # 18000 picks of 8 wavefronts (histograms of 2300 tokens): eight
                                    (90, 60, 66, 125, 24, 24),      # 8250 picks, for five workgroups: two, as 90 batch elements leave CUs for
-                                   (3, 20, 41, 100, 36, 24)],      # 4100 picks of 20 tokens, all of them hot
+                                   (3, 20, 41, 100, 132, 24)],     # 4100 picks of 20 tokens, all of them hot
                          ids=lambda s: "x".join(map(str, s)))
 def test_table_of_its_own_launch_by_several_workgroups(shape):
     B, T, E, K, I, J = shape

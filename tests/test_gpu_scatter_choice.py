@@ -66,7 +66,8 @@ def test_with_and_without_a_workspace(shape, dtype):
     ((2, 60, 50, 40, 96, 64), False),       # more than 32 picks a token
     ((6, 70, 4, 9, 32, 64), False),
     ((1, 2100, 5, 6, 64, 32), True),        # a table for long sequences is a launch of its own
-    ((2, 2100, 2150, 2, 32, 32), True),     # 4300 picks: few tokens
+    ((2, 300, 41, 100, 64, 32), True),      # 4100 picks: few tokens
+    ((2, 2100, 2150, 2, 32, 32), True),     # 4300
     ((2, 2100, 4100, 2, 32, 32), False),    # too many picks for sums without one
     ((9, 2100, 2150, 2, 32, 32), False),    # too many tokens for that many
 ], ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else str(s))

@@ -135,10 +135,11 @@ def test_weight_gradient_of_experts_with_few_picks(shape, split32, dtype):
 @pytest.mark.parametrize("dims, sums", [((6, 200, 16, 64, 256, 192), ["rows_gemm_dl_kernel", "segment_sum_kernel"]),     # the table rides along
                                         ((6, 200, 16, 64, 256, 121), ["tiled_rows_kernel", "token_sum_kernel"]),         # it would be a launch
                                         ((6, 200, 33, 125, 256, 121), ["tiled_rows_kernel", "csr_count_kernel", "segment_sum_kernel"]),  # 4125 picks
+                                        ((6, 200, 17, 241, 128, 121), ["tiled_rows_kernel", "token_sum_kernel"]),        # 4097 of short rows
                                         ((20, 120, 7, 500, 844, 25), ["tiled_rows_kernel", "csr_count_kernel", "segment_sum_kernel", "tiled_rows_kernel",
                                                                       "segment_sum_kernel"]),                            # two batch groups
                                         ((20, 120, 8, 500, 801, 24), ["tiled_rows_kernel", "token_sum_kernel"] * 2)],    # of rows read by elements
-                         ids=["rides", "few", "many", "groups", "groups-odd"])
+                         ids=["rides", "few", "many", "many-short", "groups", "groups-odd"])
 def test_which_sums_follow_the_product_rows(dims, sums):
     B, T, E, K, I, J = dims
     case = make_case(sum(dims), *dims, torch.bfloat16)
