@@ -1120,8 +1120,10 @@ int gemm_scatter_rows(const void *Y, const void *W, const void *Ind, void *Out, 
             // Few picks, and the table would be a launch of its own for one launch of sums: sums that do without it.  us, product and
             // sums with the table riding along / without a table: bf16 B54 T1123 E15 K23 I192 J320 33 / 40, B14 T2048 E64 K60 I512 J128
             // 50 / 57, B16 T512 E16 K64 I256 J256 24.5 / 26.9, B8 T2048 E32 K100 I512 J256 38.0 / 36.3; three groups of f16 B61 T1657
-            // E78 K45 I384 J384 234 / 272.  With a launch for the table: B53 T97 E29 K41 I111 J75 fp32 54 / 35; two groups of rows that
-            // the sums with the table read element by element, bf16 B58 T986 E28 K72 I443 J40 178 / 130.
+            // E78 K45 I384 J384 234 / 272.  With a launch for the table: B53 T97 E29 K41 I111 J75 fp32 54 / 35.  Groups share one table: it is the
+            // faster way for them but where rows are not whole pieces of four columns, which its sums add and store with half as many in flight: 120
+            // scatters of two to nine groups of such rows take 0.90 of the time without it (0.94 under Zipf routing; up to one pick a token 0.70, f16
+            // B101 T3838 E10 K116 I791 J47 680 / 376; from four on they are level, from sixteen on 1.04).
             if (b0 == 0)
                 token_sums = p.own_sums && !p.csr_done;
             if (rc == EGS_OK && token_sums) {

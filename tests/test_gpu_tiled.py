@@ -138,7 +138,7 @@ def test_weight_gradient_of_experts_with_few_picks(shape, split32, dtype):
                                         ((6, 200, 17, 241, 128, 121), ["tiled_rows_kernel", "token_sum_kernel"]),        # 4097 of short rows
                                         ((20, 120, 7, 500, 844, 25), ["tiled_rows_kernel", "csr_count_kernel", "segment_sum_kernel", "tiled_rows_kernel",
                                                                       "segment_sum_kernel"]),                            # two batch groups
-                                        ((20, 120, 8, 500, 801, 24), ["tiled_rows_kernel", "token_sum_kernel"] * 2)],    # of rows read by elements
+                                        ((20, 120, 8, 500, 801, 24), ["tiled_rows_kernel", "token_sum_kernel"] * 2)],    # of odd rows
                          ids=["rides", "few", "many", "many-short", "groups", "groups-odd"])
 def test_which_sums_follow_the_product_rows(dims, sums):
     B, T, E, K, I, J = dims
