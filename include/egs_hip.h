@@ -45,7 +45,8 @@ typedef enum egs_status {
     EGS_ERR_BAD_DTYPE = -3,     /* counterpart of ValueError("Unknown dtype"), reference egs/triton_kernels.py:23 */
     EGS_ERR_BAD_LAYOUT = -4,
     EGS_ERR_BAD_MODE = -5,
-    EGS_ERR_WORKSPACE = -6,     /* workspace missing, or smaller than the kernels selected for these operands need */
+    EGS_ERR_WORKSPACE = -6,     /* workspace missing, or smaller than the kernels selected for these operands need (a scatter for
+                                 * which there is a kernel that needs none takes that one instead, see egs_workspace_bytes) */
     EGS_ERR_ALIGNMENT = -7,
     EGS_ERR_HIP = -8,           /* a HIP runtime call failed; see egs_last_hip_error() */
     EGS_ERR_UNSUPPORTED = -9,
@@ -76,7 +77,8 @@ typedef enum egs_w_layout {
 } egs_w_layout;
 
 typedef enum egs_scatter_mode {
-    EGS_SCATTER_DETERMINISTIC = 0,  /* fixed summation order, bitwise reproducible, no atomics   */
+    EGS_SCATTER_DETERMINISTIC = 0,  /* fixed summation order, no atomics: the same bits from the same entry point, sizes, operand
+                                     * alignment and, where egs_workspace_bytes is not 0, any workspace of at least that size */
     EGS_SCATTER_ATOMIC = 1,         /* fp32 atomic accumulation, order of additions unspecified  */
     EGS_SCATTER_COMPACT = 2         /* DETERMINISTIC without a workspace: where the sizes allow (16-bit types, reduction
                                      * 32 / 64 / 128, output columns a multiple of 32, T <= 1024, more than 1024 picks per
@@ -110,7 +112,13 @@ const char *egs_last_hip_error(void);
 
 /* bytes of scratch the op needs for these sizes (0 is a valid answer: small experts run on
  * kernels that keep every intermediate on the CU).  `mode` is an egs_scatter_mode and only matters for ops
- * that scatter.  The answer holds for dense operands that start on a 16-byte boundary (what hipMalloc and
+ * that scatter.  Where a scatter could run as one kernel without a workspace (reduction 32, 64 or, in 16 bits, 128, output columns a
+ * multiple of 32, at most 4096 picks per batch element) but is expected to be faster as fp32 product rows, DETERMINISTIC answers
+ * with the rows' bytes (about B*E*K*I*4); a workspace that is smaller, missing or not 256-byte aligned then selects the one kernel, which
+ * has the same tolerances and its own fixed order of additions: memory that varies from call to call can vary the last bits.  COMPACT
+ * takes the one kernel there in any case and answers 0.  The two answers that contain a scatter are decided each for itself:
+ * EGS_OP_GATHER_BACKWARD may take another kernel for dX than EGS_OP_GEMM_SCATTER for the same product.
+ * The answer holds for dense operands that start on a 16-byte boundary (what hipMalloc and
  * torch return); every entry point derives the requirement again from the operands it is given, and an
  * operand off that grid can select a general kernel that needs more: the call then returns
  * EGS_ERR_WORKSPACE and launches nothing; copy such operands to aligned storage first. */
@@ -188,7 +196,8 @@ int egs_gather_gemm_fp8act(const void *X, const void *Wq, const float *w_scale, 
  * atomics, egs/triton_kernels.py:247).  The one-kernel scatter of small experts sorts the picks of a batch element by
  * token before it can add product rows in a fixed order; Ind decides that order alone, so it can be computed once per
  * Ind and reused by every scatter over the same Ind: the scatter forward, and the scatter inside the gather's backward.
- *   - egs_routing_table_bytes(): size of the table for these sizes, 0 if no kernel would read one (then pass no table).
+ *   - egs_routing_table_bytes(): size of the table for these sizes, 0 if it is not worth having one (then pass none): no
+ *     kernel would read it, or fp32 sizes of many experts with few picks, whose scatters are faster as product rows.
  *   - egs_expert_gather_forward_table(): egs_expert_gather_forward, and fills `table` from Ind in the same launch
  *     (a launch of its own when the operands do not select the small-expert gather).
  *   - egs_expert_scatter_forward_table(), egs_expert_gather_backward_table(): the plain entry points with a table that
@@ -196,9 +205,10 @@ int egs_gather_gemm_fp8act(const void *X, const void *Wq, const float *w_scale, 
  *     The table is only read.  A table built from other indices gives wrong sums without any error: the caller owns
  *     that invariant.  (Its entries are clamped to the ranges a table of these sizes can hold, so even memory that was
  *     never filled cannot make a kernel run on or touch anything but its own rows.)
- * `table` NULL makes each of these the plain entry point.  A table argument for sizes that have no use for one returns
+ * `table` NULL makes each of these the plain entry point.  A table argument for sizes that no kernel would read one for returns
  * EGS_ERR_UNSUPPORTED; `table` must be 256-byte aligned (EGS_ERR_ALIGNMENT) and at least egs_routing_table_bytes() long
- * (EGS_ERR_WORKSPACE).
+ * (EGS_ERR_WORKSPACE).  The fp32 sizes that answer 0 although a kernel could read one (see above) take a table all the same: it is
+ * filled, and must hold B*(T+1)*4 and B*E*K*4 bytes, each rounded up to 256.
  * ------------------------------------------------------------------------------------- */
 size_t egs_routing_table_bytes(const egs_dims *d, int dtype);
 
@@ -303,7 +313,10 @@ int egs_expert_scatter_backward(const void *Y, const void *W, const void *Ind, c
 
 /* scores[b,e,:] = the K largest of softmax over experts of logits[b,:,e], descending, Ind[b,e,:] their tokens.
  * logits [B,T,E] dense in fp32 / fp16 / bf16, scores fp32.  EGS_ERR_UNSUPPORTED where a column does not fit a
- * compute unit's LDS (T above about 9000) or K > 512.  Many logits per batch element need a workspace: its size, or 0. */
+ * compute unit's LDS (T above about 9000) or K > 512.  The workspace (8-byte aligned, B*T*8 bytes) holds the rows' maxima and sums, from a launch
+ * ahead of the router's; egs_expert_choice_router_workspace_bytes() is its size where it is needed or the faster way, else 0.  Up to 64
+ * experts, 96 * 1024 logits per batch element and 16 Mi of B*T*E*ceil(E/8) in all it is optional: a missing or smaller one means one launch, with the same
+ * bits.  Beyond, EGS_ERR_NULL_POINTER or EGS_ERR_WORKSPACE. */
 size_t egs_expert_choice_router_workspace_bytes(int32_t B, int32_t T, int32_t E);
 int egs_expert_choice_router(const void *logits, void *Ind, float *scores, void *workspace, size_t workspace_bytes, int32_t B,
                              int32_t T, int32_t E, int32_t K, int logits_dtype, int ind_dtype, void *stream);

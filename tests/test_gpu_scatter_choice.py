@@ -28,31 +28,37 @@ def case_of(shape, dtype):
 
 
 @pytest.mark.parametrize("dtype", list(DTYPES))
-@pytest.mark.parametrize("shape", [
-    (2, 454, 83, 5, 160, 64),       # few picks per expert: rows
-    (9, 454, 28, 5, 96, 64),        # few batch elements, many tokens: rows
-    (40, 64, 8, 32, 64, 64),        # full units: one kernel
-    (3, 33, 31, 33, 96, 64),        # 1023 picks, the second unit of one pick
-    (4, 40, 52, 40, 96, 64),        # 2080 picks: passes or rows
-    (39, 43, 49, 25, 96, 32),       # passes, short rows and few tokens
-    (12, 65, 110, 8, 64, 32),       # fp32: units of eight picks that a routing table does not make up for
-], ids=lambda s: "x".join(map(str, s)))
-def test_with_and_without_a_workspace(shape, dtype):
+@pytest.mark.parametrize("shape, by_rows", [
+    ((2, 454, 83, 5, 160, 64), ("bf16", "f16", "f32")),     # few picks per expert
+    ((9, 454, 28, 5, 96, 64), ("f32",)),                    # few batch elements, many tokens: fp32 alone
+    ((40, 64, 8, 32, 64, 64), ()),                          # full units
+    ((3, 33, 31, 33, 96, 64), ("f32",)),                    # 1023 picks, the second unit of one pick
+    ((4, 40, 52, 40, 96, 64), ("bf16", "f16", "f32")),      # 2080 picks: passes lose
+    ((39, 43, 49, 25, 96, 32), ()),                         # and win: short rows and few tokens
+    ((12, 65, 110, 8, 64, 32), ("f32",)),                   # units of eight picks that a routing table does not make up for in fp32
+], ids=lambda s: "x".join(map(str, s)) if s and isinstance(s[0], int) else None)
+def test_with_and_without_a_workspace(shape, by_rows, dtype):
     B, T, E, K, I, J = shape
     case, Ind, safe, Y = case_of(shape, DTYPES[dtype])
     L, d, code = _abi.lib(), _abi.Dims(*shape), hk.dtype_to_type_id(DTYPES[dtype])
     Yd, Ws, Indd = dev(case["Y"]), dev(case["Ws"]), dev(Ind)
     want = O.scatter_forward(Y, np64(case["Ws"]), safe, T)
     planned = L.egs_workspace_bytes(1, 0, d, code)
-    for size in sorted({planned, 0}):
-        ws = torch.empty(max(size, 256), dtype=torch.uint8, device="cuda")
+    assert (planned > 0) == (dtype in by_rows), planned
+    assert L.egs_workspace_bytes(1, _abi.SCATTER_COMPACT, d, code) == 0
+    ws = torch.empty(2 * planned + 512, dtype=torch.uint8, device="cuda")
+    # (bytes, offset): the rows with what is asked for or more, else the one kernel, which needs none
+    first = {}
+    for size, at in sorted({(planned, 0), (2 * planned, 0), (max(planned - 1, 0), 0), (planned, 8), (0, 0)}):
         out = torch.full((B, T, I), float("nan"), dtype=DTYPES[dtype], device="cuda")
         with _abi.launch_log() as log:
-            rc = L.egs_gemm_scatter(Yd.data_ptr(), Ws.data_ptr(), Indd.data_ptr(), out.data_ptr(), ws.data_ptr() if size else None, size, ctypes.byref(d),
-                                    code, _abi.IND_I64, EJI, 0, torch.cuda.current_stream().cuda_stream)
-        assert rc == 0, (rc, size, planned)
-        assert any(k.startswith("scatter_fused") for k in log.kernels) == (size == 0), (size, log.kernels)
+            rc = L.egs_gemm_scatter(Yd.data_ptr(), Ws.data_ptr(), Indd.data_ptr(), out.data_ptr(), ws.data_ptr() + at if size else None, size,
+                                    ctypes.byref(d), code, _abi.IND_I64, EJI, 0, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, (rc, size, at, planned)
+        rows = 0 < planned <= size and at == 0
+        assert any(k.startswith("scatter_fused") for k in log.kernels) != rows, (size, at, log.kernels)
         assert_close(out, want, DTYPES[dtype], "out, %d bytes of workspace" % size)
+        assert torch.equal(out, first.setdefault(rows, out)), (size, at)        # each way has its bits, whatever the memory
     dX, dW = hk.expert_gather_backward_call(dev(case["X"]), dev(case["Wg"]), Indd, Yd, torch.float32)
     wX, wW = O.gather_backward(np64(case["X"]), np64(case["Wg"]), safe, Y)
     assert_close(dX, wX, DTYPES[dtype], "dX")
