@@ -192,14 +192,6 @@ int launch_rows_strip(RowsStripParams &p, hipStream_t s)
     return EGS_OK;
 }
 
-// Mid-sized 16-bit products; `used`: rows_strip_kernel takes this one.  Against tiled_rows_kernel, us, strips / that: R768 N64 Me2048 E32 13.8 /
-// 19.3, R328 N136 Me900 E20 10 / 14, R136 N328 13.3 to 16 / 17, R800 N64 Me1628 E34 17 / 22, R64 N576 Me2814 E14 18 to 19 / 25, R896 N128
-// Me232 E83 13.2 / 16.3, R192 N64 Me92 E65 5.0 / 5.7, R704 N224 Me85 E114 12.0 / 18.4; not with little work, counted in full tiles of 128 x 64
-// (R352 N64 Me252 E18: 35, 6.2 / 5.3, R96 N48 Me576 E13: 44, 5.1 / 4.6, R160 N128 Me468 E8: 58, 5.5 / 4.8), nor up to 64 rows, which are one
-// tile of that too (773 sizes 0.89 to 1.24 of its time, level on average: R80 N1920 Me40 E248 57 / 52 with the sums, R464 N1792 Me24 E194 99 / 86;
-// 65 to 128 rows, two of them, 0.86), nor with columns mostly empty (R896 N32 Me119 E53 9.6 / 7.9, R288 N32 Me2080 E35 10.2 / 9.8) unless there are
-// many and long ones (1972 strips, R800 N32 Me2146 E116 42 / 47; but R160 N32 Me1920 E103 35.7 / 32.3).  Of 4992 such products, 1686 of them
-// taken, 21 are more than 3 % slower.
 // the parameters of either kind of weights; false: operands that the kernel can't take
 bool make_rows_strip(const RowsGemmParams &p, int act_dtype, int wes, bool gather, int epi, RowsStripParams &q)
 {
@@ -215,6 +207,15 @@ bool make_rows_strip(const RowsGemmParams &p, int act_dtype, int wes, bool gathe
     return true;
 }
 
+// Mid-sized 16-bit products; `used`: rows_strip_kernel takes this one.  Against tiled_rows_kernel, us, strips / that: R768 N64 Me2048 E32 16.4 /
+// 20.7, R328 N136 Me900 E20 10.3 / 13.9, R136 N328 12.5 / 13.8, R800 N64 Me1628 E34 18 / 22, R896 N128 Me232 E83 14.3 / 17.5, R704 N224
+// Me85 E114 12.9 / 18.4; not with little work, counted in full tiles of 128 x 64
+// (R352 N64 Me252 E18: 35, 6.2 / 5.3, R96 N48 Me576 E13: 44, 5.1 / 4.6, R160 N128 Me468 E8: 58, 5.5 / 4.8), nor up to 64 rows, which are one
+// tile of that too (773 sizes 0.89 to 1.24 of its time, level on average: R80 N1920 Me40 E248 57 / 52 with the sums, R464 N1792 Me24 E194 99 / 86;
+// 65 to 128 rows, two of them, 0.86), nor with columns mostly empty (R896 N32 Me119 E53 9.6 / 7.9, R288 N32 Me2080 E35 10.2 / 9.8) unless there are
+// many and long ones (1972 strips, R800 N32 Me2146 E116 42 / 47; but R160 N32 Me1920 E103 35.7 / 32.3).  Of 4992 such products, 1686 of them
+// taken, 21 were more than 3 % slower; since that kernel has reductions of up to four slabs written out, 105 of 895 taken ones of those are, on average
+// still 0.98 of its time (R64 N576 Me2814 E14 20.8 / 20.5; with half a strip of columns empty R72 N96 Me9699 E61 60 / 47, R48 N96 Me1560 E116 21.6 / 17.6).
 int rows_strip(RowsGemmParams &p, int act_dtype, bool w_trans, bool gather, int epi, bool &used, hipStream_t s)
 {
     used = false;

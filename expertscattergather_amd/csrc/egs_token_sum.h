@@ -4,11 +4,11 @@
 //   out[b,t,:] = sum of P[b,q,:] over the picks q of batch element b with Ind[b,q] = t, in increasing q
 //
 // With the table built by a launch of its own (csr_count_kernel, 5 .. 15 us for a few hundred picks: one workgroup per batch
-// element, a chain of phases) the table took as long as the sums.  Up to kTokenSumPicks picks per batch element it is cheaper
+// element, a chain of phases) the table took as long as the sums.  Up to kTokenSumPicks picks per batch element (kTokenSumPicksFew for few tokens) it is cheaper
 // that each workgroup reads all of the batch element's indices - a few KB out of the L2, all in flight at once - keeps those
-// of its tokens, and sorts what is left, of which there is little.  The order of the additions is the order of the picks
-// (tokens with more than kTokenSumHot of them: in contiguous shares, added in order), a function of Ind alone:
-// bitwise reproducible.
+// of its tokens, and sorts what is left, of which there is little.  The order of the additions is the order of the picks; where groups
+// of threads share a token's picks (split_log2: few tokens to a workgroup), or all of them those of a token with more than kTokenSumHot each, in
+// contiguous shares that are added in order: a function of Ind and the sizes alone, bitwise reproducible.
 #pragma once
 #include "egs_device.h"
 
@@ -18,7 +18,7 @@ constexpr int kTokenSumPicks = 4096;        // most picks per batch element
 constexpr int kTokenSumPicksFew = 8192;     // where there are few tokens, of short rows (token_sums_take)
 constexpr int kTokenSumTokens = 32;         // most tokens per workgroup
 constexpr int kTokenSumMany = 128;          // where they have few picks
-constexpr int kTokenSumHot = 64;            // longer segments are shared by the whole workgroup
+constexpr int kTokenSumHot = 64;            // picks of a group's token; longer segments are shared by the whole workgroup
 constexpr int kTokenSumOne = 32;            // a wavefront's only token: longer segments go sixteen rows at a time
 
 struct TokenSumParams {
