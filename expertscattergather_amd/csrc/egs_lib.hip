@@ -792,8 +792,12 @@ size_t dw_bytes_planned(const egs_dims *d, int act_dtype)
 // In passes (more than 1024 picks) it loses to the rows by 1.3 on average (1.85 in fp32) and by 3 with Zipf-distributed picks; the
 // model keeps 184 of 379 scatters there (1.18 of the rows' time; bf16 B78 T43 E49 K25 I96 J32 17.8 / 28.7) and one whose table comes with the
 // gather's launch, and the others take 0.55 of the time they took.
+// Up to kRowsInsteadBytes of workspace, a little more than 380000 random sizes of up to 128 batch elements ask for: a call of thousands of them would
+// want a hundred times its operands and more than a card has (bf16 B1852 T22 E252 K7 I1536 J32: 20 GB of rows for 0.36, B93597 T82 E250 K2 I1952 J32 378 GB).
+constexpr size_t kRowsInsteadBytes = 1ull << 30;
 bool fused_model_pays(const FusedPlan &fp, const egs_dims *d, int act_dtype, double extra_us, double margin = 1.15)
 {
+    if (plan_scatter(d, EGS_SCATTER_DETERMINISTIC, act_dtype, SCATTER_ROWS).bytes > kRowsInsteadBytes) return true;
     const bool f32 = act_dtype == EGS_F32, passes = fp.experts_per_pass != d->E;
     const int run_slices = passes ? 1 : fused_run(fp, d);
     if (!passes && scatter_fused_holds(d->E, d->K, d->J * elem_size(act_dtype), run_slices)) return true;     // 0.70 (fp32: 0.83) of the rows' time

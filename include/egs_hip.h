@@ -114,7 +114,7 @@ const char *egs_last_hip_error(void);
  * kernels that keep every intermediate on the CU).  `mode` is an egs_scatter_mode and only matters for ops
  * that scatter.  Where a scatter could run as one kernel without a workspace (reduction 32, 64 or, in 16 bits, 128, output columns a
  * multiple of 32, at most 4096 picks per batch element) but is expected to be faster as fp32 product rows, DETERMINISTIC answers
- * with the rows' bytes (about B*E*K*I*4); a workspace that is smaller, missing or not 256-byte aligned then selects the one kernel, which
+ * with the rows' bytes (about B*E*K*I*4, at most 1 GiB); a workspace that is smaller, missing or not 256-byte aligned then selects the one kernel, which
  * has the same tolerances and its own fixed order of additions: memory that varies from call to call can vary the last bits.  COMPACT
  * takes the one kernel there in any case and answers 0.  The two answers that contain a scatter are decided each for itself:
  * EGS_OP_GATHER_BACKWARD may take another kernel for dX than EGS_OP_GEMM_SCATTER for the same product.

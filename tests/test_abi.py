@@ -271,3 +271,31 @@ def test_which_scatter_is_planned(lib, dtype, dims, rows):
     assert (need >= B * E * K * I * 4) if rows else need == 0, need
     both = lib.egs_workspace_bytes(_abi.OP_GATHER_BACKWARD, 0, d, dtype)
     assert both == need + lib.egs_workspace_bytes(_abi.OP_DW, 0, d, dtype)
+
+
+@pytest.mark.parametrize("dtype, dims", [(_abi.BF16, (1852, 22, 252, 7, 1536, 32)), (_abi.F16, (145570, 37, 117, 3, 1440, 32)), (_abi.F32, (21682, 54, 132, 10, 1568, 32)),
+                                         (_abi.BF16, (93597, 82, 250, 2, 1952, 32))], ids=str)
+def test_large_batches_of_the_one_kernel_scatter_need_no_workspace(lib, dtype, dims):
+    """Product rows would be ten to fifty times the operands here, hundreds of GB: whatever their time, the kernel that needs none stays."""
+    d = _abi.Dims(*dims)
+    assert lib.egs_workspace_bytes(_abi.OP_GEMM_SCATTER, 0, d, dtype) == 0
+    assert lib.egs_workspace_bytes(_abi.OP_GATHER_BACKWARD, 0, d, dtype) == lib.egs_workspace_bytes(_abi.OP_DW, 0, d, dtype)
+
+
+def test_the_scatters_choice_asks_for_little(lib):
+    """Where one kernel could do without (the compact mode answers 0, with few enough picks that it always did), the rows are 1 GiB at most."""
+    import random
+    rng = random.Random(3)
+    asked = 0
+    for _ in range(20000):
+        B, T, E, K = (round(2 ** rng.uniform(0, most)) for most in (17, 11, 8, 7))
+        I, J, dtype = 32 * round(2 ** rng.uniform(0, 6)), rng.choice([32, 64]), rng.choice([_abi.F32, _abi.F16, _abi.BF16])
+        if E * K > 1024 or T > 1024 or B * E * K * J > 2 ** 29 or B * T * I > 2 ** 33:
+            continue
+        d = _abi.Dims(B, T, E, K, I, J)
+        if lib.egs_workspace_bytes(_abi.OP_GEMM_SCATTER, _abi.SCATTER_COMPACT, d, dtype) > 0:
+            continue                                        # few workgroups: no such kernel
+        need = lib.egs_workspace_bytes(_abi.OP_GEMM_SCATTER, 0, d, dtype)
+        asked += need > 0
+        assert need <= 1 << 30, (B, T, E, K, I, J, dtype, need)
+    assert asked > 500
